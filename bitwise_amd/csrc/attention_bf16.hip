@@ -707,6 +707,279 @@ __global__ __launch_bounds__(64 * FoldShape<HD>::NW) __attribute__((amdgpu_waves
   }
 }
 
+// Route 1 for heads of 64 and 128 in pages of 16 to 64 tokens.  What bounds the kernel above: eight waves in step, two a
+// SIMD, each through its reads of LDS, its matrix instructions, its exponentials and its stores of the next partition in
+// turn, so that the SIMDs issue in a third of the clocks; and half the vector instructions are addresses and copies.
+// (A SIMD's time is nearly the sum of its waves' vector instructions, 4 clocks each, 8 an exponential, and some 10 clocks
+// of every matrix instruction, which holds the registers' ports: about 1,050 clocks a tile of 128 elements and partition.)
+// Here keys travel from their page straight into LDS (no registers, no LDS write instructions) and everything a wave
+// asks for has a scalar page address and an offset that never changes, which leaves registers for four waves a SIMD: two
+// workgroups share a compute unit and drift apart.  The statements per tile are those above: the same bits.
+// 2,048 queries over 8,192 keys, 32 heads of 128 on 8: 545 us -> 349 (0.69 PFLOP/s); 2,048 tokens, 32 heads of 64: 63 -> 43.
+//
+// LDS: two buffers of a partition's keys [64][HD] and values [HD][64 keys], rows without padding; the 16-byte chunks of a
+// row are permuted by the row (fold2_k_slot; the values as fold_v_offset says), so that 16 lanes which read one chunk of
+// 16 rows hit 16 groups of banks.  A load instruction with LDS as its destination fills 1 KB of it, lane l's 16 bytes at
+// 16 l: which chunk a lane asks for is permuted instead.  Values take the way through registers (16 bytes a lane: eight
+// keys of one d): the second product's operand wants four keys of a page beside four of the next, and two 8-byte reads
+// an operand with the moves that bring them together cost more than the two 8-byte writes.
+template <int HD>
+struct Fold2Shape {
+  static constexpr int NW = 8;                                     // waves, a tile each
+  static constexpr int KROW = HD * 2, VROW = ATT_PART * 2;        // bytes from key to key, from d to d
+  static constexpr int KBYTES = ATT_PART * KROW, BYTES = KBYTES + HD * VROW;
+  static constexpr int CPR = HD / 8;                              // 16-byte chunks of a key
+  static constexpr int LOADS = HD / 8 / NW;                       // a wave's load instructions a partition: of keys, and as many of values
+  static constexpr int WAVES = 4;                                  // waves per SIMD the register budget is set for
+};
+
+template <int HD>
+__device__ __forceinline__ int fold2_k_slot(int chunk, int key) {
+  return HD == 128 ? chunk ^ (key & 15) : chunk ^ ((key >> 1) & 7);
+}
+
+// A lane's shares of a partition's loads, the same for every partition.
+template <int HD>
+struct Fold2Plan {
+  uint32_t k_off[Fold2Shape<HD>::LOADS], v_off[Fold2Shape<HD>::LOADS];   // byte offsets within a page
+  int v_lds[Fold2Shape<HD>::LOADS];                               // where the first four of the chunk's keys go in the buffer (the others: one chunk over)
+  int v_page_key[Fold2Shape<HD>::LOADS];                          // a key of the chunk's page (scalar)
+};
+
+template <int HD>
+__device__ __forceinline__ void fold2_plan(const AttnBf16Args& a, int kvh, int wave, int lane, Fold2Plan<HD>& p) {
+  using S = Fold2Shape<HD>;
+  const int per_page = HD << (a.page_shift - 3), row_shift = a.page_shift - 3;   // 16-byte chunks of a page's values (of one head), of a row (log2)
+#pragma unroll
+  for (int t = 0; t < S::LOADS; ++t) {
+    const int key = (ATT_PART / S::NW) * wave + t * (64 / S::CPR) + lane / S::CPR;
+    const int chunk = fold2_k_slot<HD>(lane % S::CPR, key);       // (the permutation is its own inverse)
+    p.k_off[t] = (uint32_t)((kvh * a.page_size + (key & (a.page_size - 1))) * HD + 8 * chunk) * 2u;
+    const int c0 = 64 * wave + 64 * S::NW * t, c = c0 + lane;            // (a page's chunks are a multiple of 64: one page a load instruction)
+    const int pi = c0 / per_page, in = c - pi * per_page;
+    const int d = in >> row_shift, slot = 8 * (in & ((1 << row_shift) - 1));
+    p.v_page_key[t] = pi << a.page_shift;
+    p.v_off[t] = (uint32_t)((kvh * HD + d) * a.page_size + slot) * 2u;
+    p.v_lds[t] = S::KBYTES + d * S::VROW + fold_v_offset((p.v_page_key[t] + slot) >> 2, d);
+  }
+}
+
+// The pages of 64 consecutive entries of the sequence's table, an entry a lane (clamped into the table's row and into the
+// pool, so this may be asked for entries past the last one): sixteen partitions' pages of 16 tokens by one load.  A
+// partition's entries never straddle two such blocks.  (Scalar loads a partition instead would make every wait for an
+// LDS operand wait for them too: they come back in no order.)
+__device__ __forceinline__ int fold2_pages(const AttnBf16Args& a, const int32_t* table, int block, int lane) {
+  const int i = 64 * block + lane;
+  return (int)min((unsigned)table[i < a.table_stride ? i : a.table_stride - 1], (unsigned)(a.num_pages - 1));
+}
+
+template <int HD>
+__device__ __forceinline__ void fold2_load(const AttnBf16Args& a, const Fold2Plan<HD>& p, int pages, int part, int wave,
+                                           unsigned char* buf, u32x4 (&v)[Fold2Shape<HD>::LOADS]) {
+  using S = Fold2Shape<HD>;
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  typedef const __attribute__((address_space(1))) void* glb_ptr;
+  const unsigned page_bytes = (unsigned)(a.kv_heads * a.page_size * HD) * 2u;
+  const int key0 = part * ATT_PART;
+  auto page = [&](int key) { return (unsigned long long)(unsigned)__builtin_amdgcn_readlane(pages, ((key0 + key) >> a.page_shift) & 63) * page_bytes; };
+  const unsigned char* k = reinterpret_cast<const unsigned char*>(a.k_cache) + page((ATT_PART / S::NW) * wave);
+#pragma unroll
+  for (int t = 0; t < S::LOADS; ++t)
+    __builtin_amdgcn_global_load_lds((glb_ptr)(k + p.k_off[t]), (lds_ptr)(buf + (wave * S::LOADS + t) * 1024), 16, 0, 0);
+#pragma unroll
+  for (int t = 0; t < S::LOADS; ++t)
+    v[t] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const unsigned char*>(a.v_cache) + page(p.v_page_key[t]) + p.v_off[t]);
+}
+
+// A partition's values from registers to LDS; where the partition is not wholly live the dead keys' values are zeroed
+// (0 times what a dead slot holds could be NaN).
+template <int HD>
+__device__ __forceinline__ void fold2_store(const AttnBf16Args& a, const Fold2Plan<HD>& p, int lane, int key0, int kmin, int kmax,
+                                            unsigned char* buf, u32x4 (&v)[Fold2Shape<HD>::LOADS]) {
+  using S = Fold2Shape<HD>;
+  if (!(key0 >= kmin && key0 + ATT_PART - 1 <= kmax)) {
+    const int slot = 8 * (lane & ((a.page_size >> 3) - 1));       // (a row's chunks divide 64)
+#pragma unroll 1
+    for (int t = 0; t < S::LOADS; ++t) {
+      uint32_t m0, m1, m2, m3;
+      int page_key = p.v_page_key[0];
+      if constexpr (S::LOADS >= 2) page_key = t == 1 ? p.v_page_key[1] : page_key;
+      if constexpr (S::LOADS >= 4) page_key = t == 2 ? p.v_page_key[2] : (t == 3 ? p.v_page_key[3] : page_key);
+      stale_masks(key0 + page_key + slot, kmin, kmax, m0, m1);
+      stale_masks(key0 + page_key + slot + 4, kmin, kmax, m2, m3);
+#pragma unroll
+      for (int i = 0; i < S::LOADS; ++i)
+        if (t == i) v[i] &= (u32x4){m0, m1, m2, m3};
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < S::LOADS; ++t) {
+    // (slots 2c and 2c + 1 of fold_v_offset lie a chunk apart: its lowest bit)
+    *reinterpret_cast<u32x2*>(buf + p.v_lds[t]) = (u32x2){v[t][0], v[t][1]};
+    *reinterpret_cast<u32x2*>(buf + (p.v_lds[t] ^ 16)) = (u32x2){v[t][2], v[t][3]};
+  }
+}
+
+// Scores of a tile whose queries all see every key of the partition -> probabilities and maximum: the statements of
+// softmax_partition without its masks.
+__device__ __forceinline__ void softmax_whole(float scale_log2, const f32x4 (&st)[4], float& m_p, u32x4 (&pf)[2]) {
+  float mx = __builtin_elementwise_maximum(st[0][0], st[0][1]);
+  mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mx, st[0][2]), st[0][3]);
+#pragma unroll
+  for (int u = 1; u < 4; ++u) {
+    mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mx, st[u][0]), st[u][1]);
+    mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mx, st[u][2]), st[u][3]);
+  }
+  mx = max_over_lane_groups(mx);
+  mx = mx * scale_log2;
+#pragma unroll
+  for (int w = 0; w < 2; ++w)
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const int u = 2 * w + (e >> 2), i = e & 3;
+      pf[w][e >> 1] = pack_bf16x2(__builtin_amdgcn_exp2f(fmaf(st[u][i], scale_log2, -mx)),
+                                  __builtin_amdgcn_exp2f(fmaf(st[u][i + 1], scale_log2, -mx)));
+    }
+  m_p = mx;
+}
+
+template <int HD, bool CAPPED>
+__global__ __launch_bounds__((64 * Fold2Shape<HD>::NW)) __attribute__((amdgpu_waves_per_eu(Fold2Shape<HD>::WAVES, Fold2Shape<HD>::WAVES))) void attention_fold2_kernel(
+    AttnBf16Args a, int groups, int items) {
+  using S = Fold2Shape<HD>;
+  constexpr int NT = HD / 16, KS = HD / 32, NW = S::NW;
+  extern __shared__ __align__(16) unsigned char lds[];
+  __shared__ int ranges[2 * NW];
+  const int wave = wave_index();
+  const int rank = fold_work_rank((int)blockIdx.x, (int)gridDim.x);
+  const int first_tile = (groups - 1 - rank / items) * S::NW;
+  GroupCtx gc;
+  TileCtx<HD> tcs[1];
+  const TileCtx<HD>& tc = tcs[0];
+  const bool live = group_setup<HD, 1>(a, first_tile + wave, rank % items, gc, tcs);
+  if (gc.lane == 0) {
+    ranges[2 * wave] = live ? gc.kmin : 0x7fffffff;
+    ranges[2 * wave + 1] = live ? gc.kmax : -1;
+  }
+  __syncthreads();
+  int kmin = 0x7fffffff, kmax = -1;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    kmin = min(kmin, ranges[2 * w]);
+    kmax = max(kmax, ranges[2 * w + 1]);
+  }
+  kmin = __builtin_amdgcn_readfirstlane(kmin);
+  kmax = __builtin_amdgcn_readfirstlane(kmax);
+  if (kmax < 0) return;                          // the same for every thread of the workgroup
+  const int32_t* table = a.block_table + (size_t)(a.tiles != nullptr ? a.tiles[first_tile * 4 + 2] : first_tile) * a.table_stride;
+  const int my_first = live ? gc.kmin / ATT_PART : 1, my_last = live ? gc.kmax / ATT_PART : 0;
+  float m = -INFINITY, l = 0.0f;
+  f32x4 o[NT];
+#pragma unroll
+  for (int dt = 0; dt < NT; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const int first = kmin / ATT_PART, last = kmax / ATT_PART;
+  Fold2Plan<HD> plan;
+  fold2_plan<HD>(a, gc.kvh, wave, gc.lane, plan);
+  // partitions whose pages one block of table entries holds (log2)
+  const int block_shift = a.page_shift;
+  int pages = fold2_pages(a, table, first >> block_shift, gc.lane);
+  u32x4 vals[S::LOADS];
+  fold2_load<HD>(a, plan, pages, first, wave, lds, vals);
+  int pages_next = fold2_pages(a, table, (first >> block_shift) + 1, gc.lane);
+  fold2_store<HD>(a, plan, gc.lane, first * ATT_PART, kmin, kmax, lds, vals);
+  // operand addresses within a buffer: key row r, chunk 4 ks + g; value row r, keys 32 w + 4 g .. and 32 w + 16 + 4 g ..
+  int k_at[KS], v_at[2];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) k_at[ks] = gc.r * S::KROW + 16 * fold2_k_slot<HD>(4 * ks + gc.g, gc.r);
+#pragma unroll
+  for (int w = 0; w < 2; ++w) v_at[w] = S::KBYTES + gc.r * S::VROW + fold_v_chunk(4 * w + gc.g, gc.r);
+  int b = 0;
+  for (int part = first; part <= last; ++part) {
+    unsigned char* buf = lds + b * S::BYTES;
+    const int key0 = part * ATT_PART;
+    // this wave's keys of the partition have landed, its values are in LDS, and it has read what it needs of the other
+    // buffer; behind the barrier that holds for every wave, and the other buffer may be filled again
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (part < last) {
+      if (((part + 1) & ((1 << block_shift) - 1)) == 0) {
+        pages = pages_next;
+        pages_next = fold2_pages(a, table, ((part + 1) >> block_shift) + 1, gc.lane);
+      }
+      fold2_load<HD>(a, plan, pages, part + 1, wave, lds + (b ^ 1) * S::BYTES, vals);
+    }
+    const bool mine = part >= my_first && part <= my_last;        // the same for the whole wave
+    float m_p = -INFINITY;
+    u32x4 pf[2], vf[2][2];
+    if (mine) {
+      // scores: the operands of the next 16 keys are read while the matrix instructions of these run
+      f32x4 st[4];
+      u32x4 kf[2][KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kf[0][ks] = *reinterpret_cast<const u32x4*>(buf + k_at[ks]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (u < 3) {
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) kf[(u + 1) & 1][ks] = *reinterpret_cast<const u32x4*>(buf + (u + 1) * 16 * S::KROW + k_at[ks]);
+        } else {
+#pragma unroll
+          for (int w = 0; w < 2; ++w) vf[0][w] = *reinterpret_cast<const u32x4*>(buf + v_at[w]);
+        }
+        st[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          st[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[u & 1][ks]), as_bf16x8(tc.qf[ks]), st[u], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x100, KS, 0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          if (u < 3 || ks < 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+      if (!CAPPED && key0 >= tc.all_lo && key0 + ATT_PART - 1 <= tc.all_hi) softmax_whole(a.scale_log2, st, m_p, pf);
+      else softmax_partition<HD>(a, gc, tc, key0, st, m_p, pf);
+    }
+    // the next partition's values, asked for a softmax ago, go to LDS while the second product runs
+    if (part < last) fold2_store<HD>(a, plan, gc.lane, key0 + ATT_PART, kmin, kmax, lds + (b ^ 1) * S::BYTES, vals);
+    if (mine) {
+      const float l_p = probability_sum(pf);
+      float mn, fa, fb;
+      fold_scalars(m, m_p, mn, fa, fb);
+      m = mn;
+      asm("s_nop 0" : "+v"(fa));                   // the wait state between the exponential unit and the assembly below
+#pragma unroll
+      for (int dt = 0; dt < NT; ++dt) {
+        if (dt + 1 < NT) {
+#pragma unroll
+          for (int w = 0; w < 2; ++w) vf[(dt + 1) & 1][w] = *reinterpret_cast<const u32x4*>(buf + 16 * (dt + 1) * S::VROW + v_at[w]);
+        }
+        f32x4 o_p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 2; ++w) o_p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf[dt & 1][w]), as_bf16x8(pf[w]), o_p, 0, 0, 0);
+        // (three-address form by hand, as in fold())
+        const f32x4 x = {o_p[0] * fb, o_p[1] * fb, o_p[2] * fb, o_p[3] * fb};
+        asm("v_fma_f32 %0, %0, %4, %5\n\tv_fma_f32 %1, %1, %4, %6\n\tv_fma_f32 %2, %2, %4, %7\n\tv_fma_f32 %3, %3, %4, %8"
+            : "+v"(o[dt][0]), "+v"(o[dt][1]), "+v"(o[dt][2]), "+v"(o[dt][3])
+            : "v"(fa), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
+      }
+      l = fmaf(l, fa, l_p * fb);
+    }
+    b ^= 1;
+  }
+  if (!live || tc.pos_c < 0) return;
+  const float inv = 1.0f / (l + sink_term(a, tc.head_c, m));
+  bf16_t* dst = a.out + (size_t)tc.row_c * a.out_stride + (size_t)tc.head_c * HD;
+#pragma unroll
+  for (int dt = 0; dt < NT; ++dt) {
+    u32x2 pk = {pack_bf16x2(o[dt][0] * inv, o[dt][1] * inv), pack_bf16x2(o[dt][2] * inv, o[dt][3] * inv)};
+    *reinterpret_cast<u32x2*>(dst + 16 * dt + 4 * gc.g) = pk;
+  }
+}
+
 // Route 2, for tiles of one token (decoded tokens): the workgroup's W waves deal the
 // partitions among themselves (wave w takes partitions w, w+W, ..., prefetching the next one's
 // keys), park every partition's partial in LDS, and after one barrier the threads fold the
@@ -1058,6 +1331,24 @@ static void decode_split_shape(int num_tiles, int items, int table_stride, int p
 }
 
 template <int HD>
+static int launch_fold2(const AttnBf16Args& a, int groups, int items, hipStream_t s) {
+  using S = Fold2Shape<HD>;
+  static_assert(S::NW == FOLD_NW(HD) * FOLD_QT(HD), "one padding of the tile lists for both kernels");
+  static bool allowed[2] = {false, false};         // more than 64 KB of dynamic LDS has to be asked for once
+  const bool capped = a.cap_over_scale > 0.0f;
+  const void* fn = capped ? (const void*)attention_fold2_kernel<HD, true> : (const void*)attention_fold2_kernel<HD, false>;
+  if (2 * S::BYTES > 48 * 1024 && !allowed[capped]) {
+    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * S::BYTES) != hipSuccess) return -8;
+    allowed[capped] = true;
+  }
+  if (capped)
+    hipLaunchKernelGGL((attention_fold2_kernel<HD, true>), dim3(groups * items), dim3(64 * S::NW), 2 * S::BYTES, s, a, groups, items);
+  else
+    hipLaunchKernelGGL((attention_fold2_kernel<HD, false>), dim3(groups * items), dim3(64 * S::NW), 2 * S::BYTES, s, a, groups, items);
+  return 0;
+}
+
+template <int HD>
 static int launch_attention(const AttnBf16Args& a, int decode, float* scratch, size_t scratch_floats, int* counters,
                             int num_counters, hipStream_t s) {
   const int items = a.kv_heads * a.nsub;
@@ -1113,6 +1404,10 @@ static int launch_attention(const AttnBf16Args& a, int decode, float* scratch, s
       allowed = true;
     }
     const int groups = (a.num_tiles + S::GROUP - 1) / S::GROUP;
+    // Heads of 64 and 128 have a kernel of their own, faster at every length (the comment at attention_fold2_kernel); it wants
+    // pages of at least 16 tokens (a wave's loads within one) and the other kernel takes what is left.
+    if constexpr (HD == 64 || HD == 128)
+      if (a.page_size >= 16) return launch_fold2<HD>(a, groups, items, s);
     hipLaunchKernelGGL((attention_fold_kernel<HD>), dim3(groups * items), dim3(64 * S::NW), lds_bytes, s, a, groups, items);
   }
   return 0;

@@ -716,6 +716,38 @@ def test_attention_prompt_tiles_equal_single_rows(gpu, bf16):
     assert (portion.cpu().double() - ref).abs().max() <= (1.5e-2 if bf16 else 3e-6) * ref.abs().max()
 
 
+@pytest.mark.parametrize("heads,kvh,hd,page", [(2, 2, 64, 16), (6, 2, 64, 64), (4, 1, 128, 16), (3, 1, 128, 32), (17, 1, 128, 64), (2, 2, 64, 8)])
+def test_prompt_attention_of_common_heads_equals_the_decode_kernel(gpu, heads, kvh, hd, page):
+    """Portions around the edges of tiles, of a workgroup's eight tiles, of partitions and of the blocks of table entries
+    (the longest sequence has more than 64 pages of 16), with dead slots full of NaN, windows, chunks, a soft cap and a sink:
+    the bits of the kernel for decoded tokens; and the plain formula within bfloat16's rounding of weights and output."""
+    n_keys = 1100 if page == 16 else 300
+    k, v, kc, vc, tab = paged_setup(gpu, True, heads, kvh, hd, page, 74 if page == 16 else 41, n_keys, seed=heads + hd, poison=True)
+    g = torch.Generator().manual_seed(page)
+    sink = torch.randn(heads, generator=g).to(gpu)
+    group = ops.fold_group_tiles(hd)
+    tpt = 16 // min(heads // kvh, 16)
+    portions = [(0, 1), (0, 64), (3, 62), (60, 9), (n_keys - 133, 133), (130, 8 * tpt + 1)] + ([(960, 140)] if page == 16 else [])
+    for first, rows in portions:
+        positions = list(range(first, first + rows))
+        q = torch.randn(rows, heads * hd, generator=g).to(torch.bfloat16)
+        tiles = [(off, min(tpt, rows - off), 0, 0) for off in range(0, rows, tpt)]
+        tiles += [(0, 0, 0, 0)] * (-len(tiles) % group)
+        for window, extra in ((0, {}), (70, {}), (0, {"chunk": 48}), (0, {"softcap": 5.0}), (0, {"sink": sink})):
+            outs = []
+            for decode, ts in ((False, tiles), (True, [(r, 1, 0, 0) for r in range(rows)])):
+                out = torch.zeros(rows, heads * hd, device=gpu, dtype=torch.bfloat16)
+                ops.attention_bf16(q.to(gpu), torch.tensor(positions, dtype=torch.int32, device=gpu), tab,
+                                   torch.tensor(ts, dtype=torch.int32, device=gpu), len(ts), kc, vc, out, heads, kvh, hd, page,
+                                   window, float(hd) ** -0.5, decode=decode, **extra)
+                outs.append(out)
+            assert torch.equal(outs[0], outs[1]), (first, rows, window, extra)
+            if window == 0 and not extra and rows <= 64:
+                ref = plain_rows(q, k, v, positions, heads)
+                # a weight and the output are rounded to 8 bits each: 2^-9 of a convex sum of values, and of the result
+                assert (outs[0].cpu().double() - ref).abs().max() <= 2.0 ** -7 * v.double().abs().max()
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 def test_attention_finds_a_far_key_and_respects_the_window(gpu, bf16):
     """One key among hundreds is made to stand out by scaling it and the query: the output must
