@@ -1040,10 +1040,189 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_tile_kernel(const float* __
     }
 }
 
+// Tiles of 64 RB x 64 outputs, four waves of 16 RB x 64 (RB 1 or 2), for the same products: v_mfma_f32_16x16x1_4b_f32 is one step
+// of k for four blocks of 16 x 16 outputs; with the A operand of the first block broadcast, 16 rows (lane i < 16 holds row i)
+// against 64 columns.  A 128 x 128 tile keeps a SIMD busy with 64 x 64 outputs, 167 to 188 clocks a step of k whatever the
+// rest of the chip does: 450 rows against 2,048 columns are 64 workgroups above, a quarter of the chip, and 256 here.
+// What bounds it is the matrix instructions' own time (33 clocks and 4 a vector instruction, which does not run under
+// them, not even another wave's): a step of k measured 51 to 58 clocks a tile of 64 x 64, 90 to 104 of 128 x 64.
+// Measured with bfloat16 weights: 450 rows, 2048 x 8192: 571 -> 211 us, 2048 x 2048: 150 -> 55, 6144 x 2048: 163 -> 135.
+template <typename WT, int RB>
+struct F32QShape {
+  static constexpr int BM = 64 * RB, BN = 64, KB = 32, STAGES = 4;
+  static constexpr int XBYTES = BM * KB * 4, WROW = KB * (int)sizeof(WT), WBYTES = BN * WROW, STAGE = XBYTES + WBYTES;
+  static constexpr int X_LOADS = XBYTES / 1024 / 4, W_LOADS = WBYTES / 1024 / 4, LPW = X_LOADS + W_LOADS;   // 1 KB instructions a wave
+  static constexpr int XQ = 4, WQ = WROW / 32;                      // 16-byte reads of a half stage: of a row of x, of a column of W
+};
+
+template <typename WT, int RB>
+__device__ __forceinline__ void f32q_issue(unsigned char* ring, __amdgpu_buffer_rsrc_t rs_x, __amdgpu_buffer_rsrc_t rs_w,
+                                           const int* voff_x, const int* voff_w, int wave, int step, int steps) {
+  using S = F32QShape<WT, RB>;
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  unsigned char* dst = ring + (step % S::STAGES) * S::STAGE;
+  const bool real = step < steps;                                  // scalar
+#pragma unroll
+  for (int t = 0; t < S::X_LOADS; ++t)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (lds_ptr)(dst + (wave * S::X_LOADS + t) * 1024), 16,
+                                             real ? voff_x[t] : 0x7ffffff0, step * S::KB * 4, 0, 0);
+#pragma unroll
+  for (int t = 0; t < S::W_LOADS; ++t)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, (lds_ptr)(dst + S::XBYTES + (wave * S::W_LOADS + t) * 1024), 16,
+                                             real ? voff_w[t] : 0x7ffffff0, step * S::WROW, 0, 0);
+}
+
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+
+// The operands of half a stage (16 steps of k), and the 16 RB matrix instructions on them.
+template <typename WT, int RB>
+struct F32QHalf {
+  f32x4 x[RB][F32QShape<WT, RB>::XQ];
+  u32x4 w[F32QShape<WT, RB>::WQ];
+};
+
+template <typename WT, int RB>
+__device__ __forceinline__ void f32q_read(const unsigned char* stage, int half, int x_off, int x_swz, int w_off, int w_swz, F32QHalf<WT, RB>& h) {
+  using S = F32QShape<WT, RB>;
+#pragma unroll
+  for (int c = 0; c < S::WQ; ++c) h.w[c] = *reinterpret_cast<const u32x4*>(stage + w_off + (((S::WQ * half + c) ^ w_swz) * 16));
+#pragma unroll
+  for (int c = 0; c < S::XQ; ++c)
+#pragma unroll
+    for (int b = 0; b < RB; ++b) h.x[b][c] = *reinterpret_cast<const f32x4*>(stage + x_off + b * 16 * 128 + (((S::XQ * half + c) ^ x_swz) * 16));
+}
+
+template <typename WT, int RB>
+__device__ __forceinline__ void f32q_run(const F32QHalf<WT, RB>& h, f32x16 (&acc)[RB]) {
+  // every weight is widened before the first matrix instruction: between a vector instruction and a matrix instruction
+  // that reads its result there are two idle slots, and a wave's vector instructions do not run under its own matrix ones
+  float wv[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    if constexpr (sizeof(WT) == 2) {                                 // bfloat16 -> 32-bit: the bits, shifted (exact)
+      const uint32_t two = h.w[k >> 3][(k >> 1) & 3];
+      wv[k] = __uint_as_float((k & 1) ? two & 0xffff0000u : two << 16);
+    } else {
+      wv[k] = __uint_as_float(h.w[k >> 2][k & 3]);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int k = 0; k < 16; ++k)                                       // ascending
+#pragma unroll
+    for (int b = 0; b < RB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(h.x[b][k >> 2][k & 3], wv[k], acc[b], 2, 0, 0);
+}
+
+template <typename WT, int RB>
+__global__ __launch_bounds__(256) void gemm_f32_mfma_columns_kernel(const float* __restrict__ x, const WT* __restrict__ w,
+                                                                   float* __restrict__ y, int M, int N, int K, int ldx, int ldy,
+                                                                   int accumulate, int m_tiles) {
+  using S = F32QShape<WT, RB>;
+  constexpr bool BF = sizeof(WT) == 2;
+  extern __shared__ __attribute__((aligned(16))) unsigned char f32q_ring[];
+  const int wave = wave_index(), lane = threadIdx.x & 63;
+  // the row tiles of a column tile run one after the other on one die: its weights come from memory once
+  int bid = blockIdx.x;
+  if (gridDim.x % 8 == 0) bid = (bid % 8) * (gridDim.x / 8) + bid / 8;
+  const int m0 = (bid % m_tiles) * S::BM, n0 = (bid / m_tiles) * S::BN;
+  const int x_rows = min(S::BM, M - m0), w_rows = min(S::BN, N - n0);
+  const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(x + (size_t)m0 * ldx), 0, (int)((((size_t)x_rows - 1) * ldx + K) * sizeof(float)), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs_w =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, (int)((size_t)w_rows * K * sizeof(WT)), 0x00020000);
+  // loads as in the kernel above.  The permutations are for the sixteen lanes that LDS serves together in a 16-byte read
+  // (0-3, 12-15, 20-27 of each half wave, and the others): rows of 128 bytes want the chunk exchanged by row / 2, rows of 64 by row / 4.
+  int voff_x[S::X_LOADS], voff_w[S::W_LOADS];
+#pragma unroll
+  for (int t = 0; t < S::X_LOADS; ++t) {
+    const int row = 8 * (wave * S::X_LOADS + t) + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
+    voff_x[t] = (min(row, x_rows - 1) * ldx + 4 * chunk) * 4;
+  }
+#pragma unroll
+  for (int t = 0; t < S::W_LOADS; ++t) {
+    if constexpr (BF) {
+      const int row = 16 * (wave * S::W_LOADS + t) + (lane >> 2), chunk = (lane & 3) ^ ((row >> 2) & 3);
+      voff_w[t] = (min(row, w_rows - 1) * K + 8 * chunk) * 2;
+    } else {
+      const int row = 8 * (wave * S::W_LOADS + t) + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
+      voff_w[t] = (min(row, w_rows - 1) * K + 4 * chunk) * 4;
+    }
+  }
+  // operand reads: rows 16 RB wave + 16 b + lane % 16 of x (the instruction uses the first sixteen lanes'), column ``lane`` of W
+  const int xr = 16 * RB * wave + (lane & 15), x_off = xr * 128, x_swz = (xr >> 1) & 7;
+  const int w_off = S::XBYTES + lane * S::WROW, w_swz = BF ? (lane >> 2) & 3 : (lane >> 1) & 7;
+  f32x16 acc[RB];
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
+  const int steps = K / S::KB;
+  // Half a stage is read from LDS while the matrix instructions of the half before run; the wait for the next stage
+  // and the barrier stand between a stage's two halves.
+  F32QHalf<WT, RB> h0, h1;
+#pragma unroll
+  for (int st = 0; st < S::STAGES - 1; ++st) f32q_issue<WT, RB>(f32q_ring, rs_x, rs_w, voff_x, voff_w, wave, st, steps);
+  __builtin_amdgcn_s_waitcnt(vmcnt_only(2 * S::LPW));                // this wave's share of stage 0 has landed
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  f32q_read<WT, RB>(f32q_ring, 0, x_off, x_swz, w_off, w_swz, h0);
+  for (int step = 0; step < steps; ++step) {
+    f32q_read<WT, RB>(f32q_ring + (step % S::STAGES) * S::STAGE, 1, x_off, x_swz, w_off, w_swz, h1);
+    __builtin_amdgcn_sched_barrier(0);
+    f32q_run<WT, RB>(h0, acc);
+    __builtin_amdgcn_sched_barrier(0);
+    // this wave's share of the next stage has landed (past K: zeros, unused); behind the barrier everyone's has, and
+    // everyone is done with the stage before this one, whose place the stage asked for next takes
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(S::LPW));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    f32q_issue<WT, RB>(f32q_ring, rs_x, rs_w, voff_x, voff_w, wave, step + S::STAGES - 1, steps);
+    f32q_read<WT, RB>(f32q_ring + ((step + 1) % S::STAGES) * S::STAGE, 0, x_off, x_swz, w_off, w_swz, h0);
+    __builtin_amdgcn_sched_barrier(0);
+    f32q_run<WT, RB>(h1, acc);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __builtin_amdgcn_s_waitcnt(vmcnt_only(0));                         // the padding loads too, before the waves end
+  // block j, register i of it, lane l: row 4 * (l / 16) + i of the 16, column 16 j + l % 16
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = m0 + 16 * RB * wave + 16 * b + 4 * (lane >> 4) + i, n = n0 + 16 * j + (lane & 15);
+        if (m < M && n < N) {
+          float* o = y + (size_t)m * ldy + n;
+          *o = accumulate ? (*o + acc[b][4 * j + i]) : acc[b][4 * j + i];
+        }
+      }
+}
+
+template <typename WT, int RB>
+static void launch_f32_mfma_columns(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s) {
+  using S = F32QShape<WT, RB>;
+  constexpr int lds_bytes = S::STAGES * S::STAGE;
+  static bool allowed = false;                       // more than 64 KB of dynamic LDS has to be asked for once
+  if (lds_bytes > 48 * 1024 && !allowed) {
+    (void)hipFuncSetAttribute((const void*)gemm_f32_mfma_columns_kernel<WT, RB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    allowed = true;
+  }
+  const int m_tiles = (M + S::BM - 1) / S::BM, n_tiles = (N + S::BN - 1) / S::BN;
+  hipLaunchKernelGGL((gemm_f32_mfma_columns_kernel<WT, RB>), dim3(m_tiles * n_tiles), dim3(256), lds_bytes, s, x, w, y, M, N, K, ldx, ldy,
+                     accumulate, m_tiles);
+}
+
 template <typename WT>
 static void launch_f32_mfma_tiles(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate,
                                   hipStream_t s) {
   using S = F32PShape<WT>;
+  // Which tiles: clocks a step of k a round of the compute units, as measured (the comment above), times the rounds.
+  auto cost = [&](int bm, int bn, int clocks) {
+    return (long long)clocks * ((((long long)(M + bm - 1) / bm) * ((N + bn - 1) / bn) + 255) / 256);
+  };
+  const long long big = cost(F32P_BM, F32P_BN, 185), one = cost(64, 64, 55), two = cost(128, 64, 103);
+  if (one < big && one <= two) return launch_f32_mfma_columns<WT, 1>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+  if (two < big) return launch_f32_mfma_columns<WT, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
   constexpr int lds_bytes = F32P_STAGES * S::STAGE;
   static bool allowed = false;                       // more than 64 KB of dynamic LDS has to be asked for once
   if (!allowed) {

@@ -122,6 +122,31 @@ def test_gemm_f32_grid_rows_and_accumulate(gpu):
             assert torch.equal(longer, before), (M, N, K, weight.dtype)
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 64, 32), (65, 1, 64), (127, 65, 96), (128, 640, 160), (129, 130, 2080), (200, 16500, 64),
+                                    (700, 6200, 96), (1030, 2050, 128), (2100, 2048, 64)])
+@pytest.mark.parametrize("wdt", [torch.bfloat16, torch.float32])
+def test_gemm_f32_prompt_tiles_are_the_chains_of_few_rows(gpu, M, N, K, wdt):
+    """Every tile shape of the 32-bit prompt products at the edges of its rows, columns and stages: the bits of the same rows
+    given sixteen at a time (the vector units' chains), written or added, from rows farther apart than they are long."""
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    wide = torch.randn(M, K + 12, generator=g, device=gpu)
+    x, w = wide[:, :K], torch.randn(N, K, generator=g, device=gpu).to(wdt)
+    want = torch.empty(M, N, device=gpu)
+    rows = list(range(0, min(M, 48), 16)) + list(range(max(48, M - 40) // 16 * 16, M, 16))
+    for r in rows:
+        n = min(16, M - r)
+        ops.gemm_f32(x[r:r + n], w, want[r:r + n], n)
+    got = torch.empty(M, N, device=gpu)
+    ops.gemm_f32(x, w, got, M)
+    base = torch.randn(M, N, generator=g, device=gpu)
+    added = base.clone()
+    ops.gemm_f32(x, w, added, M, accumulate=True)
+    for r in rows:
+        n = min(16, M - r)
+        assert torch.equal(got[r:r + n], want[r:r + n])
+        assert torch.equal(added[r:r + n], base[r:r + n] + want[r:r + n])
+
+
 def test_gemm_bf16_rows_shapes_and_epilogues(gpu):
     g = torch.Generator().manual_seed(3)
     for M, N, K in [(1, 16, 32), (5, 100, 64), (16, 64, 96), (17, 500, 96), (50, 300, 608), (130, 96, 224), (33, 72, 40),
