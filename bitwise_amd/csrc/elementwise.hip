@@ -157,26 +157,74 @@ __global__ void rmsnorm_f32_kernel(const float* __restrict__ x, const WT* __rest
 
 // The same chains and tree for rows of up to RMS32_MAX elements, a workgroup a row: its 256 threads bring the row
 // into LDS together, 16 of them run the chains from there (nothing between two steps of a chain but an LDS
-// read), and all write the result.
+// read), and all write the result.  What it costs is latency: the row and the weights are asked for together, 16 bytes a
+// load, and the chains' LDS reads run 32 links ahead (8 rows of 2,048: 7.4 -> 4.7 us inside a decode step).
 #define RMS32_MAX 8192
 template <typename WT>
 __global__ __launch_bounds__(256) void rmsnorm_f32_row_kernel(const float* __restrict__ x, const WT* __restrict__ w,
                                                               float* __restrict__ y, int dim, float eps) {
-  __shared__ float row_lds[RMS32_MAX];
+  __shared__ __attribute__((aligned(16))) float row_lds[RMS32_MAX];
   __shared__ float inv_lds;
   const float* xr = x + (size_t)blockIdx.x * dim;
-  for (int i = threadIdx.x; i < dim; i += 256) row_lds[i] = xr[i];
+  float* yr = y + (size_t)blockIdx.x * dim;
+  // rows of up to 4,096 elements that are whole vectors: a thread keeps its vectors and weights, all asked for at once
+  constexpr int NV = 4;
+  const bool vec = (dim & 3) == 0 && dim <= 1024 * NV && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)w) & 15) == 0;
+  const int nvec = dim >> 2;
+  f32x4 v[NV], wv[NV];
+  if (vec) {
+    u32x4 raw[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int c = min((int)threadIdx.x + 256 * j, nvec - 1);
+      v[j] = reinterpret_cast<const f32x4*>(xr)[c];
+      raw[j] = load_norm_w_raw(w, sizeof(WT) == 2, c);
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int c = (int)threadIdx.x + 256 * j;
+      if (c < nvec) *reinterpret_cast<f32x4*>(row_lds + 4 * c) = v[j];
+      wv[j] = norm_w_floats(raw[j], sizeof(WT) == 2);
+    }
+  } else {
+    for (int i = threadIdx.x; i < dim; i += 256) row_lds[i] = xr[i];
+  }
   __syncthreads();
   if (threadIdx.x < 16) {
     float acc = 0.0f;
-#pragma unroll 8
-    for (int i = threadIdx.x; i < dim; i += 16) acc = fmaf(row_lds[i], row_lds[i], acc);
+    // thirty-two links at a time, the next ones' elements read from LDS under these
+    const float* mine = row_lds + threadIdx.x;
+    const int links = dim / 16, whole = links & ~31;
+    float a[32], b[32];
+    if (whole) {
+#pragma unroll
+      for (int j = 0; j < 32; ++j) a[j] = mine[16 * j];
+    }
+    for (int l = 0; l < whole; l += 32) {
+      const int nx = l + 32 < whole ? l + 32 : l;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) b[j] = mine[16 * (nx + j)];
+#pragma unroll
+      for (int j = 0; j < 32; ++j) acc = fmaf(a[j], a[j], acc);
+#pragma unroll
+      for (int j = 0; j < 32; ++j) a[j] = b[j];
+    }
+    for (int i = 16 * whole + (int)threadIdx.x; i < dim; i += 16) acc = fmaf(row_lds[i], row_lds[i], acc);
     acc = row16_sum(acc);
     if (threadIdx.x == 0) inv_lds = 1.0f / sqrtf(acc / (float)dim + eps);
   }
   __syncthreads();
   const float inv = inv_lds;
-  float* yr = y + (size_t)blockIdx.x * dim;
+  if (vec) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int c = (int)threadIdx.x + 256 * j;
+      if (c < nvec)
+        reinterpret_cast<f32x4*>(yr)[c] = (f32x4){(v[j][0] * inv) * wv[j][0], (v[j][1] * inv) * wv[j][1], (v[j][2] * inv) * wv[j][2],
+                                                  (v[j][3] * inv) * wv[j][3]};
+    }
+    return;
+  }
   for (int i = threadIdx.x; i < dim; i += 256) {
     float wi;
     if constexpr (sizeof(WT) == 2) wi = bf16_to_f32(w[i]);
@@ -341,19 +389,36 @@ extern "C" int bw_convert(const void* src, int src_is_bf16, void* dst, int dst_i
 }
 
 // h = g * (1/(1+exp(-g))) * u over rows laid out [gate | up] (src/kernels.cpp:291-298).
-__global__ void swiglu_f32_kernel(const float* __restrict__ gate_up, float* __restrict__ h, int rows, int inter) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)rows * inter) return;
-  const int r = (int)(i / inter), c = (int)(i % inter);
-  const float g = gate_up[(size_t)r * 2 * inter + c];
-  const float u = gate_up[(size_t)r * 2 * inter + inter + c];
-  h[i] = g * (1.0f / (1.0f + bw_expf(-g))) * u;
+// (A row a y index: a thread's element number divided by the row length was most of the kernel at 8 rows of 8,192, 4.9 us.)
+template <int VEC>
+__global__ __launch_bounds__(256) void swiglu_f32_kernel(const float* __restrict__ gate_up, float* __restrict__ h, int inter) {
+  const int c = ((int)blockIdx.x * 256 + (int)threadIdx.x) * VEC;
+  if (c >= inter) return;
+  const float* g0 = gate_up + (size_t)blockIdx.y * 2 * inter + c;
+  float* dst = h + (size_t)blockIdx.y * inter + c;
+  if constexpr (VEC == 4) {
+    const f32x4 g = *reinterpret_cast<const f32x4*>(g0), u = *reinterpret_cast<const f32x4*>(g0 + inter);
+    f32x4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = g[j] * (1.0f / (1.0f + bw_expf(-g[j]))) * u[j];
+    *reinterpret_cast<f32x4*>(dst) = o;
+  } else {
+    const float g = g0[0], u = g0[inter];
+    dst[0] = g * (1.0f / (1.0f + bw_expf(-g))) * u;
+  }
 }
 
 extern "C" int bw_swiglu_f32(const float* gate_up, float* h, int rows, int inter, void* stream) {
   if (rows <= 0) return 0;
-  size_t n = (size_t)rows * inter;
-  hipLaunchKernelGGL(swiglu_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, gate_up, h, rows, inter);
+  // four elements a thread where there are rows enough to fill the chip with such threads (else one: more workgroups)
+  const bool vec = inter % 4 == 0 && (((uintptr_t)gate_up | (uintptr_t)h) & 15) == 0 && (size_t)rows * inter >= (size_t)1 << 18;
+  for (int r = 0; r < rows; r += 65535) {
+    const int n = rows - r < 65535 ? rows - r : 65535;
+    const float* g = gate_up + (size_t)r * 2 * inter;
+    float* o = h + (size_t)r * inter;
+    if (vec) hipLaunchKernelGGL(swiglu_f32_kernel<4>, dim3((unsigned)((inter / 4 + 255) / 256), n), dim3(256), 0, (hipStream_t)stream, g, o, inter);
+    else hipLaunchKernelGGL(swiglu_f32_kernel<1>, dim3((unsigned)((inter + 255) / 256), n), dim3(256), 0, (hipStream_t)stream, g, o, inter);
+  }
   return BW_LAUNCH_CHECK();
 }
 
@@ -389,87 +454,125 @@ struct RopeArgs {
   int rows, heads, kv_heads, head_dim, page_size, table_stride, write_cache;
 };
 
-// 32-bit: q and k are rotated in place; k and v go to cache[page][kv_head][slot][hd]
-// (src/model.cpp:291-296, src/kernels.h:97-99).
-__global__ void rope_kvwrite_f32_kernel(RopeArgs a, float* qkv_rw, float* __restrict__ k_cache,
-                                        float* __restrict__ v_cache) {
-  const int row = blockIdx.x;
-  const int pos = a.positions[row];
-  if (pos < 0) return;
-  const int hd = a.head_dim, half = hd / 2;
-  const int q_dim = a.heads * hd, kv_dim = a.kv_heads * hd;
-  float* r = qkv_rw + (size_t)row * (q_dim + 2 * kv_dim);
-  const int page = a.block_table[(size_t)a.row_seq[row] * a.table_stride + pos / a.page_size];
-  const int slot = pos % a.page_size;
-  const float* ct = a.cos_table + (size_t)pos * half;
-  const float* st = a.sin_table + (size_t)pos * half;
-  const int pairs = (a.heads + a.kv_heads) * half;
-  for (int e = threadIdx.x; e < pairs; e += blockDim.x) {
-    const int hh = e / half, i = e % half;
-    float* v = r + hh * hd;
-    const float x1 = v[i], x2 = v[i + half];
-    const float c = ct[i], s = st[i];
-    const float o1 = x1 * c - x2 * s;
-    const float o2 = x2 * c + x1 * s;
-    v[i] = o1;
-    v[i + half] = o2;
-    if (hh >= a.heads && a.write_cache) {
-      const int h = hh - a.heads;
-      float* dst = k_cache + (((size_t)page * a.kv_heads + h) * a.page_size + slot) * hd;
-      dst[i] = o1;
-      dst[i + half] = o2;
-    }
+// A thread takes VEC neighbouring pairs of one row and head (blocks y < qk_blocks), or a value column: every load of a row is
+// asked for at once, where a workgroup a row walked its pairs 256 at a time, a round trip to memory each (8 rows of 32
+// heads of 64 in 32 bits: 7.9 -> 4.7 us; 777 rows of 32 + 8 heads of 128 in bfloat16: 12.8 -> 9.3, 2,048 rows: 20.9 -> 17.2, of
+// which the bytes take 15).
+// 32-bit: q and k are rotated in place; k and v go to cache[page][kv_head][slot][hd] (src/model.cpp:291-296,
+// src/kernels.h:97-99).  bfloat16: rotation in 32-bit from the 32-bit projections; q goes to q_out [rows, q_dim], k to
+// cache[page][kv_head][slot][hd], v transposed to cache[page][kv_head][hd][slot], each rounded once; a thread there has
+// four rows of a value column, whose slots most often are four neighbours that start at a multiple of four: one 8-byte
+// store instead of four of two bytes a page row apart.
+template <int VEC>
+struct RopeVec {
+  float v[VEC];
+};
+
+template <int VEC>
+__device__ __forceinline__ RopeVec<VEC> rope_load(const float* p) {
+  RopeVec<VEC> r;
+  if constexpr (VEC == 4) {
+    const f32x4 q = *reinterpret_cast<const f32x4*>(p);
+    r.v[0] = q[0]; r.v[1] = q[1]; r.v[2] = q[2]; r.v[3] = q[3];
+  } else {
+    r.v[0] = p[0];
   }
-  if (a.write_cache) {
-    const float* vsrc = r + q_dim + kv_dim;
-    for (int e = threadIdx.x; e < kv_dim; e += blockDim.x) {
-      const int h = e / hd, d = e % hd;
-      v_cache[(((size_t)page * a.kv_heads + h) * a.page_size + slot) * hd + d] = vsrc[e];
+  return r;
+}
+
+template <int VEC>
+__device__ __forceinline__ void rope_store(float* p, const RopeVec<VEC>& r) {
+  if constexpr (VEC == 4) *reinterpret_cast<f32x4*>(p) = (f32x4){r.v[0], r.v[1], r.v[2], r.v[3]};
+  else p[0] = r.v[0];
+}
+
+template <int VEC>
+__device__ __forceinline__ void rope_store(bf16_t* p, const RopeVec<VEC>& r) {
+  if constexpr (VEC == 4) *reinterpret_cast<u32x2*>(p) = (u32x2){pack_bf16x2(r.v[0], r.v[1]), pack_bf16x2(r.v[2], r.v[3])};
+  else p[0] = f32_to_bf16(r.v[0]);
+}
+
+template <typename CT, int VEC>
+__global__ __launch_bounds__(256) void rope_kvwrite_kernel(RopeArgs a, float* qkv_rw, bf16_t* __restrict__ q_out, CT* __restrict__ k_cache,
+                                                           CT* __restrict__ v_cache, int qk_blocks) {
+  constexpr bool BF = sizeof(CT) == 2;
+  const int hd = a.head_dim, half = hd / 2;
+  const int q_dim = a.heads * hd, kv_dim = a.kv_heads * hd, width = q_dim + 2 * kv_dim;
+  if ((int)blockIdx.y < qk_blocks) {
+    const int row = blockIdx.x, per_head = half / VEC;
+    const int e = (int)blockIdx.y * 256 + (int)threadIdx.x;
+    if (e >= (a.heads + a.kv_heads) * per_head) return;
+    const int hh = e / per_head, i = (e % per_head) * VEC;
+    const int pos = a.positions[row];
+    if (pos < 0) return;
+    float* v = qkv_rw + (size_t)row * width + hh * hd + i;
+    const RopeVec<VEC> x1 = rope_load<VEC>(v), x2 = rope_load<VEC>(v + half);
+    const RopeVec<VEC> c = rope_load<VEC>(a.cos_table + (size_t)pos * half + i), s = rope_load<VEC>(a.sin_table + (size_t)pos * half + i);
+    RopeVec<VEC> o1, o2;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      o1.v[j] = x1.v[j] * c.v[j] - x2.v[j] * s.v[j];
+      o2.v[j] = x2.v[j] * c.v[j] + x1.v[j] * s.v[j];
     }
+    if constexpr (!BF) {
+      rope_store<VEC>(v, o1);
+      rope_store<VEC>(v + half, o2);
+    } else if (hh < a.heads) {
+      bf16_t* dst = q_out + (size_t)row * q_dim + hh * hd + i;
+      rope_store<VEC>(dst, o1);
+      rope_store<VEC>(dst + half, o2);
+    }
+    if (hh >= a.heads && a.write_cache) {
+      const int page = a.block_table[(size_t)a.row_seq[row] * a.table_stride + pos / a.page_size];
+      CT* dst = k_cache + (((size_t)page * a.kv_heads + (hh - a.heads)) * a.page_size + pos % a.page_size) * hd + i;
+      rope_store<VEC>(dst, o1);
+      rope_store<VEC>(dst + half, o2);
+    }
+    return;
+  }
+  const int e = ((int)blockIdx.y - qk_blocks) * 256 + (int)threadIdx.x;
+  if constexpr (!BF) {
+    const int row = blockIdx.x;
+    if (e * VEC >= kv_dim) return;
+    const int pos = a.positions[row];
+    if (pos < 0) return;
+    const RopeVec<VEC> x = rope_load<VEC>(qkv_rw + (size_t)row * width + q_dim + kv_dim + e * VEC);
+    const int page = a.block_table[(size_t)a.row_seq[row] * a.table_stride + pos / a.page_size];
+    rope_store<VEC>(v_cache + (((size_t)page * a.kv_heads + (e * VEC) / hd) * a.page_size + pos % a.page_size) * hd + (e * VEC) % hd, x);
+  } else {
+    const int row0 = 4 * (int)blockIdx.x;
+    if (row0 >= a.rows || e >= kv_dim) return;
+    const int h = e / hd, d = e % hd;
+    int pos[4];
+    size_t page[4];
+    float x[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int row = min(row0 + t, a.rows - 1);
+      pos[t] = row0 + t < a.rows ? a.positions[row] : -1;
+      x[t] = qkv_rw[(size_t)row * width + q_dim + kv_dim + e];
+      const int seq = pos[t] >= 0 ? a.row_seq[row] : 0;
+      page[t] = (size_t)a.block_table[(size_t)seq * a.table_stride + (pos[t] > 0 ? pos[t] : 0) / a.page_size];
+    }
+    auto at = [&](int t) { return v_cache + ((page[t] * a.kv_heads + h) * hd + d) * a.page_size + pos[t] % a.page_size; };
+    const bool four = VEC == 4 && pos[0] >= 0 && (pos[0] & 3) == 0 && (a.page_size & 3) == 0 && pos[1] == pos[0] + 1 && pos[2] == pos[0] + 2 &&
+                      pos[3] == pos[0] + 3 && page[1] == page[0] && page[2] == page[0] && page[3] == page[0];
+    if (four) {
+      *reinterpret_cast<u32x2*>(at(0)) = (u32x2){pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
+      return;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (pos[t] >= 0) *at(t) = f32_to_bf16(x[t]);
   }
 }
 
-// bfloat16: rotation in 32-bit from the 32-bit projections; q goes to q_out [rows, q_dim],
-// k to cache[page][kv_head][slot][hd], v transposed to cache[page][kv_head][hd][slot], each
-// rounded once.
-__global__ void rope_kvwrite_bf16_kernel(RopeArgs a, bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cache,
-                                         bf16_t* __restrict__ v_cache) {
-  const int row = blockIdx.x;
-  const int pos = a.positions[row];
-  if (pos < 0) return;
-  const int hd = a.head_dim, half = hd / 2;
-  const int q_dim = a.heads * hd, kv_dim = a.kv_heads * hd;
-  const float* r = a.qkv + (size_t)row * (q_dim + 2 * kv_dim);
-  const int page = a.block_table[(size_t)a.row_seq[row] * a.table_stride + pos / a.page_size];
-  const int slot = pos % a.page_size;
-  const float* ct = a.cos_table + (size_t)pos * half;
-  const float* st = a.sin_table + (size_t)pos * half;
-  const int pairs = (a.heads + a.kv_heads) * half;
-  for (int e = threadIdx.x; e < pairs; e += blockDim.x) {
-    const int hh = e / half, i = e % half;
-    const float* v = r + hh * hd;
-    const float x1 = v[i], x2 = v[i + half];
-    const float c = ct[i], s = st[i];
-    const float o1 = x1 * c - x2 * s;
-    const float o2 = x2 * c + x1 * s;
-    if (hh < a.heads) {
-      bf16_t* dst = q_out + (size_t)row * q_dim + hh * hd;
-      dst[i] = f32_to_bf16(o1);
-      dst[i + half] = f32_to_bf16(o2);
-    } else if (a.write_cache) {
-      const int h = hh - a.heads;
-      bf16_t* dst = k_cache + (((size_t)page * a.kv_heads + h) * a.page_size + slot) * hd;
-      dst[i] = f32_to_bf16(o1);
-      dst[i + half] = f32_to_bf16(o2);
-    }
-  }
-  if (a.write_cache) {
-    const float* vsrc = r + q_dim + kv_dim;
-    for (int e = threadIdx.x; e < kv_dim; e += blockDim.x) {
-      const int h = e / hd, d = e % hd;
-      v_cache[(((size_t)page * a.kv_heads + h) * hd + d) * a.page_size + slot] = f32_to_bf16(vsrc[e]);
-    }
-  }
+template <typename CT, int VEC>
+static void launch_rope(const RopeArgs& a, float* qkv, void* q_out, void* k_cache, void* v_cache, hipStream_t s) {
+  const int qk = ((a.heads + a.kv_heads) * (a.head_dim / 2 / VEC) + 255) / 256;
+  const int per_block = sizeof(CT) == 2 ? 256 : 256 * VEC;
+  const int v = a.write_cache ? (a.kv_heads * a.head_dim + per_block - 1) / per_block : 0;
+  hipLaunchKernelGGL((rope_kvwrite_kernel<CT, VEC>), dim3(a.rows, qk + v), dim3(256), 0, s, a, qkv, (bf16_t*)q_out, (CT*)k_cache, (CT*)v_cache, qk);
 }
 
 extern "C" int bw_rope_kvwrite(float* qkv, void* q_out, const int32_t* positions, const int32_t* row_seq,
@@ -482,9 +585,15 @@ extern "C" int bw_rope_kvwrite(float* qkv, void* q_out, const int32_t* positions
   RopeArgs a{qkv, positions, row_seq, block_table, cos_table, sin_table,
              rows, heads, kv_heads, head_dim, page_size, table_stride, write_cache};
   hipStream_t s = (hipStream_t)stream;
-  if (is_bf16)
-    hipLaunchKernelGGL(rope_kvwrite_bf16_kernel, dim3(rows), dim3(256), 0, s, a, (bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache);
-  else
-    hipLaunchKernelGGL(rope_kvwrite_f32_kernel, dim3(rows), dim3(256), 0, s, a, qkv, (float*)k_cache, (float*)v_cache);
+  // four pairs a thread where halves of heads are whole vectors and everything starts at one
+  const bool vec = head_dim % 8 == 0 && (((uintptr_t)qkv | (uintptr_t)cos_table | (uintptr_t)sin_table | (uintptr_t)k_cache | (uintptr_t)v_cache |
+                                         (uintptr_t)q_out) & 15) == 0;
+  if (is_bf16) {
+    if (vec) launch_rope<bf16_t, 4>(a, qkv, q_out, k_cache, v_cache, s);
+    else launch_rope<bf16_t, 1>(a, qkv, q_out, k_cache, v_cache, s);
+  } else {
+    if (vec) launch_rope<float, 4>(a, qkv, q_out, k_cache, v_cache, s);
+    else launch_rope<float, 1>(a, qkv, q_out, k_cache, v_cache, s);
+  }
   return BW_LAUNCH_CHECK();
 }

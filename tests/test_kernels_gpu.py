@@ -515,6 +515,63 @@ def test_rope_and_cache_write(gpu, bf16):
 
 # ----------------------------------------------------------------------------- attention
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("heads,kvh,hd,page", [(4, 2, 64, 16), (3, 1, 20, 4), (6, 2, 128, 8), (1, 1, 8, 2), (33, 3, 16, 64)])
+def test_rope_of_mixed_rows_equals_the_rows_alone(gpu, bf16, heads, kvh, hd, page):
+    """Portions that start anywhere in a page, single tokens and padding rows (vectors of four pairs and single ones, four
+    rows of a value column and fewer): every row gets the bits it gets alone, padding and foreign slots are not written, and
+    the numbers are the formula's within a rounding."""
+    g = torch.Generator().manual_seed(hd)
+    segs = [(page - 1, page + 5), (0, 9), (4 * page + 2, 1), (3, 2 * page + 3)]
+    rows = sum(n for _, n in segs)
+    width = (max(p + n for p, n in segs) + page - 1) // page
+    table = torch.randperm(len(segs) * width, generator=g).int().view(len(segs), width)
+    pos = torch.cat([torch.arange(p, p + n, dtype=torch.int32) for p, n in segs])
+    seq = torch.cat([torch.full((n,), i, dtype=torch.int32) for i, (_, n) in enumerate(segs)])
+    pos[5] = pos[rows - 2] = -1
+    qkv = torch.randn(rows, (heads + 2 * kvh) * hd, generator=g)
+    cos, sin = torch.randn(2, 6 * page + 40, hd // 2, generator=g)
+    dt = torch.bfloat16 if bf16 else torch.float32
+
+    def run(which):
+        x, n = qkv[which].to(gpu).contiguous(), len(which)
+        kc = torch.full((len(segs) * width, kvh * page * hd), 7.0, dtype=dt, device=gpu)
+        vc = kc.clone()
+        q = torch.full((n, heads * hd), 7.0, dtype=torch.bfloat16, device=gpu) if bf16 else None
+        ops.rope_kvwrite(x, q, pos[which].to(gpu), seq[which].to(gpu), table.to(gpu), cos.to(gpu), sin.to(gpu), kc, vc, n, heads, kvh, hd, page)
+        return [t.cpu() for t in ((q if bf16 else x), kc, vc)]
+
+    together = run(list(range(rows)))
+    k_alone, v_alone = torch.full_like(together[1], 7.0), torch.full_like(together[2], 7.0)
+    for r in range(rows):
+        one = run([r])
+        assert torch.equal(one[0][0], together[0][r]), r
+        for alone, now in ((k_alone, one[1]), (v_alone, one[2])):
+            touched = now != 7.0
+            alone[touched] = now[touched]
+    assert torch.equal(together[1], k_alone) and torch.equal(together[2], v_alone)
+    r, half = 7, hd // 2
+    x1, x2 = qkv[r, :half].double(), qkv[r, half:hd].double()
+    c, s = cos[pos[r]].double(), sin[pos[r]].double()
+    want = torch.cat([x1 * c - x2 * s, x2 * c + x1 * s])
+    scale = torch.cat([(x1 * c).abs() + (x2 * s).abs(), (x2 * c).abs() + (x1 * s).abs()])
+    assert ((together[0][r, :hd].double() - want).abs() <= (2.0 ** -8 if bf16 else 2.0 ** -22) * scale).all()
+
+
+@pytest.mark.parametrize("dim", [15, 97, 512, 528, 2048, 4096, 4100, 8192])
+@pytest.mark.parametrize("wdt", [torch.bfloat16, torch.float32])
+def test_rmsnorm_f32_rows_are_the_chains_of_the_definition(gpu, dim, wdt):
+    """Sixteen chains i % 16 and their tree, in 32-bit steps on the host, for rows that are whole vectors and rows that are not."""
+    g = torch.Generator().manual_seed(dim)
+    x, w = torch.randn(3, dim, generator=g), (1 + 0.1 * torch.randn(dim, generator=g)).to(wdt)
+    out = torch.zeros(3, dim, device=gpu)
+    ops.rmsnorm(x.to(gpu), w.to(gpu), out, 3, 1e-5)
+    for r in range(3):
+        inv = np.float32(1.0) / np.sqrt(canonical_sumsq(x[r].numpy()) / np.float32(dim) + np.float32(1e-5), dtype=np.float32)
+        want = (x[r].numpy() * inv) * w.float().numpy()
+        assert np.array_equal(out[r].cpu().numpy(), want), r
+
+
 def paged_setup(gpu, bf16, heads, kvh, hd, page, pages, n_keys, seed, poison=False):
     """A sequence of n_keys keys and values scattered over pages by the reference's table
     (i*7+3) % pages (tests/test_main.cpp:146-147); everything else is poison."""
