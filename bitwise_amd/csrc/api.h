@@ -123,6 +123,7 @@ int bw_norm_shift(const float* x, int ldx, const float* w, const float* mix, flo
 // q is multiplied by qscale, k by kscale; heads_per_key neighbouring heads share one q and one k.
 // (silu 1, fixed decay only: q, k and v pass SiLU on their way in; few 1: the requests bring a few rows each, which picks the
 // kernel that favours many waves over long walks, the same bits)
+int bw_decay_rows(float* z, int ld, const float* bias, float param, int rows, int cols, void* stream);
 int bw_linear_recurrence(int mode, const float* proj, int ldp, int q_off, int k_off, int v_off, const float* gate, int ldg,
                          int gate_off, int gate2_off, const float* bias, const float* bias2, float param, float qscale,
                          float kscale, const float* skip, int heads_per_key, int silu, int few, float* state, long long state_ld, float* out,

@@ -96,6 +96,7 @@ _SIGS = {
     "bw_side_gate": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "bw_norm_mean": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_float, c_void_p],
     "bw_norm_mean_add": [c_void_p, c_void_p, c_void_p, c_int, c_float, c_void_p, c_float, c_float, c_void_p, c_int, c_int, c_int, c_void_p],
+    "bw_decay_rows": [c_void_p, c_int, c_void_p, c_float, c_int, c_int, c_void_p],
     "bw_linear_recurrence": [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p,
                              c_float, c_float, c_float, c_void_p, c_int, c_int, c_int, c_void_p, c_longlong, c_void_p, c_int, c_void_p, c_void_p,
                              c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_longlong, c_void_p],
@@ -796,7 +797,7 @@ def gemm_qkv_rope_bf16(x: torch.Tensor, w_qkv: torch.Tensor, q_out: torch.Tensor
 # ------------------------------------------------------------------------------ mixers with a state per request
 
 RECUR_DECAY_PER_CHANNEL, RECUR_SCALAR_GATES, RECUR_BONUS_DECAY, RECUR_FIXED_DECAY, RECUR_STEP_DECAY = 0, 1, 2, 3, 4
-RECUR_DELTA = 5
+RECUR_DELTA, RECUR_DECAY_GIVEN = 5, 6
 RECUR_MAX_DIM = 256          # key channels of a head that the recurrence keeps in a lane's registers
 GATE_SIGMOID, GATE_SILU = 0, 1
 ACT_SILU, ACT_GELU_TANH, ACT_CLAMPED_SWISH = 0, 1, 2
@@ -853,6 +854,16 @@ def recurrence_state(mode: int, heads: int, dim: int, vdim: int) -> int:
     return n
 
 
+def decay_rows(z: torch.Tensor, bias: torch.Tensor, param: float, rows: int) -> None:
+    """z[r, c] <- exp(logsigmoid(z[r, c] + bias[c]) * param) for the first ``rows`` rows, in place: what RECUR_DECAY_PER_CHANNEL
+    makes of its logits, for RECUR_DECAY_GIVEN."""
+    _need_strided(z, torch.float32, "z")
+    _need(bias, torch.float32, "bias")
+    if z.shape[0] < rows or bias.numel() != z.shape[1]:
+        raise ValueError("decay_rows: rows or bias do not fit")
+    _check(_fn("bw_decay_rows")(z.data_ptr(), z.stride(0), bias.data_ptr(), float(param), int(rows), z.shape[1], _stream()), "decay_rows")
+
+
 def linear_recurrence(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_off: int, gate: Optional[torch.Tensor], gate_off: int,
                       gate2_off: int, bias: Optional[torch.Tensor], bias2: Optional[torch.Tensor], param: float, qscale: float,
                       state: torch.Tensor, out: torch.Tensor, seq_rows: torch.Tensor, slots: torch.Tensor,
@@ -863,6 +874,7 @@ def linear_recurrence(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_o
     to ``state`` [slots, elements].  RECUR_DECAY_PER_CHANNEL: decay = exp(logsigmoid(gate + bias) * param) per key
     channel (``gate`` [rows, >= gate_off + heads*dim]).  RECUR_SCALAR_GATES: capped input and forget gates per head
     (columns gate_off + h and gate2_off + h of ``gate``), a normaliser and a running maximum in the state; param = cap.
+    RECUR_DECAY_GIVEN: as per channel with the decays themselves in ``gate`` (``decay_rows``; ``bias`` None).
     RECUR_BONUS_DECAY: decay = exp(-exp(gate + bias)) per key channel, and the read-out comes before the update:
     o = (S + diag(bias2) k v^T)^T q with the S the token before left (``bias2`` [heads*dim]: the weight of the token's own
     k v^T), then S <- decay * S + k v^T.  RECUR_FIXED_DECAY: one constant decay a head (``bias`` [heads]; ``gate`` None).
@@ -885,7 +897,7 @@ def linear_recurrence(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_o
     _need_strided(proj, torch.float32, "proj")            # (may be a column slice of a wider product)
     if mode != RECUR_FIXED_DECAY:
         _need_strided(gate, torch.float32, "gate")
-    if bias is not None or mode != RECUR_DELTA:
+    if bias is not None or mode not in (RECUR_DELTA, RECUR_DECAY_GIVEN):
         _need(bias, torch.float32, "bias")
     if silu and mode != RECUR_FIXED_DECAY:
         raise ValueError("linear_recurrence: SiLU on the way in comes with a constant decay only")
@@ -924,7 +936,7 @@ def linear_recurrence(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_o
             _need(bias2, torch.float32, "bias2")
             if bias2.numel() != heads * dim:
                 raise ValueError("linear_recurrence: the weights of the token's own k v^T do not fit heads x dim")
-        if bias.numel() != heads * dim or gate_off + heads * dim > gate.shape[1]:
+        if (mode != RECUR_DECAY_GIVEN and bias.numel() != heads * dim) or gate_off + heads * dim > gate.shape[1]:
             raise ValueError("linear_recurrence: decay logits or bias do not fit heads x dim")
         need = heads * dim * vdim
     if state.dim() != 2 or state.shape[1] < need:

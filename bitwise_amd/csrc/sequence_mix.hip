@@ -29,6 +29,9 @@ __device__ __forceinline__ float softplus(float z) {
   return fmaxf(z, 0.0f) + log1pf(bw_expf(-fabsf(z)));
 }
 
+// The decay of a key channel from its logit.
+__device__ __forceinline__ float channel_decay(float z, float param) { return bw_expf(log_sigmoid(z) * param); }
+
 __device__ __forceinline__ float silu(float z) { return z * (1.0f / (1.0f + bw_expf(-z))); }
 
 template <typename OT>
@@ -252,7 +255,8 @@ __global__ __launch_bounds__(256) void norm_shift_row_kernel(const float* __rest
 
 // ------------------------------------------------------------------------- the linear recurrence
 
-enum { RECUR_DECAY_PER_CHANNEL = 0, RECUR_SCALAR_GATES = 1, RECUR_BONUS_DECAY = 2, RECUR_FIXED_DECAY = 3, RECUR_STEP_DECAY = 4, RECUR_DELTA = 5 };
+enum { RECUR_DECAY_PER_CHANNEL = 0, RECUR_SCALAR_GATES = 1, RECUR_BONUS_DECAY = 2, RECUR_FIXED_DECAY = 3, RECUR_STEP_DECAY = 4, RECUR_DELTA = 5,
+       RECUR_DECAY_GIVEN = 6 };
 
 // The sum over the SPLIT neighbouring lanes that hold the parts of one column (every one of them gets it): an addition a
 // stage whose second operand comes through a data-parallel move within a row of 16 lanes.  Behind the first two stages the
@@ -311,6 +315,9 @@ struct RecurArgs {
 //
 // RECUR_BONUS_DECAY:  alpha[d] = exp(-exp(z[d] + bias[d]));  o[j] = sum_d (S[d][j] + u[d] k[d] v[j]) q[d] with the S of the token
 //   before (the token's own k v^T is read through the bonus u = bias2 [heads*dim]), then S[d][j] <- alpha[d] S[d][j] + k[d] v[j].
+// RECUR_DECAY_GIVEN:  as per channel, with the decays themselves in place of their logits (decay_rows_kernel).  Steps of more
+//   than a few rows a request: on the way to LDS every workgroup of a head took the two exponentials and the logarithm of the
+//   same elements, a third of a portion's time.
 // RECUR_FIXED_DECAY:  as per channel with one constant decay a head, alpha[d] = bias[head]; no logits are read.
 // RECUR_STEP_DECAY:  a step size per head and token, delta = softplus(z + bias[head]) with z at gate_off + head;
 //   S[d][j] <- e^(-bias2[head] delta) S[d][j] + k[d] (delta v[j]),  o[j] = (S^T q)[j] + skip[head] v[j].
@@ -352,11 +359,20 @@ struct RecurOps {
   float k[N][DH], q[N][DH], a[CHANNELS ? N : 1][CHANNELS ? DH : 1], v[N], g1[N], g2[N], kq[N];
 };
 
+// f(0), f(2 TU), f(4 TU) ... below RUN, the numbers known at compile time.
+template <int B, int RUN, int TU, typename F>
+__device__ __forceinline__ void run_groups(F f) {
+  if constexpr (B < RUN) {
+    f(std::integral_constant<int, B>{});
+    run_groups<B + 2 * TU, RUN, TU>(f);
+  }
+}
+
 template <int MODE, int DPAD, int PHASE>
 __global__ __launch_bounds__(64 * RW) void linear_recurrence_kernel(RecurArgs a) {
   constexpr bool GATES = MODE == RECUR_SCALAR_GATES;
   constexpr bool BONUS = MODE == RECUR_BONUS_DECAY, FIXED = MODE == RECUR_FIXED_DECAY, STEP = MODE == RECUR_STEP_DECAY;
-  constexpr bool DELTA = MODE == RECUR_DELTA;
+  constexpr bool DELTA = MODE == RECUR_DELTA, GIVEN = MODE == RECUR_DECAY_GIVEN;
   constexpr bool CHANNELS = !GATES && !STEP && !DELTA && !FIXED;   // a decay per channel comes through LDS
   constexpr int NN = (DPAD + 63) / 64;
   constexpr bool READ_OUT = PHASE != 1;
@@ -368,10 +384,22 @@ __global__ __launch_bounds__(64 * RW) void linear_recurrence_kernel(RecurArgs a)
   constexpr int RC = PHASE == 4 && DPAD >= 64 ? 4 : (PHASE == 0 && DPAD <= 128 ? 32 : 16);     // tokens staged together
   constexpr int NQ = RC * DPAD / (64 * RW), NV = (RC * WCOLS + 64 * RW - 1) / (64 * RW);
   static_assert(NQ * 64 * RW == RC * DPAD && RC % TU == 0, "a chunk is whole loads and whole groups of tokens");
+  // What the gates and the normaliser make of a chunk's tokens does not depend on the wave's columns, and only the running
+  // maximum is a chain: a portion walked whole prepares it for a chunk at once, a token a lane (three exponentials a
+  // chunk instead of three a token) and the tokens' n.q shared out over the workgroup's waves.  The same statements.
+  // (8 heads of 128 x 256, 2,048 tokens: 963 us -> 520, with the runs below.)
+  constexpr bool HOIST = GATES && PHASE == 0;
+  static_assert(!HOIST || RC <= 64, "a token a lane");
+  // tokens of a whole chunk that leave together: one division and one store for as many as a column has lanes
+  // (a column of fewer lanes: every group's own)
+  constexpr bool GATHER = SPLIT >= 2 * TU;
+  constexpr int RUN = GATHER ? (SPLIT < RC ? SPLIT : RC) : 2 * TU;
+  static_assert(PHASE != 0 || RC % RUN == 0, "runs fill a chunk");
+  __shared__ float nqs[HOIST ? RC : 1], ems[HOIST ? RC : 1];
   __shared__ __attribute__((aligned(16))) float qs[BUFS][RC][DPAD];
   __shared__ __attribute__((aligned(16))) float ks[BUFS][RC][DPAD];
   __shared__ __attribute__((aligned(16))) float as[CHANNELS ? BUFS : 1][CHANNELS ? RC : 1][CHANNELS ? DPAD : 4];
-  __shared__ float gi[BUFS][RC], gf[BUFS][RC], gd[DELTA ? BUFS : 1][DELTA ? RC : 1];
+  __shared__ __attribute__((aligned(16))) float gi[BUFS][RC], gf[BUFS][RC], gd[DELTA ? BUFS : 1][DELTA ? RC : 1];
   __shared__ float vs[BUFS][RC][WCOLS];
   const int lane = threadIdx.x & 63, wv = wave_index();
   const int h = blockIdx.y;
@@ -453,7 +481,7 @@ __global__ __launch_bounds__(64 * RW) void linear_recurrence_kernel(RecurArgs a)
   // q, k and decay logits as 16-byte vectors where the rows allow it: vector u of a thread is elements 4u .. 4u + 3 of its rq
   constexpr bool WIDE = NQ % 4 == 0;
   const bool vectors = WIDE && (dim & 3) == 0 && ((a.q_off | a.k_off | a.ldp) & 3) == 0 && (reinterpret_cast<uintptr_t>(a.proj) & 15) == 0 &&
-                       (!CHANNELS || (((a.ldg | a.gate_off) & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.gate) | reinterpret_cast<uintptr_t>(a.bias)) & 15) == 0));   // (scalar)
+                       (!CHANNELS || (((a.ldg | a.gate_off) & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.gate) | (GIVEN ? 0 : reinterpret_cast<uintptr_t>(a.bias))) & 15) == 0));   // (scalar)
   float rq[NQ], rk[NQ], rz[CHANNELS ? NQ : 1], rv[NV], rg[3];
   auto fetch = [&](int t0) {
     if (t0 >= count) return;                             // (scalar)
@@ -468,8 +496,8 @@ __global__ __launch_bounds__(64 * RW) void linear_recurrence_kernel(RecurArgs a)
           const float* pr = a.proj + row * a.ldp + hk * dim + d;
           const f32x4 q4 = *reinterpret_cast<const f32x4*>(pr + a.q_off), k4 = *reinterpret_cast<const f32x4*>(pr + a.k_off);
           f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
-          if constexpr (CHANNELS)
-            z4 = *reinterpret_cast<const f32x4*>(a.gate + row * a.ldg + a.gate_off + h * dim + d) + *reinterpret_cast<const f32x4*>(a.bias + h * dim + d);
+          if constexpr (CHANNELS) z4 = *reinterpret_cast<const f32x4*>(a.gate + row * a.ldg + a.gate_off + h * dim + d);
+          if constexpr (CHANNELS && !GIVEN) z4 = z4 + *reinterpret_cast<const f32x4*>(a.bias + h * dim + d);
 #pragma unroll
           for (int x = 0; x < 4; ++x) {
             rq[4 * u + x] = q4[x];
@@ -488,7 +516,8 @@ __global__ __launch_bounds__(64 * RW) void linear_recurrence_kernel(RecurArgs a)
           const float* pr = a.proj + row * a.ldp;
           rq[u] = pr[a.q_off + hk * dim + d];
           rk[u] = pr[a.k_off + hk * dim + d];
-          if constexpr (CHANNELS) rz[u] = a.gate[row * a.ldg + a.gate_off + h * dim + d] + a.bias[h * dim + d];
+          if constexpr (CHANNELS) rz[u] = a.gate[row * a.ldg + a.gate_off + h * dim + d];
+          if constexpr (CHANNELS && !GIVEN) rz[u] += a.bias[h * dim + d];
         }
       }
     }
@@ -507,7 +536,10 @@ __global__ __launch_bounds__(64 * RW) void linear_recurrence_kernel(RecurArgs a)
       rg[2] = DELTA ? gr[a.gate2_off + a.heads + hk] : 0.0f;
     }
   };
-  auto decay_of = [&](float z) { return BONUS ? bw_expf(-bw_expf(z)) : bw_expf(log_sigmoid(z) * a.param); };
+  auto decay_of = [&](float z) {
+    if constexpr (GIVEN) return z;
+    else return BONUS ? bw_expf(-bw_expf(z)) : channel_decay(z, a.param);
+  };
   auto stash = [&](int t0, int buf) {
     if (t0 >= count) return;
     const int tc = min(RC, count - t0);
@@ -611,9 +643,86 @@ __global__ __launch_bounds__(64 * RW) void linear_recurrence_kernel(RecurArgs a)
     }
   };
 
-  // those tokens one after the other
-  auto run_tokens = [&](auto& O, int t0, int buf, int t) {
+  // HOIST: the chunk's gates (lane t: token t's factors; its e^-m' for everybody), and the tokens' n.q
+  float fa_lane = 0.0f, ib_lane = 0.0f;
+  auto prepare_chunk = [&](int buf, int tc) {
+    if constexpr (HOIST) {
+      float fm = 0.0f, mx = 0.0f;
+      for (int t4 = 0; t4 < tc; t4 += 4) {
+        // (reads past the chunk's tokens bring what an earlier chunk left: not used)
+        const f32x4 f4 = *reinterpret_cast<const f32x4*>(&gf[buf][t4]), i4 = *reinterpret_cast<const f32x4*>(&gi[buf][t4]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (t4 + e >= tc) break;                       // (scalar)
+          const float x = f4[e] + m, mn = fmaxf(x, i4[e]);
+          fm = lane == t4 + e ? x : fm;
+          mx = lane == t4 + e ? mn : mx;
+          m = mn;
+        }
+      }
+      const float ig = gi[buf][lane < RC ? lane : 0];
+      fa_lane = bw_expf(fm - mx);
+      ib_lane = bw_expf(ig - mx);
+      const float em = bw_expf(-mx);
+      if (wv == 0 && lane < tc) ems[lane] = em;
+      // every wave carries the normaliser through all the tokens; the sum over the lanes of each is one wave's.  Four
+      // tokens at a time, the next four's keys read under these.
+      float kc[RW][NN], kn[RW][NN];
+      auto read_keys = [&](float (&k)[RW][NN], int t) {
+#pragma unroll
+        for (int e = 0; e < RW; ++e)
+#pragma unroll
+          for (int i = 0; i < NN; ++i) k[e][i] = ks[buf][min(t + e, RC - 1)][(lane + 64 * i) & (DPAD - 1)];
+      };
+      read_keys(kc, 0);
+      for (int t4 = 0; t4 < tc; t4 += RW) {
+        read_keys(kn, t4 + RW);
+        float qv[NN], nn[NN];
+        const int mine_t = min(t4 + wv, RC - 1);
+#pragma unroll
+        for (int i = 0; i < NN; ++i) {
+          qv[i] = qs[buf][mine_t][(lane + 64 * i) & (DPAD - 1)];
+          nn[i] = 0.0f;
+        }
+#pragma unroll
+        for (int e = 0; e < RW; ++e) {
+          if (t4 + e >= tc) break;                       // (scalar)
+          const float fa = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(fa_lane), t4 + e));
+          const float ib = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(ib_lane), t4 + e));
+#pragma unroll
+          for (int i = 0; i < NN; ++i) {
+            if (lane + 64 * i < DPAD) nreg[i] = fmaf(fa, nreg[i], ib * kc[e][i]);
+            if (e == wv) nn[i] = nreg[i];                // (scalar)
+          }
+        }
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NN; ++i)
+          if (lane + 64 * i < DPAD) sum = fmaf(nn[i], qv[i], sum);
+        const float nq = wave_sum(sum);
+        if (lane == 0 && t4 + wv < tc) nqs[t4 + wv] = nq;
+#pragma unroll
+        for (int e = 0; e < RW; ++e)
+#pragma unroll
+          for (int i = 0; i < NN; ++i) kc[e][i] = kn[e][i];
+      }
+      __syncthreads();
+    }
+  };
+
+  // What a column's lanes have gathered of a run of tokens leaves: part p of it stores token ``t`` + p (p < n).
+  auto flush = [&](float mine, int t0, int t, int n) {
+    if constexpr (HOIST) {
+      const int at = t + (part < n ? part : 0);
+      mine = mine / (fmaxf(fabsf(nqs[at]), ems[at]) + 1e-6f);
+    }
+    if (live && part < n) a.out[(size_t)(first + t0 + t + part) * a.ldo + h * vdim + j] = mine;
+  };
+  // those tokens one after the other (``base``: where in a run that is flushed together the tokens stand; a run of their own: -1)
+  float gathered = 0.0f;
+  auto run_tokens = [&](auto& O, int t0, int buf, int t, auto base) {
     constexpr int N = std::remove_reference_t<decltype(O)>::N;
+    constexpr int BASE = decltype(base)::value;
     float o[N], w[DELTA ? N : 1];
 #pragma unroll
     for (int n = 0; n < N; ++n) {
@@ -667,47 +776,57 @@ __global__ __launch_bounds__(64 * RW) void linear_recurrence_kernel(RecurArgs a)
             if (lane + 64 * i < DPAD) nreg[i] *= FIXED ? fixed_decay : as[CHANNELS ? buf : 0][CHANNELS ? t + n : 0][CHANNELS ? lane + 64 * i : 0];
         }
       } else {
-        const float ig = O.g1[n], fg = O.g2[n];
-        const float mn = fmaxf(fg + m, ig);
-        const float fa = bw_expf(fg + m - mn);
-        const float ib = bw_expf(ig - mn);
-        m = mn;
-        fsum += fg;
+        float fa, ib, mn = 0.0f;
+        if constexpr (HOIST) {
+          fa = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(fa_lane), t + n));
+          ib = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(ib_lane), t + n));
+        } else {
+          const float ig = O.g1[n], fg = O.g2[n];
+          mn = fmaxf(fg + m, ig);
+          fa = bw_expf(fg + m - mn);
+          ib = bw_expf(ig - mn);
+          m = mn;
+          fsum += fg;
+        }
         const float bv = ib * O.v[n];
 #pragma unroll
         for (int d = 0; d < DH; ++d) {
           Sreg[d] = fmaf(fa, Sreg[d], O.k[n][d] * bv);
           if constexpr (READ_OUT) o[n] = fmaf(Sreg[d], O.q[n][d], o[n]);
         }
-        float sum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < NN; ++i) {
-          const int d = lane + 64 * i;
-          if (d < DPAD) {
-            nreg[i] = fmaf(fa, nreg[i], ib * ks[buf][t + n][d]);
-            sum = fmaf(nreg[i], qs[buf][t + n][d], sum);
-          }
-        }
-        if constexpr (READ_OUT) {
+        if constexpr (HOIST) {
           o[n] = join_parts<SPLIT>(o[n]);
-          const float nq = wave_sum(sum);
-          o[n] = o[n] / (fmaxf(fabsf(nq), bw_expf(-mn)) + 1e-6f);
+        } else {
+          float sum = 0.0f;
+#pragma unroll
+          for (int i = 0; i < NN; ++i) {
+            const int d = lane + 64 * i;
+            if (d < DPAD) {
+              nreg[i] = fmaf(fa, nreg[i], ib * ks[buf][t + n][d]);
+              sum = fmaf(nreg[i], qs[buf][t + n][d], sum);
+            }
+          }
+          if constexpr (READ_OUT) {
+            o[n] = join_parts<SPLIT>(o[n]);
+            const float nq = wave_sum(sum);
+            o[n] = o[n] / (fmaxf(fabsf(nq), bw_expf(-mn)) + 1e-6f);
+          }
         }
       }
     }
     if constexpr (READ_OUT) {
-      float* orow = a.out + (size_t)(first + t0 + t) * a.ldo + h * vdim + j;
-      // (part n of a column stores token t + n)
-      float mine = 0.0f;
+      // (part n of a column keeps token t + n)
+      if (BASE <= 0) gathered = 0.0f;
 #pragma unroll
       for (int n = 0; n < N; ++n) {
         float v = o[n];
         if constexpr (!GATES) v = join_parts<SPLIT>(v);
         if constexpr (STEP) v = fmaf(skip, O.v[n], v);
         if constexpr (DELTA) v = fmaf(O.g2[n], v, w[n]);
-        mine = part == n ? v : mine;
+        gathered = part == (BASE < 0 ? 0 : BASE) + n ? v : gathered;
       }
-      if (live && part < N) orow[(size_t)part * a.ldo] = mine;
+      if constexpr (BASE < 0) flush(gathered, t0, t, N);
+      else if constexpr (BASE + N == RUN) flush(gathered, t0, t - BASE, RUN);
     }
   };
   using Group = RecurOps<TU, DH, CHANNELS>;
@@ -729,31 +848,35 @@ __global__ __launch_bounds__(64 * RW) void linear_recurrence_kernel(RecurArgs a)
       stash(t0, 0);
       __syncthreads();
     }
+    prepare_chunk(buf, tc);
     int t = 0;
     if (BUFS == 2 && tc == RC) {
       // a whole chunk: a group's operands are on their way while the group before it is worked on
       Group even, odd;
       load_tokens(even, buf, 0);
 #pragma unroll
-      for (int g = 0; g < RC / TU; g += 2) {
-        load_tokens(odd, buf, (g + 1) * TU);
-        __builtin_amdgcn_sched_barrier(0);
-        run_tokens(even, t0, buf, g * TU);
-        if (g + 2 < RC / TU) load_tokens(even, buf, (g + 2) * TU);
-        __builtin_amdgcn_sched_barrier(0);
-        run_tokens(odd, t0, buf, (g + 1) * TU);
-      }
+      for (int r = 0; r < RC; r += RUN)
+        run_groups<0, RUN, TU>([&](auto base) {
+          constexpr int B = decltype(base)::value;
+          const int at = r + B;
+          load_tokens(odd, buf, at + TU);
+          __builtin_amdgcn_sched_barrier(0);
+          run_tokens(even, t0, buf, at, std::integral_constant<int, GATHER ? B : -1>{});
+          if (at + 2 * TU < RC) load_tokens(even, buf, at + 2 * TU);
+          __builtin_amdgcn_sched_barrier(0);
+          run_tokens(odd, t0, buf, at + TU, std::integral_constant<int, GATHER ? B + TU : -1>{});
+        });
       t = RC;
     }
     for (; t + TU <= tc; t += TU) {
       Group group;
       load_tokens(group, buf, t);
-      run_tokens(group, t0, buf, t);
+      run_tokens(group, t0, buf, t, std::integral_constant<int, -1>{});
     }
     for (; t < tc; ++t) {
       Single single;
       load_tokens(single, buf, t);
-      run_tokens(single, t0, buf, t);
+      run_tokens(single, t0, buf, t, std::integral_constant<int, -1>{});
     }
     if constexpr (BUFS == 2) {
       stash(t0 + RC, buf ^ 1);
@@ -1054,7 +1177,15 @@ __global__ __launch_bounds__(256) void tanh_rows_kernel(float* __restrict__ x, i
   *p = tanhf(*p);
 }
 
-// x <- silu(x) likewise
+// Decay logits of a memory with a decay per channel -> decays, in place (RECUR_DECAY_GIVEN).
+__global__ __launch_bounds__(256) void decay_rows_kernel(float* __restrict__ z, int ld, const float* __restrict__ bias, float param, int rows, int cols) {
+  const int c = (int)blockIdx.x * 256 + (int)threadIdx.x;
+  if (c >= cols) return;
+  const float b = bias[c];
+  for (int r = blockIdx.y; r < rows; r += gridDim.y) z[(size_t)r * ld + c] = channel_decay(z[(size_t)r * ld + c] + b, param);
+}
+
+// x <- silu(x) over [rows, cols] of 32-bit values
 __global__ __launch_bounds__(256) void silu_rows_kernel(float* __restrict__ x, int ld, int rows, int cols) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= cols) return;
@@ -1109,7 +1240,7 @@ extern "C" int bw_linear_recurrence(int mode, const float* proj, int ldp, int q_
   const long long need = (long long)heads * dim * vdim + (mode == RECUR_SCALAR_GATES ? (long long)recur_blocks(dim, vdim) * ((long long)heads * dim + heads) : 0);
   if (state_ld < need) return -2;
   if (silu && mode != RECUR_FIXED_DECAY) return -2;
-  if ((bias == nullptr && mode != RECUR_DELTA) || (mode != RECUR_FIXED_DECAY && gate == nullptr) || ((mode == RECUR_SCALAR_GATES || mode == RECUR_BONUS_DECAY || mode == RECUR_STEP_DECAY) && bias2 == nullptr))
+  if ((bias == nullptr && mode != RECUR_DELTA && mode != RECUR_DECAY_GIVEN) || (mode != RECUR_FIXED_DECAY && gate == nullptr) || ((mode == RECUR_SCALAR_GATES || mode == RECUR_BONUS_DECAY || mode == RECUR_STEP_DECAY) && bias2 == nullptr))
     return -2;
   RecurArgs a{proj, ldp, q_off, k_off, v_off, gate, ldg, gate_off, gate2_off, bias, bias2, skip, heads_per_key, param, qscale, kscale, silu, state, state_ld,
               out, ldo, seq_rows, slots, positions, heads, dim, vdim, chunks, scan_local, scan_start};
@@ -1119,8 +1250,17 @@ extern "C" int bw_linear_recurrence(int mode, const float* proj, int ldp, int q_
   if (mode == RECUR_BONUS_DECAY) return launch_recurrence_passes<RECUR_BONUS_DECAY>(a, nseq, few != 0, nchunks, spans, nspans, s);
   if (mode == RECUR_FIXED_DECAY) return launch_recurrence_passes<RECUR_FIXED_DECAY>(a, nseq, few != 0, nchunks, spans, nspans, s);
   if (mode == RECUR_STEP_DECAY) return launch_recurrence_passes<RECUR_STEP_DECAY>(a, nseq, few != 0, nchunks, spans, nspans, s);
+  if (mode == RECUR_DECAY_GIVEN) return launch_recurrence_passes<RECUR_DECAY_GIVEN>(a, nseq, few != 0, nchunks, spans, nspans, s);
   if (mode == RECUR_DELTA) return launch_recurrence_passes<RECUR_DELTA>(a, nseq, few != 0, nchunks, spans, nspans, s);
   return -2;
+}
+
+extern "C" int bw_decay_rows(float* z, int ld, const float* bias, float param, int rows, int cols, void* stream) {
+  if (rows <= 0 || cols <= 0) return 0;
+  if (ld < cols) return -2;
+  const int y = rows < 1024 ? rows : 1024;
+  hipLaunchKernelGGL(decay_rows_kernel, dim3((cols + 255) / 256, y), dim3(256), 0, (hipStream_t)stream, z, ld, bias, param, rows, cols);
+  return BW_LAUNCH_CHECK();
 }
 
 extern "C" long long bw_recurrence_record(int dim, int vdim) { return (long long)recur_record(dim, vdim); }

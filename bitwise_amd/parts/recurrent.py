@@ -138,9 +138,9 @@ class _MatrixMemoryMixer(Mixer):
         return y
 
     def _recur(self, ctx, call, y, gate, gate_off, gate2_off, bias, bias2, param, raw, kscale: float = 1.0, at=None, state=None,
-               heads_per_key: int = 1, skip=None, silu: bool = False) -> None:
+               heads_per_key: int = 1, skip=None, silu: bool = False, mode: Optional[int] = None) -> None:
         """``at``: where q (or r), k and v lie in a row of ``y``, if not at the stacked projection's own
-        offsets.  ``state``: the memories' part of the slots, if they do not fill them."""
+        offsets.  ``state``: the memories' part of the slots, if they do not fill them.  ``mode``: the recurrence, if not the class's."""
         at = self.offsets if at is None else at
         plan = _scan_plan(ctx) if self.passes and self.heads * self.dim * self.vdim < self.walk_from else None
         seq_rows, nseq, scan = ctx.seq_rows, ctx.nseq, None
@@ -151,7 +151,7 @@ class _MatrixMemoryMixer(Mixer):
             local = ctx.ws.buffer("recur_scan_local", most * rec, torch.float32, rows=1)
             start = ctx.ws.buffer("recur_scan_start", most * rec, torch.float32, rows=1)
             scan = (chunks, nchunks, spans, nspans, local, start)
-        ops.linear_recurrence(self.mode, y, at["r"] if "q" not in at else at["q"], at["k"], at["v"], gate, gate_off, gate2_off,
+        ops.linear_recurrence(self.mode if mode is None else mode, y, at["r"] if "q" not in at else at["q"], at["k"], at["v"], gate, gate_off, gate2_off,
                               bias, bias2, param, self.qscale, call.state if state is None else state, raw, seq_rows, ctx.slots, ctx.positions, nseq,
                               self.heads, self.dim, self.vdim, scan=scan, kscale=kscale, heads_per_key=heads_per_key, skip=skip, silu=silu,
                               few_rows=max_seq_rows(ctx) <= FEW_SEQ_ROWS)
@@ -210,7 +210,13 @@ class GatedLinearAttention(_MatrixMemoryMixer):
         z = ws.buffer("gla_decay_logits", self.heads * self.dim, torch.float32)
         self.a2.store(ws, low, z, rows)
         raw = ws.buffer("recur_out", self.heads * self.vdim, torch.float32)
-        self._recur(ctx, call, y, z, 0, 0, self.a2_bias, None, 1.0 / self.tau, raw)
+        # a step of a few rows a request makes the decays where it uses them; in longer ones every workgroup of a head would
+        # (the same function either way: the same bits)
+        if max_seq_rows(ctx) <= FEW_SEQ_ROWS:
+            self._recur(ctx, call, y, z, 0, 0, self.a2_bias, None, 1.0 / self.tau, raw)
+        else:
+            ops.decay_rows(z, self.a2_bias, 1.0 / self.tau, rows)
+            self._recur(ctx, call, y, z, 0, 0, None, None, 1.0 / self.tau, raw, mode=ops.RECUR_DECAY_GIVEN)
         self._finish(ctx, y, raw, residual)
 
 

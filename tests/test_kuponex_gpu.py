@@ -398,3 +398,46 @@ def test_recurrences_remember_the_first_token(folders):
     for cuts in ([200], [3], [64, 64, 64]):
         assert pk.logits_error(run_cut(rp, "m", toks, cuts), want) < TOL["float32"]
         assert pk.logits_error(run_cut(rp, "o", other, cuts), want_other) < TOL["float32"]
+
+
+@pytest.mark.parametrize("dim,vdim", [(16, 24), (32, 33), (64, 40), (100, 48), (128, 17), (256, 20)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_memory_walked_in_chunks_equals_token_by_token(gpu, dim, vdim, gated):
+    """A portion around the kernel's chunks and runs of tokens (the gates, the normaliser's products and the decays prepared
+    for many tokens at once) against the same tokens one a step, which prepare them where they are used: outputs and
+    state bit for bit, beside a second request and from a state that is not zero."""
+    from bitwise_amd.csrc import ops
+    heads, dev = 2, gpu
+    g = torch.Generator(device=dev).manual_seed(dim + vdim + gated)
+    mode = ops.RECUR_SCALAR_GATES if gated else ops.RECUR_DECAY_PER_CHANNEL
+    need = ops.recurrence_state(mode, heads, dim, vdim)
+    for counts in ((1, 31), (32, 33), (70, 5), (15, 129)):
+        rows = sum(counts)
+        proj = torch.randn(rows, heads * (2 * dim + vdim), generator=g, device=dev)
+        gate = 2.0 * torch.randn(rows, 2 * heads if gated else heads * dim, generator=g, device=dev)
+        bias = torch.randn(heads if gated else heads * dim, generator=g, device=dev)
+        bias2 = torch.randn(heads, generator=g, device=dev) if gated else None
+        param = 15.0 if gated else 1.0 / 16.0
+        start = 0.1 * torch.randn(2, need, generator=g, device=dev)
+        if gated:                                    # every workgroup's copy of the normaliser and the maximum is the same
+            one = heads * (dim + 1)
+            tail = start[:, heads * dim * vdim:].view(2, -1, one)
+            tail[:] = tail[:, :1].clone()
+        slots = torch.tensor([1, 0], dtype=torch.int32, device=dev)
+        positions = torch.zeros(rows, dtype=torch.int32, device=dev)
+
+        def run(state, out, seq_rows, few, given):
+            z, b, m = gate, bias, mode
+            if given:
+                z, b, m = gate.clone(), None, ops.RECUR_DECAY_GIVEN
+                ops.decay_rows(z, bias, param, rows)
+            ops.linear_recurrence(m, proj, 0, heads * dim, 2 * heads * dim, z, 0, heads if gated else 0, b, bias2, param, dim ** -0.5, state,
+                                  out, torch.tensor(seq_rows, dtype=torch.int32, device=dev), slots, positions, 2, heads, dim, vdim, few_rows=few)
+
+        whole, single = start.clone(), start.clone()
+        out_w, out_s = torch.zeros(2, rows, heads * vdim, device=dev)
+        run(whole, out_w, [0, counts[0], counts[0], counts[1]], False, not gated)
+        for t in range(max(counts)):
+            run(single, out_s, [min(t, counts[0] - 1), int(t < counts[0]), counts[0] + min(t, counts[1] - 1), int(t < counts[1])], True, False)
+        assert torch.equal(out_w, out_s), counts
+        assert torch.equal(whole, single), counts
