@@ -1171,6 +1171,35 @@ __device__ __forceinline__ void store_partial(const AttnBf16Args& a, const Group
     for (int i = 0; i < 4; ++i) put(2 + 16 * dt + 4 * gc.g + i, o_p[dt][i]);
 }
 
+#define DECODE_W 8               // waves a workgroup of the decode kernel
+#define DECODE_W_MANY 4          // waves a workgroup where there are two workgroups or more for every compute unit: two of
+                                 // these share a compute unit, and a token's first keys do not wait for a whole
+                                 // generation of eight-wave workgroups before it (16 requests of 32 heads: 2.61 -> 2.52 ms
+                                 // a step at 2,048-token contexts, 1.76 -> 1.69 at 512)
+
+// The tile of rank ``rank`` when tiles of one token (tile t: row t) are ordered by their number of partitions, the most first,
+// tiles of equally many by their number; at most 64 tiles.  Every lane of every wave gets the answer.  A radix selection over
+// ballots: some seven scalar instructions a bit.
+__device__ __forceinline__ int tile_of_rank(const AttnBf16Args& a, int rank) {
+  const int lane = threadIdx.x & 63;
+  const int pos = lane < a.num_tiles ? a.positions[lane] : -1;
+  const unsigned key = lane < a.num_tiles ? (unsigned)(pos < 0 ? 0 : pos / ATT_PART + 1) : 0u;
+  unsigned long long left = a.num_tiles >= 64 ? ~0ull : (1ull << a.num_tiles) - 1;
+  const int parts = (a.table_stride * a.page_size + ATT_PART - 1) / ATT_PART + 1;     // no key is larger
+  for (int bit = 31 - __builtin_clz((unsigned)parts); bit >= 0; --bit) {
+    const unsigned long long with = __ballot((key >> bit) & 1u) & left;
+    const int n = __popcll(with);
+    if (rank < n) left = with;
+    else {
+      rank -= n;
+      left &= ~with;
+    }
+  }
+  const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(left >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)left, 0u));
+  const unsigned long long me = __ballot(((left >> lane) & 1ull) != 0 && before == rank);
+  return me != 0 ? (int)__builtin_ctzll(me) : 0;
+}
+
 template <int HD, int W, bool SPLIT>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void attention_decode_kernel(AttnBf16Args a, int pcap, float* __restrict__ scratch,
                                                                   int* __restrict__ counters, int max_parts) {
@@ -1188,18 +1217,42 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
   // Without a window and with the implicit tile list the first partition is partition 0 of sequence blockIdx.x
   // whatever the position says: its pages are asked for beside the position, not after it (the table index is
   // clamped into the row and the pages into the pool, so a sequence shorter than that costs a wasted load).
+  int tile = blockIdx.x, head_item = blockIdx.y;
+  const bool queued = W == DECODE_W_MANY && !SPLIT && gridDim.x * gridDim.y > 512u;
+  if (queued) {
+    // More workgroups than places on the chip (two a compute unit): the longest contexts go first, or one that starts last is
+    // worked on alone.  Eight neighbours of that order run at a time, through the heads, a die each (forward and
+    // backward in turn: no die gets the longest of every eight).  Rows of a step without a tile list are ordered below; a
+    // tile list comes in that order.  32 heads of 64: 43 requests of 97 to 4,000 tokens 210 us -> 128 (688 MB); 64 of 2,048
+    // each, where only the dies matter, 192 -> 180.
+    const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x), per = 8 * (int)gridDim.y, eight = id / per;
+    tile = id / (int)gridDim.y;
+    head_item = id % (int)gridDim.y;
+    if (8 * eight + 8 <= (int)gridDim.x) {
+      tile = 8 * eight + ((eight & 1) ? 7 - (id & 7) : id & 7);
+      head_item = (id % per) >> 3;
+    }
+  }
   const bool early = a.window == 0 && a.chunk == 0 && a.tiles == nullptr;
   PartPages pg_first;
   if (early) {
     gc.r = threadIdx.x & 15;
     gc.g = (threadIdx.x & 63) >> 4;
-    gc.table = a.block_table + (size_t)blockIdx.x * a.table_stride;
+    gc.table = a.block_table + (size_t)tile * a.table_stride;
     load_pages(a, gc, (SPLIT ? (int)blockIdx.z * W : 0) + wave, pg_first);
   }
-  const bool live = group_setup<HD, 1>(a, blockIdx.x, blockIdx.y, gc, tc);   // uniform over the workgroup
+  if (queued && a.tiles == nullptr && a.num_tiles <= 64) {
+    const int ranked = tile_of_rank(a, tile);
+    if (early && ranked != tile) {                 // (contexts of one length are in order: the pages asked for above are theirs)
+      gc.table = a.block_table + (size_t)ranked * a.table_stride;
+      load_pages(a, gc, wave, pg_first);
+    }
+    tile = ranked;
+  }
+  const bool live = group_setup<HD, 1>(a, tile, head_item, gc, tc);   // uniform over the workgroup
   if (!SPLIT && !live) return;
   const int first = gc.kmin / ATT_PART, last = gc.kmax / ATT_PART;
-  const int row = a.tiles != nullptr ? a.tiles[blockIdx.x * 4] : blockIdx.x;
+  const int row = a.tiles != nullptr ? a.tiles[tile * 4] : tile;
   if constexpr (SPLIT) {
     const int item = blockIdx.x * gridDim.y + blockIdx.y;
     float* mine = scratch + (size_t)item * max_parts * a.hpt * CELL;
@@ -1308,12 +1361,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
   }
 }
 
-#define DECODE_W 8
 #define BW_LDS_BYTES (160 * 1024 - 256)   // a compute unit's LDS less the kernels' few static words
-#define DECODE_W_MANY 4          // waves a workgroup where there are two workgroups or more for every compute unit: two of
-                                 // these share a compute unit, and a token's first keys do not wait for a whole
-                                 // generation of eight-wave workgroups before it (16 requests of 32 heads: 2.61 -> 2.52 ms
-                                 // a step at 2,048-token contexts, 1.76 -> 1.69 at 512)
 #define DECODE_MANY 257          // that many workgroups: more than there are compute units
 #define DECODE_MANY_LONG 1024    // heads of 128 or more in a cache laid out for long contexts (more than 80 partitions a
                                  // request): eight waves' loads in flight are worth more there up to this many (64

@@ -54,6 +54,7 @@ def plan_tiles(ctx, tokens_per_tile: int, group_tiles: int = 1) -> AttentionPlan
                 fold.append((r0 + off, min(tokens_per_tile, n - off), i, 0))
             while len(fold) % group_tiles:
                 fold.append((r0, 0, i, 0))
+        split.sort(key=lambda t: -ctx.segments[t[2]].pos0)       # (the longest contexts first: the kernel starts them in this order)
         both = np.asarray(fold + split, np.int32).reshape(-1, 4)
         dev = torch.from_numpy(both).to(ctx.device)
         return AttentionPlan(dev[:len(fold)].contiguous() if fold else None, len(fold),

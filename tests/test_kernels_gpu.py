@@ -798,6 +798,28 @@ def test_attention_prompt_tiles_equal_single_rows(gpu, bf16):
     assert (portion.cpu().double() - ref).abs().max() <= (1.5e-2 if bf16 else 3e-6) * ref.abs().max()
 
 
+@pytest.mark.parametrize("rows,heads,kvh,hd", [(64, 16, 16, 64), (33, 32, 16, 64), (17, 32, 32, 64), (63, 32, 16, 128), (65, 16, 16, 64)])
+def test_decode_attention_of_a_queue_equals_each_row_alone(gpu, rows, heads, kvh, hd):
+    """More workgroups than places: rows are handed out by their contexts' lengths.  Contexts of all lengths, equal ones and
+    padding rows among them (65: more rows than the order covers): every row has the bits of a launch of its own."""
+    page, width = 16, 20
+    g = torch.Generator(device=gpu).manual_seed(rows)
+    pos = torch.randint(0, page * width, (rows,), generator=g, device=gpu, dtype=torch.int32)
+    pos[1], pos[rows // 2], pos[3], pos[4] = -1, -1, pos[5], 319
+    table = torch.arange(rows * width, dtype=torch.int32, device=gpu).view(rows, width)
+    kc, vc = torch.randn(2, rows * width, kvh * page * hd, generator=g, device=gpu).bfloat16()
+    q = torch.randn(rows, heads * hd, generator=g, device=gpu).bfloat16()
+    for window in (0, 100):
+        out = torch.zeros_like(q)
+        ops.attention_bf16(q, pos, table, None, rows, kc, vc, out, heads, kvh, hd, page, window, 0.125, decode=True)
+        for r in range(rows):
+            if pos[r] >= 0:
+                one = torch.zeros_like(q[:1])
+                ops.attention_bf16(q[r:r + 1], pos[r:r + 1].clone(), table[r:r + 1].clone(), None, 1, kc, vc, one, heads, kvh, hd, page, window, 0.125,
+                                   decode=True)
+                assert torch.equal(out[r], one[0]), r
+
+
 @pytest.mark.parametrize("heads,kvh,hd,page", [(2, 2, 64, 16), (6, 2, 64, 64), (4, 1, 128, 16), (3, 1, 128, 32), (17, 1, 128, 64), (2, 2, 64, 8)])
 def test_prompt_attention_of_common_heads_equals_the_decode_kernel(gpu, heads, kvh, hd, page):
     """Portions around the edges of tiles, of a workgroup's eight tiles, of partitions and of the blocks of table entries
