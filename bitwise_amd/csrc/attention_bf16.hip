@@ -1172,6 +1172,7 @@ __device__ __forceinline__ void store_partial(const AttnBf16Args& a, const Group
 }
 
 #define DECODE_W 8               // waves a workgroup of the decode kernel
+#define DECODE_ALONE 2           // rounds of partitions that a workgroup of a split launch takes by itself
 #define DECODE_W_MANY 4          // waves a workgroup where there are two workgroups or more for every compute unit: two of
                                  // these share a compute unit, and a token's first keys do not wait for a whole
                                  // generation of eight-wave workgroups before it (16 requests of 32 heads: 2.61 -> 2.52 ms
@@ -1233,13 +1234,35 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
       head_item = (id % per) >> 3;
     }
   }
+  int z = SPLIT ? (int)blockIdx.z : 0, nz = SPLIT ? (int)gridDim.z : 1;
   const bool early = a.window == 0 && a.chunk == 0 && a.tiles == nullptr;
   PartPages pg_first;
   if (early) {
     gc.r = threadIdx.x & 15;
     gc.g = (threadIdx.x & 63) >> 4;
     gc.table = a.block_table + (size_t)tile * a.table_stride;
-    load_pages(a, gc, (SPLIT ? (int)blockIdx.z * W : 0) + wave, pg_first);
+    load_pages(a, gc, z * W + wave, pg_first);
+  }
+  if (SPLIT && a.tiles == nullptr && a.num_tiles > 1 && a.num_tiles <= 64) {
+    // A captured step's rows past its requests are padding: the rows that are live share all the workgroups (5 requests in
+    // the graph of 8, 8 key heads of 128, 4,500 tokens: 44 us -> 37).
+    const int lane = threadIdx.x & 63;
+    const unsigned long long rows = __ballot(lane < a.num_tiles && a.positions[lane < a.num_tiles ? lane : 0] >= 0);
+    const int live_rows = __popcll(rows), live_items = live_rows * (int)gridDim.y;
+    if (live_items == 0) return;
+    const int id = (int)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x);
+    nz = (int)(gridDim.x * gridDim.y * gridDim.z) / live_items;
+    z = id / live_items;
+    if (z >= nz) return;
+    const int index = id % live_items, nth = index % live_rows;    // (no padding: what blockIdx says)
+    head_item = index / live_rows;
+    const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(rows >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)rows, 0u));
+    const int mine = (int)__builtin_ctzll(__ballot(((rows >> lane) & 1ull) != 0 && before == nth));
+    if (early && (mine != tile || z != (int)blockIdx.z)) {
+      gc.table = a.block_table + (size_t)mine * a.table_stride;
+      load_pages(a, gc, z * W + wave, pg_first);
+    }
+    tile = mine;
   }
   if (queued && a.tiles == nullptr && a.num_tiles <= 64) {
     const int ranked = tile_of_rank(a, tile);
@@ -1254,14 +1277,36 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
   const int first = gc.kmin / ATT_PART, last = gc.kmax / ATT_PART;
   const int row = a.tiles != nullptr ? a.tiles[tile * 4] : tile;
   if constexpr (SPLIT) {
-    const int item = blockIdx.x * gridDim.y + blockIdx.y;
+    // A context of few partitions is one workgroup's, which folds them where it is: the meeting in device memory costs
+    // more than a second round of loads (331 tokens of one request, 32 heads of 64: 9.3 us -> 7.3).
+    const int count = live ? last - first + 1 : 0;
+    if (count <= DECODE_ALONE * W && count <= pcap) {
+      if (z != 0 || !live) return;
+      for (int part = first + wave; part <= last; part += W) {
+        PartPages pg;
+        KFrags<HD> kf;
+        VFrags<HD> vf;
+        if (early && part == wave) pg = pg_first;
+        else load_pages(a, gc, part, pg);
+        load_keys<HD>(a, gc, part, pg, kf);
+        load_values<HD>(a, gc, pg, vf);
+        float m_p, l_p;
+        f32x4 o_p[NT];
+        partition_partial<HD>(a, gc, tc[0], part, pg, kf, vf, m_p, l_p, o_p);
+        store_partial<HD, false>(a, gc, parts + (size_t)(part - first) * a.hpt * CELL, m_p, l_p, o_p);
+      }
+      __syncthreads();
+      decode_fold_pass<HD, W>(a, gc, lds, count, 0, true, row);
+      return;
+    }
+    const int item = tile * gridDim.y + head_item;
     float* mine = scratch + (size_t)item * max_parts * a.hpt * CELL;
     if (live) {
       PartPages pg;
       KFrags<HD> kf;
       VFrags<HD> vf;
-      for (int part = first + blockIdx.z * W + wave; part <= last; part += W * gridDim.z) {
-        if (early && part == (int)blockIdx.z * W + wave) pg = pg_first;
+      for (int part = first + z * W + wave; part <= last; part += W * nz) {
+        if (early && part == z * W + wave) pg = pg_first;
         else load_pages(a, gc, part, pg);
         load_keys<HD>(a, gc, part, pg, kf);
         load_values<HD>(a, gc, pg, vf);
@@ -1288,7 +1333,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     // after that barrier.
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
     __syncthreads();
-    if (threadIdx.x == 0) is_last = atomicAdd(&counters[item], 1) == (int)gridDim.z - 1;
+    if (threadIdx.x == 0) is_last = atomicAdd(&counters[item], 1) == nz - 1;
     __syncthreads();
     if (!is_last) return;
     if (threadIdx.x == 0) counters[item] = 0;

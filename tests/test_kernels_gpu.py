@@ -820,6 +820,33 @@ def test_decode_attention_of_a_queue_equals_each_row_alone(gpu, rows, heads, kvh
                 assert torch.equal(out[r], one[0]), r
 
 
+@pytest.mark.parametrize("rows,heads,kvh,hd", [(1, 4, 4, 64), (8, 2, 1, 64), (8, 32, 8, 128), (4, 6, 3, 32), (64, 2, 2, 16)])
+def test_split_decode_attention_with_padding_and_short_contexts(gpu, rows, heads, kvh, hd):
+    """Launches of few tiles, split over workgroups that share the live rows' work: padding anywhere, all padding, contexts
+    around what one workgroup takes by itself; the bits of launches that are not split, and the counters back at zero."""
+    page, width = 16, 150
+    g = torch.Generator(device=gpu).manual_seed(rows + heads)
+    table = torch.randperm(rows * width, generator=g, device=gpu).int().view(rows, width)
+    kc, vc = torch.randn(2, rows * width, kvh * page * hd, generator=g, device=gpu).bfloat16()
+    q = torch.randn(rows, heads * hd, generator=g, device=gpu).bfloat16()
+    floats, counters = ops.attention_decode_scratch(rows, heads, kvh, hd, width, page)
+    assert floats and counters
+    scratch = (torch.full((floats,), float("nan"), device=gpu), torch.zeros(counters, dtype=torch.int32, device=gpu))
+    contexts = [0, 63, 64, 511, 512, 1023, 1024, 1100, 2390]
+    for trial in range(6):
+        pos = torch.tensor([contexts[(3 * i + trial) % len(contexts)] for i in range(rows)], dtype=torch.int32)
+        if rows > 1:
+            pos[torch.randperm(rows)[: trial * rows // 6]] = -1
+        if trial == 5:
+            pos[:] = -1
+        pos = pos.to(gpu)
+        out, want = torch.zeros_like(q), torch.zeros_like(q)
+        ops.attention_bf16(q, pos, table, None, rows, kc, vc, out, heads, kvh, hd, page, 0, 0.125, decode=True, scratch=scratch)
+        ops.attention_bf16(q, pos, table, None, rows, kc, vc, want, heads, kvh, hd, page, 0, 0.125, decode=True)
+        assert torch.equal(out, want), trial
+        assert not scratch[1].any()
+
+
 @pytest.mark.parametrize("heads,kvh,hd,page", [(2, 2, 64, 16), (6, 2, 64, 64), (4, 1, 128, 16), (3, 1, 128, 32), (17, 1, 128, 64), (2, 2, 64, 8)])
 def test_prompt_attention_of_common_heads_equals_the_decode_kernel(gpu, heads, kvh, hd, page):
     """Portions around the edges of tiles, of a workgroup's eight tiles, of partitions and of the blocks of table entries
