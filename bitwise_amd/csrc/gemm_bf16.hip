@@ -50,7 +50,7 @@
 #include "layout.h"        // the epilogues' numbers, GEMM_SEG, MidShape and the LDS layout of the rows normalised in the kernel
 
 // What the rotary epilogue of the stacked q|k|v product needs: the statements of
-// rope_kvwrite_bf16_kernel on the 32-bit products while they are still in registers.
+// rope_kvwrite_kernel on the 32-bit products while they are still in registers.
 struct QkvRopeArgs {
   const int32_t* positions;    // [rows]; negative = padding row
   const int32_t* row_seq;      // [rows] -> row of the block table

@@ -347,7 +347,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // groups of banks.  LDS is a ring of five slots of 32 KB, filled in the order A0 B0 A1 B1 A2 ... (a
 // step's tile of x, then its tile of W): while the waves work on step s, B(s+1) and A(s+2) are in
 // flight and A(s+1) has landed or is landing, so the memory pipe never runs dry at a step's edge;
-// one barrier a step.  Rows past M or N lie outside the buffer descriptors.  K a multiple of 64 and
+// one barrier a step.  A step's eight loads of a wave are spread over it, one in front of every eight matrix
+// instructions: a compute unit's path to LDS takes some 16 clocks a load, so 64 of them at the barrier held all waves, and
+// with them the matrix cores, for up to half a step (2,048 rows: gate|up of 8192 x 2048 121 to 130 us -> 116, q|k|v with its
+// rotary epilogue 66 -> 60, the down projection of 2048 x 8192 in segments 81 -> 77).  Rows past M or N lie outside the buffer descriptors.  K a multiple of 64 and
 // one segment; for products with enough tiles to go round.
 #define BIG_BM 256
 #define BIG_SLOT (32 * 1024)
@@ -394,18 +397,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     voff_b[t] = ((b_row0 + 8 * t + lrow) * K + 8 * chunk) * 2;
   }
   typedef __attribute__((address_space(3))) void* lds_ptr;
-  // load number n of the ring: A of step n / 2 (n even) or B of it (n odd), into slot n % 5
-  auto issue_a = [&](int step) {
-    unsigned char* dst = big_lds + ((2 * step) % BIG_SLOTS) * BIG_SLOT + (4 * wave) * 1024;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (lds_ptr)(dst + t * 1024), 16, voff_a[t], k_base * 2 + step * 128, 0, 0);
+  const int steps = gridDim.y > 1 ? ((K - k_base) < GEMM_SEG ? K - k_base : GEMM_SEG) / 64 : K / 64;
+  // load number n of the ring: A of step n / 2 (n even) or B of it (n odd), into slot n % 5; quarter t of a wave's share (past
+  // K: outside the descriptors, no traffic, into slots that nobody reads any more)
+  auto issue_a = [&](int step, int t) {
+    unsigned char* dst = big_lds + ((2 * step) % BIG_SLOTS) * BIG_SLOT + (4 * wave + t) * 1024;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (lds_ptr)dst, 16, step < steps ? voff_a[t] : 0x7ffffff0, k_base * 2 + step * 128, 0, 0);
   };
-  auto issue_b = [&](int step) {
-    unsigned char* dst = big_lds + ((2 * step + 1) % BIG_SLOTS) * BIG_SLOT + (4 * wave) * 1024;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, (lds_ptr)(dst + t * 1024), 16, voff_b[t], k_base * 2 + step * 128, 0, 0);
+  auto issue_b = [&](int step, int t) {
+    unsigned char* dst = big_lds + ((2 * step + 1) % BIG_SLOTS) * BIG_SLOT + (4 * wave + t) * 1024;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, (lds_ptr)dst, 16, step < steps ? voff_b[t] : 0x7ffffff0, k_base * 2 + step * 128, 0, 0);
   };
 
   f32x4 acc[8][4];
@@ -423,20 +424,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int a_frag = (8 * wy) * 2048, b_frag = (GLU ? 2 * wx : 4 * wx) * 2048;
   auto b_off = [&](int j) { return GLU ? ((j & 1) + 8 * (j >> 1)) * 2048 : j * 2048; };
 
-  const int steps = gridDim.y > 1 ? ((K - k_base) < GEMM_SEG ? K - k_base : GEMM_SEG) / 64 : K / 64;
-  issue_a(0);
-  issue_b(0);
-  if (steps > 1) issue_a(1);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) issue_a(0, t);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) issue_b(0, t);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) issue_a(1, t);
   for (int step = 0; step < steps; ++step) {
     // A(step) and B(step) have landed (only A(step + 1), the wave's last four loads, may still be in
     // flight), for every wave; and every wave is done with the slots of the step before, which the
     // next loads overwrite
-    if (step + 1 < steps) __builtin_amdgcn_s_waitcnt(BIG_WAIT_BUT_4);
-    else __builtin_amdgcn_s_waitcnt(BIG_WAIT_ALL);
+    __builtin_amdgcn_s_waitcnt(BIG_WAIT_BUT_4);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (step + 1 < steps) issue_b(step + 1);
-    if (step + 2 < steps) issue_a(step + 2);
     const unsigned char* a_slot = big_lds + ((2 * step) % BIG_SLOTS) * BIG_SLOT + a_frag;
     const unsigned char* b_slot = big_lds + ((2 * step + 1) % BIG_SLOTS) * BIG_SLOT + b_frag;
     __builtin_amdgcn_sched_barrier(0);
@@ -464,42 +464,39 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     };
     read_b(0);
     read_a(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
       for (int pair = 0; pair < 4; ++pair) {
+        if (kk == 0) issue_b(step + 1, pair);
+        else issue_a(step + 2, pair);
+        __builtin_amdgcn_sched_barrier(0);
         if (pair < 3) read_a(kk, pair + 1);
         else if (kk == 0) {
           read_b(1);
           read_a(1, 0);
         }
         multiply(kk, pair);
-      }
-    __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-#pragma unroll
-      for (int pair = 0; pair < 3; ++pair) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-      }
-      if (kk == 0) {
-#pragma unroll
-        for (int t = 0; t < 6; ++t) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (pair < 3) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+        } else if (kk == 0) {
+#pragma unroll
+          for (int t = 0; t < 6; ++t) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          }
+          __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-      } else {
-        __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+        __builtin_amdgcn_sched_barrier(0);
       }
-    }
-    __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
   }
+  __builtin_amdgcn_s_waitcnt(BIG_WAIT_ALL);                            // the padding loads too
   if constexpr (EPI == EPI_QKV_ROPE) {
     // What the rows of the tile need from memory is fetched once for the workgroup, into the ring (free now), not
     // by every lane for each of its rows: position and page of each of the 256 rows (a thread a row), then the
@@ -811,7 +808,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // a step pulls 48 KB for twice the 128 x 128 tile's products (which pulls 32), and a wave's 64 accumulators leave room
 // for the sums of the segments before, so that a K of several segments, which the 256 x 256 kernel does not take,
 // runs on these where there are enough of them.  Three stages of 48 KB (x 16 KB | W 32 KB); a wave issues six loads a
-// stage.  Plain, residual, SwiGLU and (one segment, heads of 64) rotary epilogues; segments joined left to right in registers (a residual add's chain
+// stage, one in front of every four matrix instructions of the first three quarters of a step (as in the big-tile kernel; all
+// of them at the barrier: gate|up of 14336 x 4096 at 2,048 rows 527 us -> 512, down of 4096 x 14336 263 -> 251).  Plain, residual, SwiGLU and (one segment, heads of 64) rotary epilogues; segments joined left to right in registers (a residual add's chain
 // starts at the residual, which is read when the first segment ends).  K a multiple of 64.
 #define T256_STAGE (48 * 1024)
 #define T256_STAGES 3
@@ -858,17 +856,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   typedef __attribute__((address_space(3))) void* lds_ptr;
   const int steps = K / 64;
-  auto issue = [&](int step) {
+  auto issue = [&](int step, int n) {                                   // load n of a wave's six: two of x, four of W
     unsigned char* dst = t256_lds + (step % T256_STAGES) * T256_STAGE;
     const bool real = step < steps;                                     // scalar; past K: outside the descriptors
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (lds_ptr)(dst + (2 * wave + t) * 1024), 16, real ? voff_a[t] : 0x7ffffff0,
+    if (n < 2)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (lds_ptr)(dst + (2 * wave + n) * 1024), 16, real ? voff_a[n] : 0x7ffffff0,
                                                k_base * 2 + step * 128, 0, 0);
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, (lds_ptr)(dst + 16 * 1024 + (4 * wave + t) * 1024), 16,
-                                               real ? voff_b[t] : 0x7ffffff0, k_base * 2 + step * 128, 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, (lds_ptr)(dst + 16 * 1024 + (4 * wave + n - 2) * 1024), 16,
+                                               real ? voff_b[n - 2] : 0x7ffffff0, k_base * 2 + step * 128, 0, 0);
   };
   f32x4 acc[4][4], tot[4][4];
 #pragma unroll
@@ -888,37 +884,47 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int b_frag = 16 * 1024 + (GLU ? 2 * wx : 4 * wx) * 2048;
   auto b_off = [&](int j) { return GLU ? ((j & 1) + 8 * (j >> 1)) * 2048 : j * 2048; };
 #pragma unroll
-  for (int st = 0; st < T256_STAGES - 1; ++st) issue(st);
+  for (int st = 0; st < T256_STAGES - 1; ++st)
+#pragma unroll
+    for (int n = 0; n < 6; ++n) issue(st, n);
   for (int step = 0; step < steps; ++step) {
     __builtin_amdgcn_s_waitcnt(vmcnt_only(6 * (T256_STAGES - 2)));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    issue(step + T256_STAGES - 1);                                      // into the stage worked on a step ago
     const unsigned char* stage = t256_lds + (step % T256_STAGES) * T256_STAGE;
     __builtin_amdgcn_sched_barrier(0);
     // 16 operand reads and 32 matrix instructions a step, the second half's reads under the first half's products
     u32x4 fa[2][4], fb[2][4];
+    // (and the loads of the step after next, into the stage worked on a step ago, spread over it: see the big-tile kernel)
+    auto read_b = [&](int kk, int j) { fb[kk][j] = *reinterpret_cast<const u32x4*>(stage + b_frag + b_off(j) + slot_off[kk]); };
+    auto read_a = [&](int kk, int i) { fa[kk][i] = *reinterpret_cast<const u32x4*>(stage + a_frag + i * 2048 + slot_off[kk]); };
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
+    for (int j = 0; j < 4; ++j) read_b(0, j);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) fb[kk][j] = *reinterpret_cast<const u32x4*>(stage + b_frag + b_off(j) + slot_off[kk]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) fa[kk][i] = *reinterpret_cast<const u32x4*>(stage + a_frag + i * 2048 + slot_off[kk]);
-    }
+    for (int i = 0; i < 4; ++i) read_a(0, i);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i) {
+        if (4 * kk + i < 6) issue(step + T256_STAGES - 1, 4 * kk + i);
+        __builtin_amdgcn_sched_barrier(0);
+        if (kk == 0) {
+          read_b(1, i);
+          read_a(1, i);
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(fa[kk][i]), as_bf16x8(fb[kk][j]), acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+        if (kk == 0) {
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+          for (int t = 0; t < 2; ++t) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
     const int kn = (step + 1) * 64;
