@@ -25,7 +25,8 @@
 // Work shapes: the fold kernel (prompt portions) gives a workgroup of up to 8 waves as many
 // tiles of one sequence and kv head, a tile a wave; the threads together stage each partition's
 // keys and values once in LDS (the next partition's loads fly meanwhile), and every wave whose
-// queries see the partition folds it into its own state.  The decode kernel (tiles of one
+// queries see the partition folds it into its own state; heads of 64 and 128 have a fold kernel
+// of their own with the same statements (attention_fold2_kernel).  The decode kernel (tiles of one
 // token) gives a workgroup one tile and each of its 8 waves one partition at a time, operands
 // straight from the pages into registers; the partials meet in LDS and are folded there in
 // partition order.
