@@ -1173,7 +1173,14 @@ __device__ __forceinline__ void store_partial(const AttnBf16Args& a, const Group
 }
 
 #define DECODE_W 8               // waves a workgroup of the decode kernel
-#define DECODE_ALONE 2           // rounds of partitions that a workgroup of a split launch takes by itself
+// Partitions that a workgroup of a split launch takes by itself: the meeting in device memory costs some 2 us whatever the
+// head, a second round of loads behind the first as much as its bytes, so it grows with the head.  Up to a round it always pays
+// (300 keys, 1 to 16 rows: 32 heads of 64 8.5 us -> 6.4, 8 heads of 128 10.4 -> 8.6, 4 of 256 18.6 -> 16.5); 16 partitions
+// met -> alone: heads of 32 0.89 to 1.02 of the time, of 64 1.04 to 1.13, of 128 1.20 to 1.37; 10: of 64 0.88 to 1.01, of 128 0.93
+// to 1.05; 9: of 128 0.84 to 1.02, of 192 and 256 1.18 to 1.30.
+constexpr int decode_alone(int head_dim) {
+  return DECODE_W + (head_dim <= 32 ? 8 : head_dim <= 48 ? 4 : head_dim <= 64 ? 2 : head_dim <= 128 ? 1 : 0);
+}
 #define DECODE_W_MANY 4          // waves a workgroup where there are two workgroups or more for every compute unit: two of
                                  // these share a compute unit, and a token's first keys do not wait for a whole
                                  // generation of eight-wave workgroups before it (16 requests of 32 heads: 2.61 -> 2.52 ms
@@ -1278,10 +1285,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
   const int first = gc.kmin / ATT_PART, last = gc.kmax / ATT_PART;
   const int row = a.tiles != nullptr ? a.tiles[tile * 4] : tile;
   if constexpr (SPLIT) {
-    // A context of few partitions is one workgroup's, which folds them where it is: the meeting in device memory costs
-    // more than a second round of loads (331 tokens of one request, 32 heads of 64: 9.3 us -> 7.3).
+    // A context of few partitions is one workgroup's, which folds them where it is (331 tokens of one request, 32 heads of
+    // 64: 9.3 us -> 7.3).
     const int count = live ? last - first + 1 : 0;
-    if (count <= DECODE_ALONE * W && count <= pcap) {
+    if (count <= decode_alone(HD) && count <= pcap) {
       if (z != 0 || !live) return;
       for (int part = first + wave; part <= last; part += W) {
         PartPages pg;

@@ -847,6 +847,27 @@ def test_split_decode_attention_with_padding_and_short_contexts(gpu, rows, heads
         assert not scratch[1].any()
 
 
+@pytest.mark.parametrize("heads,kvh,hd,line", [(4, 2, 32, 16), (4, 2, 48, 12), (4, 4, 64, 10), (8, 2, 128, 9), (4, 2, 192, 8), (32, 2, 256, 8)])
+def test_split_decode_attention_where_one_workgroup_takes_a_context(gpu, heads, kvh, hd, line):
+    """Contexts of ``line`` partitions (folded by one workgroup), one fewer and one more (met in device memory), their last
+    partition full or of one key, side by side in a launch: the bits of a launch that is not split."""
+    page, width, rows = 16, 120, 6
+    g = torch.Generator(device=gpu).manual_seed(hd)
+    table = torch.randperm(rows * width, generator=g, device=gpu).int().view(rows, width)
+    kc, vc = torch.randn(2, rows * width, kvh * page * hd, generator=g, device=gpu).bfloat16()
+    q = torch.randn(rows, heads * hd, generator=g, device=gpu).bfloat16()
+    floats, counters = ops.attention_decode_scratch(rows, heads, kvh, hd, width, page)
+    assert floats and counters
+    scratch = (torch.full((floats,), float("nan"), device=gpu), torch.zeros(counters, dtype=torch.int32, device=gpu))
+    pos = torch.tensor([64 * n + last for n in (line - 2, line - 1, line) for last in (0, 63)], dtype=torch.int32, device=gpu)
+    for window in (0, 64 * (line - 1)):
+        out, want = torch.zeros_like(q), torch.zeros_like(q)
+        ops.attention_bf16(q, pos, table, None, rows, kc, vc, out, heads, kvh, hd, page, window, 0.125, decode=True, scratch=scratch)
+        ops.attention_bf16(q, pos, table, None, rows, kc, vc, want, heads, kvh, hd, page, window, 0.125, decode=True)
+        assert torch.equal(out, want), window
+        assert not scratch[1].any()
+
+
 @pytest.mark.parametrize("heads,kvh,hd,page", [(2, 2, 64, 16), (6, 2, 64, 64), (4, 1, 128, 16), (3, 1, 128, 32), (17, 1, 128, 64), (2, 2, 64, 8)])
 def test_prompt_attention_of_common_heads_equals_the_decode_kernel(gpu, heads, kvh, hd, page):
     """Portions around the edges of tiles, of a workgroup's eight tiles, of partitions and of the blocks of table entries
