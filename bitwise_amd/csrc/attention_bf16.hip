@@ -72,9 +72,12 @@ struct TileCtx {
   u32x4 qf[KS];
 };
 
+#define POS_UNREAD (-0x7fffffff - 1)       // group_setup: the position is still to be read
+
+// ``known_pos``: the position of a tile of one row, where the caller has it.
 template <int HD, int QT>
 __device__ __forceinline__ bool group_setup(const AttnBf16Args& a, int first_tile, int head_item, GroupCtx& gc,
-                                            TileCtx<HD> (&tc)[QT]) {
+                                            TileCtx<HD> (&tc)[QT], int known_pos = POS_UNREAD) {
   gc.lane = threadIdx.x & 63;
   gc.r = gc.lane & 15;
   gc.g = gc.lane >> 4;
@@ -99,7 +102,8 @@ __device__ __forceinline__ bool group_setup(const AttnBf16Args& a, int first_til
     const bool ok = col_in && tok < ntok;
     tc[t].row_c = row0 + (ok ? tok : 0);
     tc[t].head_c = gc.kvh * group + gc.sub * a.hpt + (ok ? hh : 0);
-    tc[t].pos_c = ok ? a.positions[tc[t].row_c] : -1;
+    tc[t].pos_c = ok ? known_pos : -1;
+    if (known_pos == POS_UNREAD && ok) tc[t].pos_c = a.positions[tc[t].row_c];      // (scalar, or known at compile time)
     if (a.chunk > 0) tc[t].lo_c = tc[t].pos_c > 0 ? tc[t].pos_c - tc[t].pos_c % a.chunk : 0;
     else tc[t].lo_c = (a.window > 0 && tc[t].pos_c - a.window + 1 > 0) ? tc[t].pos_c - a.window + 1 : 0;
     kmax = max(kmax, tc[t].pos_c);
@@ -1244,6 +1248,12 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
   }
   int z = SPLIT ? (int)blockIdx.z : 0, nz = SPLIT ? (int)gridDim.z : 1;
   const bool early = a.window == 0 && a.chunk == 0 && a.tiles == nullptr;
+  // Split launches hand their workgroups out by the rows' positions: row l's in lane l, one load for that and for the tile's own
+  // (8 rows of 1,100 keys, 8 heads of 128, no padding: 14.5 us with a load behind the other, 13.7 so).  Without a split the
+  // branch on a known position costs more than the second load (128 rows of up to 300 keys 51 us -> 53).
+  const bool by_position = SPLIT && a.tiles == nullptr && a.num_tiles <= 64;
+  int row_pos = -1, known_pos = POS_UNREAD;
+  if (by_position) row_pos = a.positions[min((int)threadIdx.x & 63, a.num_tiles - 1)];
   PartPages pg_first;
   if (early) {
     gc.r = threadIdx.x & 15;
@@ -1251,26 +1261,30 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     gc.table = a.block_table + (size_t)tile * a.table_stride;
     load_pages(a, gc, z * W + wave, pg_first);
   }
-  if (SPLIT && a.tiles == nullptr && a.num_tiles > 1 && a.num_tiles <= 64) {
+  if (by_position) {
     // A captured step's rows past its requests are padding: the rows that are live share all the workgroups (5 requests in
     // the graph of 8, 8 key heads of 128, 4,500 tokens: 44 us -> 37).
     const int lane = threadIdx.x & 63;
-    const unsigned long long rows = __ballot(lane < a.num_tiles && a.positions[lane < a.num_tiles ? lane : 0] >= 0);
-    const int live_rows = __popcll(rows), live_items = live_rows * (int)gridDim.y;
-    if (live_items == 0) return;
-    const int id = (int)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x);
-    nz = (int)(gridDim.x * gridDim.y * gridDim.z) / live_items;
-    z = id / live_items;
-    if (z >= nz) return;
-    const int index = id % live_items, nth = index % live_rows;    // (no padding: what blockIdx says)
-    head_item = index / live_rows;
-    const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(rows >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)rows, 0u));
-    const int mine = (int)__builtin_ctzll(__ballot(((rows >> lane) & 1ull) != 0 && before == nth));
-    if (early && (mine != tile || z != (int)blockIdx.z)) {
-      gc.table = a.block_table + (size_t)mine * a.table_stride;
-      load_pages(a, gc, z * W + wave, pg_first);
+    const unsigned long long rows = __ballot(lane < a.num_tiles && row_pos >= 0);
+    const int live_rows = __popcll(rows);
+    if (live_rows < a.num_tiles) {                 // (without padding: what blockIdx says)
+      const int live_items = live_rows * (int)gridDim.y;
+      if (live_items == 0) return;
+      const int id = (int)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x);
+      nz = (int)(gridDim.x * gridDim.y * gridDim.z) / live_items;
+      z = id / live_items;
+      if (z >= nz) return;
+      const int index = id % live_items, nth = index % live_rows;
+      head_item = index / live_rows;
+      const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(rows >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)rows, 0u));
+      const int mine = (int)__builtin_ctzll(__ballot(((rows >> lane) & 1ull) != 0 && before == nth));
+      if (early && (mine != tile || z != (int)blockIdx.z)) {
+        gc.table = a.block_table + (size_t)mine * a.table_stride;
+        load_pages(a, gc, z * W + wave, pg_first);
+      }
+      tile = mine;
     }
-    tile = mine;
+    known_pos = __builtin_amdgcn_readlane(row_pos, tile);
   }
   if (queued && a.tiles == nullptr && a.num_tiles <= 64) {
     const int ranked = tile_of_rank(a, tile);
@@ -1280,7 +1294,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
     tile = ranked;
   }
-  const bool live = group_setup<HD, 1>(a, tile, head_item, gc, tc);   // uniform over the workgroup
+  const bool live = group_setup<HD, 1>(a, tile, head_item, gc, tc, known_pos);   // uniform over the workgroup
   if (!SPLIT && !live) return;
   const int first = gc.kmin / ATT_PART, last = gc.kmax / ATT_PART;
   const int row = a.tiles != nullptr ? a.tiles[tile * 4] : tile;
