@@ -391,8 +391,10 @@ __global__ __launch_bounds__(64 * RW) void linear_recurrence_kernel(RecurArgs a)
   constexpr bool HOIST = GATES && PHASE == 0;
   static_assert(!HOIST || RC <= 64, "a token a lane");
   // tokens of a whole chunk that leave together: one division and one store for as many as a column has lanes
-  // (a column of fewer lanes: every group's own)
-  constexpr bool GATHER = SPLIT >= 2 * TU;
+  // (a column of fewer lanes: every group's own).  2,048 tokens of 128 channels: 7 % less with a constant decay, a step size or
+  // a delta memory, 3 % with a bonus.  Not where it takes the registers of a second wave a SIMD (a step size or a
+  // delta memory of 256 channels: 239 -> 261 and 293; 8 portions of 5 tokens, 8 heads of 256 x 256, 11.4 us -> 17.6).
+  constexpr bool GATHER = SPLIT >= 2 * TU && !((STEP || DELTA) && DPAD == 256);
   constexpr int RUN = GATHER ? (SPLIT < RC ? SPLIT : RC) : 2 * TU;
   static_assert(PHASE != 0 || RC % RUN == 0, "runs fill a chunk");
   __shared__ float nqs[HOIST ? RC : 1], ems[HOIST ? RC : 1];
