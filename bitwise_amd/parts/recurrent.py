@@ -36,6 +36,12 @@ from .linear import Linear
 
 
 FEW_SEQ_ROWS = 4         # steps whose requests bring up to so many rows each run the recurrence's kernel for decoding
+# A launch that makes the decays of all rows first costs some 1.7 us and takes the exponentials and the logarithm out of the walk,
+# where every workgroup of a head repeats them.  One portion gets that back from about 1,200 rows x channels on (microseconds,
+# without -> with; 32 heads of 64: 16 rows 6.8 -> 7.2, 24 rows 9.5 -> 8.4; 8 of 128: 8 rows 6.3 -> 6.7, 12 rows 8.6 -> 7.5; 16 of 32: 32 rows 8.1
+# -> 8.7, 48 rows 12.3 -> 11.0; 16 of 16: 64 rows 11.6 -> 12.0, 96 rows 16.2 -> 15.5), heads of 64 channels and more sooner where
+# the step's requests together fill the chip (8 x 5 rows: 32 heads of 64 10.7 -> 9.3, 8 of 128 20.4 -> 15.8).
+DECAYS_AHEAD_CHAIN, DECAYS_AHEAD_COLUMNS = 1200, 40960
 SCAN_CHUNK = 32          # rows of a chunk of a long portion
 SCAN_MIN_ROWS = 96       # portions from this many rows on run in three passes over chunks (shorter ones are walked whole),
                          # where the engine allows logits to depend on the cut in their last bits (Workspace.exact_cuts False)
@@ -166,6 +172,14 @@ class _MatrixMemoryMixer(Mixer):
             self.o.store(ctx.ws, act, target, ctx.rows)
 
 
+def decays_ahead(longest: int, rows: int, heads: int, dim: int, vdim: int) -> bool:
+    """Whether a step of ``rows`` rows, up to ``longest`` a request, makes a per-channel memory's decays in a launch of their own.
+    (Every portion long enough for passes over chunks does: SCAN_MIN_ROWS * 16 is past the line.)"""
+    if longest <= FEW_SEQ_ROWS:
+        return False
+    return longest * max(dim, 16) >= DECAYS_AHEAD_CHAIN or (dim >= 64 and rows * heads * vdim >= DECAYS_AHEAD_COLUMNS)
+
+
 @register_mixer("gla")
 class GatedLinearAttention(_MatrixMemoryMixer):
     """params as the base, plus tau and rank (the inner size of the decay's low-rank projection).
@@ -210,13 +224,12 @@ class GatedLinearAttention(_MatrixMemoryMixer):
         z = ws.buffer("gla_decay_logits", self.heads * self.dim, torch.float32)
         self.a2.store(ws, low, z, rows)
         raw = ws.buffer("recur_out", self.heads * self.vdim, torch.float32)
-        # a step of a few rows a request makes the decays where it uses them; in longer ones every workgroup of a head would
         # (the same function either way: the same bits)
-        if max_seq_rows(ctx) <= FEW_SEQ_ROWS:
-            self._recur(ctx, call, y, z, 0, 0, self.a2_bias, None, 1.0 / self.tau, raw)
-        else:
+        if decays_ahead(max_seq_rows(ctx), rows, self.heads, self.dim, self.vdim):
             ops.decay_rows(z, self.a2_bias, 1.0 / self.tau, rows)
             self._recur(ctx, call, y, z, 0, 0, None, None, 1.0 / self.tau, raw, mode=ops.RECUR_DECAY_GIVEN)
+        else:
+            self._recur(ctx, call, y, z, 0, 0, self.a2_bias, None, 1.0 / self.tau, raw)
         self._finish(ctx, y, raw, residual)
 
 

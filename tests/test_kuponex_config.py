@@ -88,3 +88,13 @@ def test_plain_recurrences_equal_their_unrolled_sums():
     assert torch.allclose(pk.norm_around_zero(x, torch.zeros(32, dtype=torch.float64), 0.0).pow(2).mean(-1), torch.ones(2, dtype=torch.float64))
     lg = pk.forward(cfg, w, [1, 2, 3, 4, 5])
     assert lg.shape == (5, 53) and torch.allclose(pk.forward(cfg, w, [1, 2, 3])[-1], lg[2])     # causal
+
+
+def test_decays_get_a_launch_of_their_own_where_it_pays():
+    """Steps timed both ways (longest portion, rows, heads, channels, columns): the launch only where it was the faster one, never
+    for single tokens, and always for portions that run in passes over chunks."""
+    from bitwise_amd.parts.recurrent import SCAN_MIN_ROWS, decays_ahead
+    slower = [(5, 5, 16, 16, 64), (64, 512, 16, 16, 64), (32, 256, 16, 32, 64), (16, 16, 32, 64, 64), (5, 5, 8, 128, 256), (1, 64, 32, 64, 64)]
+    faster = [(96, 96, 16, 16, 64), (48, 48, 16, 32, 64), (24, 24, 32, 64, 64), (5, 40, 32, 64, 64), (12, 12, 8, 128, 256), (5, 40, 8, 128, 128), (5, 5, 8, 256, 256)]
+    assert not any(decays_ahead(*s) for s in slower) and all(decays_ahead(*s) for s in faster)
+    assert all(decays_ahead(SCAN_MIN_ROWS, SCAN_MIN_ROWS, 1, dim, 1) for dim in (1, 4, 16, 256))

@@ -441,3 +441,50 @@ def test_memory_walked_in_chunks_equals_token_by_token(gpu, dim, vdim, gated):
             run(single, out_s, [min(t, counts[0] - 1), int(t < counts[0]), counts[0] + min(t, counts[1] - 1), int(t < counts[1])], True, False)
         assert torch.equal(out_w, out_s), counts
         assert torch.equal(whole, single), counts
+
+
+@pytest.mark.parametrize("dim,vdim", [(12, 20), (64, 40), (100, 48)])
+def test_decays_made_ahead_equal_decays_made_in_the_walk(gpu, dim, vdim):
+    """One memory with a decay per channel over portions of 5, 33 and 100 tokens: decays handed over and decays made in the walk leave
+    the same bits, and passes over the chunks of the portion of 100 stay within the rounding of their sums."""
+    from bitwise_amd.csrc import ops
+    heads, dev, counts, chunk = 2, gpu, (5, 33, 100), 32
+    rows, hd, hv = sum(counts), heads * dim, heads * vdim
+    g = torch.Generator(device=dev).manual_seed(dim)
+    proj = torch.randn(rows, 2 * hd + hv, generator=g, device=dev)
+    logits, bias = 2.0 * torch.randn(rows, hd, generator=g, device=dev), torch.randn(hd, generator=g, device=dev)
+    start = 0.1 * torch.randn(3, hd * vdim, generator=g, device=dev)
+    dev32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    slots, positions, first = dev32([2, 0, 1]), dev32([0] * rows), [0, 5, 38]
+    given = logits.clone()
+    ops.decay_rows(given, bias, 1.0 / 16.0, rows)
+
+    def run(mode, gate, b, counts, scan=None):
+        state, out = start.clone(), torch.zeros(rows, hv, device=dev)
+        seq_rows = dev32([x for f, n in zip(first, counts) for x in (f, n)])
+        ops.linear_recurrence(mode, proj, 0, hd, 2 * hd, gate, 0, 0, b, None, 1.0 / 16.0, dim ** -0.5, state, out, seq_rows, slots, positions, 3,
+                              heads, dim, vdim, scan=scan)
+        return out, state
+
+    out, state = run(ops.RECUR_DECAY_GIVEN, given, None, counts)
+    out_w, state_w = run(ops.RECUR_DECAY_PER_CHANNEL, logits, bias, counts)
+    assert torch.equal(out, out_w) and torch.equal(state, state_w)
+    chunks = [(38 + c, min(chunk, 100 - c), 2, int(c + chunk >= 100)) for c in range(0, 100, chunk)]
+    rec = len(chunks) * heads * ops.recurrence_record(dim, vdim)
+    scan = (dev32(chunks), len(chunks), dev32([2, 0, len(chunks)]), 1, torch.zeros(rec, device=dev), torch.zeros(rec, device=dev))
+    out_s, state_s = run(ops.RECUR_DECAY_GIVEN, given, None, (5, 33, 0), scan)
+    assert torch.equal(out_s[:38], out[:38]) and torch.equal(state_s[[0, 2]], state[[0, 2]])
+    # the portion of 100 in 64 bits, beside the sums of the terms' sizes: every output and state element of either order is
+    # a sum of at most 100 terms a channel, each through up to 100 + 4 products (an output: dim of them)
+    p, a = proj[38:].double(), given[38:].double().view(100, heads, dim, 1)
+    q, k, v = p[:, :hd].view(100, heads, dim, 1) * dim ** -0.5, p[:, hd:2 * hd].view(100, heads, dim, 1), p[:, 2 * hd:].view(100, heads, 1, vdim)
+    S = start[1].double().view(heads, vdim, dim).transpose(1, 2)
+    size = S.abs()
+    for t in range(100):
+        S, size = a[t] * S + k[t] * v[t], a[t] * size + (k[t] * v[t]).abs()
+        bound = (210 + dim) * 2.0 ** -24 * (q[t].abs() * size).sum(1).reshape(-1)
+        for o in (out, out_s):
+            assert ((o[38 + t].double() - (q[t] * S).sum(1).reshape(-1)).abs() <= bound).all(), t
+    for s in (state, state_s):
+        got = s[1].double().view(heads, vdim, dim).transpose(1, 2)
+        assert ((got - S).abs() <= 210 * 2.0 ** -24 * size).all()
