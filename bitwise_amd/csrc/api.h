@@ -120,10 +120,12 @@ int bw_norm_shift(const float* x, int ldx, const float* w, const float* mix, flo
 // k v^T weighted by bias2 [heads*dim]; mode 3: one constant decay a head, bias [heads] (gate is not read).
 // mode 4: a step size per head, delta = softplus(logit at gate_off + head + bias[head]); decay exp(-bias2[head] delta), the
 // token enters as k (delta v)^T, skip[head] v (optional) joins the read-out.
+// mode 5: the delta rule, S <- a S + k (b (v - a S^T k))^T with step sizes b at gate_off + head, decays a at gate2_off + head and
+// the products k.q of the key heads behind them (no bias; one pass only).
+// mode 6: mode 0 with the decays themselves in gate (bw_decay_rows; no bias).  Passes over chunks: this in place of mode 0.
 // q is multiplied by qscale, k by kscale; heads_per_key neighbouring heads share one q and one k.
 // (silu 1, fixed decay only: q, k and v pass SiLU on their way in; few 1: the requests bring a few rows each, which picks the
 // kernel that favours many waves over long walks, the same bits)
-int bw_decay_rows(float* z, int ld, const float* bias, float param, int rows, int cols, void* stream);
 int bw_linear_recurrence(int mode, const float* proj, int ldp, int q_off, int k_off, int v_off, const float* gate, int ldg,
                          int gate_off, int gate2_off, const float* bias, const float* bias2, float param, float qscale,
                          float kscale, const float* skip, int heads_per_key, int silu, int few, float* state, long long state_ld, float* out,
@@ -131,6 +133,8 @@ int bw_linear_recurrence(int mode, const float* proj, int ldp, int q_off, int k_
                          const int32_t* slots, const int32_t* positions, int nseq, int heads, int dim, int vdim,
                          const int32_t* chunks, int nchunks, const int32_t* spans, int nspans, float* scan_local,
                          float* scan_start, long long scan_floats, void* stream);
+// z[r][c] <- exp(logsigmoid(z[r][c] + bias[c]) * param), in place: the decays of mode 0 for mode 6
+int bw_decay_rows(float* z, int ld, const float* bias, float param, int rows, int cols, void* stream);
 long long bw_recurrence_record(int dim, int vdim);      // floats that scan_local and scan_start hold per chunk and head
 // gate 0: sigmoid, 1: SiLU.  weight: [heads, wstride] (wstride 0: one weight vector for all heads).
 // Up to two sections of [heads][dim] 32-bit elements a row (at columns off0, off1) turned in place: of a head's first rot

@@ -954,6 +954,10 @@ def linear_recurrence(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_o
     chunks = spans = local = start = None
     nchunks = nspans = 0
     if scan is not None:
+        if mode == RECUR_DECAY_PER_CHANNEL:               # the passes exist for decays that are given
+            decays = gate[:, gate_off:gate_off + heads * dim].clone(memory_format=torch.contiguous_format)
+            decay_rows(decays, bias, param, decays.shape[0])
+            mode, gate, gate_off, bias = RECUR_DECAY_GIVEN, decays, 0, None
         chunks, nchunks, spans, nspans, local, start = scan
         _need(chunks, torch.int32, "chunks")
         _need(spans, torch.int32, "spans")

@@ -977,12 +977,17 @@ int launch_recurrence(const RecurArgs& a, int units, hipStream_t s) {
 
 template <int MODE>
 int launch_recurrence_passes(const RecurArgs& a, int nseq, bool few, int nchunks, const int32_t* spans, int nspans, hipStream_t s) {
+  // (Decays that are given come with portions of more than a few rows: the walk takes what there is of others, the same bits.
+  // Passes over chunks come with a per-channel memory's decays given, never with their logits.)
+  constexpr bool FEW = MODE != RECUR_DECAY_GIVEN, PASSES = MODE != RECUR_DELTA && MODE != RECUR_DECAY_PER_CHANNEL;
+  if (nchunks > 0 && !PASSES) return -2;
   int rc = 0;
-  if (nseq > 0) rc = few ? launch_recurrence<MODE, 4>(a, nseq, s) : launch_recurrence<MODE, 0>(a, nseq, s);
+  if (nseq > 0) {
+    if constexpr (FEW) rc = few ? launch_recurrence<MODE, 4>(a, nseq, s) : launch_recurrence<MODE, 0>(a, nseq, s);
+    else rc = launch_recurrence<MODE, 0>(a, nseq, s);
+  }
   if (rc != 0 || nchunks <= 0) return rc;
-  if constexpr (MODE == RECUR_DELTA) {
-    return -2;
-  } else {
+  if constexpr (PASSES) {
     rc = launch_recurrence<MODE, 1>(a, nchunks, s);
     if (rc != 0) return rc;
     const int mine = a.dim * a.vdim + (MODE == RECUR_SCALAR_GATES ? a.dim + 1 : 0);
@@ -991,6 +996,7 @@ int launch_recurrence_passes(const RecurArgs& a, int nseq, bool few, int nchunks
     if (rc != 0) return rc;
     return launch_recurrence<MODE, 3>(a, nchunks, s);
   }
+  return rc;
 }
 
 // ------------------------------------------------------------------------- per-head RMS norm and output gate

@@ -474,6 +474,8 @@ def test_decays_made_ahead_equal_decays_made_in_the_walk(gpu, dim, vdim):
     scan = (dev32(chunks), len(chunks), dev32([2, 0, len(chunks)]), 1, torch.zeros(rec, device=dev), torch.zeros(rec, device=dev))
     out_s, state_s = run(ops.RECUR_DECAY_GIVEN, given, None, (5, 33, 0), scan)
     assert torch.equal(out_s[:38], out[:38]) and torch.equal(state_s[[0, 2]], state[[0, 2]])
+    out_p, state_p = run(ops.RECUR_DECAY_PER_CHANNEL, logits, bias, (5, 33, 0), scan)
+    assert torch.equal(out_p, out_s) and torch.equal(state_p, state_s)
     # the portion of 100 in 64 bits, beside the sums of the terms' sizes: every output and state element of either order is
     # a sum of at most 100 terms a channel, each through up to 100 + 4 products (an output: dim of them)
     p, a = proj[38:].double(), given[38:].double().view(100, heads, dim, 1)
