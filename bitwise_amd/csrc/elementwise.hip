@@ -157,22 +157,24 @@ __global__ void rmsnorm_f32_kernel(const float* __restrict__ x, const WT* __rest
 
 // The same chains and tree for rows of up to RMS32_MAX elements, a workgroup a row: its 256 threads bring the row
 // into LDS together, 16 of them run the chains from there (nothing between two steps of a chain but an LDS
-// read), and all write the result.  What it costs is latency: the row and the weights are asked for together, 16 bytes a
-// load, and the chains' LDS reads run 32 links ahead (8 rows of 2,048: 7.4 -> 4.7 us inside a decode step).
+// read), and all write the result.  What it costs is latency.  LONG, rows of 1,024 to 4,096 elements that are whole
+// vectors: the row and the weights are asked for together, 16 bytes a load, and the chains' LDS reads run 32 links ahead (8
+// rows of 2,048: 4.6 us -> 3.4 alone, 7.4 -> 4.7 inside a decode step; 2,048 rows 10.1 -> 8.2).  Shorter rows have nothing to run
+// ahead of and pay for its registers (2,048 rows of 256: 3.5 us -> 5.6; 8 rows of 768: 2.8 -> 3.2).
 #define RMS32_MAX 8192
-template <typename WT>
+#define RMS32_LONG 1024
+#define RMS32_VECS 4             // vectors a thread keeps of a long row
+template <typename WT, bool LONG>
 __global__ __launch_bounds__(256) void rmsnorm_f32_row_kernel(const float* __restrict__ x, const WT* __restrict__ w,
                                                               float* __restrict__ y, int dim, float eps) {
-  __shared__ __attribute__((aligned(16))) float row_lds[RMS32_MAX];
+  constexpr int NV = LONG ? RMS32_VECS : 1;
+  __shared__ __attribute__((aligned(16))) float row_lds[LONG ? 1024 * NV : RMS32_MAX];
   __shared__ float inv_lds;
   const float* xr = x + (size_t)blockIdx.x * dim;
   float* yr = y + (size_t)blockIdx.x * dim;
-  // rows of up to 4,096 elements that are whole vectors: a thread keeps its vectors and weights, all asked for at once
-  constexpr int NV = 4;
-  const bool vec = (dim & 3) == 0 && dim <= 1024 * NV && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)w) & 15) == 0;
   const int nvec = dim >> 2;
   f32x4 v[NV], wv[NV];
-  if (vec) {
+  if constexpr (LONG) {
     u32x4 raw[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
@@ -192,30 +194,33 @@ __global__ __launch_bounds__(256) void rmsnorm_f32_row_kernel(const float* __res
   __syncthreads();
   if (threadIdx.x < 16) {
     float acc = 0.0f;
-    // thirty-two links at a time, the next ones' elements read from LDS under these
-    const float* mine = row_lds + threadIdx.x;
-    const int links = dim / 16, whole = links & ~31;
-    float a[32], b[32];
-    if (whole) {
+    int done = 0;
+    if constexpr (LONG) {
+      // thirty-two links at a time, the next ones' elements read from LDS under these
+      const float* mine = row_lds + threadIdx.x;
+      const int whole = (dim / 16) & ~31;
+      float a[32], b[32];
 #pragma unroll
       for (int j = 0; j < 32; ++j) a[j] = mine[16 * j];
+      for (int l = 0; l < whole; l += 32) {
+        const int nx = l + 32 < whole ? l + 32 : l;
+#pragma unroll
+        for (int j = 0; j < 32; ++j) b[j] = mine[16 * (nx + j)];
+#pragma unroll
+        for (int j = 0; j < 32; ++j) acc = fmaf(a[j], a[j], acc);
+#pragma unroll
+        for (int j = 0; j < 32; ++j) a[j] = b[j];
+      }
+      done = 16 * whole;
     }
-    for (int l = 0; l < whole; l += 32) {
-      const int nx = l + 32 < whole ? l + 32 : l;
-#pragma unroll
-      for (int j = 0; j < 32; ++j) b[j] = mine[16 * (nx + j)];
-#pragma unroll
-      for (int j = 0; j < 32; ++j) acc = fmaf(a[j], a[j], acc);
-#pragma unroll
-      for (int j = 0; j < 32; ++j) a[j] = b[j];
-    }
-    for (int i = 16 * whole + (int)threadIdx.x; i < dim; i += 16) acc = fmaf(row_lds[i], row_lds[i], acc);
+#pragma unroll 8
+    for (int i = done + (int)threadIdx.x; i < dim; i += 16) acc = fmaf(row_lds[i], row_lds[i], acc);
     acc = row16_sum(acc);
     if (threadIdx.x == 0) inv_lds = 1.0f / sqrtf(acc / (float)dim + eps);
   }
   __syncthreads();
   const float inv = inv_lds;
-  if (vec) {
+  if constexpr (LONG) {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int c = (int)threadIdx.x + 256 * j;
@@ -223,14 +228,22 @@ __global__ __launch_bounds__(256) void rmsnorm_f32_row_kernel(const float* __res
         reinterpret_cast<f32x4*>(yr)[c] = (f32x4){(v[j][0] * inv) * wv[j][0], (v[j][1] * inv) * wv[j][1], (v[j][2] * inv) * wv[j][2],
                                                   (v[j][3] * inv) * wv[j][3]};
     }
-    return;
+  } else {
+    for (int i = threadIdx.x; i < dim; i += 256) {
+      float wi;
+      if constexpr (sizeof(WT) == 2) wi = bf16_to_f32(w[i]);
+      else wi = w[i];
+      yr[i] = (row_lds[i] * inv) * wi;
+    }
   }
-  for (int i = threadIdx.x; i < dim; i += 256) {
-    float wi;
-    if constexpr (sizeof(WT) == 2) wi = bf16_to_f32(w[i]);
-    else wi = w[i];
-    yr[i] = (row_lds[i] * inv) * wi;
-  }
+}
+
+template <typename WT>
+static void launch_rmsnorm_f32_rows(const float* x, const WT* w, float* y, int rows, int dim, float eps, hipStream_t s) {
+  if (dim >= RMS32_LONG && dim <= 1024 * RMS32_VECS && (dim & 3) == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)w) & 15) == 0)
+    hipLaunchKernelGGL((rmsnorm_f32_row_kernel<WT, true>), dim3(rows), dim3(256), 0, s, x, w, y, dim, eps);
+  else
+    hipLaunchKernelGGL((rmsnorm_f32_row_kernel<WT, false>), dim3(rows), dim3(256), 0, s, x, w, y, dim, eps);
 }
 
 // ------------------------------------------------------------------------- RMSNorm, bfloat16 out
@@ -313,10 +326,8 @@ extern "C" int bw_rmsnorm(const float* x, const void* weight, int weight_is_bf16
   } else {
     if (ldy != dim) return -2;
     if (dim <= RMS32_MAX) {
-      if (weight_is_bf16)
-        hipLaunchKernelGGL(rmsnorm_f32_row_kernel<bf16_t>, dim3(rows), dim3(256), 0, s, x, (const bf16_t*)weight, (float*)y, dim, eps);
-      else
-        hipLaunchKernelGGL(rmsnorm_f32_row_kernel<float>, dim3(rows), dim3(256), 0, s, x, (const float*)weight, (float*)y, dim, eps);
+      if (weight_is_bf16) launch_rmsnorm_f32_rows(x, (const bf16_t*)weight, (float*)y, rows, dim, eps, s);
+      else launch_rmsnorm_f32_rows(x, (const float*)weight, (float*)y, rows, dim, eps, s);
       return BW_LAUNCH_CHECK();
     }
     dim3 grid((rows + 15) / 16), block(256);

@@ -572,6 +572,20 @@ def test_rmsnorm_f32_rows_are_the_chains_of_the_definition(gpu, dim, wdt):
         assert np.array_equal(out[r].cpu().numpy(), want), r
 
 
+@pytest.mark.parametrize("dim", [1020, 1023, 1024, 1028, 1100, 1548, 4092])
+def test_rmsnorm_f32_long_rows_begin_where_the_short_ones_end(gpu, dim):
+    """Rows around the length from which the chains read ahead, whole vectors and not, and rows that start off a vector."""
+    g = torch.Generator().manual_seed(dim)
+    x, w = torch.randn(5, dim, generator=g), 1 + 0.1 * torch.randn(dim, generator=g)
+    want = np.stack([(r * (np.float32(1.0) / np.sqrt(canonical_sumsq(r) / np.float32(dim) + np.float32(1e-5), dtype=np.float32))) * w.numpy()
+                     for r in x.numpy()])
+    for off in (0, 1):
+        xs, out = (torch.zeros(5 * dim + off, device=gpu)[off:].view(5, dim) for _ in range(2))
+        xs.copy_(x)
+        ops.rmsnorm(xs, w.to(gpu), out, 5, 1e-5)
+        assert np.array_equal(out.cpu().numpy(), want), off
+
+
 def paged_setup(gpu, bf16, heads, kvh, hd, page, pages, n_keys, seed, poison=False):
     """A sequence of n_keys keys and values scattered over pages by the reference's table
     (i*7+3) % pages (tests/test_main.cpp:146-147); everything else is poison."""
