@@ -108,6 +108,20 @@ def test_swiglu_and_the_exponential_bits(gpu):
     assert (np.abs(e - ref) <= 2.0 * np.spacing(ref.astype(np.float32)).astype(np.float64)).all()
 
 
+@pytest.mark.parametrize("rows,inter", [(1, 1), (5, 63), (7, 64), (66, 65), (3, 1023), (2, 1024), (260, 1020), (1030, 300), (65, 4100), (64, 4092),
+                                        (65537, 4)])
+def test_swiglu_of_every_width_and_height_of_workgroup(gpu, rows, inter):
+    """Rows narrower and wider than a workgroup, one element a thread and four, row counts that fill no workgroup, more rows than a
+    grid is high; the element behind the result stays what it was."""
+    g = torch.Generator().manual_seed(rows + inter)
+    gu = 3 * torch.randn(rows, 2 * inter, generator=g)
+    h = torch.full((rows + 1, inter), 7.0, device=gpu)
+    ops.swiglu_f32(gu.to(gpu), h, rows)
+    got = h.cpu().numpy()
+    assert np.array_equal(bits(got[:rows]), bits(ps.swiglu(gu[:, :inter].contiguous().numpy(), gu[:, inter:].contiguous().numpy())))
+    assert (got[rows] == 7.0).all()
+
+
 @pytest.mark.parametrize("heads,kvh,hd,page,window", [(4, 2, 16, 16, 0), (3, 1, 32, 8, 0), (2, 2, 64, 16, 37),
                                                       (2, 1, 128, 16, 0), (5, 5, 80, 32, 0)])
 def test_attention_bits(gpu, heads, kvh, hd, page, window):
