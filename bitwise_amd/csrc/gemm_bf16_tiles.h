@@ -502,7 +502,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // by every lane for each of its rows: position and page of each of the 256 rows (a thread a row), then the
     // rows' cosines and sines (16-byte loads; a row of 32 + 32 floats, 36 apart against bank conflicts).
     constexpr int CS = 36;
-    __builtin_amdgcn_s_waitcnt(BIG_WAIT_ALL);
     __syncthreads();                                                // every wave is done with the ring
     int* pos_lds = reinterpret_cast<int*>(big_lds);                 // [256]
     int* page_lds = pos_lds + BIG_BM;                               // [256]
@@ -773,6 +772,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
     }
   }
+  __builtin_amdgcn_s_waitcnt(vmcnt_only(0));                         // the padding loads too, before the waves end
   if (EPI != EPI_ADD_F32 && steps > GEMM_SEG / 64) {
 #pragma unroll
     for (int i = 0; i < NI; ++i)
@@ -949,6 +949,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
     }
   }
+  __builtin_amdgcn_s_waitcnt(vmcnt_only(0));                         // the padding loads too, before the waves end
   if (K > GEMM_SEG) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
