@@ -33,6 +33,8 @@ int bw_rope_kvwrite(float* qkv, void* q_out, const int32_t* positions, const int
                     int page_size, int write_cache, void* stream);
 int bw_gemm_f32(const float* x, const void* w, int w_is_bf16, float* y, int M, int N, int K, int ldx, int ldy,
                 int accumulate, void* stream);
+// rows and columns of the tiles that a product of more than 64 rows gets (K a multiple of 32, whole vectors)
+int bw_gemm_f32_prompt_tile(int M, int N, int* rows, int* columns);
 int bw_gemm_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, int epilogue,
                  void* stream);
 int bw_gemm_clamped_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, float limit,

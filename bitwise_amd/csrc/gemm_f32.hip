@@ -1212,17 +1212,39 @@ static void launch_f32_mfma_columns(const float* x, const WT* w, float* y, int M
                      accumulate, m_tiles);
 }
 
-template <typename WT>
-static void launch_f32_mfma_tiles(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate,
-                                  hipStream_t s) {
-  using S = F32PShape<WT>;
-  // Which tiles: clocks a step of k a round of the compute units, as measured (the comment above), times the rounds.
+// Which tiles a prompt's product gets, rows x columns: clocks a step of k a round of the compute units, as measured with bfloat16
+// weights (the comment at F32QShape), times the rounds.  With 32-bit weights, which need no widening, every tile takes about a tenth
+// less, so the same rule holds: over 65 to 2,048 rows, 512 to 16,384 columns and K of 512 to 8,192 its choice took 0.33 to 1.01
+// of the 128 x 128 tiles' time with either (450 rows, 2048 x 8192: 519 us -> 174 with 32-bit weights, 572 -> 194 with bfloat16).
+struct F32PromptTile {
+  int rows, columns;
+};
+
+static F32PromptTile f32_prompt_tile(int M, int N) {
   auto cost = [&](int bm, int bn, int clocks) {
     return (long long)clocks * ((((long long)(M + bm - 1) / bm) * ((N + bn - 1) / bn) + 255) / 256);
   };
   const long long big = cost(F32P_BM, F32P_BN, 185), one = cost(64, 64, 55), two = cost(128, 64, 103);
-  if (one < big && one <= two) return launch_f32_mfma_columns<WT, 1>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
-  if (two < big) return launch_f32_mfma_columns<WT, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+  if (one < big && one <= two) return {64, 64};
+  if (two < big) return {128, 64};
+  return {F32P_BM, F32P_BN};
+}
+
+extern "C" int bw_gemm_f32_prompt_tile(int M, int N, int* rows, int* columns) {
+  if (M <= 0 || N <= 0) return -2;
+  const F32PromptTile t = f32_prompt_tile(M, N);
+  *rows = t.rows;
+  *columns = t.columns;
+  return 0;
+}
+
+template <typename WT>
+static void launch_f32_mfma_tiles(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate,
+                                  hipStream_t s) {
+  using S = F32PShape<WT>;
+  const F32PromptTile tile = f32_prompt_tile(M, N);
+  if (tile.rows == 64) return launch_f32_mfma_columns<WT, 1>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+  if (tile.columns == 64) return launch_f32_mfma_columns<WT, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
   constexpr int lds_bytes = F32P_STAGES * S::STAGE;
   static bool allowed = false;                       // more than 64 KB of dynamic LDS has to be asked for once
   if (!allowed) {
@@ -1264,8 +1286,8 @@ extern "C" int bw_gemm_f32(const float* x, const void* w, int w_is_bf16, float* 
   const int wc = w_is_bf16 ? 8 : 4;
   // 17 to 64 rows, K in whole stages: the chains run on the matrix cores (offsets within x and within a wave's rows
   // of W must fit the buffer descriptors' 31 bits).  Up to 16 rows stay on the vector unit: a matrix instruction that
-  // depends on the one before it issues some 40 clocks later, a vector one 4, and so few rows have too few chains
-  // to fill the gap.
+  // depends on the one before it issues some 40 clocks later, a vector multiply-add 9, and so few rows have too few
+  // chains to fill the gap.
   if (M > 16 && M <= 64 && K % 64 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 &&
       (size_t)M * ldx * 4 < ((size_t)1 << 31) && (size_t)64 * K * 4 < ((size_t)1 << 31)) {
     if (w_is_bf16) launch_f32_mfma_rows<bf16_t>(x, (const bf16_t*)w, y, M, N, K, ldx, ldy, accumulate, s);

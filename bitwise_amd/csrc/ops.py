@@ -49,6 +49,7 @@ _SIGS = {
     "bw_gemm_f32": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_clamped_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],
+    "bw_gemm_f32_prompt_tile": [c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_add_scratch": [c_int, c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_add_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_longlong, c_void_p,
                          c_int, c_void_p],
@@ -156,7 +157,7 @@ _fns = {}
 # what waits.
 _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
-    "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
+    "bw_gemm_f32_prompt_tile", "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
     "bw_chain_flush", "bw_chain_end",
 })
@@ -446,6 +447,13 @@ def gemm_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows: int, acc
         raise ValueError(f"gemm_f32: x {tuple(x.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not match")
     _check(_fn("bw_gemm_f32")(x.data_ptr(), w.data_ptr(), _is_bf16(w, "weight"), out.data_ptr(), rows, N, K,
                               x.stride(0), out.stride(0), int(accumulate), _stream()), "gemm_f32")
+
+
+def gemm_f32_prompt_tile(rows: int, N: int) -> Tuple[int, int]:
+    """(rows, columns) of the tiles that ``gemm_f32`` gives a product of more than 64 rows, K in whole stages of 32."""
+    r, c = ctypes.c_int(0), ctypes.c_int(0)
+    _check(_fn("bw_gemm_f32_prompt_tile")(rows, N, ctypes.addressof(r), ctypes.addressof(c)), "gemm_f32_prompt_tile")
+    return int(r.value), int(c.value)
 
 
 @functools.lru_cache(maxsize=None)

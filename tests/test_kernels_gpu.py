@@ -84,7 +84,7 @@ def test_gemm_f32_grid_rows_and_accumulate(gpu):
     before = batch.clone()
     ops.gemm_f32(x, wb, batch, 9, accumulate=True)
     assert torch.equal(batch, before + before)                     # y + acc, one addition per output
-    # prompt portions (128 x 128 tiles, or 64 x 64 where K is no multiple of 16): a row's bits are those of the row alone
+    # prompt portions (64 x 64 tiles on the matrix cores, or on the vector units where K is no multiple of 32): a row's bits are those of the row alone
     # (and 17 to 64 rows: the chain-per-thread kernel with two or four blocks of rows)
     for M, N, K in [(150, 200, 1024), (129, 130, 64), (300, 77, 48), (70, 140, 1000), (40, 130, 1024), (20, 77, 264),
                     (64, 50, 136), (33, 16, 8)]:
@@ -122,8 +122,20 @@ def test_gemm_f32_grid_rows_and_accumulate(gpu):
             assert torch.equal(longer, before), (M, N, K, weight.dtype)
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 64, 32), (65, 1, 64), (127, 65, 96), (128, 640, 160), (129, 130, 2080), (200, 16500, 64),
-                                    (700, 6200, 96), (1030, 2050, 128), (2100, 2048, 64)])
+PROMPT_TILES = {            # tile -> products (M, N, K) that the rule gives it, at the edges of its rows, columns and stages
+    (64, 64): [(65, 64, 32), (65, 1, 64), (127, 65, 96), (128, 640, 160), (129, 130, 2080), (200, 16500, 64), (700, 6200, 96),
+               (1030, 2050, 128), (2100, 2048, 64)],
+    (128, 64): [(1000, 2040, 64), (2040, 1020, 96), (2048, 1024, 32), (897, 1985, 160)],
+    (128, 128): [(2040, 2040, 64), (450, 16380, 32), (2048, 2048, 96), (257, 10753, 160)],
+}
+
+
+def test_gemm_f32_prompt_products_reach_every_tile():
+    for tile, shapes in PROMPT_TILES.items():
+        assert [ops.gemm_f32_prompt_tile(M, N) for M, N, _ in shapes] == [tile] * len(shapes)
+
+
+@pytest.mark.parametrize("M,N,K", sum(PROMPT_TILES.values(), []))
 @pytest.mark.parametrize("wdt", [torch.bfloat16, torch.float32])
 def test_gemm_f32_prompt_tiles_are_the_chains_of_few_rows(gpu, M, N, K, wdt):
     """Every tile shape of the 32-bit prompt products at the edges of its rows, columns and stages: the bits of the same rows
