@@ -846,6 +846,32 @@ def test_decode_attention_of_a_queue_equals_each_row_alone(gpu, rows, heads, kvh
                 assert torch.equal(out[r], one[0]), r
 
 
+@pytest.mark.parametrize("rows,heads,kvh,hd,width", [(33, 16, 16, 64, 20), (70, 32, 8, 128, 20), (64, 12, 12, 128, 400), (100, 16, 8, 64, 20)])
+def test_decode_attention_of_a_tile_list_in_any_order(gpu, rows, heads, kvh, hd, width):
+    """The single tokens of a step that has portions beside them come as a list, the longest contexts first: more workgroups than
+    places in that order, in the rows' and in a shuffled one, in four waves and in eight (heads of 128 in a wide table), every
+    row at another sequence's place: the bits of a launch of its own."""
+    page = 16
+    g = torch.Generator(device=gpu).manual_seed(rows + hd)
+    pos = torch.randint(0, page * 20, (rows,), generator=g, device=gpu, dtype=torch.int32)
+    pos[2], pos[rows // 2] = 319, 0
+    seqs = torch.randperm(rows, generator=g, device=gpu).int()
+    table = torch.zeros(rows, width, dtype=torch.int32, device=gpu)
+    table[:, :20] = torch.randperm(rows * 20, generator=g, device=gpu).int().view(rows, 20)
+    kc, vc = torch.randn(2, rows * 20, kvh * page * hd, generator=g, device=gpu).bfloat16()
+    q = torch.randn(rows, heads * hd, generator=g, device=gpu).bfloat16()
+    want = torch.zeros_like(q)
+    for r in range(rows):
+        ops.attention_bf16(q[r:r + 1], pos[r:r + 1].clone(), table[seqs[r]:seqs[r] + 1].clone(), None, 1, kc, vc, want[r:r + 1], heads, kvh, hd, page,
+                           0, 0.125, decode=True)
+    longest = sorted(range(rows), key=lambda r: -int(pos[r]))
+    for order in (longest, list(range(rows)), torch.randperm(rows, generator=g, device=gpu).tolist()):
+        tiles = torch.tensor([(r, 1, int(seqs[r]), 0) for r in order], dtype=torch.int32, device=gpu)
+        out = torch.zeros_like(q)
+        ops.attention_bf16(q, pos, table, tiles, rows, kc, vc, out, heads, kvh, hd, page, 0, 0.125, decode=True)
+        assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("rows,heads,kvh,hd", [(1, 4, 4, 64), (8, 2, 1, 64), (8, 32, 8, 128), (4, 6, 3, 32), (64, 2, 2, 16)])
 def test_split_decode_attention_with_padding_and_short_contexts(gpu, rows, heads, kvh, hd):
     """Launches of few tiles, split over workgroups that share the live rows' work: padding anywhere, all padding, contexts
