@@ -72,12 +72,10 @@ struct TileCtx {
   u32x4 qf[KS];
 };
 
-#define POS_UNREAD (-0x7fffffff - 1)       // group_setup: the position is still to be read
-
-// ``known_pos``: the position of a tile of one row, where the caller has it.
-template <int HD, int QT>
+// KNOWN: the caller has read the position of a tile of one row.
+template <int HD, int QT, bool KNOWN = false>
 __device__ __forceinline__ bool group_setup(const AttnBf16Args& a, int first_tile, int head_item, GroupCtx& gc,
-                                            TileCtx<HD> (&tc)[QT], int known_pos = POS_UNREAD) {
+                                            TileCtx<HD> (&tc)[QT], int known_pos = -1) {
   gc.lane = threadIdx.x & 63;
   gc.r = gc.lane & 15;
   gc.g = gc.lane >> 4;
@@ -102,8 +100,8 @@ __device__ __forceinline__ bool group_setup(const AttnBf16Args& a, int first_til
     const bool ok = col_in && tok < ntok;
     tc[t].row_c = row0 + (ok ? tok : 0);
     tc[t].head_c = gc.kvh * group + gc.sub * a.hpt + (ok ? hh : 0);
-    tc[t].pos_c = ok ? known_pos : -1;
-    if (known_pos == POS_UNREAD && ok) tc[t].pos_c = a.positions[tc[t].row_c];      // (scalar, or known at compile time)
+    if constexpr (KNOWN) tc[t].pos_c = ok ? known_pos : -1;
+    else tc[t].pos_c = ok ? a.positions[tc[t].row_c] : -1;
     if (a.chunk > 0) tc[t].lo_c = tc[t].pos_c > 0 ? tc[t].pos_c - tc[t].pos_c % a.chunk : 0;
     else tc[t].lo_c = (a.window > 0 && tc[t].pos_c - a.window + 1 > 0) ? tc[t].pos_c - a.window + 1 : 0;
     kmax = max(kmax, tc[t].pos_c);
@@ -1190,27 +1188,66 @@ constexpr int decode_alone(int head_dim) {
                                  // generation of eight-wave workgroups before it (16 requests of 32 heads: 2.61 -> 2.52 ms
                                  // a step at 2,048-token contexts, 1.76 -> 1.69 at 512)
 
-// The tile of rank ``rank`` when tiles of one token (tile t: row t) are ordered by their number of partitions, the most first,
-// tiles of equally many by their number; at most 64 tiles.  Every lane of every wave gets the answer.  A radix selection over
-// ballots: some seven scalar instructions a bit.
-__device__ __forceinline__ int tile_of_rank(const AttnBf16Args& a, int rank) {
-  const int lane = threadIdx.x & 63;
-  const int pos = lane < a.num_tiles ? a.positions[lane] : -1;
-  const unsigned key = lane < a.num_tiles ? (unsigned)(pos < 0 ? 0 : pos / ATT_PART + 1) : 0u;
-  unsigned long long left = a.num_tiles >= 64 ? ~0ull : (1ull << a.num_tiles) - 1;
-  const int parts = (a.table_stride * a.page_size + ATT_PART - 1) / ATT_PART + 1;     // no key is larger
-  for (int bit = 31 - __builtin_clz((unsigned)parts); bit >= 0; --bit) {
-    const unsigned long long with = __ballot((key >> bit) & 1u) & left;
-    const int n = __popcll(with);
-    if (rank < n) left = with;
-    else {
-      rank -= n;
-      left &= ~with;
-    }
+// From so many keys on (rounds of a workgroup, five of four waves) the longest context is worth putting the rows in order,
+// which holds every workgroup up by some 0.3 us at 64 rows and 0.6 at 256 (32 heads of 64, ranked and not: 43 rows of up to 600
+// keys 35.1 us and 32.3, 65 rows of up to 1,100 66 and 64, 33 rows 36.6 and 32.8; 65 of up to 2,000 105 and 119).  Asking
+// whether one is that long costs short launches 0 to 4 % (256 rows of 300 keys, 3 key heads of 64: 20.1 us -> 20.8).
+#define QUEUE_KEYS (20 * ATT_PART)
+#define QUEUE_ROWS 256           // rows that a queue without a tile list puts in order
+
+// Positions of the rows of a launch of tiles of one token (tile t: row t), 64 to a load: lane l has those of rows l, 64 + l ...
+struct QueueRows {
+  static constexpr int G = QUEUE_ROWS / 64;
+  int at[G];
+};
+
+// The tile of rank ``rank`` when the tiles are ordered by the rounds that a workgroup of W waves makes over their
+// partitions, the most first, tiles of equally many by their number, padding rows last.  Every lane of every wave gets the
+// answer.  A radix selection over ballots: some seven scalar instructions a bit and 64 tiles.
+template <int G, int W>
+__device__ __forceinline__ int tile_of_rank(const AttnBf16Args& a, const QueueRows& rows, int rank) {
+  unsigned long long left[G];
+  unsigned key[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int n = a.num_tiles - 64 * g;
+    left[g] = n >= 64 ? ~0ull : n > 0 ? (1ull << n) - 1 : 0;
+    key[g] = rows.at[g] >= 0 ? (unsigned)rows.at[g] / (ATT_PART * W) + 1u : 0u;
   }
-  const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(left >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)left, 0u));
-  const unsigned long long me = __ballot(((left >> lane) & 1ull) != 0 && before == rank);
-  return me != 0 ? (int)__builtin_ctzll(me) : 0;
+  const unsigned most = (unsigned)(a.table_stride * a.page_size) / (ATT_PART * W) + 1u;      // no key is larger
+  for (int bit = 31 - __builtin_clz(most); bit >= 0; --bit) {
+    unsigned long long with[G];
+    int n = 0;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      with[g] = __ballot((key[g] >> bit) & 1u) & left[g];
+      n += __popcll(with[g]);
+    }
+    const bool among = rank < n;
+    if (!among) rank -= n;
+#pragma unroll
+    for (int g = 0; g < G; ++g) left[g] = among ? with[g] : left[g] & ~with[g];
+  }
+  int tile = 0;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(left[g] >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)left[g], 0u));
+    const unsigned long long me = __ballot(((left[g] >> (threadIdx.x & 63)) & 1ull) != 0 && before == rank);
+    if (me != 0) tile = 64 * g + (int)__builtin_ctzll(me);
+    rank -= __popcll(left[g]);
+  }
+  return tile;
+}
+
+// Place ``index`` of the order is whose turn it is: tile, and head.
+__device__ __forceinline__ void queue_place(int& index, int& head_item) {
+  const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x), per = 8 * (int)gridDim.y, eight = id / per;
+  index = id / (int)gridDim.y;
+  head_item = id % (int)gridDim.y;
+  if (8 * eight + 8 <= (int)gridDim.x) {
+    index = 8 * eight + ((eight & 1) ? 7 - (id & 7) : id & 7);
+    head_item = (id % per) >> 3;
+  }
 }
 
 template <int HD, int W, bool SPLIT>
@@ -1231,29 +1268,31 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
   // whatever the position says: its pages are asked for beside the position, not after it (the table index is
   // clamped into the row and the pages into the pool, so a sequence shorter than that costs a wasted load).
   int tile = blockIdx.x, head_item = blockIdx.y;
+  // More workgroups than places on the chip (two a compute unit): where a context is long (QUEUE_KEYS) the longest go
+  // first, or one that starts last is worked on alone; a tile list comes in that order, other rows are ranked here.  Eight
+  // neighbours of that order run at a time, through the heads, a die each (forward and backward in turn: no die
+  // gets the longest of every eight).  Short contexts leave no tail worth the ranking: rows in whole eights take the dies'
+  // order as they are, others keep blockIdx's, which spreads a row over the dies.  (32 heads of 64: 43 rows of up to 2,000
+  // keys 82 us -> 70, 65 rows 119 -> 105, 128 rows 222 -> 191; 64 of 2,000 each, where only the dies matter, 190 -> 182.)
   const bool queued = W == DECODE_W_MANY && !SPLIT && gridDim.x * gridDim.y > 512u;
-  if (queued) {
-    // More workgroups than places on the chip (two a compute unit): the longest contexts go first, or one that starts last is
-    // worked on alone.  Eight neighbours of that order run at a time, through the heads, a die each (forward and
-    // backward in turn: no die gets the longest of every eight).  Rows of a step without a tile list are ordered below; a
-    // tile list comes in that order.  32 heads of 64: 43 requests of 97 to 4,000 tokens 210 us -> 128 (688 MB); 64 of 2,048
-    // each, where only the dies matter, 192 -> 180.
-    const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x), per = 8 * (int)gridDim.y, eight = id / per;
-    tile = id / (int)gridDim.y;
-    head_item = id % (int)gridDim.y;
-    if (8 * eight + 8 <= (int)gridDim.x) {
-      tile = 8 * eight + ((eight & 1) ? 7 - (id & 7) : id & 7);
-      head_item = (id % per) >> 3;
-    }
-  }
+  const bool placed = queued && (a.tiles != nullptr || gridDim.x % 8 == 0);
+  if (placed) queue_place(tile, head_item);
   int z = SPLIT ? (int)blockIdx.z : 0, nz = SPLIT ? (int)gridDim.z : 1;
   const bool early = a.window == 0 && a.chunk == 0 && a.tiles == nullptr;
-  // Split launches hand their workgroups out by the rows' positions: row l's in lane l, one load for that and for the tile's own
-  // (8 rows of 1,100 keys, 8 heads of 128, no padding: 14.5 us with a load behind the other, 13.7 so).  Without a split the
-  // branch on a known position costs more than the second load (128 rows of up to 300 keys 51 us -> 53).
+  // The tile's position is asked for once, in front of the pages (loads come back in order): here, or out of all rows' where
+  // those are read anyway, row l's in lane l (8 rows of 1,100 keys, 8 heads of 128: 14.5 us with one load behind the other, 13.7 so;
+  // 256 rows of 300 keys, 8 of 64: 39.8 and 39.0).
   const bool by_position = SPLIT && a.tiles == nullptr && a.num_tiles <= 64;
-  int row_pos = -1, known_pos = POS_UNREAD;
+  int row = tile;
+  if (a.tiles != nullptr) row = a.tiles[tile * 4 + 1] > 0 ? a.tiles[tile * 4] : 0;       // (an empty tile: any row)
+  int row_pos = -1, pos = a.positions[row];
   if (by_position) row_pos = a.positions[min((int)threadIdx.x & 63, a.num_tiles - 1)];
+  const bool ranked = queued && a.tiles == nullptr && a.num_tiles <= QUEUE_ROWS;
+  QueueRows queue;
+  if (ranked) {
+#pragma unroll
+    for (int g = 0; g < QueueRows::G; ++g) queue.at[g] = a.positions[min(((int)threadIdx.x & 63) + 64 * g, a.num_tiles - 1)];
+  }
   PartPages pg_first;
   if (early) {
     gc.r = threadIdx.x & 15;
@@ -1284,20 +1323,27 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
       }
       tile = mine;
     }
-    known_pos = __builtin_amdgcn_readlane(row_pos, tile);
+    row = tile;
+    pos = __builtin_amdgcn_readlane(row_pos, tile);
   }
-  if (queued && a.tiles == nullptr && a.num_tiles <= 64) {
-    const int ranked = tile_of_rank(a, tile);
-    if (early && ranked != tile) {                 // (contexts of one length are in order: the pages asked for above are theirs)
-      gc.table = a.block_table + (size_t)ranked * a.table_stride;
-      load_pages(a, gc, wave, pg_first);
+  if (ranked) {
+    bool lengthy = false;
+#pragma unroll
+    for (int g = 0; g < QueueRows::G; ++g) lengthy = lengthy || queue.at[g] >= QUEUE_KEYS;
+    if (__ballot(lengthy) != 0) {
+      if (!placed) queue_place(tile, head_item);
+      tile = a.num_tiles <= 64 ? tile_of_rank<1, W>(a, queue, tile) : tile_of_rank<QueueRows::G, W>(a, queue, tile);
+      row = tile;
+      pos = a.positions[row];
+      if (early) {
+        gc.table = a.block_table + (size_t)tile * a.table_stride;
+        load_pages(a, gc, wave, pg_first);
+      }
     }
-    tile = ranked;
   }
-  const bool live = group_setup<HD, 1>(a, tile, head_item, gc, tc, known_pos);   // uniform over the workgroup
+  const bool live = group_setup<HD, 1, true>(a, tile, head_item, gc, tc, pos);   // uniform over the workgroup
   if (!SPLIT && !live) return;
   const int first = gc.kmin / ATT_PART, last = gc.kmax / ATT_PART;
-  const int row = a.tiles != nullptr ? a.tiles[tile * 4] : tile;
   if constexpr (SPLIT) {
     // A context of few partitions is one workgroup's, which folds them where it is (331 tokens of one request, 32 heads of
     // 64: 9.3 us -> 7.3).

@@ -827,7 +827,7 @@ def test_attention_prompt_tiles_equal_single_rows(gpu, bf16):
 @pytest.mark.parametrize("rows,heads,kvh,hd", [(64, 16, 16, 64), (33, 32, 16, 64), (17, 32, 32, 64), (63, 32, 16, 128), (65, 16, 16, 64)])
 def test_decode_attention_of_a_queue_equals_each_row_alone(gpu, rows, heads, kvh, hd):
     """More workgroups than places: rows are handed out by their contexts' lengths.  Contexts of all lengths, equal ones and
-    padding rows among them (65: more rows than the order covers): every row has the bits of a launch of its own."""
+    padding rows among them, none long enough to be ranked: every row has the bits of a launch of its own."""
     page, width = 16, 20
     g = torch.Generator(device=gpu).manual_seed(rows)
     pos = torch.randint(0, page * width, (rows,), generator=g, device=gpu, dtype=torch.int32)
@@ -844,6 +844,28 @@ def test_decode_attention_of_a_queue_equals_each_row_alone(gpu, rows, heads, kvh
                 ops.attention_bf16(q[r:r + 1], pos[r:r + 1].clone(), table[r:r + 1].clone(), None, 1, kc, vc, one, heads, kvh, hd, page, window, 0.125,
                                    decode=True)
                 assert torch.equal(out[r], one[0]), r
+
+
+@pytest.mark.parametrize("rows,heads,kvh,hd", [(33, 16, 16, 64), (64, 18, 9, 64), (65, 8, 8, 128), (130, 4, 4, 32), (256, 6, 3, 64), (257, 2, 2, 64)])
+def test_decode_attention_of_a_queue_with_long_contexts(gpu, rows, heads, kvh, hd):
+    """Contexts from which on the rows are ranked, up to the 256 that are (257: as they come), in whole eights and not, one
+    context just at that length or one under it, padding first, last and in between: the bits of a launch of its own."""
+    page, width = 16, 100
+    g = torch.Generator(device=gpu).manual_seed(rows)
+    table = torch.randperm(rows * width, generator=g, device=gpu).int().view(rows, width)
+    kc, vc = torch.randn(2, rows * width, kvh * page * hd, generator=g, device=gpu).bfloat16()
+    q = torch.randn(rows, heads * hd, generator=g, device=gpu).bfloat16()
+    for top, window in ((page * width, 0), (1281, 0), (1280, 0), (page * width, 200)):
+        pos = torch.randint(0, top, (rows,), generator=g, device=gpu, dtype=torch.int32)
+        pos[rows - 2], pos[5] = top - 1, top - 1
+        pos[0], pos[rows - 1], pos[rows // 2] = -1, -1, -1
+        out = torch.zeros_like(q)
+        ops.attention_bf16(q, pos, table, None, rows, kc, vc, out, heads, kvh, hd, page, window, 0.125, decode=True)
+        want = torch.zeros_like(q)
+        for r in range(rows):
+            ops.attention_bf16(q[r:r + 1], pos[r:r + 1].clone(), table[r:r + 1].clone(), None, 1, kc, vc, want[r:r + 1], heads, kvh, hd, page, window,
+                               0.125, decode=True)
+        assert torch.equal(out, want), (top, window)
 
 
 @pytest.mark.parametrize("rows,heads,kvh,hd,width", [(33, 16, 16, 64, 20), (70, 32, 8, 128, 20), (64, 12, 12, 128, 400), (100, 16, 8, 64, 20)])
