@@ -475,17 +475,21 @@ struct RopeArgs {
   const int32_t* block_table;
   const float* cos_table;    // [max_pos, hd/2]
   const float* sin_table;
-  int rows, heads, kv_heads, head_dim, page_size, table_stride, write_cache;
+  int rows, heads, kv_heads, head_dim, page_size, page_shift, table_stride, write_cache;      // (page_shift: log2 of page_size, or -1)
+  // entry of a request's table, and slot of that page
+  __device__ __forceinline__ int entry(int pos) const { return page_shift >= 0 ? pos >> page_shift : pos / page_size; }
+  __device__ __forceinline__ int slot(int pos) const { return page_shift >= 0 ? pos & (page_size - 1) : pos % page_size; }
 };
 
 // A thread takes VEC neighbouring pairs of one row and head (blocks y < qk_blocks), or a value column: every load of a row is
 // asked for at once, where a workgroup a row walked its pairs 256 at a time, a round trip to memory each (8 rows of 32
-// heads of 64 in 32 bits: 7.9 -> 4.7 us; 777 rows of 32 + 8 heads of 128 in bfloat16: 12.8 -> 9.3, 2,048 rows: 20.9 -> 17.2, of
-// which the bytes take 15).
+// heads of 64 in 32 bits: 4.7 -> 2.4 us; 777 rows of 32 + 8 heads of 128 in bfloat16: 11.5 -> 7.0, 2,048 rows: 19.5 -> 15.7, of
+// which the bytes take 15).  Pages of a power of two are found by shifts: with divisions the four rows of a value column
+// were the longest chain (64 rows of 4 + 2 heads of 16: 2.3 us a workgroup a row, 2.7 with divisions, 2.4 now).
 // 32-bit: q and k are rotated in place; k and v go to cache[page][kv_head][slot][hd] (src/model.cpp:291-296,
 // src/kernels.h:97-99).  bfloat16: rotation in 32-bit from the 32-bit projections; q goes to q_out [rows, q_dim], k to
-// cache[page][kv_head][slot][hd], v transposed to cache[page][kv_head][hd][slot], each rounded once; a thread there has
-// four rows of a value column, whose slots most often are four neighbours that start at a multiple of four: one 8-byte
+// cache[page][kv_head][slot][hd], v transposed to cache[page][kv_head][hd][slot], each rounded once; with vectors
+// a thread there has four rows of a value column, whose slots most often are four neighbours that start at a multiple of four: one 8-byte
 // store instead of four of two bytes a page row apart.
 template <int VEC>
 struct RopeVec {
@@ -526,7 +530,7 @@ __global__ __launch_bounds__(256) void rope_kvwrite_kernel(RopeArgs a, float* qk
     const int row = blockIdx.x, per_head = half / VEC;
     const int e = (int)blockIdx.y * 256 + (int)threadIdx.x;
     if (e >= (a.heads + a.kv_heads) * per_head) return;
-    const int hh = e / per_head, i = (e % per_head) * VEC;
+    const int hh = (int)((unsigned)e / (unsigned)per_head), i = (e - hh * per_head) * VEC;
     const int pos = a.positions[row];
     if (pos < 0) return;
     float* v = qkv_rw + (size_t)row * width + hh * hd + i;
@@ -547,28 +551,27 @@ __global__ __launch_bounds__(256) void rope_kvwrite_kernel(RopeArgs a, float* qk
       rope_store<VEC>(dst + half, o2);
     }
     if (hh >= a.heads && a.write_cache) {
-      const int page = a.block_table[(size_t)a.row_seq[row] * a.table_stride + pos / a.page_size];
-      CT* dst = k_cache + (((size_t)page * a.kv_heads + (hh - a.heads)) * a.page_size + pos % a.page_size) * hd + i;
+      const int page = a.block_table[(size_t)a.row_seq[row] * a.table_stride + a.entry(pos)];
+      CT* dst = k_cache + (((size_t)page * a.kv_heads + (hh - a.heads)) * a.page_size + a.slot(pos)) * hd + i;
       rope_store<VEC>(dst, o1);
       rope_store<VEC>(dst + half, o2);
     }
     return;
   }
   const int e = ((int)blockIdx.y - qk_blocks) * 256 + (int)threadIdx.x;
-  if constexpr (!BF) {
+  if constexpr (!BF || VEC == 1) {
     const int row = blockIdx.x;
     if (e * VEC >= kv_dim) return;
     const int pos = a.positions[row];
     if (pos < 0) return;
     const RopeVec<VEC> x = rope_load<VEC>(qkv_rw + (size_t)row * width + q_dim + kv_dim + e * VEC);
-    const int page = a.block_table[(size_t)a.row_seq[row] * a.table_stride + pos / a.page_size];
-    rope_store<VEC>(v_cache + (((size_t)page * a.kv_heads + (e * VEC) / hd) * a.page_size + pos % a.page_size) * hd + (e * VEC) % hd, x);
+    const int page = a.block_table[(size_t)a.row_seq[row] * a.table_stride + a.entry(pos)];
+    if constexpr (BF) rope_store<VEC>(v_cache + ((size_t)page * kv_dim + e) * a.page_size + a.slot(pos), x);
+    else rope_store<VEC>(v_cache + (((size_t)page * a.kv_heads + (e * VEC) / hd) * a.page_size + a.slot(pos)) * hd + (e * VEC) % hd, x);
   } else {
     const int row0 = 4 * (int)blockIdx.x;
     if (row0 >= a.rows || e >= kv_dim) return;
-    const int h = e / hd, d = e % hd;
-    int pos[4];
-    size_t page[4];
+    int pos[4], page[4];
     float x[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -576,10 +579,10 @@ __global__ __launch_bounds__(256) void rope_kvwrite_kernel(RopeArgs a, float* qk
       pos[t] = row0 + t < a.rows ? a.positions[row] : -1;
       x[t] = qkv_rw[(size_t)row * width + q_dim + kv_dim + e];
       const int seq = pos[t] >= 0 ? a.row_seq[row] : 0;
-      page[t] = (size_t)a.block_table[(size_t)seq * a.table_stride + (pos[t] > 0 ? pos[t] : 0) / a.page_size];
+      page[t] = a.block_table[(size_t)seq * a.table_stride + a.entry(pos[t] > 0 ? pos[t] : 0)];
     }
-    auto at = [&](int t) { return v_cache + ((page[t] * a.kv_heads + h) * hd + d) * a.page_size + pos[t] % a.page_size; };
-    const bool four = VEC == 4 && pos[0] >= 0 && (pos[0] & 3) == 0 && (a.page_size & 3) == 0 && pos[1] == pos[0] + 1 && pos[2] == pos[0] + 2 &&
+    auto at = [&](int t) { return v_cache + ((size_t)page[t] * kv_dim + e) * a.page_size + a.slot(pos[t]); };
+    const bool four = pos[0] >= 0 && (pos[0] & 3) == 0 && (a.page_size & 3) == 0 && pos[1] == pos[0] + 1 && pos[2] == pos[0] + 2 &&
                       pos[3] == pos[0] + 3 && page[1] == page[0] && page[2] == page[0] && page[3] == page[0];
     if (four) {
       *reinterpret_cast<u32x2*>(at(0)) = (u32x2){pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
@@ -607,7 +610,7 @@ extern "C" int bw_rope_kvwrite(float* qkv, void* q_out, const int32_t* positions
   if (rows <= 0) return 0;
   if (head_dim % 2 || page_size <= 0) return -2;
   RopeArgs a{qkv, positions, row_seq, block_table, cos_table, sin_table,
-             rows, heads, kv_heads, head_dim, page_size, table_stride, write_cache};
+             rows, heads, kv_heads, head_dim, page_size, page_size & (page_size - 1) ? -1 : __builtin_ctz((unsigned)page_size), table_stride, write_cache};
   hipStream_t s = (hipStream_t)stream;
   // four pairs a thread where halves of heads are whole vectors and everything starts at one
   const bool vec = head_dim % 8 == 0 && (((uintptr_t)qkv | (uintptr_t)cos_table | (uintptr_t)sin_table | (uintptr_t)k_cache | (uintptr_t)v_cache |

@@ -528,7 +528,7 @@ def test_rope_and_cache_write(gpu, bf16):
 # ----------------------------------------------------------------------------- attention
 
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("heads,kvh,hd,page", [(4, 2, 64, 16), (3, 1, 20, 4), (6, 2, 128, 8), (1, 1, 8, 2), (33, 3, 16, 64)])
+@pytest.mark.parametrize("heads,kvh,hd,page", [(4, 2, 64, 16), (3, 1, 20, 4), (6, 2, 128, 8), (1, 1, 8, 2), (33, 3, 16, 64), (2, 2, 32, 12), (2, 1, 12, 6)])
 def test_rope_of_mixed_rows_equals_the_rows_alone(gpu, bf16, heads, kvh, hd, page):
     """Portions that start anywhere in a page, single tokens and padding rows (vectors of four pairs and single ones, four
     rows of a value column and fewer): every row gets the bits it gets alone, padding and foreign slots are not written, and
