@@ -718,7 +718,7 @@ __global__ __launch_bounds__(64 * FoldShape<HD>::NW) __attribute__((amdgpu_waves
 // Here keys travel from their page straight into LDS (no registers, no LDS write instructions) and everything a wave
 // asks for has a scalar page address and an offset that never changes, which leaves registers for four waves a SIMD: two
 // workgroups share a compute unit and drift apart.  The statements per tile are those above: the same bits.
-// 2,048 queries over 8,192 keys, 32 heads of 128 on 8: 545 us -> 349 (0.69 PFLOP/s); 2,048 tokens, 32 heads of 64: 63 -> 43.
+// 2,048 queries behind 6,144 keys, 32 heads of 128 on 8, alone: 502 us -> 309 (0.78 PFLOP/s); 2,048 tokens, 32 heads of 64: 58 -> 41.
 //
 // LDS: two buffers of a partition's keys [64][HD] and values [HD][64 keys], rows without padding; the 16-byte chunks of a
 // row are permuted by the row (fold2_k_slot; the values as fold_v_offset says), so that 16 lanes which read one chunk of

@@ -264,7 +264,7 @@ static AddRoute add_route(int M, int N, int K, int ldo, int& tiles64) {
   const long long whole = ((t128 + 255) / 256) * (K / 64);
   const long long tile_split = ((t128 * S + 255) / 256) * (GEMM_SEG / 64) + join;
   const long long big_split = M >= 2 * BIG_BM ? ((tbig * S + 255) / 256) * 2 * (GEMM_SEG / 64) + join : whole;
-  // 128 x 256 tiles: a step of theirs takes 1.0 us (1.6 to 1.75 of the 128 x 128 tile's).  With all of K, the
+  // 128 x 256 tiles: a step of theirs takes 0.85 to 0.92 us (1.6 to 1.7 of the 128 x 128 tile's).  With all of K, the
   // segments joined in registers: no scratch, no join.  A workgroup per tile and segment: where that is one round of
   // the chip and 128 x 128 tiles would be two (1,024 rows of K = 8192 into 2048 columns).
   const long long t256 = (long long)((M + 127) / 128) * ((N + 255) / 256);
@@ -495,7 +495,8 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
       // tile, a head a wave as in the 128 x 128 tiles: 1,024 rows 45.8 us there)
       constexpr int COLS256 = epi_is_glu(EPI) ? 128 : 256;
       const int mt = (M + 127) / 128, nt = (N + COLS256 - 1) / COLS256;
-      // (in rounds of 256 workgroups; a step of these takes 1.0 us where a 128 x 128 tile's takes 0.58)
+      // (in rounds of 256 workgroups; a step of these takes 0.85 to 0.92 us where a 128 x 128 tile's takes 0.54 to 0.57, 1.6 to 1.7
+      // times, and prologue and epilogue some 8 us against 5: a round of K = 4096 66 us and 40)
       const int rounds256 = (mt * nt + 255) / 256, rounds128 = (mt * ((N + COLS256 / 2 - 1) / (COLS256 / 2)) + 255) / 256;
       if (K % 64 == 0 && 7 * rounds256 <= 4 * rounds128) return launch_tile256<EPI>(x, w, out, M, N, K, ldx, ldo, s, rp);
     }
