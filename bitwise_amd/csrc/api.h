@@ -37,6 +37,9 @@ int bw_gemm_f32(const float* x, const void* w, int w_is_bf16, float* y, int M, i
 int bw_gemm_f32_prompt_tile(int M, int N, int* rows, int* columns);
 int bw_gemm_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, int epilogue,
                  void* stream);
+// rows and rows of W of the tiles that a bfloat16 product of more than 64 rows gets where all of K is one workgroup's and the
+// kernels for few rows do not take it (K a multiple of 64; gated: the stacked weight of a gated epilogue)
+int bw_gemm_prompt_tile(int M, long long w_rows, int K, int gated, int* rows, int* columns);
 int bw_gemm_clamped_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, float limit,
                              float alpha, void* stream);
 int bw_gemm_add_scratch(int M, int N, int K, long long* scratch_floats, int* counters);

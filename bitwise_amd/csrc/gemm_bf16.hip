@@ -27,22 +27,18 @@
 //         works because loads complete in the order they are issued and nothing else is loaded meanwhile;
 //       - anything else (K no multiple of 64, SwiGLU with few columns): the "skinny" kernel, a wave per strip
 //         and segment streaming through a ring of registers;
-//   * more rows (prompt portions): 128 x 128 x 64 tiles, eight waves, fed through a four-stage LDS ring by the
-//     same kind of loads ("tile128"; several segments are joined in registers, or for the residual add added
-//     into the output as they end), and for products with at least 128 tiles of 256 x 256 the "big" kernel,
-//     which computes twice as much per byte it fetches (a ring of five 32 KB slots, operand reads pipelined
-//     under the matrix instructions; one segment, or for a residual add with scratch a workgroup per tile and
-//     segment, the segments' sums joined in order by a second kernel); 128 x 256 tiles ("tile256": eight waves of
-//     64 x 64, room in the registers for the sums of the segments before) where they make fewer rounds of the compute
-//     units than the 128 x 128 ones by enough, which is where K has several segments and the big kernel does not
-//     run; the "wide" kernel (128 x 128 tiles staged through registers by four waves) takes what those do not: K no
-//     multiple of 64.
+//   * more rows (prompt portions): tiles of 128 x 128 to 256 x 256 outputs, eight waves, steps of 64 along K fed through
+//     rings in LDS by the same kind of loads (gemm_bf16_ring.h); the shape is the one whose rounds of the compute units
+//     take the least time.  Several segments are joined in registers, or, for a residual add with scratch and few tiles, a
+//     workgroup per tile and segment leaves its sums for a second kernel that joins them in order.  The "wide" kernel (128 x
+//     128 tiles staged through registers by four waves) takes K that is no multiple of 64.
 //
 // Epilogues: store 32-bit, store bfloat16, add into a 32-bit residual (each output owned
 // by one lane: no atomics), SwiGLU of two products (gate rows n, up rows N+n of a
 // stacked weight) stored as bfloat16: h = g * (1/(1+exp(-g))) * u in 32-bit, the exact GELU stored as bfloat16, or rotary encoding of the
 // stacked q|k|v product and the write of k and v to their page slots (heads of 64; up to 64 rows: head sizes
 // in multiples of 64).
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -179,6 +175,7 @@ static int chain_record_rows(int kind, const RowsCall& c, int wgs, int waves, in
 
 #include "gemm_bf16_skinny.h"
 #include "gemm_bf16_tiles.h"
+#include "gemm_bf16_ring.h"
 #include "gemm_bf16_rows.h"
 #include "gemm_bf16_phases.h"
 
@@ -188,7 +185,7 @@ static int chain_record_rows(int kind, const RowsCall& c, int wgs, int waves, in
 // as there are compute units, if the product has them), a workgroup per tile and segment of K if there are several
 // (they meet in device scratch the caller brings).  tiles 0: it does not run there.
 // out = (((out + p[0]) + p[1]) + ...) + p[S-1], element by element: the segments of a residual add that
-// gemm_bf16_big_kernel left in scratch ([S][M][N]), joined in segment order (ADD false: a store, the chain starts at p[0]).
+// the tiles left in scratch ([S][M][N]), joined in segment order (ADD false: a store, the chain starts at p[0]).
 template <bool ADD>
 __global__ __launch_bounds__(256) void add_segments_kernel(float* __restrict__ out, const float* __restrict__ parts, int S,
                                                            int M, int N, int ldo) {
@@ -212,26 +209,23 @@ static void add_rows_shape(int M, int N, int K, int& tiles, bool& narrow) {
   if (tiles * S < 32) tiles = 0;
 }
 
-// How a residual add of more than 64 rows is laid out.  One workgroup of the tile kernels fits a compute unit, so
-// a product goes in rounds of 256 workgroups, and a workgroup that has all of K to itself takes K / 64 steps
-// whatever else is idle: an output of 2048 columns and 128 rows is 16 tiles (76 us for K = 8192).
-//   whole       128 x 128 tiles with all of K, each finished segment added into the output: needs no scratch.
-//   row blocks  the kernel for up to 64 rows once per block of 64 rows, with its workgroup per 32 or 64 columns and
-//               segment of K (its scratch if K has several segments): up to 128 rows and three segments, where a
-//               launch more costs less than the join below (K = 2048: 16 and 19 us at 65 and 128 rows, for 24).
-//   tile split  a 128 x 128 workgroup per tile and segment, the segments' sums whole in scratch and joined in order
-//               afterwards (128 rows of K = 8192: 25 us).
-//   big split   the same with 256 x 256 tiles, which fetch half as many bytes a flop: for 512 rows or more.
-//   tile256     128 x 256 tiles with all of K, the segments joined in registers: needs no scratch.
-//   blocks at once  one segment of K only: the kernel for up to 64 rows with all blocks of 64 rows in one launch (its
+// How a residual add (or 32-bit store) of more than 64 rows is laid out.
+//   blocks at once  the kernel for up to 64 rows with all blocks of 64 rows in one launch (its
 //               grid's third dimension), while the workgroups fit the chip at once (512): the output projection of
 //               2048 columns takes 8.4 us at 128 rows and 13.3 at 512, where 128 x 128 tiles took 16.4 and 21.6.  The
 //               q|k|v product with rotation and cache write goes the same way (launch_qkv_rope_mid).
-// All five give the same bits.  The choice is by a count of steps: rounds times the steps of a workgroup (a step of
-// a 256 x 256 tile counts twice); the join moves 8 bytes an element and segment (about 500,000 elements in the
-// time of a step) and is a launch more (8 steps); a split has to win by a tenth.  tiles64: what the 64-row
-// kernel's scratch is sized by.
-enum AddRoute { ADD_WHOLE, ADD_ROW_BLOCKS, ADD_TILE_SPLIT, ADD_BIG_SPLIT, ADD_TILE256, ADD_TILE256_SPLIT };
+//   row blocks  the kernel for up to 64 rows once per block of 64 rows, with its workgroup per 32 or 64 columns and
+//               segment of K (its scratch if K has several segments): up to 128 rows and three segments, where a
+//               launch more costs less than the join below (K = 2048: 16 and 19 us at 65 and 128 rows, for 24).
+//   whole       a workgroup per tile with all of K, the segments joined in registers: needs no scratch.
+//   split       a workgroup per tile and segment, the segments' sums whole in scratch and joined in order
+//               afterwards: where few tiles of all of K would leave most of the chip idle (128 rows of 2048 columns are 16
+//               of 128 x 128, each 128 steps long for K = 8192: 76 us; 25 split).
+// All give the same bits.  Which shapes are asked to bring scratch for a split is a count of rounds and steps
+// (add_takes_scratch: what callers size their scratch by, so it stays as it is while the kernels change); whether one that
+// brings it is split or goes whole, and in which tiles, the estimated times decide (add_split_shape).
+// tiles64: what the 64-row kernel's scratch is sized by.
+enum AddRoute { ADD_WHOLE, ADD_ROW_BLOCKS, ADD_SPLIT };
 
 // "Blocks at once" for a residual add of more than 64 rows: how many blocks of 64 rows, tiles of 64 or (narrow) 32
 // columns; tiles 0: it does not run that way (more than 512 workgroups, or too few to matter).  Several segments of K
@@ -249,6 +243,21 @@ static void add_blocks_shape(int M, int N, int K, int& tiles, bool& narrow, int&
   if (t * zb * S >= 32 && t * zb * S <= ADD_BLOCKS_MAX_WGS) tiles = t;
 }
 
+// Steps of a round times rounds, a step of 256 x 256 tiles counted as two of 128 x 128 and one of 128 x 256 as 8/5 (with
+// all of K) or 7/4; the join as the steps it takes time for.  Scratch where a split of some shape saves a tenth.
+static bool add_takes_scratch(int M, int N, int K, int ldo) {
+  const int S = (K + GEMM_SEG - 1) / GEMM_SEG;
+  if (S < 2 || N % 4 || ldo % 4) return false;
+  auto tiles = [&](int rows, int cols) { return (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols); };
+  auto rounds = [](long long wgs) { return (wgs + 255) / 256; };
+  const long long seg = GEMM_SEG / 64, join = (long long)S * M * N / 500000 + 8;
+  const long long whole = rounds(tiles(128, 128)) * (K / 64), whole256 = rounds(tiles(128, 256)) * (K / 64) * 8 / 5;
+  const long long by128 = rounds(tiles(128, 128) * S) * seg + join, by256 = rounds(tiles(128, 256) * S) * seg * 7 / 4 + join;
+  const long long by_big = M >= 512 ? rounds(tiles(256, 256) * S) * 2 * seg + join : whole;
+  const long long split = std::min(std::min(by128, by_big), by256);
+  return !(whole256 < whole && whole256 <= split) && 10 * split < 9 * whole;
+}
+
 static AddRoute add_route(int M, int N, int K, int ldo, int& tiles64) {
   const int S = (K + GEMM_SEG - 1) / GEMM_SEG;
   tiles64 = 0;
@@ -257,25 +266,26 @@ static AddRoute add_route(int M, int N, int K, int ldo, int& tiles64) {
   add_rows_shape(64, N, K, tiles64, narrow);
   if (tiles64 && M <= 128 && S <= 3) return ADD_ROW_BLOCKS;
   tiles64 = 0;
-  if (S < 2 || N % 4 || ldo % 4) return ADD_WHOLE;
-  const long long t128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
-  const long long tbig = (long long)((M + BIG_BM - 1) / BIG_BM) * ((N + 255) / 256);
-  const long long join = (long long)S * M * N / 500000 + 8;
-  const long long whole = ((t128 + 255) / 256) * (K / 64);
-  const long long tile_split = ((t128 * S + 255) / 256) * (GEMM_SEG / 64) + join;
-  const long long big_split = M >= 2 * BIG_BM ? ((tbig * S + 255) / 256) * 2 * (GEMM_SEG / 64) + join : whole;
-  // 128 x 256 tiles: a step of theirs takes 0.85 to 0.92 us (1.6 to 1.7 of the 128 x 128 tile's).  With all of K, the
-  // segments joined in registers: no scratch, no join.  A workgroup per tile and segment: where that is one round of
-  // the chip and 128 x 128 tiles would be two (1,024 rows of K = 8192 into 2048 columns).
-  const long long t256 = (long long)((M + 127) / 128) * ((N + 255) / 256);
-  const long long whole256 = ((t256 + 255) / 256) * (K / 64) * 8 / 5;
-  const long long t256_split = ((t256 * S + 255) / 256) * (GEMM_SEG / 64) * 7 / 4 + join;
-  const long long split3 = tile_split <= big_split ? tile_split : big_split;
-  const long long split = t256_split < split3 ? t256_split : split3;
-  if (whole256 < whole && whole256 <= split) return ADD_TILE256;
-  if (10 * split >= 9 * whole) return ADD_WHOLE;
-  if (t256_split < split3) return ADD_TILE256_SPLIT;
-  return tile_split <= big_split ? ADD_TILE_SPLIT : ADD_BIG_SPLIT;
+  return add_takes_scratch(M, N, K, ldo) ? ADD_SPLIT : ADD_WHOLE;
+}
+
+// The tiles of a split that takes less time than all of K a workgroup; -1: none does.  The join is a launch (3 us) and moves 8
+// bytes an element and segment and 8 more an element, the stores of the sums among them (2048 x 2048, four segments: 28 us in
+// all), at about 7 TB/s.
+static int add_split_shape(int M, int N, int K) {
+  const int S = (K + GEMM_SEG - 1) / GEMM_SEG;
+  long long least;
+  int shape = -1;
+  ring_choice(M, N, K, false, &least);
+  const long long join = (8LL * S + 8) * M * N / 70000 + 300;
+  for (int i = 0; i < RING_SHAPES; ++i) {
+    const long long t = ring_time(ring_costs[i], ring_tiles(ring_costs[i], M, N) * S, GEMM_SEG) + join;
+    if (t < least) {
+      least = t;
+      shape = i;
+    }
+  }
+  return shape;
 }
 
 template <int EPI>
@@ -404,7 +414,7 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
       }
       int tiles;
       AddRoute route = add_route(M, N, K, ldo, tiles);
-      // (a store has whole-K kernels with larger tiles further down: it splits only what leaves compute units idle there)
+      // (a store splits only what leaves compute units idle)
       if (EPI == EPI_F32 && ((M + 127) / 128) * ((N + 127) / 128) >= 256) route = ADD_WHOLE;
       if (EPI == EPI_ADD_F32 && route == ADD_ROW_BLOCKS && (size_t)M * ldx * 2 < ((size_t)1 << 31) &&
           (S == 1 || (sp.scratch != nullptr && sp.counters != nullptr && scratch_floats >= (size_t)tiles * S * 4096 &&
@@ -416,47 +426,17 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
         }
         return 0;
       }
-      if (EPI == EPI_ADD_F32 && route == ADD_TILE256) return launch_tile256<EPI>(x, w, out, M, N, K, ldx, ldo, s);
-      if (route == ADD_BIG_SPLIT && sp.scratch != nullptr && ((uintptr_t)out & 15) == 0) {
+      if (route == ADD_SPLIT && sp.scratch != nullptr && ((uintptr_t)out & 15) == 0) {
         if (scratch_floats < (size_t)S * M * N) return -6;
-        const int bm = (M + BIG_BM - 1) / BIG_BM, bn = (N + 255) / 256;
-        static bool allowed = false;                 // more than 64 KB of dynamic LDS has to be asked for once
-        if (!allowed) {
-          (void)hipFuncSetAttribute((const void*)gemm_bf16_big_kernel<EPI_F32>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    BIG_SLOTS * BIG_SLOT);
-          allowed = true;
+        const int shape = add_split_shape(M, N, K);
+        if (shape >= 0) {
+          const int rc = launch_ring<EPI_F32>(shape, x, w, (void*)sp.scratch, M, N, K, ldx, N, s, QkvRopeArgs{}, S, (size_t)M * N);
+          if (rc) return rc;
+          const size_t quads = (size_t)M * (N >> 2);
+          BW_LAUNCH(add_segments_kernel<EPI == EPI_ADD_F32>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, (float*)out, sp.scratch, S,
+                             M, N, ldo);
+          return BW_LAUNCH_CHECK();
         }
-        BW_LAUNCH((gemm_bf16_big_kernel<EPI_F32>), dim3(bm * bn, S), dim3(512), BIG_SLOTS * BIG_SLOT, s, x, w,
-                           (void*)sp.scratch, M, N, K, ldx, N, bm, bn, rp, (size_t)M * N);
-        const size_t quads = (size_t)M * (N >> 2);
-        BW_LAUNCH(add_segments_kernel<EPI == EPI_ADD_F32>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, (float*)out, sp.scratch, S,
-                           M, N, ldo);
-        return BW_LAUNCH_CHECK();
-      }
-      if (route == ADD_TILE256_SPLIT && sp.scratch != nullptr && ((uintptr_t)out & 15) == 0) {
-        if (scratch_floats < (size_t)S * M * N) return -6;
-        const int rc = launch_tile256<EPI_F32>(x, w, (void*)sp.scratch, M, N, K, ldx, N, s, QkvRopeArgs{}, S, (size_t)M * N);
-        if (rc) return rc;
-        const size_t quads = (size_t)M * (N >> 2);
-        BW_LAUNCH(add_segments_kernel<EPI == EPI_ADD_F32>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, (float*)out, sp.scratch, S,
-                           M, N, ldo);
-        return BW_LAUNCH_CHECK();
-      }
-      if (route == ADD_TILE_SPLIT && sp.scratch != nullptr && ((uintptr_t)out & 15) == 0) {
-        if (scratch_floats < (size_t)S * M * N) return -6;
-        const int mt = (M + 127) / 128, nt = (N + 127) / 128;
-        static bool allowed = false;
-        if (!allowed) {
-          (void)hipFuncSetAttribute((const void*)gemm_bf16_tile128_kernel<EPI_F32>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    T128_STAGES * T128_STAGE);
-          allowed = true;
-        }
-        BW_LAUNCH((gemm_bf16_tile128_kernel<EPI_F32>), dim3(mt * nt, S), dim3(512), T128_STAGES * T128_STAGE, s, x, w,
-                           (void*)sp.scratch, M, N, K, ldx, N, mt, nt, rp, (size_t)M * N);
-        const size_t quads = (size_t)M * (N >> 2);
-        BW_LAUNCH(add_segments_kernel<EPI == EPI_ADD_F32>, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, (float*)out, sp.scratch, S,
-                           M, N, ldo);
-        return BW_LAUNCH_CHECK();
       }
     }
     if constexpr (EPI == EPI_F32 || EPI == EPI_BF16 || EPI == EPI_GELU_BF16) {
@@ -466,57 +446,12 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
       if (K % 64 == 0 && wgs >= 64 && wgs * zb <= ADD_BLOCKS_MAX_WGS && (size_t)M * ldx * 2 < ((size_t)1 << 31))
         return launch_mid<EPI, 4, false>(x, w, out, M, N, K, ldx, ldo, wgs, s, MidNormArgs{}, QkvRopeArgs{}, 1, MidSplitArgs{}, zb);
     }
-    if constexpr (EPI != EPI_ADD_F32) {
-      // enough 256-row tiles to go round the compute units (a second round at least half full)
-      constexpr int BIG_COLS = epi_is_glu(EPI) ? 128 : 256;
-      const int bm = (M + BIG_BM - 1) / BIG_BM, bn = (N + BIG_COLS - 1) / BIG_COLS;
-      // (fewer of these tiles than compute units while the 128-row tiles below would fill the chip in one round: a step
-      // of those takes half as long, so they win: gate|up of 512 rows 62 us here, half the chip idle)
-      bool half_tiles_win = false;
-      if constexpr (EPI == EPI_F32 || EPI == EPI_BF16 || EPI == EPI_GELU_BF16 || epi_is_glu(EPI)) {
-        const int t256 = ((M + 127) / 128) * bn;
-        half_tiles_win = (t256 + 255) / 256 < 2 * ((bm * bn + 255) / 256);
-      }
-      if (S == 1 && K % 64 == 0 && M >= 2 * BIG_BM && bm * bn >= 128 && !half_tiles_win) {
-        static bool allowed = false;                 // more than 64 KB of dynamic LDS has to be asked for once
-        if (!allowed) {
-          (void)hipFuncSetAttribute((const void*)gemm_bf16_big_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    BIG_SLOTS * BIG_SLOT);
-          allowed = true;
-        }
-        BW_LAUNCH((gemm_bf16_big_kernel<EPI>), dim3(bm * bn), dim3(512), BIG_SLOTS * BIG_SLOT, s, x, w, out, M, N, K, ldx,
-                           ldo, bm, bn, rp, (size_t)0);
-        return BW_LAUNCH_CHECK();
-      }
-    }
-    if constexpr (EPI == EPI_F32 || EPI == EPI_BF16 || EPI == EPI_GELU_BF16 || epi_is_glu(EPI) || EPI == EPI_QKV_ROPE) {
-      // 128 x 256 tiles where they go round the compute units (the 256 x 256 kernel above took what it takes: one
-      // segment of K and enough of its tiles); the q|k|v product of 600 to 1,200 rows among them (four heads of 64 a
-      // tile, a head a wave as in the 128 x 128 tiles: 1,024 rows 45.8 us there)
-      constexpr int COLS256 = epi_is_glu(EPI) ? 128 : 256;
-      const int mt = (M + 127) / 128, nt = (N + COLS256 - 1) / COLS256;
-      // (in rounds of 256 workgroups; a step of these takes 0.85 to 0.92 us where a 128 x 128 tile's takes 0.54 to 0.57, 1.6 to 1.7
-      // times, and prologue and epilogue some 8 us against 5: a round of K = 4096 66 us and 40)
-      const int rounds256 = (mt * nt + 255) / 256, rounds128 = (mt * ((N + COLS256 / 2 - 1) / (COLS256 / 2)) + 255) / 256;
-      if (K % 64 == 0 && 7 * rounds256 <= 4 * rounds128) return launch_tile256<EPI>(x, w, out, M, N, K, ldx, ldo, s, rp);
-    }
+    // K in whole steps of 64: tiles through LDS rings, of the shape that takes the least time
+    if (K % 64 == 0)
+      return launch_ring<EPI>(ring_choice(M, epi_is_glu(EPI) ? 2LL * N : N, K, epi_is_glu(EPI), nullptr), x, w, out, M, N, K, ldx, ldo, s, rp);
     constexpr int COLS = epi_is_glu(EPI) ? 64 : 128;
     const int m_tiles = (M + WIDE_BM - 1) / WIDE_BM, n_tiles = (N + COLS - 1) / COLS;
     dim3 grid(m_tiles * n_tiles), block(256);
-    {
-      // K in whole steps of 64: the tiles go straight into an LDS ring
-      if (K % 64 == 0) {
-        static bool allowed = false;                   // more than 64 KB of dynamic LDS has to be asked for once
-        if (!allowed) {
-          (void)hipFuncSetAttribute((const void*)gemm_bf16_tile128_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    T128_STAGES * T128_STAGE);
-          allowed = true;
-        }
-        BW_LAUNCH((gemm_bf16_tile128_kernel<EPI>), grid, dim3(512), T128_STAGES * T128_STAGE, s, x, w, out, M, N, K, ldx,
-                           ldo, m_tiles, n_tiles, rp, (size_t)0);
-        return BW_LAUNCH_CHECK();
-      }
-    }
     if (S > 1)
       BW_LAUNCH((gemm_bf16_wide_kernel<EPI, true, false>), grid, block, 0, s, x, w, out, M, N, K, ldx, ldo, m_tiles, n_tiles, rp);
     else if (K % (2 * WIDE_BK) == 0)
@@ -543,7 +478,7 @@ extern "C" int bw_gemm_add_scratch(int M, int N, int K, long long* scratch_float
     }
   }
   const AddRoute route = M > 64 && N > 0 ? add_route(M, N, K, 4, tiles) : ADD_WHOLE;
-  if (route == ADD_TILE_SPLIT || route == ADD_BIG_SPLIT || route == ADD_TILE256_SPLIT) {      // a prompt portion: the segments' sums, whole
+  if (route == ADD_SPLIT) {      // a prompt portion: the segments' sums, whole
     *scratch_floats = (long long)S * M * N;
     *counters = 1;                                          // (none is used)
     return 0;

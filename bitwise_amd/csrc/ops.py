@@ -50,6 +50,7 @@ _SIGS = {
     "bw_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_clamped_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],
     "bw_gemm_f32_prompt_tile": [c_int, c_int, c_void_p, c_void_p],
+    "bw_gemm_prompt_tile": [c_int, c_longlong, c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_add_scratch": [c_int, c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_add_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_longlong, c_void_p,
                          c_int, c_void_p],
@@ -157,7 +158,7 @@ _fns = {}
 # what waits.
 _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
-    "bw_gemm_f32_prompt_tile", "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
+    "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
     "bw_chain_flush", "bw_chain_end",
 })
@@ -453,6 +454,14 @@ def gemm_f32_prompt_tile(rows: int, N: int) -> Tuple[int, int]:
     """(rows, columns) of the tiles that ``gemm_f32`` gives a product of more than 64 rows, K in whole stages of 32."""
     r, c = ctypes.c_int(0), ctypes.c_int(0)
     _check(_fn("bw_gemm_f32_prompt_tile")(rows, N, ctypes.addressof(r), ctypes.addressof(c)), "gemm_f32_prompt_tile")
+    return int(r.value), int(c.value)
+
+
+def gemm_prompt_tile(rows: int, w_rows: int, K: int, gated: bool = False) -> Tuple[int, int]:
+    """(rows, rows of W) of the tiles that ``gemm_bf16`` gives a product of more than 64 rows, K in whole steps of 64, where
+    all of K is one workgroup's and the kernels for few rows do not take it."""
+    r, c = ctypes.c_int(0), ctypes.c_int(0)
+    _check(_fn("bw_gemm_prompt_tile")(rows, w_rows, K, int(gated), ctypes.addressof(r), ctypes.addressof(c)), "gemm_prompt_tile")
     return int(r.value), int(c.value)
 
 

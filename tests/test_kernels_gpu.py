@@ -159,6 +159,45 @@ def test_gemm_f32_prompt_tiles_are_the_chains_of_few_rows(gpu, M, N, K, wdt):
         assert torch.equal(added[r:r + n], base[r:r + n] + want[r:r + n])
 
 
+BF16_PROMPT_TILES = {       # tile -> products (M, rows of W, K) that the rule gives it, at the edges of its rows, columns and steps
+    (128, 128): [(65, 200, 64), (129, 2100, 2112), (300, 1000, 4160)],
+    (128, 256): [(385, 12000, 2048), (300, 16000, 4160), (193, 16000, 192)],
+    (160, 256): [(700, 12000, 2112), (1345, 6144, 2048), (577, 16000, 2112)],
+    (192, 256): [(641, 16000, 192), (513, 16000, 4096)],
+    (256, 192): [(2040, 6136, 2112), (2000, 6000, 1024), (2047, 6140, 2048)],
+    (256, 256): [(1345, 8200, 64), (2047, 16000, 64), (1500, 8200, 192)],
+}
+
+
+def test_gemm_bf16_prompt_products_reach_every_tile():
+    for tile, shapes in BF16_PROMPT_TILES.items():
+        assert [ops.gemm_prompt_tile(M, N, K) for M, N, K in shapes] == [tile] * len(shapes)
+    assert ops.gemm_prompt_tile(1345, 8200, 64, gated=True) == (256, 256)
+    for M, K in ((64, 64), (65, 72)):
+        with pytest.raises(RuntimeError, match="out of the kernel's range"):
+            ops.gemm_prompt_tile(M, 200, K)
+
+
+@pytest.mark.parametrize("M,N,K", sum(BF16_PROMPT_TILES.values(), []))
+def test_gemm_bf16_prompt_tiles_are_the_bits_of_few_rows(gpu, M, N, K):
+    """Every tile of the bfloat16 prompt products: the bits of the same rows given sixteen at a time (kernels for few rows),
+    stored, added and gated, from rows farther apart than they are long."""
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    wide = torch.randn(M, K + 16, generator=g, device=gpu).bfloat16()
+    x, w = wide[:, :K], (torch.randn(N, K, generator=g, device=gpu) * K ** -0.5).bfloat16()
+    base = torch.randn(M, N, generator=g, device=gpu)
+    for epi, cols, dtype in ((ops.EPI_F32, N, torch.float32), (ops.EPI_ADD_F32, N, torch.float32), (ops.EPI_SWIGLU_BF16, N // 2, torch.bfloat16)):
+        got = base.clone() if epi == ops.EPI_ADD_F32 else torch.full((M, cols), 7.0, device=gpu, dtype=dtype)
+        ops.gemm_bf16(x, w, got, M, epi)
+        for r in sorted({0, 16, 112, 128, 144, 160, 176, 192, 240, M // 32 * 16, (M - 1) // 16 * 16}):
+            n = min(16, M - r)
+            if n <= 0:
+                continue
+            want = base[r:r + n].clone() if epi == ops.EPI_ADD_F32 else torch.zeros(n, cols, device=gpu, dtype=dtype)
+            ops.gemm_bf16(x[r:r + n], w, want, n, epi)
+            assert torch.equal(got[r:r + n], want), (epi, r)
+
+
 def test_gemm_bf16_rows_shapes_and_epilogues(gpu):
     g = torch.Generator().manual_seed(3)
     for M, N, K in [(1, 16, 32), (5, 100, 64), (16, 64, 96), (17, 500, 96), (50, 300, 608), (130, 96, 224), (33, 72, 40),
@@ -1138,6 +1177,38 @@ def test_fused_norm_products_equal_the_separate_kernels(gpu):
         live = [0, 1, 2, 3, 4, 6]                                  # the row with position -1 is padding
         assert torch.equal(outs[0][0][live], outs[1][0][live])
         assert torch.equal(outs[0][1], outs[1][1]) and torch.equal(outs[0][2], outs[1][2])
+
+
+@pytest.mark.parametrize("heads,kvh,M,tile", [(72, 12, 700, (128, 256)), (71, 13, 1345, (160, 256)), (125, 17, 1000, (192, 256)),
+                                              (71, 12, 2041, (256, 192)), (75, 11, 2041, (256, 256))])
+def test_rotary_epilogue_of_every_prompt_tile(gpu, heads, kvh, M, tile):
+    """q|k|v of heads of 64 in each tile shape, last tiles ragged in rows and heads: the bits of product + rope_kvwrite."""
+    K, page = 1024, 16
+    assert ops.gemm_prompt_tile(M, (heads + 2 * kvh) * 64, K) == tile
+    g = torch.Generator(device=gpu).manual_seed(M)
+    h = torch.randn(M, K, generator=g, device=gpu).bfloat16()
+    w = (torch.randn((heads + 2 * kvh) * 64, K, generator=g, device=gpu) * 0.05).bfloat16()
+    cos, sin = rope_tables(10000.0, 64, M + 8, gpu)
+    pos = [r if r < M // 2 else r - M // 2 + 3 for r in range(M)]
+    pos[7] = pos[2] = pos[M - 2] = -1
+    positions = torch.tensor(pos, dtype=torch.int32, device=gpu)
+    row_seq = torch.tensor([int(r >= M // 2) for r in range(M)], dtype=torch.int32, device=gpu)
+    per = M // page + 2
+    table = torch.randperm(2 * per, generator=torch.Generator().manual_seed(M)).to(torch.int32).view(2, per).to(gpu)
+    outs = []
+    for fused in (False, True):
+        kc = torch.full((2 * per, kvh * page * 64), 3.0, dtype=torch.bfloat16, device=gpu)
+        vc = torch.full((2 * per, kvh * page * 64), 3.0, dtype=torch.bfloat16, device=gpu)
+        q = torch.zeros(M, heads * 64, dtype=torch.bfloat16, device=gpu)
+        if fused:
+            ops.gemm_qkv_rope_bf16(h, w, q, positions, row_seq, table, cos, sin, kc, vc, M, heads, kvh, 64, page)
+        else:
+            qkv = torch.zeros(M, w.shape[0], device=gpu)
+            ops.gemm_bf16(h, w, qkv, M, ops.EPI_F32)
+            ops.rope_kvwrite(qkv, q, positions, row_seq, table, cos, sin, kc, vc, M, heads, kvh, 64, page)
+        outs.append((q[positions >= 0], kc, vc))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
 
 
 def test_prompt_qkv_product_with_rotary_epilogue_equals_the_separate_kernels(gpu):
