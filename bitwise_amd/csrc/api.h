@@ -42,6 +42,8 @@ int bw_gemm_bf16(const void* x, const void* w, void* out, int M, int N, int K, i
 int bw_gemm_prompt_tile(int M, long long w_rows, int K, int gated, int* rows, int* columns);
 int bw_gemm_clamped_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, float limit,
                              float alpha, void* stream);
+// the same with the GELU (tanh form) of the gate instead of the clamped unit
+int bw_gemm_gelu_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, void* stream);
 int bw_gemm_add_scratch(int M, int N, int K, long long* scratch_floats, int* counters);
 // out = bf16(gelu_tanh(x W^T) * table[token of the row]): up to 16 rows, K in steps of 64, fewer than 4,096 columns (-7: another shape)
 int bw_gemm_side_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, const int32_t* tokens,

@@ -103,6 +103,13 @@ __device__ __forceinline__ float gelu_tanh(float z) {
   return 0.5f * z * (1.0f + tanhf(inner));
 }
 
+// The gated GELU (tanh form), gelu(g) u, as the activation kernel and the products' epilogue both compute it: one sequence of
+// operations, so both give the same bits.
+__device__ __forceinline__ float gelu_tanh_times(float g, float u) {
+  const float inner = 0.7978845608028654f * (g + 0.044715f * ((g * g) * g));
+  return ((0.5f * g) * (1.0f + tanhf(inner))) * u;
+}
+
 // Lane exchanges from register to register (no trip through LDS).  The halves and quarters of the wave by gfx950's
 // lane swaps: of (v, v) swapped, the first result holds in every lane the value of its partner or its own in the
 // lower half (32: lanes 0-31; 16: the even rows of 16 lanes), the second the one in the upper half; an operation

@@ -132,6 +132,7 @@ __device__ __forceinline__ void epilogue_store(void* __restrict__ out, size_t o,
   else if constexpr (EPI == EPI_ADD_F32) st_f32<DEV>((float*)out + o, ld_f32<DEV>((const float*)out + o) + v);
   else if constexpr (EPI == EPI_SWIGLU_BF16) st_bf16<DEV>((bf16_t*)out + o, f32_to_bf16(silu_times(v, u)));
   else if constexpr (EPI == EPI_CLAMPED_GLU_BF16) st_bf16<DEV>((bf16_t*)out + o, f32_to_bf16(clamped_swish_times<true>(v, u, limit, alpha)));
+  else if constexpr (EPI == EPI_GELU_GLU_BF16) st_bf16<DEV>((bf16_t*)out + o, f32_to_bf16(gelu_tanh_times(v, u)));
 }
 
 // EPI_SIDE_BF16 (up to 16 rows): an output is the GELU (tanh form) of its sum times the element of its row's token in a table, rounded
@@ -297,8 +298,8 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
   // a 32-bit store may give the segments of K workgroups of their own, too, where the caller brings the scratch
   const bool split_ok = sp.scratch != nullptr && sp.counters != nullptr;
   if (M <= 64) {
-    // (the rotary epilogue belongs to the wide kernel; the clamped unit of few rows is a kernel behind the 32-bit product)
-    if constexpr (EPI == EPI_QKV_ROPE || EPI == EPI_CLAMPED_GLU_BF16) return -2;
+    // (the rotary epilogue belongs to the wide kernel; the clamped and the GELU unit of few rows are a kernel behind the 32-bit product)
+    if constexpr (EPI == EPI_QKV_ROPE || EPI == EPI_CLAMPED_GLU_BF16 || EPI == EPI_GELU_GLU_BF16) return -2;
     else {
       // one segment and enough columns: the rows of x are shared through LDS
       constexpr int MID_COLS = epi_is_glu(EPI) ? 32 : 64;
@@ -558,6 +559,16 @@ extern "C" int bw_gemm_clamped_glu_bf16(const void* x, const void* w, void* out,
   rp.glu_alpha = alpha;
   return launch_gemm_bf16<EPI_CLAMPED_GLU_BF16>((const bf16_t*)x, (const bf16_t*)w, out, M, N, K, ldx, ldo,
                                                 (hipStream_t)stream, rp);
+}
+
+// The same with the GELU (tanh form) of the gate: out[m, n] = bf16(gelu(x.W[n]) (x.W[N + n])).  The bits of gemm_bf16
+// (32-bit store) + glu.
+extern "C" int bw_gemm_gelu_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, void* stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (M <= 64) return -2;
+  if (K <= 0 || (K % 8) || (ldx % 8) || ldx < K || ldo < N) return -2;
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) return -3;
+  return launch_gemm_bf16<EPI_GELU_GLU_BF16>((const bf16_t*)x, (const bf16_t*)w, out, M, N, K, ldx, ldo, (hipStream_t)stream);
 }
 
 // The stacked q|k|v product with rotation and cache write in its epilogue (heads of 64 elements, K of one

@@ -54,6 +54,7 @@ struct RingTile {
 template <int EPI>
 __device__ __forceinline__ float glu_value(float g, float u, const QkvRopeArgs& rp) {
   if constexpr (EPI == EPI_CLAMPED_GLU_BF16) return clamped_swish_times<true>(g, u, rp.glu_limit, rp.glu_alpha);
+  else if constexpr (EPI == EPI_GELU_GLU_BF16) return gelu_tanh_times(g, u);
   else return silu_times(g, u);
 }
 

@@ -49,6 +49,7 @@ _SIGS = {
     "bw_gemm_f32": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_clamped_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],
+    "bw_gemm_gelu_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_f32_prompt_tile": [c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_prompt_tile": [c_int, c_longlong, c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_add_scratch": [c_int, c_int, c_int, c_void_p, c_void_p],
@@ -512,7 +513,7 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows: int, ep
                                epilogue, _stream()), "gemm_bf16")
 
 
-CLAMPED_GLU_MIN_ROWS = 65      # steps of fewer rows run the clamped unit as a kernel behind the 32-bit product
+CLAMPED_GLU_MIN_ROWS = 65      # steps of fewer rows run the clamped and the GELU unit as a kernel behind the 32-bit product
 
 
 def gemm_clamped_glu_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows: int, limit: float, alpha: float) -> None:
@@ -536,6 +537,23 @@ def gemm_clamped_glu_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, r
 # ------------------------------------------------------------------------------ decode fusions
 
 _decode_ok = {}
+
+
+def gemm_gelu_glu_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows: int) -> None:
+    """out[:rows, n] = bf16(gelu(x . w[n]) (x . w[N + n])), the tanh form: the stacked product [2N, K] of a prompt portion (more
+    than 64 rows) with the gated GELU in its epilogue; the bits of gemm_bf16 with a 32-bit store followed by ``glu``."""
+    _need(x, torch.bfloat16, "x")
+    _need(w, torch.bfloat16, "weight")
+    _need(out, torch.bfloat16, "out")
+    if w.dim() != 2 or w.shape[0] % 2:
+        raise ValueError("gemm_gelu_glu_bf16: weight must be the stacked [2N, K]")
+    N, K = w.shape[0] // 2, w.shape[1]
+    if x.shape[1] != K or out.shape[1] != N or x.shape[0] < rows or out.shape[0] < rows:
+        raise ValueError(f"gemm_gelu_glu_bf16: x {tuple(x.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not match")
+    if rows < CLAMPED_GLU_MIN_ROWS or K % 8:
+        raise ValueError("gemm_gelu_glu_bf16: more than 64 rows and an inner size in multiples of 8")
+    _check(_fn("bw_gemm_gelu_glu_bf16")(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, N, K, x.stride(0), out.stride(0),
+                                        _stream()), "gemm_gelu_glu_bf16")
 
 
 def norm_gemm_supported(rows: int, inner: int) -> bool:

@@ -1106,8 +1106,7 @@ __global__ void glu_kernel(const float* __restrict__ gu, int ldg, OT* __restrict
   float g = gu[row * ldg + c], u = gu[row * ldg + inter + c];
   float h;
   if (act == ACT_GELU_TANH) {
-    const float inner = 0.7978845608028654f * (g + 0.044715f * ((g * g) * g));
-    h = ((0.5f * g) * (1.0f + tanhf(inner))) * u;
+    h = gelu_tanh_times(g, u);
   } else if (act == ACT_CLAMPED_SWISH) {
     h = clamped_swish_times<sizeof(OT) == 2>(g, u, limit, alpha);
   } else {

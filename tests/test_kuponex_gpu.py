@@ -490,3 +490,38 @@ def test_decays_made_ahead_equal_decays_made_in_the_walk(gpu, dim, vdim):
     for s in (state, state_s):
         got = s[1].double().view(heads, vdim, dim).transpose(1, 2)
         assert ((got - S).abs() <= 210 * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("rows,inter,width", [(65, 64, 64), (130, 136, 72), (513, 512, 192), (700, 6000, 2112), (1345, 4100, 64)])
+def test_gelu_unit_in_the_products_epilogue(gpu, rows, inter, width):
+    """Prompt portions compute the gated GELU in the stacked product's epilogue: the bits of the 32-bit product followed by the
+    activation kernel, and the float64 values to one bfloat16 rounding and the sums' own error; gates of every size among
+    them, infinities and NaN where the product has them."""
+    from bitwise_amd.csrc import ops
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, width, generator=g).bfloat16()
+    w = (torch.randn(2 * inter, width, generator=g) * (3.0 / width ** 0.5)).bfloat16()
+    xd, wd = x.to(gpu), w.to(gpu)
+    fused = torch.zeros(rows, inter, dtype=torch.bfloat16, device=gpu)
+    ops.gemm_gelu_glu_bf16(xd, wd, fused, rows)
+    sums = torch.zeros(rows, 2 * inter, device=gpu)
+    ops.gemm_bf16(xd, wd, sums, rows, ops.EPI_F32)
+    apart = torch.zeros(rows, inter, dtype=torch.bfloat16, device=gpu)
+    ops.glu(sums, apart, rows, ops.ACT_GELU_TANH)
+    assert torch.equal(fused.view(torch.int16), apart.view(torch.int16))
+    a, b = sums.double().split(inter, dim=1)
+    want = torch.nn.functional.gelu(a, approximate="tanh") * b
+    # half a bfloat16 step of the value, and the rounding of 1 + tanh beside it
+    assert ((fused.double() - want).abs() <= 2.0 ** -8 * want.abs() * 1.01 + 2.0 ** -21 * (a * b).abs()).all()
+    few = torch.zeros(64, 2 * inter, device=gpu)
+    ops.gemm_bf16(xd[:64].contiguous(), wd, few, 64, ops.EPI_F32)
+    ops.glu(few, apart, 64, ops.ACT_GELU_TANH)
+    assert torch.equal(fused[:64].view(torch.int16), apart[:64].view(torch.int16))
+    edges = torch.tensor([[float("inf"), -float("inf"), float("nan"), 0.0, -0.0, 3e38, -3e38, 40.0, -40.0, 1e-30, -5.5, 2.0],
+                          [1.0] * 12], device=gpu).view(1, 24)
+    out = torch.zeros(1, 12, dtype=torch.bfloat16, device=gpu)
+    ops.glu(edges, out, 1, ops.ACT_GELU_TANH)
+    inf = float("inf")
+    got = out[0].float().cpu()
+    assert got[0] == inf and got[1].isnan() and got[2].isnan() and got[3] == 0 and got[4] == 0 and got[5] > 2.9e38 and got[6] == 0
+    assert got[7] == 40 and got[8] == 0 and abs(got[9] / 5e-31 - 1) < 2 ** -7 and abs(got[11] - 1.9545977) < 2 ** -7
