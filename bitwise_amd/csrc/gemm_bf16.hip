@@ -441,10 +441,11 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
       }
     }
     if constexpr (EPI == EPI_F32 || EPI == EPI_BF16 || EPI == EPI_GELU_BF16) {
-      // few enough workgroups of the 64-row kernel to be on the chip at once: all blocks of 64 rows in one launch (a
-      // product of 6144 columns at 128 rows 13 us against 20 on 128 x 128 tiles; the SwiGLU product gains nothing)
+      // two blocks of 64 rows and few enough workgroups of the 64-row kernel to be on the chip at once: both in one launch (6144
+      // columns of K = 2048 at 128 rows 11.9 us against 13.2 in 64 x 128 tiles; three blocks 14.6 against 13.5, five 16.9
+      // against 14.3, and K = 4096 likewise)
       const int wgs = (N + 63) / 64, zb = (M + 63) / 64;
-      if (K % 64 == 0 && wgs >= 64 && wgs * zb <= ADD_BLOCKS_MAX_WGS && (size_t)M * ldx * 2 < ((size_t)1 << 31))
+      if (K % 64 == 0 && wgs >= 64 && zb <= 2 && wgs * zb <= ADD_BLOCKS_MAX_WGS && (size_t)M * ldx * 2 < ((size_t)1 << 31))
         return launch_mid<EPI, 4, false>(x, w, out, M, N, K, ldx, ldo, wgs, s, MidNormArgs{}, QkvRopeArgs{}, 1, MidSplitArgs{}, zb);
     }
     // K in whole steps of 64: tiles through LDS rings, of the shape that takes the least time

@@ -411,13 +411,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // The shapes, and how long a round of the compute units takes with one (hundredths of a microsecond, all 256 at work):
 // ``step`` for each 64 of K, ``ends`` for its first loads and its epilogue.  Measured on products of 2,048 rows whose tiles are
 // whole rounds, K = 2048 and 4096.  A tile of 256 x 256 has no registers left for the sums of earlier segments.
-enum { RING_128, RING_128X256, RING_160X256, RING_192X256, RING_256X192, RING_256X256, RING_SHAPES };
+// (The two of 8,192 outputs are for products that would leave half of the chip idle in larger ones: gate|up of 117 x 16384 x 2048
+// 23.4 us in 128 x 128 tiles, 18.6 in 128 x 64; 320 rows of 6144 x 2048 18.7 and 14.3 in 64 x 128.)
+enum { RING_128, RING_128X256, RING_160X256, RING_192X256, RING_256X192, RING_256X256, RING_128X64, RING_64X128, RING_SHAPES };
 struct RingCost {
   int rows, cols, step, ends;
   bool joins;
 };
 static const RingCost ring_costs[RING_SHAPES] = {{128, 128, 52, 650, true},  {128, 256, 81, 750, true},  {160, 256, 98, 750, true},
-                                                 {192, 256, 107, 840, true}, {256, 192, 117, 940, true}, {256, 256, 141, 900, false}};
+                                                 {192, 256, 107, 840, true}, {256, 192, 117, 940, true}, {256, 256, 141, 900, false},
+                                                 {128, 64, 38, 500, true},   {64, 128, 38, 500, true}};
 
 // The time of a product's tiles in that measure.  A last round that is part empty runs faster than a full one, the memory and
 // the L2s being shared by fewer (0.6 of its time at the least; 160 x 256 tiles of 777 x 28672 x 4096, 2.19 rounds: 190 us
@@ -476,6 +479,8 @@ static int launch_ring(int shape, const bf16_t* x, const bf16_t* w, void* out, i
   constexpr bool JOIN = EPI != EPI_QKV_ROPE;     // (the rotary product has one segment)
   switch (shape) {
     case RING_128: return launch_ring_shape<EPI, 2, 4, 2, JOIN>(x, w, out, M, N, K, ldx, ldo, s, rp, segments, seg_stride);
+    case RING_128X64: return launch_ring_shape<EPI, 4, 2, 2, JOIN>(x, w, out, M, N, K, ldx, ldo, s, rp, segments, seg_stride);
+    case RING_64X128: return launch_ring_shape<EPI, 2, 2, 2, JOIN>(x, w, out, M, N, K, ldx, ldo, s, rp, segments, seg_stride);
     case RING_128X256: return launch_ring_shape<EPI, 2, 4, 4, JOIN>(x, w, out, M, N, K, ldx, ldo, s, rp, segments, seg_stride);
     case RING_160X256: return launch_ring_shape<EPI, 2, 5, 4, JOIN>(x, w, out, M, N, K, ldx, ldo, s, rp, segments, seg_stride);
     case RING_192X256: return launch_ring_shape<EPI, 2, 6, 4, JOIN>(x, w, out, M, N, K, ldx, ldo, s, rp, segments, seg_stride);

@@ -160,7 +160,9 @@ def test_gemm_f32_prompt_tiles_are_the_chains_of_few_rows(gpu, M, N, K, wdt):
 
 
 BF16_PROMPT_TILES = {       # tile -> products (M, rows of W, K) that the rule gives it, at the edges of its rows, columns and steps
-    (128, 128): [(65, 200, 64), (129, 2100, 2112), (300, 1000, 4160)],
+    (128, 128): [(330, 6144, 64), (600, 4090, 4160), (1200, 2040, 2112), (200, 8200, 128)],
+    (128, 64): [(65, 200, 64), (117, 16380, 2112), (128, 8192, 4096), (500, 2100, 64)],
+    (64, 128): [(190, 6144, 2048), (257, 6100, 4160), (320, 6144, 192), (129, 2100, 2112)],
     (128, 256): [(385, 12000, 2048), (300, 16000, 4160), (193, 16000, 192)],
     (160, 256): [(700, 12000, 2112), (1345, 6144, 2048), (577, 16000, 2112)],
     (192, 256): [(641, 16000, 192), (513, 16000, 4096)],
@@ -1179,7 +1181,8 @@ def test_fused_norm_products_equal_the_separate_kernels(gpu):
         assert torch.equal(outs[0][1], outs[1][1]) and torch.equal(outs[0][2], outs[1][2])
 
 
-@pytest.mark.parametrize("heads,kvh,M,tile", [(72, 12, 700, (128, 256)), (71, 13, 1345, (160, 256)), (125, 17, 1000, (192, 256)),
+@pytest.mark.parametrize("heads,kvh,M,tile", [(71, 13, 300, (64, 128)), (101, 12, 250, (128, 64)), (71, 13, 384, (128, 128)),
+                                              (72, 12, 700, (128, 256)), (71, 13, 1345, (160, 256)), (125, 17, 1000, (192, 256)),
                                               (71, 12, 2041, (256, 192)), (75, 11, 2041, (256, 256))])
 def test_rotary_epilogue_of_every_prompt_tile(gpu, heads, kvh, M, tile):
     """q|k|v of heads of 64 in each tile shape, last tiles ragged in rows and heads: the bits of product + rope_kvwrite."""
