@@ -563,7 +563,7 @@ extern "C" int bw_gemm_clamped_glu_bf16(const void* x, const void* w, void* out,
 }
 
 // The same with the GELU (tanh form) of the gate: out[m, n] = bf16(gelu(x.W[n]) (x.W[N + n])).  The bits of gemm_bf16
-// (32-bit store) + glu.
+// (32-bit store) + glu, which at 2,048 rows of 2 x 8192 columns and K = 2048 write and read 134 MB of sums: 122 + 38 us -> 121.
 extern "C" int bw_gemm_gelu_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, void* stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M <= 64) return -2;
