@@ -278,9 +278,15 @@ static int add_split_shape(int M, int N, int K) {
   long long least;
   int shape = -1;
   ring_choice(M, N, K, false, &least);
+  // (up to 192 rows the weights' way from memory takes the time, not the matrix cores: rounds and steps are counted as where
+  // scratch is asked for.  4096 columns of K = 14336, 130 rows: 43 us, 50 by the times below; 6144 of K = 4096 22 and 24.)
+  if (M <= 192) {
+    const long long wgs128 = ring_tiles(ring_costs[RING_128], M, N) * S, wgs256 = ring_tiles(ring_costs[RING_128X256], M, N) * S;
+    return (wgs256 + 255) / 256 * 7 < (wgs128 + 255) / 256 * 4 ? RING_128X256 : RING_128;
+  }
   const long long join = (8LL * S + 8) * M * N / 70000 + 300;
   for (int i = 0; i < RING_SHAPES; ++i) {
-    const long long t = ring_time(ring_costs[i], ring_tiles(ring_costs[i], M, N) * S, GEMM_SEG) + join;
+    const long long t = ring_time(ring_costs[i], ring_tiles(ring_costs[i], M, N) * S, GEMM_SEG, false) + join;
     if (t < least) {
       least = t;
       shape = i;
@@ -443,9 +449,9 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
     if constexpr (EPI == EPI_F32 || EPI == EPI_BF16 || EPI == EPI_GELU_BF16) {
       // two blocks of 64 rows and few enough workgroups of the 64-row kernel to be on the chip at once: both in one launch (6144
       // columns of K = 2048 at 128 rows 11.9 us against 13.2 in 64 x 128 tiles; three blocks 14.6 against 13.5, five 16.9
-      // against 14.3, and K = 4096 likewise)
+      // against 14.3; of K = 4096 three blocks 23 against 24.5, four 27.4 against 25.6)
       const int wgs = (N + 63) / 64, zb = (M + 63) / 64;
-      if (K % 64 == 0 && wgs >= 64 && zb <= 2 && wgs * zb <= ADD_BLOCKS_MAX_WGS && (size_t)M * ldx * 2 < ((size_t)1 << 31))
+      if (K % 64 == 0 && wgs >= 64 && zb <= (S == 1 ? 2 : 3) && wgs * zb <= ADD_BLOCKS_MAX_WGS && (size_t)M * ldx * 2 < ((size_t)1 << 31))
         return launch_mid<EPI, 4, false>(x, w, out, M, N, K, ldx, ldo, wgs, s, MidNormArgs{}, QkvRopeArgs{}, 1, MidSplitArgs{}, zb);
     }
     // K in whole steps of 64: tiles through LDS rings, of the shape that takes the least time

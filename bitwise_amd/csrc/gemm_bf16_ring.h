@@ -45,6 +45,9 @@ struct RingTile {
   // loads of a wave that are younger than those of the next step, when a step has issued all of its own
   static constexpr int YOUNGER = (DA - 1) * LA + (DB - 1) * LB;
   static constexpr int U = 2 * MI;                                 // a step's turns: one block of x rows times NJ blocks of W rows
+  // Three or four steps of both in LDS: the turn before which load n of a step is issued.  The first of them stand behind the
+  // barrier, in the last two turns (-2, -1) of the step before, whose slots they overwrite.
+  static constexpr int turn(int n) { return n * U / (LA + LB) - 2; }
   static constexpr int NA = U % 4 == 0 && MI < 6 ? 4 : (U % 3 == 0 ? 3 : (U % 4 == 0 ? 4 : 5));   // registers' ring of x blocks; divides U
   static constexpr int BPT = (NJ + MI - 2) / (MI - 1);             // W blocks of the second half read a turn
   static constexpr int B_FROM = MI - 1 - (NJ + BPT - 1) / BPT;     // and from which turn on
@@ -174,6 +177,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   __builtin_amdgcn_s_waitcnt(vmcnt_only(T::YOUNGER));
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
+  if constexpr (!T::MID) {
+#pragma unroll
+    for (int n = 0; n < T::LA + T::LB; ++n)
+      if (T::turn(n) < 0) {
+        if (n < T::LA) issue_a(T::RA - 1, T::RA - 1, n);
+        else issue_b(T::RB - 1, T::RB - 1, n - T::LA);
+      }
+  }
 #pragma unroll
   for (int j = 0; j < NJ; ++j) read_b(0, 0, j);
   read_a(0, 0, 0, 0);
@@ -205,7 +216,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       } else
 #pragma unroll
       for (int n = 0; n < T::LA + T::LB; ++n)
-        if (n * (U - 2) / (T::LA + T::LB) == u) {
+        if (T::turn(n) == u) {
           if (n < T::LA) issue_a(step + T::RA - 1, sa_fill, n);
           else issue_b(step + T::RB - 1, sb_fill, n - T::LA);
         }
@@ -215,6 +226,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         __builtin_amdgcn_s_waitcnt(vmcnt_only(T::YOUNGER) & ~0x0f00);
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+      }
+      if constexpr (!T::MID) {
+        // (this step's own slots, from here on)
+#pragma unroll
+        for (int n = 0; n < T::LA + T::LB; ++n)
+          if (T::turn(n) + U == u) {
+            if (n < T::LA) issue_a(step + T::RA, sa, n);
+            else issue_b(step + T::RB, sb, n - T::LA);
+          }
       }
       __builtin_amdgcn_sched_barrier(0);
       if (u + 2 < U) read_a(sa, (u + 2) / MI, (u + 2) % MI, (u + 2) % NA);
@@ -424,10 +444,11 @@ static const RingCost ring_costs[RING_SHAPES] = {{128, 128, 52, 650, true},  {12
 
 // The time of a product's tiles in that measure.  A last round that is part empty runs faster than a full one, the memory and
 // the L2s being shared by fewer (0.6 of its time at the least; 160 x 256 tiles of 777 x 28672 x 4096, 2.19 rounds: 190 us
-// against 67.5 a full round).
-static long long ring_time(const RingCost& c, long long tiles, int K) {
+// against 67.5 a full round); not where one tile takes all rows: the weights' way through fewer compute units is what takes
+// the time there (130 x 28672 x 4096: 112 tiles of 160 x 256 69 us, 224 of 128 x 256 60).
+static long long ring_time(const RingCost& c, long long tiles, int K, bool one_row_tile) {
   const long long last = tiles % 256;
-  const long long rounds256 = tiles / 256 * 256 + (last ? 154 + last * 102 / 256 : 0);
+  const long long rounds256 = tiles / 256 * 256 + (last ? (one_row_tile ? 256 : 154 + last * 102 / 256) : 0);
   return rounds256 * ((long long)(K / 64) * c.step + c.ends) / 256;
 }
 static long long ring_tiles(const RingCost& c, int M, long long cols) { return (long long)((M + c.rows - 1) / c.rows) * ((cols + c.cols - 1) / c.cols); }
@@ -439,7 +460,7 @@ static int ring_choice(int M, long long cols, int K, bool gated, long long* time
   for (int i = 0; i < RING_SHAPES; ++i) {
     if (K > GEMM_SEG && !ring_costs[i].joins) continue;
     if (gated && i == RING_256X192) continue;
-    const long long t = ring_time(ring_costs[i], ring_tiles(ring_costs[i], M, cols), K);
+    const long long t = ring_time(ring_costs[i], ring_tiles(ring_costs[i], M, cols), K, M <= ring_costs[i].rows);
     if (least < 0 || t < least) {
       least = t;
       best = i;

@@ -161,8 +161,8 @@ def test_gemm_f32_prompt_tiles_are_the_chains_of_few_rows(gpu, M, N, K, wdt):
 
 BF16_PROMPT_TILES = {       # tile -> products (M, rows of W, K) that the rule gives it, at the edges of its rows, columns and steps
     (128, 128): [(330, 6144, 64), (600, 4090, 4160), (1200, 2040, 2112), (200, 8200, 128)],
-    (128, 64): [(65, 200, 64), (117, 16380, 2112), (128, 8192, 4096), (500, 2100, 64)],
-    (64, 128): [(190, 6144, 2048), (257, 6100, 4160), (320, 6144, 192), (129, 2100, 2112)],
+    (128, 64): [(117, 16380, 2112), (500, 2100, 2112), (500, 2100, 64)],
+    (64, 128): [(65, 200, 64), (128, 8192, 4096), (190, 6144, 2048), (257, 6100, 4160), (320, 6144, 192), (129, 2100, 2112)],
     (128, 256): [(385, 12000, 2048), (300, 16000, 4160), (193, 16000, 192)],
     (160, 256): [(700, 12000, 2112), (1345, 6144, 2048), (577, 16000, 2112)],
     (192, 256): [(641, 16000, 192), (513, 16000, 4096)],
