@@ -541,8 +541,9 @@ _decode_ok = {}
 
 def gemm_gelu_glu_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows: int) -> None:
     """out[:rows, n] = bf16(gelu(x . w[n]) (x . w[N + n])), the tanh form: the stacked product [2N, K] of a prompt portion (more
-    than 64 rows) with the gated GELU in its epilogue; the bits of gemm_bf16 with a 32-bit store followed by ``glu``."""
-    _need(x, torch.bfloat16, "x")
+    than 64 rows) with the gated GELU in its epilogue; the bits of gemm_bf16 with a 32-bit store followed by ``glu``.  ``x`` may be a
+    column slice of a wider matrix, as there."""
+    _need_strided(x, torch.bfloat16, "x")
     _need(w, torch.bfloat16, "weight")
     _need(out, torch.bfloat16, "out")
     if w.dim() != 2 or w.shape[0] % 2:

@@ -525,3 +525,20 @@ def test_gelu_unit_in_the_products_epilogue(gpu, rows, inter, width):
     got = out[0].float().cpu()
     assert got[0] == inf and got[1].isnan() and got[2].isnan() and got[3] == 0 and got[4] == 0 and got[5] > 2.9e38 and got[6] == 0
     assert got[7] == 40 and got[8] == 0 and abs(got[9] / 5e-31 - 1) < 2 ** -7 and abs(got[11] - 1.9545977) < 2 ** -7
+
+
+def test_gelu_unit_takes_rows_of_a_wider_matrix(gpu):
+    """Rows that are a column slice of a wider matrix, as the 32-bit store that the epilogue stands for takes them; rows whose
+    elements do not lie next to each other stay refused."""
+    from bitwise_amd.csrc import ops
+    g = torch.Generator().manual_seed(12)
+    wide = torch.randn(200, 320, generator=g).bfloat16().to(gpu)
+    w = (torch.randn(2 * 96, 192, generator=g) * 0.1).bfloat16().to(gpu)
+    want, got = (torch.zeros(200, 96, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    ops.gemm_gelu_glu_bf16(wide[:, 64:256].contiguous(), w, want, 200)
+    ops.gemm_gelu_glu_bf16(wide[:, 64:256], w, got, 200)
+    assert torch.equal(want, got) and want.any()
+    with pytest.raises(ValueError, match="rows are contiguous"):
+        ops.gemm_gelu_glu_bf16(wide.T[:200], w[:, :200].contiguous(), got, 200)
+    with pytest.raises(RuntimeError):
+        ops.gemm_gelu_glu_bf16(wide[:, 3:195], w, got, 200)          # (16-byte loads: not from any column)
