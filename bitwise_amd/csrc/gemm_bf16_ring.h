@@ -345,9 +345,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       bool quad = pos4[0] >= 0 && (pos4[0] & 3) == 0;
 #pragma unroll
       for (int t = 1; t < 4; ++t) quad = quad && pos4[t] == pos4[0] + t && page4[t] == page4[0];
+      // (one or two pairs a wave belong to one head, and the stores to a row of it lie next to each other: by pairs instead, a
+      // row's second half eight stores behind its first, 256 x 256 tiles took 3 us a round more)
+      constexpr int OF_HEAD = NH <= 2 ? NH : 1;
 #pragma unroll
-      for (int j = 0; j < NH; ++j) {
-        const int p = NH * wx + j, head = first_head + (p >> 1), d = 16 * (p & 1) + r;    // pairs (d, d + 32) of the head
+      for (int j0 = 0; j0 < NH; j0 += OF_HEAD) {
+        const int p0 = NH * wx + j0, head = first_head + (p0 >> 1);
         if (head < rp.heads + rp.kv_heads) {
           if (head >= rp.heads && !rp.write_cache) continue;
 #pragma unroll
@@ -358,28 +361,36 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             bf16_t* dst = head < rp.heads
                               ? (bf16_t*)out + (size_t)m * q_dim + (size_t)head * 64
                               : rp.k_cache + (((size_t)page4[q] * rp.kv_heads + (head - rp.heads)) * rp.page_size + (pos & (rp.page_size - 1))) * 64;
-            const float c = cos_lds[(lrow0 + q) * CS + d], sn = sin_lds[(lrow0 + q) * CS + d];
-            const float x1 = acc[i][j][q], x2 = acc[i][j + NH][q];
-            dst[d] = f32_to_bf16(x1 * c - x2 * sn);
-            dst[d + 32] = f32_to_bf16(x2 * c + x1 * sn);
+#pragma unroll
+            for (int j = j0; j < j0 + OF_HEAD; ++j) {
+              const int d = 16 * ((p0 & 1) + j - j0) + r;           // pairs (d, d + 32) of the head
+              const float c = cos_lds[(lrow0 + q) * CS + d], sn = sin_lds[(lrow0 + q) * CS + d];
+              const float x1 = acc[i][j][q], x2 = acc[i][j + NH][q];
+              dst[d] = f32_to_bf16(x1 * c - x2 * sn);
+              dst[d + 32] = f32_to_bf16(x2 * c + x1 * sn);
+            }
           }
         } else if (head < rp.heads + 2 * rp.kv_heads && rp.write_cache) {
           const int vh = head - rp.heads - rp.kv_heads;
-          if (quad) {
-            bf16_t* dst = rp.v_cache + ((size_t)page4[0] * rp.kv_heads + vh) * 64 * rp.page_size + (pos4[0] & (rp.page_size - 1));
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const f32x4& a = acc[i][j + h * NH];
-              const u32x2 four = {pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])};
-              *reinterpret_cast<u32x2*>(dst + (size_t)(d + 32 * h) * rp.page_size) = four;
-            }
-          } else {
+          for (int j = j0; j < j0 + OF_HEAD; ++j) {
+            const int d = 16 * ((p0 & 1) + j - j0) + r;
+            if (quad) {
+              bf16_t* dst = rp.v_cache + ((size_t)page4[0] * rp.kv_heads + vh) * 64 * rp.page_size + (pos4[0] & (rp.page_size - 1));
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              if (pos4[q] < 0) continue;
-              bf16_t* dst = rp.v_cache + ((size_t)page4[q] * rp.kv_heads + vh) * 64 * rp.page_size + (pos4[q] & (rp.page_size - 1));
+              for (int h = 0; h < 2; ++h) {
+                const f32x4& a = acc[i][j + h * NH];
+                const u32x2 four = {pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])};
+                *reinterpret_cast<u32x2*>(dst + (size_t)(d + 32 * h) * rp.page_size) = four;
+              }
+            } else {
 #pragma unroll
-              for (int h = 0; h < 2; ++h) dst[(size_t)(d + 32 * h) * rp.page_size] = f32_to_bf16(acc[i][j + h * NH][q]);
+              for (int q = 0; q < 4; ++q) {
+                if (pos4[q] < 0) continue;
+                bf16_t* dst = rp.v_cache + ((size_t)page4[q] * rp.kv_heads + vh) * 64 * rp.page_size + (pos4[q] & (rp.page_size - 1));
+#pragma unroll
+                for (int h = 0; h < 2; ++h) dst[(size_t)(d + 32 * h) * rp.page_size] = f32_to_bf16(acc[i][j + h * NH][q]);
+              }
             }
           }
         }
