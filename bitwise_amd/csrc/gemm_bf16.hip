@@ -212,9 +212,10 @@ static void add_rows_shape(int M, int N, int K, int& tiles, bool& narrow) {
 
 // How a residual add (or 32-bit store) of more than 64 rows is laid out.
 //   blocks at once  the kernel for up to 64 rows with all blocks of 64 rows in one launch (its
-//               grid's third dimension), while the workgroups fit the chip at once (512): the output projection of
-//               2048 columns takes 8.4 us at 128 rows and 13.3 at 512, where 128 x 128 tiles took 16.4 and 21.6.  The
-//               q|k|v product with rotation and cache write goes the same way (launch_qkv_rope_mid).
+//               grid's third dimension), while the workgroups fit the chip at once (512; a store of one segment: as
+//               store_in_blocks has it): the output projection of 2048 columns takes 8.4 us at 128 rows and 13.3 at 512,
+//               where 128 x 128 tiles took 16.4 and 21.6.  The q|k|v product with rotation and cache write goes the
+//               same way (launch_qkv_rope_mid).
 //   row blocks  the kernel for up to 64 rows once per block of 64 rows, with its workgroup per 32 or 64 columns and
 //               segment of K (its scratch if K has several segments): up to 128 rows and three segments, where a
 //               launch more costs less than the join below (K = 2048: 16 and 19 us at 65 and 128 rows, for 24).
@@ -242,6 +243,19 @@ static void add_blocks_shape(int M, int N, int K, int& tiles, bool& narrow, int&
   narrow = wide * zb * S < 192;
   const int t = narrow ? (N + 31) / 32 : wide;
   if (t * zb * S >= 32 && t * zb * S <= ADD_BLOCKS_MAX_WGS) tiles = t;
+}
+
+// A store of more than 64 rows and one workgroup for all of K: the 64-row kernel with all blocks of 64 rows in one launch, or
+// tiles?  While every workgroup has a compute unit to itself (256) the blocks take 0.75 to 0.9 of the tiles' time at any K; two of
+// them on a compute unit take turns, and from 257 to 512 workgroups the blocks win only where K is short (0.96 to 1.03 of the tiles'
+// time at K = 512, 1.04 to 1.17 at K = 2048; the exact GELU's many instructions run beside the other's products: 0.85 to 0.96 up to K = 1024),
+// up to 384 of them at K = 2048 for the GELU (0.95 to 0.99) and for three blocks (192 rows of 8192 columns 15.4 us and 17.0), and up to 320
+// for K of several segments (0.92 to 1.02; 1.04 to 1.4 beyond).
+static bool store_in_blocks(int M, int N, int K, bool erf) {
+  const long long wgs = (long long)((N + 63) / 64) * ((M + 63) / 64);
+  if (K <= (erf ? 1024 : 512)) return wgs <= 512;
+  if (K <= GEMM_SEG) return wgs <= (erf || M <= 192 ? 384 : 256);
+  return wgs <= 320;
 }
 
 // Steps of a round times rounds, a step of 256 x 256 tiles counted as two of 128 x 128 and one of 128 x 256 as 8/5 (with
@@ -410,6 +424,8 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
         int tiles, zb;
         bool narrow;
         add_blocks_shape(M, N, K, tiles, narrow, zb);
+        // (a store of one segment whose workgroups would share compute units: by time, further down)
+        if (EPI == EPI_F32 && S == 1 && !narrow && !store_in_blocks(M, N, K, false)) tiles = 0;
         const bool scratch_ok = S == 1 || (split_ok &&
                                            scratch_floats >= (size_t)tiles * zb * S * 4096 && num_counters >= tiles * zb);
         if (tiles && scratch_ok) {
@@ -447,11 +463,8 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
       }
     }
     if constexpr (EPI == EPI_F32 || EPI == EPI_BF16 || EPI == EPI_GELU_BF16) {
-      // two blocks of 64 rows and few enough workgroups of the 64-row kernel to be on the chip at once: both in one launch (6144
-      // columns of K = 2048 at 128 rows 11.9 us against 13.2 in 64 x 128 tiles; three blocks 14.6 against 13.5, five 16.9
-      // against 14.3; of K = 4096 three blocks 23 against 24.5, four 27.4 against 25.6)
       const int wgs = (N + 63) / 64, zb = (M + 63) / 64;
-      if (K % 64 == 0 && wgs >= 64 && zb <= (S == 1 ? 2 : 3) && wgs * zb <= ADD_BLOCKS_MAX_WGS && (size_t)M * ldx * 2 < ((size_t)1 << 31))
+      if (K % 64 == 0 && wgs >= 64 && store_in_blocks(M, N, K, EPI == EPI_GELU_BF16) && (size_t)M * ldx * 2 < ((size_t)1 << 31))
         return launch_mid<EPI, 4, false>(x, w, out, M, N, K, ldx, ldo, wgs, s, MidNormArgs{}, QkvRopeArgs{}, 1, MidSplitArgs{}, zb);
     }
     // K in whole steps of 64: tiles through LDS rings, of the shape that takes the least time

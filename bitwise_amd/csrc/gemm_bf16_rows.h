@@ -590,8 +590,8 @@ static int launch_qkv_rope_mid(const bf16_t* x, int ldx, const bf16_t* w_qkv, vo
   if (M > 64) {
     // a short prompt portion: blocks of 64 rows in one launch, while all of them fit the chip at once
     const int zb = (M + 63) / 64;
-    // (heads of 64 and one segment of K: more than three blocks are faster in tiles; 96 heads, K = 2048: 160 rows 16.8 us here
-    // and 17.1 there, 192 18.7 and 18.2, 256 20.5 and 18.0, 320 23.3 and 18.8)
+    // (heads of 64 and one segment of K: more than three blocks are faster in tiles.  64 to 192 heads, K of 256 to 2048, both ways
+    // timed: tiles take 0.64 to 0.92 of the time with four blocks and more, 0.62 to 0.96 with three, 0.56 to 1.27 with two)
     if (wide_tiles * zb > 512 || (hd == 64 && K <= GEMM_SEG && zb > 3)) return -7;
     if (2 * wide_tiles * zb <= 256 && wide_tiles < ROPE_NARROW_BELOW)      // (half heads only while they leave compute units idle)
       return launch_mid<EPI_QKV_ROPE, 4, false, true>(x, w_qkv, q_out, M, N, K, ldx, ldo, 2 * wide_tiles, s, MidNormArgs{}, rp, 1,
