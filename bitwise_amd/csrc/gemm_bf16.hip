@@ -27,7 +27,7 @@
 //         works because loads complete in the order they are issued and nothing else is loaded meanwhile;
 //       - anything else (K no multiple of 64, SwiGLU with few columns): the "skinny" kernel, a wave per strip
 //         and segment streaming through a ring of registers;
-//   * more rows (prompt portions): tiles of 128 x 128 to 256 x 256 outputs, eight waves, steps of 64 along K fed through
+//   * more rows (prompt portions): tiles of 8,192 to 65,536 outputs (64 x 128 to 256 x 256), eight waves, steps of 64 along K fed through
 //     rings in LDS by the same kind of loads (gemm_bf16_ring.h); the shape is the one whose rounds of the compute units
 //     take the least time.  Several segments are joined in registers, or, for a residual add with scratch and few tiles, a
 //     workgroup per tile and segment leaves its sums for a second kernel that joins them in order.  The "wide" kernel (128 x
@@ -469,7 +469,7 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
     }
     // K in whole steps of 64: tiles through LDS rings, of the shape that takes the least time
     if (K % 64 == 0)
-      return launch_ring<EPI>(ring_choice(M, epi_is_glu(EPI) ? 2LL * N : N, K, epi_is_glu(EPI), nullptr), x, w, out, M, N, K, ldx, ldo, s, rp);
+      return launch_ring<EPI>(ring_choice(M, epi_is_glu(EPI) ? 2LL * N : N, K, epi_is_glu(EPI), nullptr, EPI == EPI_GELU_BF16), x, w, out, M, N, K, ldx, ldo, s, rp);
     constexpr int COLS = epi_is_glu(EPI) ? 64 : 128;
     const int m_tiles = (M + WIDE_BM - 1) / WIDE_BM, n_tiles = (N + COLS - 1) / COLS;
     dim3 grid(m_tiles * n_tiles), block(256);

@@ -480,38 +480,47 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // The shapes, and how long a round of the compute units takes with one (hundredths of a microsecond, all 256 at work):
-// ``step`` for each 64 of K, ``ends`` for its first loads and its epilogue.  Measured on products of 2,048 rows whose tiles are
-// whole rounds, K = 2048 and 4096.  A tile of 256 x 256 has no registers left for the sums of earlier segments.
+// ``step`` for each 64 of K, ``ends`` for its first loads and its epilogue, ``brief`` the same for one or two steps, where nothing
+// hides either and tiles of twice the size take more nearly twice as long, ``erf`` what the exact GELU adds, ``far`` what a step takes
+// more from K = 4096 on (64 x 128: its rows are fewer than its rows of W, which come from memory and not from the L2s where K
+// is long: 320 rows of 4096 x 4096 29 us, 25 in 128 x 64; of K = 14336 101 and 78).  Measured on products of 65 to 2,048 rows, 512 to 14336
+// columns and K of 64 to 14336, every shape timed at each; over those with K of 512 or more a product takes 0.7 % more than in the
+// shape that is best for it (mean; 7 % in one of 100).
+// A tile of 256 x 256 has no registers left for the sums of earlier segments.
 // (The two of 8,192 outputs are for products that would leave half of the chip idle in larger ones: gate|up of 117 x 16384 x 2048
 // 23.4 us in 128 x 128 tiles, 18.6 in 128 x 64; 320 rows of 6144 x 2048 18.7 and 14.3 in 64 x 128.)
 enum { RING_128, RING_128X256, RING_160X256, RING_192X256, RING_256X192, RING_256X256, RING_128X64, RING_64X128, RING_SHAPES };
 struct RingCost {
-  int rows, cols, step, ends;
+  int rows, cols, step, ends, brief, erf, far;
   bool joins;
 };
-static const RingCost ring_costs[RING_SHAPES] = {{128, 128, 52, 650, true},  {128, 256, 81, 750, true},  {160, 256, 98, 750, true},
-                                                 {192, 256, 107, 840, true}, {256, 192, 117, 940, true}, {256, 256, 141, 900, false},
-                                                 {128, 64, 38, 500, true},   {64, 128, 38, 500, true}};
+static const RingCost ring_costs[RING_SHAPES] = {{128, 128, 52, 650, 330, 240, 0, true},  {128, 256, 81, 750, 480, 500, 0, true},
+                                                 {160, 256, 98, 820, 570, 600, 0, true},  {192, 256, 107, 865, 670, 740, 0, true},
+                                                 {256, 192, 117, 940, 715, 740, 0, true}, {256, 256, 141, 900, 840, 980, 0, false},
+                                                 {128, 64, 37, 500, 220, 110, 0, true},   {64, 128, 38, 500, 217, 110, 6, true}};
 
 // The time of a product's tiles in that measure.  A last round that is part empty runs faster than a full one, the memory and
 // the L2s being shared by fewer (0.6 of its time at the least; 160 x 256 tiles of 777 x 28672 x 4096, 2.19 rounds: 190 us
-// against 67.5 a full round); not where one tile takes all rows: the weights' way through fewer compute units is what takes
-// the time there (130 x 28672 x 4096: 112 tiles of 160 x 256 69 us, 224 of 128 x 256 60).
-static long long ring_time(const RingCost& c, long long tiles, int K, bool one_row_tile) {
+// against 67.5 a full round; 0.73 of one or two steps); not where one tile takes all rows: the weights' way through fewer compute units
+// is what takes the time there (130 x 28672 x 4096: 112 tiles of 160 x 256 69 us, 224 of 128 x 256 60).
+static long long ring_time(const RingCost& c, long long tiles, int K, bool one_row_tile, bool erf = false, int least_of_256 = 154) {
+  const bool brief = K <= 128;
+  if (brief) least_of_256 = 187;
   const long long last = tiles % 256;
-  const long long rounds256 = tiles / 256 * 256 + (last ? (one_row_tile ? 256 : 154 + last * 102 / 256) : 0);
-  return rounds256 * ((long long)(K / 64) * c.step + c.ends) / 256;
+  const long long rounds256 =
+      tiles / 256 * 256 + (last ? (one_row_tile && !brief ? 256 : least_of_256 + last * (256 - least_of_256) / 256) : 0);
+  return rounds256 * ((long long)(K / 64) * (c.step + (K >= 2 * GEMM_SEG ? c.far : 0)) + (brief ? c.brief : c.ends) + (erf ? c.erf : 0)) / 256;
 }
 static long long ring_tiles(const RingCost& c, int M, long long cols) { return (long long)((M + c.rows - 1) / c.rows) * ((cols + c.cols - 1) / c.cols); }
 
 // The shape that takes the least time, all of K a workgroup.  ``cols``: rows of W; ``gated``: the outputs are half of those.
-static int ring_choice(int M, long long cols, int K, bool gated, long long* time) {
+static int ring_choice(int M, long long cols, int K, bool gated, long long* time, bool erf = false) {
   int best = RING_128;
   long long least = -1;
   for (int i = 0; i < RING_SHAPES; ++i) {
     if (K > GEMM_SEG && !ring_costs[i].joins) continue;
     if (gated && i == RING_256X192) continue;
-    const long long t = ring_time(ring_costs[i], ring_tiles(ring_costs[i], M, cols), K, M <= ring_costs[i].rows);
+    const long long t = ring_time(ring_costs[i], ring_tiles(ring_costs[i], M, cols), K, M <= ring_costs[i].rows, erf);
     if (least < 0 || t < least) {
       least = t;
       best = i;
@@ -523,7 +532,7 @@ static int ring_choice(int M, long long cols, int K, bool gated, long long* time
 
 extern "C" int bw_gemm_prompt_tile(int M, long long w_rows, int K, int gated, int* rows, int* columns) {
   if (M <= 64 || w_rows <= 0 || K <= 0 || K % 64 || rows == nullptr || columns == nullptr) return -2;
-  const RingCost& c = ring_costs[ring_choice(M, w_rows, K, gated != 0, nullptr)];
+  const RingCost& c = ring_costs[ring_choice(M, w_rows, K, gated == 1, nullptr, gated == 2)];
   *rows = c.rows;
   *columns = c.cols;
   return 0;

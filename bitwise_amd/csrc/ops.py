@@ -458,11 +458,12 @@ def gemm_f32_prompt_tile(rows: int, N: int) -> Tuple[int, int]:
     return int(r.value), int(c.value)
 
 
-def gemm_prompt_tile(rows: int, w_rows: int, K: int, gated: bool = False) -> Tuple[int, int]:
+def gemm_prompt_tile(rows: int, w_rows: int, K: int, gated: bool = False, erf: bool = False) -> Tuple[int, int]:
     """(rows, rows of W) of the tiles that ``gemm_bf16`` gives a product of more than 64 rows, K in whole steps of 64, where
-    all of K is one workgroup's and the kernels for few rows do not take it."""
+    all of K is one workgroup's and the kernels for few rows do not take it; ``gated``: of a gated epilogue, ``erf``: of the exact
+    GELU."""
     r, c = ctypes.c_int(0), ctypes.c_int(0)
-    _check(_fn("bw_gemm_prompt_tile")(rows, w_rows, K, int(gated), ctypes.addressof(r), ctypes.addressof(c)), "gemm_prompt_tile")
+    _check(_fn("bw_gemm_prompt_tile")(rows, w_rows, K, 2 if erf else int(gated), ctypes.addressof(r), ctypes.addressof(c)), "gemm_prompt_tile")
     return int(r.value), int(c.value)
 
 
