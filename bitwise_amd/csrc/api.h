@@ -45,6 +45,9 @@ int bw_gemm_clamped_glu_bf16(const void* x, const void* w, void* out, int M, int
 // the same with the GELU (tanh form) of the gate instead of the clamped unit
 int bw_gemm_gelu_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, void* stream);
 int bw_gemm_add_scratch(int M, int N, int K, long long* scratch_floats, int* counters);
+// whether (and in which tiles; 0, 0: it does not) the sums of a split go into that scratch; the most rows with which they do
+int bw_gemm_split_tile(int M, int N, int K, int store, int* rows, int* columns);
+int bw_gemm_split_rows(int max_rows, int N, int K, int store);
 // out = bf16(gelu_tanh(x W^T) * table[token of the row]): up to 16 rows, K in steps of 64, fewer than 4,096 columns (-7: another shape)
 int bw_gemm_side_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, const int32_t* tokens,
                       const int32_t* feedback, const void* table, int ldt, int vocab, void* stream);

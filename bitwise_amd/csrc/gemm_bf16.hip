@@ -224,8 +224,9 @@ static void add_rows_shape(int M, int N, int K, int& tiles, bool& narrow) {
 //               afterwards: where few tiles of all of K would leave most of the chip idle (128 rows of 2048 columns are 16
 //               of 128 x 128, each 128 steps long for K = 8192: 76 us; 25 split).
 // All give the same bits.  Which shapes are asked to bring scratch for a split is a count of rounds and steps
-// (add_takes_scratch: what callers size their scratch by, so it stays as it is while the kernels change); whether one that
-// brings it is split or goes whole, and in which tiles, the estimated times decide (add_split_shape).
+// (add_takes_scratch: what callers of bw_gemm_add_scratch size by, so it stays as it is while the kernels change); whether one that
+// brings it is split or goes whole, and in which tiles, the estimated times decide (split_shape, which bw_gemm_split_tile
+// and bw_gemm_split_rows tell callers that do not want to hold scratch for nothing).
 // tiles64: what the 64-row kernel's scratch is sized by.
 enum AddRoute { ADD_WHOLE, ADD_ROW_BLOCKS, ADD_SPLIT };
 
@@ -284,21 +285,25 @@ static AddRoute add_route(int M, int N, int K, int ldo, int& tiles64) {
   return add_takes_scratch(M, N, K, ldo) ? ADD_SPLIT : ADD_WHOLE;
 }
 
-// The tiles of a split that takes less time than all of K a workgroup; -1: none does.  The join is a launch (3 us) and moves 8
-// bytes an element and segment and 8 more an element, the stores of the sums among them (2048 x 2048, four segments: 28 us in
-// all), at about 7 TB/s.
+// The join is a launch (3 us) and moves 8 bytes an element and segment and 8 more an element, the stores of the sums among them
+// (2048 x 2048, four segments: 28 us in all), at about 9 TB/s, much of it in caches.
+static long long add_join_time(int M, int N, int S) { return (8LL * S + 8) * M * N / 90000 + 300; }
+
+// The tiles of a split.  Up to 192 rows always one of 128 x 128 or 128 x 256, counted in rounds and steps as where scratch is asked
+// for: the weights' way from memory takes the time there, not the matrix cores, and the times below do not see it (33 products of 129
+// to 192 rows, 4096 to 8192 columns and K of 4096 to 14336, every shape timed, split and whole: by the count four take more than 5 %
+// longer than the best, up to 27 %; by the times ten, up to 18 %).  More rows: the shape that takes less time than all of K a
+// workgroup; -1: none does (204 products of up to 2,048 rows: 0.8 % from the best in the mean).
 static int add_split_shape(int M, int N, int K) {
   const int S = (K + GEMM_SEG - 1) / GEMM_SEG;
-  long long least;
-  int shape = -1;
-  ring_choice(M, N, K, false, &least);
-  // (up to 192 rows the weights' way from memory takes the time, not the matrix cores: rounds and steps are counted as where
-  // scratch is asked for.  4096 columns of K = 14336, 130 rows: 43 us, 50 by the times below; 6144 of K = 4096 22 and 24.)
   if (M <= 192) {
     const long long wgs128 = ring_tiles(ring_costs[RING_128], M, N) * S, wgs256 = ring_tiles(ring_costs[RING_128X256], M, N) * S;
     return (wgs256 + 255) / 256 * 7 < (wgs128 + 255) / 256 * 4 ? RING_128X256 : RING_128;
   }
-  const long long join = (8LL * S + 8) * M * N / 70000 + 300;
+  long long least;
+  int shape = -1;
+  ring_choice(M, N, K, false, &least);
+  const long long join = add_join_time(M, N, S);
   for (int i = 0; i < RING_SHAPES; ++i) {
     const long long t = ring_time(ring_costs[i], ring_tiles(ring_costs[i], M, N) * S, GEMM_SEG, false) + join;
     if (t < least) {
@@ -307,6 +312,18 @@ static int add_split_shape(int M, int N, int K) {
     }
   }
   return shape;
+}
+
+// The tiles in which a residual add (store: a 32-bit store) of more than 64 rows leaves its segments' sums in scratch of S M N
+// floats; -1: it does not, whatever scratch it is given for that.
+static int split_shape(int M, int N, int K, int ldo, bool store) {
+  int tiles, zb;
+  bool narrow;
+  add_blocks_shape(M, N, K, tiles, narrow, zb);
+  if (tiles || add_route(M, N, K, ldo, tiles) != ADD_SPLIT) return -1;
+  // (a store splits only what leaves compute units idle)
+  if (store && ((M + 127) / 128) * ((N + 127) / 128) >= 256) return -1;
+  return add_split_shape(M, N, K);
 }
 
 template <int EPI>
@@ -481,6 +498,25 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
       BW_LAUNCH((gemm_bf16_wide_kernel<EPI, false, false>), grid, block, 0, s, x, w, out, M, N, K, ldx, ldo, m_tiles, n_tiles, rp);
   }
   return BW_LAUNCH_CHECK();
+}
+
+// bw_gemm_add_scratch asks for the S M N floats of a split by a count that its callers rely on; whether one takes place goes by time.
+// The tiles (rows, columns) in which a residual add (store: a 32-bit store) of M > 64 rows leaves its segments' sums there; 0, 0: it
+// goes whole, with the scratch as without.
+extern "C" int bw_gemm_split_tile(int M, int N, int K, int store, int* rows, int* columns) {
+  if (M <= 0 || N <= 0 || K <= 0 || rows == nullptr || columns == nullptr) return -2;
+  const int shape = M > 64 ? split_shape(M, N, K, 4, store != 0) : -1;
+  *rows = shape < 0 ? 0 : ring_costs[shape].rows;
+  *columns = shape < 0 ? 0 : ring_costs[shape].cols;
+  return 0;
+}
+
+// The most rows, up to max_rows, with which it does; 0: it never does.
+extern "C" int bw_gemm_split_rows(int max_rows, int N, int K, int store) {
+  if (N <= 0 || K <= 0) return 0;
+  for (int M = max_rows; M > 64; --M)
+    if (split_shape(M, N, K, 4, store != 0) >= 0) return M;
+  return 0;
 }
 
 // What a residual add wants beside its operands to give every segment of K workgroups of its own: floats of

@@ -1,9 +1,10 @@
 // Part of gemm_bf16.hip (included there behind gemm_bf16_tiles.h; not a unit of its own): the tiles of prompt portions,
 // fed through LDS rings.
 //
-// What bounds them: a compute unit's loads from the L2s (64 KB a step of 256 x 256 outputs), the operand reads from LDS (24 a
-// wave and step beside 64 matrix instructions) and the matrix cores take 0.8, 1.0 and 1.0 us a step of their own at the
-// 2.0 GHz that the part runs at under this load; what is lost is where they wait for each other.  So
+// What bounds them, a step of 256 x 256 outputs: a compute unit's loads from the L2s take 0.8 us (64 KB at the 80 KB a microsecond
+// that a kernel of nothing but such loads gets), its operand reads 0.4 (24 a wave, by the counter of LDS at work), the matrix
+// instructions 1.0 (64 a wave), at the 2.0 GHz that the part runs at under this load; the step takes 1.41.  What is lost is where
+// they wait for each other.  So
 //   * the wait for a step and its barrier stand two turns before the end of the step before, and the step's first operands
 //     are read under the last turns' matrix instructions: no wave starts a step by waiting for LDS;
 //   * where only two steps of W fit beside three of x, a barrier in the middle of a step gives the half ring back early, so that
@@ -11,10 +12,10 @@
 //   * the tile's shape goes by the product (ring_choice): as few bytes an output as its registers allow, but rounds of the
 //     256 compute units that are not left part empty.
 // Against one kernel each for 256 x 256, 128 x 256 and 128 x 128 tiles that waited at the step's edge and were chosen by counts
-// of steps (one machine, both in turn, us): gate|up + SwiGLU of 2048 x 16384 x 2048 118 -> 108, of 2048 x 28672 x 4096 442 -> 383 (in
-// 192 x 256 tiles, 1.26 PFLOP/s), of 777 rows 216 -> 190 (160 x 256); q|k|v of 2048 x 6144 x 2048 56 -> 46 and of K = 4096
-// 120 -> 85 (256 x 192, one round), of 1348 rows 48 -> 36 (160 x 256); the residual adds of 2048 x 2048 x 8192 102 -> 74 without
-// scratch, of 777 x 4096 x 4096 51 -> 36, of K = 14336 126 in two launches -> 102.  The results are the same bits.
+// of steps (one machine, both in turn, us): gate|up + SwiGLU of 2048 x 16384 x 2048 107 -> 99, of 2048 x 28672 x 4096 420 -> 365 (in
+// 192 x 256 tiles, 1.32 PFLOP/s), of 777 rows 209 -> 186 (160 x 256); q|k|v with rotation of 2048 x 6144 x 2048 53 -> 46, of 1348 rows
+// 51 -> 41, the plain product of K = 4096 118 -> 81 (256 x 192, one round); the residual adds of 2048 x 2048 x 8192 78 -> 73 (before with
+// 67 MB of scratch, now without), of 777 x 4096 x 4096 48 -> 34, of K = 14336 120 in two launches -> 102.  The results are the same bits.
 #pragma once
 
 // A workgroup of eight waves computes BM x BN outputs (gated epilogues: BM x BN / 2, from BN / 2 gate and BN / 2 up rows of
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   typedef __attribute__((address_space(3))) void* lds_ptr;
   const int steps = K / 64;
-  // (past K: outside the descriptors, no traffic, into slots that nobody reads any more)
+  // (past K: outside the descriptors, no traffic, zeros into slots that the last step reads ahead from and whose values nobody uses)
   auto issue_a = [&](int step, int slot, int t) {
     const int q = T::LA * wave + t;
     const int at = T::JUNK && q >= BM / 8 ? T::JUNK_AT : slot * T::A_SLOT + q * 1024;

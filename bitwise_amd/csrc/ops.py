@@ -52,6 +52,8 @@ _SIGS = {
     "bw_gemm_gelu_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_f32_prompt_tile": [c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_prompt_tile": [c_int, c_longlong, c_int, c_int, c_void_p, c_void_p],
+    "bw_gemm_split_tile": [c_int, c_int, c_int, c_int, c_void_p, c_void_p],
+    "bw_gemm_split_rows": [c_int, c_int, c_int, c_int],
     "bw_gemm_add_scratch": [c_int, c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_add_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_longlong, c_void_p,
                          c_int, c_void_p],
@@ -159,7 +161,8 @@ _fns = {}
 # what waits.
 _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
-    "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
+    "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_split_tile", "bw_gemm_split_rows",
+    "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
     "bw_chain_flush", "bw_chain_end",
 })
@@ -475,6 +478,21 @@ def gemm_add_scratch(rows: int, N: int, K: int) -> Tuple[int, int]:
     floats, counters = ctypes.c_longlong(0), ctypes.c_int(0)
     _check(_fn("bw_gemm_add_scratch")(rows, N, K, ctypes.addressof(floats), ctypes.addressof(counters)), "gemm_add_scratch")
     return int(floats.value), int(counters.value)
+
+
+@functools.lru_cache(maxsize=None)
+def gemm_split_tile(rows: int, N: int, K: int, store: bool = False) -> Optional[Tuple[int, int]]:
+    """(rows, columns) of the tiles that leave the sums of a residual add's (``store``: a 32-bit store's) segments of K in the
+    whole-sized scratch of ``gemm_add_scratch`` (the one with a single counter); None: the product goes whole and does not touch it."""
+    r, c = ctypes.c_int(0), ctypes.c_int(0)
+    _check(_fn("bw_gemm_split_tile")(rows, N, K, int(store), ctypes.addressof(r), ctypes.addressof(c)), "gemm_split_tile")
+    return (int(r.value), int(c.value)) if r.value else None
+
+
+@functools.lru_cache(maxsize=None)
+def gemm_split_rows(max_rows: int, N: int, K: int, store: bool = False) -> int:
+    """The most rows, up to ``max_rows``, with which a product leaves its segments' sums there; 0: it never does."""
+    return int(_fn("bw_gemm_split_rows")(max_rows, N, K, int(store)))
 
 
 def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows: int, epilogue: int,

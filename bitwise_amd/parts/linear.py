@@ -45,20 +45,22 @@ class Linear:
         ops.convert(x, buf, rows)
         return buf
 
-    def _scratch(self, ws, rows: int):
+    def _scratch(self, ws, rows: int, store: bool = False):
         """17 rows or more and a long inner size: every 2048-segment of it gets workgroups of its own, which meet in device
         scratch.  For up to 64 rows (or a few blocks of 64) that is a fixed size; for a prompt portion it holds the
-        segments' sums whole and is sized for the longest step, so that one buffer serves every portion."""
+        segments' sums whole (one counter asked for) and is sized for the longest step that splits, so that one buffer serves every
+        portion; a portion whose product goes whole gets none."""
         if rows <= 16:
             return None
-        floats, counters = ops.gemm_add_scratch(rows, self.out_features, self.in_features)
-        if floats and rows > 64:
-            longest = ops.gemm_add_scratch(ws.max_rows, self.out_features, self.in_features)
-            floats, counters = max(floats, longest[0]), max(counters, longest[1])
-            if floats > longest[0]:        # (the longest step needs none: a size per power of two, not one per number of rows)
-                floats = 1 << (floats - 1).bit_length()
-        if not floats:
+        N, K = self.out_features, self.in_features
+        floats, counters = ops.gemm_add_scratch(rows, N, K)
+        if not floats or (counters == 1 and ops.gemm_split_tile(rows, N, K, store) is None):
             return None
+        if rows > 64:
+            counters = max(counters, ops.gemm_add_scratch(ws.max_rows, N, K)[1])
+            split_rows = ops.gemm_split_rows(ws.max_rows, N, K, store)
+            if split_rows:
+                floats = max(floats, ops.gemm_add_scratch(split_rows, N, K)[0])
         return (ws.buffer("gemm_add_split", floats, torch.float32, rows=1),
                 ws.buffer("gemm_add_split_count", counters, torch.int32, rows=1))
 
@@ -79,7 +81,7 @@ class Linear:
             if out.dtype == torch.bfloat16:
                 ops.gemm_bf16(x, self.weight, out, rows, ops.EPI_BF16)
             else:
-                ops.gemm_bf16(x, self.weight, out, rows, ops.EPI_F32, scratch=self._scratch(ws, rows))
+                ops.gemm_bf16(x, self.weight, out, rows, ops.EPI_F32, scratch=self._scratch(ws, rows, store=True))
         elif out.dtype == torch.float32:
             ops.gemm_f32(self._x32(ws, x, rows), self.weight, out, rows)
         else:
