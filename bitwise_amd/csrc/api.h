@@ -44,6 +44,7 @@ int bw_gemm_clamped_glu_bf16(const void* x, const void* w, void* out, int M, int
                              float alpha, void* stream);
 // the same with the GELU (tanh form) of the gate instead of the clamped unit
 int bw_gemm_gelu_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, void* stream);
+int bw_gemm_gelu_glu_wins(int M, int N, int K);   // 1: faster than the 32-bit store and the activation kernel behind it
 int bw_gemm_add_scratch(int M, int N, int K, long long* scratch_floats, int* counters);
 // whether (and in which tiles; 0, 0: it does not) the sums of a split go into that scratch; the most rows with which they do
 int bw_gemm_split_tile(int M, int N, int K, int store, int* rows, int* columns);

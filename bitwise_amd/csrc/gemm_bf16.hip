@@ -500,6 +500,46 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
   return BW_LAUNCH_CHECK();
 }
 
+// Whether a gated GELU of more than 64 rows takes less time in the epilogue of its stacked product (bw_gemm_gelu_glu_bf16) than as a
+// kernel behind the 32-bit store.  The epilogue saves the sums' way through memory (writing 2 N of them a row, reading them, a
+// launch: 2,048 rows of 2 x 8192 columns and K = 2048 122 + 38 us -> 111), but its product goes in tiles with all of K a workgroup, where
+// the store of few rows or few columns gives blocks of 64 rows or segments of K workgroups of their own (128 rows of 2 x 512 columns and K =
+// 14336: 20 us and 70).  Both times are estimated, in hundredths of a microsecond: a workgroup of the 64-row kernel 300 and 25 a
+// step of 64 (15 with 32 columns), half as much again where two share a compute unit, 200 more where segments meet; tiles as in
+// ring_time, a part-empty round counted as 0.73 of a full one at the least; the activation 250 and its bytes at 3.5 TB/s.  K of several
+// segments in tiles of few rows is slower than that (the weights' way), so there the epilogue has to win by a quarter.  Over
+// 1,704 products (65 to 2,048 rows, 2 x 512 to 2 x 14336 columns, K of 64 to 14336) both ways timed: no choice more than 5 % slower than the
+// kernel behind the store, 0.3 % from the better one in the mean.
+extern "C" int bw_gemm_gelu_glu_wins(int M, int N, int K) {
+  if (M <= 64 || N <= 0 || K <= 0 || N > (1 << 29)) return 0;
+  if (K % 64) return 1;                                     // (the same kernel either way)
+  const int S = (K + GEMM_SEG - 1) / GEMM_SEG, cols = 2 * N, per = std::min(K, GEMM_SEG) / 64;
+  const long long squares = (long long)((cols + 31) / 32) * ((M + 31) / 32);
+  long long store;
+  int tiles, zb;
+  bool narrow;
+  add_blocks_shape(M, cols, K, tiles, narrow, zb);
+  if (S == 1 && squares >= 32 && squares <= 256) {
+    store = 300 + 15 * per;
+  } else if (tiles && (S > 1 || narrow || store_in_blocks(M, cols, K, false))) {
+    store = 300 + (narrow ? 15 : 25) * per;
+    if ((long long)tiles * zb * S > 256) store = store * 29 / 20;
+    if (S > 1) store += 200;
+  } else {
+    const int shape = split_shape(M, cols, K, cols, true);
+    if (shape < 0) return 1;
+    store = ring_time(ring_costs[shape], ring_tiles(ring_costs[shape], M, cols) * S, GEMM_SEG, false) + add_join_time(M, cols, S);
+  }
+  long long epilogue = -1;
+  for (int i = 0; i < RING_SHAPES; ++i) {
+    if (i == RING_256X192 || (K > GEMM_SEG && !ring_costs[i].joins)) continue;
+    const long long t = ring_time(ring_costs[i], ring_tiles(ring_costs[i], M, cols), K, M <= ring_costs[i].rows, false, 187);
+    if (epilogue < 0 || t < epilogue) epilogue = t;
+  }
+  if (S > 1) epilogue = epilogue * 5 / 4;
+  return epilogue <= store + 250 + 5LL * M * cols / 70000;
+}
+
 // bw_gemm_add_scratch asks for the S M N floats of a split by a count that its callers rely on; whether one takes place goes by time.
 // The tiles (rows, columns) in which a residual add (store: a 32-bit store) of M > 64 rows leaves its segments' sums there; 0, 0: it
 // goes whole, with the scratch as without.
@@ -618,7 +658,8 @@ extern "C" int bw_gemm_clamped_glu_bf16(const void* x, const void* w, void* out,
 }
 
 // The same with the GELU (tanh form) of the gate: out[m, n] = bf16(gelu(x.W[n]) (x.W[N + n])).  The bits of gemm_bf16
-// (32-bit store) + glu, which at 2,048 rows of 2 x 8192 columns and K = 2048 write and read 134 MB of sums: 122 + 38 us -> 121.
+// (32-bit store) + glu, which at 2,048 rows of 2 x 8192 columns and K = 2048 write and read 134 MB of sums: 122 + 38 us -> 111
+// (bw_gemm_gelu_glu_wins: where it is the faster way).
 extern "C" int bw_gemm_gelu_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, void* stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M <= 64) return -2;

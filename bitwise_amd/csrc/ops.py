@@ -52,6 +52,7 @@ _SIGS = {
     "bw_gemm_gelu_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_f32_prompt_tile": [c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_prompt_tile": [c_int, c_longlong, c_int, c_int, c_void_p, c_void_p],
+    "bw_gemm_gelu_glu_wins": [c_int, c_int, c_int],
     "bw_gemm_split_tile": [c_int, c_int, c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_split_rows": [c_int, c_int, c_int, c_int],
     "bw_gemm_add_scratch": [c_int, c_int, c_int, c_void_p, c_void_p],
@@ -161,7 +162,7 @@ _fns = {}
 # what waits.
 _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
-    "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_split_tile", "bw_gemm_split_rows",
+    "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_gelu_glu_wins", "bw_gemm_split_tile", "bw_gemm_split_rows",
     "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
     "bw_chain_flush", "bw_chain_end",
@@ -553,9 +554,10 @@ def gemm_clamped_glu_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, r
                                            float(limit), float(alpha), _stream()), "gemm_clamped_glu_bf16")
 
 
-# ------------------------------------------------------------------------------ decode fusions
-
-_decode_ok = {}
+@functools.lru_cache(maxsize=None)
+def gelu_glu_in_epilogue(rows: int, inter: int, K: int) -> bool:
+    """Whether ``gemm_gelu_glu_bf16`` is faster for these sizes than the 32-bit store and ``glu`` behind it (the same bits)."""
+    return bool(_fn("bw_gemm_gelu_glu_wins")(rows, inter, K))
 
 
 def gemm_gelu_glu_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows: int) -> None:
@@ -574,6 +576,11 @@ def gemm_gelu_glu_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows
         raise ValueError("gemm_gelu_glu_bf16: more than 64 rows and an inner size in multiples of 8")
     _check(_fn("bw_gemm_gelu_glu_bf16")(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, N, K, x.stride(0), out.stride(0),
                                         _stream()), "gemm_gelu_glu_bf16")
+
+
+# ------------------------------------------------------------------------------ decode fusions
+
+_decode_ok = {}
 
 
 def norm_gemm_supported(rows: int, inner: int) -> bool:

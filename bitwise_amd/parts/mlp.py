@@ -84,8 +84,8 @@ class SwiGLU(FeedForward):
 @register_feed_forward("geglu")
 class GeGLU(SwiGLU):
     """The same arrangement with the tanh form of GELU on the gate.  Prompt portions of more than 64 rows compute the activation
-    and the product with ``up`` in the stacked product's epilogue (bfloat16 mode, weights the matrix cores take); otherwise the
-    product leaves 32-bit sums and one kernel behind it rounds once for the down projection.  Both are the same sequence
+    and the product with ``up`` in the stacked product's epilogue where that is faster (bfloat16 mode, weights the matrix cores
+    take); otherwise the product leaves 32-bit sums and one kernel behind it rounds once for the down projection.  Both are the same sequence
     of operations on the same sums, so a row's bits do not depend on the route."""
 
     act = ops.ACT_GELU_TANH
@@ -112,7 +112,7 @@ class GeGLU(SwiGLU):
 
     def forward(self, ctx, h, residual) -> None:
         if (self.act == ops.ACT_GELU_TANH and self.rt.bf16 and self.gate_up.mfma and self.gate_up.bias is None
-                and ctx.rows >= ops.CLAMPED_GLU_MIN_ROWS):
+                and ops.gelu_glu_in_epilogue(ctx.rows, self.inter, self.width)):
             act = ctx.ws.buffer("mlp_h", self.inter, torch.bfloat16)
             ops.gemm_gelu_glu_bf16(h, self.gate_up.weight, act, ctx.rows)
             self.down.add_into(ctx.ws, act, residual, ctx.rows)

@@ -45,6 +45,21 @@ def test_part_empty_rounds_of_a_short_inner_size_do_not_take_the_larger_of_two_t
     assert ops.gemm_prompt_tile(M, N, K) in ((128, 256), (128, 128))
 
 
+def test_gated_gelu_in_the_epilogue_only_where_it_is_faster():
+    # both ways timed, us behind the store and in the epilogue
+    for (M, inter, K), wins in {(128, 512, 14336): False,         # 19.7 and 69.9
+                                (192, 1024, 14336): False,        # 30.1 and 101
+                                (65, 512, 2048): False,           # 7.2 and 13.6
+                                (96, 512, 1024): False,           # 6.4 and 8.8
+                                (128, 2048, 4096): False,         # 64 workgroups with all of K
+                                (2048, 8192, 2048): True,         # 151 and 111
+                                (117, 8192, 2048): True,
+                                (2048, 512, 64): True, (65, 512, 72): True}.items():
+        assert ops.gelu_glu_in_epilogue(M, inter, K) == wins, (M, inter, K)
+    for M in (1, 16, 64):
+        assert not ops.gelu_glu_in_epilogue(M, 8192, 2048)        # (no epilogue for steps of so few rows)
+
+
 class Workspace:
     """Keeps what is asked of it, as the real one does: a buffer by name and size, for good."""
 
