@@ -235,8 +235,8 @@ def test_gemm_bf16_rows_shapes_and_epilogues(gpu):
             ops.gemm_bf16(x[:, k0:k0 + 2048].contiguous(), w[:, k0:k0 + 2048].contiguous(), part, M, ops.EPI_F32)
             want = want + part
         assert torch.equal(acc, want), (M, N, K)
-    # enough 256 x 256 tiles for the big-tile kernel: the bits of the same rows in slices that other kernels take
-    # (3696 columns: SwiGLU outputs of whole 16-byte pieces, which leave that kernel through LDS a row at a time)
+    # many tiles (160 x 256; the others: tests of the prompt products by tile): the bits of the same rows in slices that go another way
+    # (3696 columns: SwiGLU outputs of whole 16-byte pieces, which leave the tiles through LDS a row at a time)
     for M, N, K in ((2100, 3700, 192), (2100, 3696, 192)):
         x = torch.randn(M, K, generator=g).bfloat16().to(gpu)
         w = torch.randn(N, K, generator=g).bfloat16().to(gpu)
@@ -275,16 +275,16 @@ def test_gemm_bf16_rows_shapes_and_epilogues(gpu):
             assert torch.equal(got, want) and not scratch[1].any(), (M, N, K)
     # a residual add of more than 64 rows whose 128 x 128 tiles with all of K would leave compute units idle: up to
     # 128 rows and three segments in blocks of 64 rows through that kernel (its scratch if K has several segments);
-    # else a workgroup per tile (128 x 128, 128 x 256, or 256 x 256 from 512 rows) and segment, the segments' sums whole in
-    # scratch and joined in order afterwards; or 128 x 256 tiles with all of K where those go round the compute units
-    # once (no scratch).  The bits of the rows alone, 16 at a time, with and without scratch,
+    # else, where that is faster, a workgroup per tile and segment, the segments' sums whole in scratch and joined in order
+    # afterwards (2,048 rows of 2048 x 8192 and 513 of 8192 x 4096 are asked for scratch and go whole).  The bits of the rows
+    # alone, 16 at a time, with and without scratch,
     # twice on the same scratch (full of NaN at first, larger than needed); ragged edges, a short last segment
     S = lambda K: (K + 2047) // 2048
     # ("at once": up to 512 workgroups of the 64-row kernel, a block of 64 rows, a tile of columns and a segment each, in
     # one launch; their scratch is the same size whatever the shape)
     for M, N, K, kind in [(65, 2048, 4096, "at once"), (128, 1100, 2048 * 2 + 320, "at once"), (100, 2048, 2048, None),
                           (129, 2048, 2048, None), (81, 2048, 4096 + 72, None), (640, 4096, 4096, None),
-                          (2048, 4096, 4096, None),       # 128 x 256 tiles, the two segments joined in registers
+                          (2048, 4096, 4096, None),       # tiles with all of K, the two segments joined in registers
                           (65, 2048, 8192, "at once"), (145, 2048, 8192, "at once"), (300, 1000, 2 * 2048 + 192, "at once"),
                           (256, 2048, 8192, "at once"), (320, 2048, 8192, "sums"),
                           (768, 2048, 8192, "sums"), (700, 3000, 4 * 2048 + 128, "sums"), (2048, 2048, 8192, "sums"),

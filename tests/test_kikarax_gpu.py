@@ -420,8 +420,8 @@ def test_clamped_unit_and_row_gate(gpu, act_dtype):
                                               (1024, 2048, 512), (1500, 96, 2112)])
 def test_clamped_unit_in_the_products_epilogue(gpu, rows, inter, width):
     """Prompt portions compute the clamped unit in the stacked product's epilogue: the bits of the product's 32-bit sums
-    followed by the activation kernel (what steps of few rows run), over every tiling the product chooses, and the
-    float64 values; inputs large enough for all three clamps to bite."""
+    followed by the activation kernel (what steps of few rows run), in the smaller tiles (the others: the tests of the prompt
+    products by tile), and the float64 values; inputs large enough for all three clamps to bite."""
     from bitwise_amd.csrc import ops
     g = torch.Generator().manual_seed(rows)
     x = torch.randn(rows, width, generator=g).bfloat16()

@@ -495,8 +495,8 @@ def test_decays_made_ahead_equal_decays_made_in_the_walk(gpu, dim, vdim):
 @pytest.mark.parametrize("rows,inter,width", [(65, 64, 64), (130, 136, 72), (513, 512, 192), (700, 6000, 2112), (1345, 4100, 64)])
 def test_gelu_unit_in_the_products_epilogue(gpu, rows, inter, width):
     """Prompt portions compute the gated GELU in the stacked product's epilogue: the bits of the 32-bit product followed by the
-    activation kernel, and the float64 values to one bfloat16 rounding and the sums' own error; gates of every size among
-    them, infinities and NaN where the product has them."""
+    activation kernel, and the float64 values to one bfloat16 rounding and the sums' own error; then the activation kernel at
+    infinities, NaN and gates of every size (the epilogue at those: the tests of the prompt products by tile)."""
     from bitwise_amd.csrc import ops
     g = torch.Generator().manual_seed(rows)
     x = torch.randn(rows, width, generator=g).bfloat16()
