@@ -533,7 +533,7 @@ static int ring_choice(int M, long long cols, int K, bool gated, long long* time
 
 extern "C" int bw_gemm_prompt_tile(int M, long long w_rows, int K, int gated, int* rows, int* columns) {
   if (M <= 64 || w_rows <= 0 || K <= 0 || K % 64 || rows == nullptr || columns == nullptr) return -2;
-  const RingCost& c = ring_costs[ring_choice(M, w_rows, K, gated == 1, nullptr, gated == 2)];
+  const RingCost& c = ring_costs[ring_choice(M, w_rows, K, gated != 0 && gated != 2, nullptr, gated == 2)];
   *rows = c.rows;
   *columns = c.cols;
   return 0;
