@@ -333,145 +333,13 @@ __global__ __launch_bounds__(256) void gemm_f32_rows_kernel(const float* __restr
   }
 }
 
-// ------------------------------------------------------------------------------ up to 16 rows: a wave a row
-
-// Decoded tokens, the same chains with the operands brought another way.  A workgroup owns 64 columns and all
-// (up to 16) rows; wave m is row m, lane l the chain of (row m, column n0 + l).  Weights and rows travel from
-// memory straight into LDS (buffer loads with LDS as destination: 8 rows of W, 128 bytes each, or 4 rows of x, 256
-// bytes each, an instruction; whole cache lines, the 16-byte chunks of a row of W permuted against bank conflicts;
-// a ring of stages, waits by counting loads).  The weights stay packed there: a lane reads its column's 16-byte
-// chunks and widens them in registers.  A row's elements are the same for the whole wave: every lane reads the same
-// address, which costs LDS one access.  Against the kernel above (every thread reads a 32-bit element of x and one
-// of W from LDS for each multiply-add) a multiply-add here needs 2 bytes of W from LDS (bfloat16 weights) instead of
-// 4 of W and 4 of x.  For products with at least as many blocks of 64 columns as there are compute units.
-// K a multiple of a stage (64 bfloat16 or 32 32-bit elements), rows 16-byte aligned.
-#define F32L_MIN_BLOCKS 256                                           // fewer blocks of 64 columns than compute units: the kernel above (16 columns a workgroup)
-#define F32L_STAGES 8
-#define F32L_W (64 * 128)                                             // 64 rows of W, 128 bytes each
-#define F32L_X (16 * 256)                                             // 16 rows of x, up to 64 elements each
-#define F32L_STAGE (F32L_W + F32L_X)
-
-// A wave's loads of one stage (a device function rather than a lambda in the kernel: the host pass drops, without a
-// word, kernel templates whose lambdas capture arrays of dependent size): LPW of W and one of x.
-template <int LPW>
-__device__ __forceinline__ void lanes_issue(unsigned char* lds, __amdgpu_buffer_rsrc_t rs_w, __amdgpu_buffer_rsrc_t rs_x, const int* voff,
-                                            int voff_x, int wave, int nwaves, int step, int steps, int w_step, int x_step) {
-  typedef __attribute__((address_space(3))) void* lds_ptr;
-  unsigned char* dst = lds + (step % F32L_STAGES) * F32L_STAGE;
-  unsigned char* dump = lds + F32L_STAGES * F32L_STAGE;               // where loads that bring nothing put their zeros
-  const bool real = step < steps;                                     // scalar
-#pragma unroll
-  for (int t = 0; t < LPW; ++t) {
-    const int blk = wave + t * nwaves;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, (lds_ptr)(blk < 8 ? dst + blk * 1024 : dump), 16, real ? voff[t] : 0x7ffffff0,
-                                             step * w_step, 0, 0);
-  }
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (lds_ptr)(wave < 4 ? dst + F32L_W + wave * 1024 : dump), 16,
-                                           real ? voff_x : 0x7ffffff0, step * x_step, 0, 0);
-}
-
-// LPW: loads of W a wave issues per stage (8 in all; waves past the eighth, and what does not divide, issue loads
-// outside the descriptor: no traffic, zeros into a spare KB behind the ring), so that every wave counts alike.
-template <typename WT, int LPW>
-__global__ __launch_bounds__(1024) void gemm_f32_lanes_kernel(const float* __restrict__ x, const WT* __restrict__ w,
-                                                              float* __restrict__ y, int M, int N, int K, int ldx, int ldy,
-                                                              int accumulate) {
-  constexpr int EPC = 16 / (int)sizeof(WT);                           // elements in a 16-byte chunk
-  constexpr int KS = 128 / (int)sizeof(WT);                           // elements of k a stage
-  extern __shared__ __attribute__((aligned(16))) unsigned char lanes_lds[];   // [stages][W: 64 rows of 128 B | x: 16 rows of 256 B], 1 KB
-  const int wave = wave_index(), lane = threadIdx.x & 63, nwaves = blockDim.x >> 6;
-  const int n0 = blockIdx.x * 64;
-  const int w_rows = min(64, N - n0);
-  const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0,
-                                                                        (int)((size_t)w_rows * K * sizeof(WT)), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, (int)((((size_t)M - 1) * ldx + K) * 4), 0x00020000);
-  // loads of W: lane l of a load fetches row l / 8 of its 8 rows, chunk (l % 8) ^ (row within 16 >> 1) of the row's 128 bytes
-  const int lrow = lane >> 3, lslot = lane & 7;
-  int voff[LPW];
-#pragma unroll
-  for (int t = 0; t < LPW; ++t) {
-    const int blk = wave + t * nwaves;                                // which 8 rows of the 64
-    const int row = 8 * blk + lrow;
-    voff[t] = blk < 8 ? (int)((row * K) * (int)sizeof(WT) + 16 * (lslot ^ ((row & 15) >> 1))) : 0x7ffffff0;
-  }
-  // loads of x (waves 0 to 3): lane l fetches row 4 wave + l / 16, its chunk l % 16 of the stage's KS elements (rows
-  // past M and, with 32-bit weights, chunks past the stage: outside, or never read)
-  const int xrow = 4 * wave + (lane >> 4), xchunk = lane & 15;
-  const int voff_x = (wave < 4 && xrow < M && 4 * xchunk < KS) ? (xrow * ldx + 4 * xchunk) * 4 : 0x7ffffff0;
-  const int steps = K / KS;
-#pragma unroll
-  for (int st = 0; st < F32L_STAGES - 1; ++st) lanes_issue<LPW>(lanes_lds, rs_w, rs_x, voff, voff_x, wave, nwaves, st, steps, 128, KS * 4);
-  // this lane's row of the tile: chunk j lies in slot j ^ (row within 16 >> 1)
-  const int my = (lane >> 3) * 1024 + (lane & 7) * 128, swz = (lane & 15) >> 1;
-  float acc = 0.0f;
-  for (int step = 0; step < steps; ++step) {
-    __builtin_amdgcn_s_waitcnt(vmcnt_only((LPW + 1) * (F32L_STAGES - 2)));   // all but the loads of the stages after this one have landed
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    lanes_issue<LPW>(lanes_lds, rs_w, rs_x, voff, voff_x, wave, nwaves, step + F32L_STAGES - 1, steps, 128, KS * 4);   // into the stage worked on a step ago
-    const unsigned char* stage = lanes_lds + (step % F32L_STAGES) * F32L_STAGE;
-    const unsigned char* xs = stage + F32L_W + wave * 256;            // the wave's row: the same address in every lane
-    u32x4 v[8];                                                       // the stage's eight chunks of W, asked for at once
-    f32x4 xv[KS / 4];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const u32x4*>(stage + my + ((j ^ swz) * 16));
-#pragma unroll
-    for (int j = 0; j < KS / 4; ++j) xv[j] = *reinterpret_cast<const f32x4*>(xs + 16 * j);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if constexpr (sizeof(WT) == 2) {                                // bfloat16 -> 32-bit: the bits, shifted (exact)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          acc = fmaf(xv[2 * j + (e >> 1)][2 * (e & 1)], __uint_as_float(v[j][e] << 16), acc);
-          acc = fmaf(xv[2 * j + (e >> 1)][2 * (e & 1) + 1], __uint_as_float(v[j][e] & 0xffff0000u), acc);
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc = fmaf(xv[j][e], __uint_as_float(v[j][e]), acc);
-      }
-    }
-    asm volatile("" ::: "memory");
-  }
-  __builtin_amdgcn_s_waitcnt(vmcnt_only(0));                          // the padding loads too, before the wave ends
-  const int n = n0 + lane;
-  if (n >= N) return;
-  float* o = y + (size_t)wave * ldy + n;
-  *o = accumulate ? (*o + acc) : acc;
-}
-
-template <typename WT, int LPW>
-static void launch_lanes_lpw(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate,
-                             hipStream_t s) {
-  constexpr int lds_bytes = F32L_STAGES * F32L_STAGE + 1024;
-  static_assert((LPW + 1) * (F32L_STAGES - 2) < 64, "the wait count has six bits");
-  static bool allowed = false;                       // 64 KB of dynamic LDS and more has to be asked for once
-  if (!allowed) {
-    (void)hipFuncSetAttribute((const void*)gemm_f32_lanes_kernel<WT, LPW>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    allowed = true;
-  }
-  hipLaunchKernelGGL((gemm_f32_lanes_kernel<WT, LPW>), dim3((N + 63) / 64), dim3(64 * M), lds_bytes, s, x, w, y, M, N, K, ldx, ldy,
-                     accumulate);
-}
-
-template <typename WT>
-static void launch_lanes(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate,
-                         hipStream_t s) {
-  switch ((8 + M - 1) / M) {                         // loads a wave and stage: 8 over the waves, rounded up
-    case 8: launch_lanes_lpw<WT, 8>(x, w, y, M, N, K, ldx, ldy, accumulate, s); break;
-    case 4: launch_lanes_lpw<WT, 4>(x, w, y, M, N, K, ldx, ldy, accumulate, s); break;
-    case 3: launch_lanes_lpw<WT, 3>(x, w, y, M, N, K, ldx, ldy, accumulate, s); break;
-    case 2: launch_lanes_lpw<WT, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s); break;
-    default: launch_lanes_lpw<WT, 1>(x, w, y, M, N, K, ldx, ldy, accumulate, s); break;
-  }
-}
-
 // ------------------------------------------------------------------------------ a wave a row, the row four elements a register
 
-// Decoded tokens once more: a wave is a row and 64 columns, lane l the chain of (row, column n0 + l), weights and
-// rows in an LDS ring as above (weights packed).  What is new is how a row's elements reach the multiply-adds.
-// x[row][k] is the same number for every lane of the wave; read as such from LDS it costs what any read costs (LDS
-// returns 128 bytes a clock whatever the addresses: above, the rows took two thirds of what LDS returned).  Here lane
+// A decoded token alone: a wave is a row and 64 columns, lane l the chain of (row, column n0 + l); weights and rows travel from
+// memory straight into an LDS ring (buffer loads with LDS as destination: 8 rows of W, 128 bytes each, or 4 rows of x, 256
+// bytes each, an instruction; whole cache lines, the 16-byte chunks of a row of W permuted against bank conflicts; a ring of
+// stages, waits by counting loads).  The weights stay packed there: a lane reads its column's 16-byte chunks and widens them in
+// registers.  x[row][k] is the same number for every lane of the wave; read as such from LDS it costs what any read costs.  Here lane
 // l reads the 16 bytes at element 4 * (l % 4) of a run of sixteen, so that a register holds four elements of the row,
 // the same four in every quad of lanes, and the multiply-add picks its element with the quad permutation of its
 // first operand (v_fmac_f32 with quad_perm [i,i,i,i]: the same fused multiply-add, the operand routed on the way
@@ -673,12 +541,12 @@ __global__ __launch_bounds__(64 * (8 + F32C_LOADERS)) void gemm_f32_chain_kernel
   *o = accumulate ? (*o + acc) : acc;
 }
 
-// For products with at least as many blocks of 64 columns as there are compute units and up to 8 rows: a workgroup
-// a block of columns with all the rows (there it is faster than the kernels above: gate|up of 16,384 columns
-// at 8 rows 26.6 us against 29.1, a head of 49,152 columns 65 against 85; with fewer columns a chain wave has a
-// compute unit to itself in either kernel and both take what the chain takes).
+// For one row and at least as many blocks of 64 columns as there are compute units: 16,384 columns, K = 2048: 14.4 us, 15.0 to 15.8
+// on the matrix cores (gemm_f32_matrix.h), a head of 49,152 columns 36.6 against 37.4.  From two rows on those are faster (15.4
+// against 15.0, 36.7 and 37.3; three rows 17.9 against 15.4, eight 25 against 16 and 62 against 38).
 #define F32C_STAGES 7
-#define F32C_MAX_ROWS 8
+#define F32C_MAX_ROWS 1
+#define F32C_MIN_BLOCKS 256                                           // blocks of 64 columns
 
 template <typename WT>
 static void launch_chain(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s) {
@@ -696,526 +564,13 @@ static void launch_chain(const float* x, const WT* w, float* y, int M, int N, in
                      M, N, K, ldx, ldy, accumulate);
 }
 
-// ------------------------------------------------------------------------------ up to 64 rows on the matrix cores
+#include "gemm_f32_matrix.h"
 
-// v_mfma_f32_4x4x1_16b_f32 computes, for 16 blocks of 4 x 4 outputs at once, D[r][j] = fma(A[r], B[j], D[r][j]):
-// one step of k, a true 32-bit fused multiply-add with a single rounding (denormal numbers, infinities and all;
-// the tests hold it against std::fma bit for bit).  A chain of them over k ascending from a zero accumulator is
-// therefore the scalar chain of the definition, and it needs one element of x and one of W a lane and step where
-// the vector unit needs one of each per output: the operands' way through LDS no longer bounds the product.
-//
-// A wave owns 4 * CG columns and up to 16 rows (MR such blocks of rows for up to 64): block (rg, cg) of the
-// instruction is rows 4 rg .. 4 rg + 3 of x against columns 4 cg .. 4 cg + 3 of the wave's, RG row groups times
-// CG = 16 / RG column groups; the blocks of a row group share their A operand (the instruction broadcasts it from
-// the group's first block).  Lane (block, i) holds row 4 rg + i of x as A, column 4 cg + i of W as B, and the
-// outputs of rows 4 rg .. 4 rg + 3 at its column.  Both operands stream through a ring in LDS that is the wave's
-// own (buffer loads with LDS as destination, in whole 128-byte or 256-byte runs, the 16-byte chunks of a row
-// permuted so that operand reads hit distinct banks; bfloat16 weights are widened when they are read).  Nothing is
-// shared between waves, so the loop has no barrier; loads complete in issue order and every stage has the same
-// number of them (stages past K are asked for outside the descriptors: zeros, no traffic), so "all but the last
-// PENDING loads have landed" is the wait for the stage at hand.  K a multiple of 64.
-template <typename WT, int RG, int MR>
-struct F32MShape {
-  static constexpr int CG = 16 / RG, NCW = 4 * CG;                  // column groups, columns a wave
-  static constexpr int CBSZ = RG == 1 ? 4 : (RG == 2 ? 3 : 2);      // log2 of the blocks that share an A operand
-  static constexpr int XROWS = 4 * RG * MR;                         // rows of x a stage holds
-  static constexpr int WROW = 64 * (int)sizeof(WT);                 // bytes of a row of W a stage (64 steps of k)
-  static constexpr int X_LOADS = XROWS / 4, W_LOADS = NCW * WROW / 1024;   // 1 KB an instruction
-  static constexpr int LPW = X_LOADS + W_LOADS;
-  static constexpr int XBYTES = XROWS * 256, STAGE = XBYTES + NCW * WROW;
-  static constexpr int BY_COUNT = 63 / LPW + 2, BY_ROOM = 65536 / STAGE;
-  static constexpr int STAGES = BY_COUNT < BY_ROOM ? (BY_COUNT < 12 ? BY_COUNT : 12) : (BY_ROOM < 12 ? BY_ROOM : 12);
-  static constexpr int PENDING = LPW * (STAGES - 2);
-  static_assert(STAGES >= 3 && PENDING < 64, "the ring needs three stages and the wait count has six bits");
-  static_assert(MR == 1 || RG == 4, "more than 16 rows: blocks of 16");
-};
-
-template <typename WT, int RG, int MR>
-__device__ __forceinline__ void f32m_issue(unsigned char* ring, __amdgpu_buffer_rsrc_t rs_x, __amdgpu_buffer_rsrc_t rs_w,
-                                           const int* voff_x, const int* voff_w, int step, int steps) {
-  using S = F32MShape<WT, RG, MR>;
-  typedef __attribute__((address_space(3))) void* lds_ptr;
-  unsigned char* dst = ring + (step % S::STAGES) * S::STAGE;
-  const bool real = step < steps;                                  // scalar
-#pragma unroll
-  for (int t = 0; t < S::X_LOADS; ++t)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (lds_ptr)(dst + t * 1024), 16, real ? voff_x[t] : 0x7ffffff0, step * 256, 0, 0);
-#pragma unroll
-  for (int t = 0; t < S::W_LOADS; ++t)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, (lds_ptr)(dst + S::XBYTES + t * 1024), 16, real ? voff_w[t] : 0x7ffffff0,
-                                             step * S::WROW, 0, 0);
-}
-
-template <typename WT, int RG, int MR>
-__global__ __launch_bounds__(64) void gemm_f32_mfma_kernel(const float* __restrict__ x, const WT* __restrict__ w,
-                                                           float* __restrict__ y, int M, int N, int K, int ldx, int ldy,
-                                                           int accumulate) {
-  using S = F32MShape<WT, RG, MR>;
-  constexpr bool BF = sizeof(WT) == 2;
-  extern __shared__ __attribute__((aligned(16))) unsigned char f32m_ring[];
-  const int lane = threadIdx.x, blk = lane >> 2, i = lane & 3;
-  const int rg = blk / S::CG, cg = blk % S::CG;
-  const int n0 = blockIdx.x * S::NCW;
-  const int w_rows = min(S::NCW, N - n0);
-  const __amdgpu_buffer_rsrc_t rs_w =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, (int)((size_t)w_rows * K * sizeof(WT)), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rs_x =
-      __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, (int)((((size_t)M - 1) * ldx + K) * sizeof(float)), 0x00020000);
-  // loads: an instruction brings 1 KB: 4 rows of x (16 chunks of 4 elements each), 8 rows of bfloat16 weights (8 chunks
-  // of 8 elements) or 4 rows of 32-bit ones; the lane that fills slot s of a row fetches chunk s ^ (row % 8).  Rows
-  // past M or N are clamped to the last: what they bring ends in outputs that are never stored.
-  int voff_x[S::X_LOADS], voff_w[S::W_LOADS];
-#pragma unroll
-  for (int t = 0; t < S::X_LOADS; ++t) {
-    const int row = 4 * t + (lane >> 4), chunk = (lane & 15) ^ (row & 7);
-    voff_x[t] = (min(row, M - 1) * ldx + 4 * chunk) * 4;
-  }
-#pragma unroll
-  for (int t = 0; t < S::W_LOADS; ++t) {
-    if constexpr (BF) {
-      const int row = 8 * t + (lane >> 3), chunk = (lane & 7) ^ (row & 7);
-      voff_w[t] = (min(row, w_rows - 1) * K + 8 * chunk) * 2;
-    } else {
-      const int row = 4 * t + (lane >> 4), chunk = (lane & 15) ^ (row & 7);
-      voff_w[t] = (min(row, w_rows - 1) * K + 4 * chunk) * 4;
-    }
-  }
-  // operand reads: this lane's row of x in every block of 16 rows, and its column's row of W
-  int x_base[MR], x_swz[MR];
-#pragma unroll
-  for (int mr = 0; mr < MR; ++mr) {
-    const int row = 16 * mr + 4 * rg + i;
-    x_base[mr] = row * 256;
-    x_swz[mr] = row & 7;
-  }
-  const int wr = 4 * cg + i;
-  const int w_base = S::XBYTES + wr * S::WROW, w_swz = wr & 7;
-  f32x4 acc[MR];
-#pragma unroll
-  for (int mr = 0; mr < MR; ++mr) acc[mr] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const int steps = K / 64;
-  // A stage is worked on in PH phases of CH chunks of 8 steps of k.  The operands of a phase are read from LDS
-  // into one of two sets of registers while the phase before runs out of the other: an LDS read takes longer than
-  // the few matrix instructions the compiler would put between it and its use.
-  constexpr int CH = MR == 4 ? 2 : 4, PH = 8 / CH;
-  constexpr int WQ = BF ? CH : 2 * CH;                              // 16-byte reads of W a phase
-  u32x4 w_a[WQ], w_b[WQ];
-  f32x4 x_a[MR][2 * CH], x_b[MR][2 * CH];
-  auto read_phase = [&](const unsigned char* stage, int ph, u32x4 (&wq)[WQ], f32x4 (&xq)[MR][2 * CH]) {
-#pragma unroll
-    for (int c = 0; c < WQ; ++c) wq[c] = *reinterpret_cast<const u32x4*>(stage + w_base + (((ph * WQ + c) ^ w_swz) * 16));
-#pragma unroll
-    for (int c = 0; c < 2 * CH; ++c)
-#pragma unroll
-      for (int mr = 0; mr < MR; ++mr)
-        xq[mr][c] = *reinterpret_cast<const f32x4*>(stage + x_base[mr] + (((ph * 2 * CH + c) ^ x_swz[mr]) * 16));
-  };
-  auto run_phase = [&](const u32x4 (&wq)[WQ], const f32x4 (&xq)[MR][2 * CH]) {
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      float wv[8];
-      if constexpr (BF) {                                           // bfloat16 -> 32-bit: the bits, shifted (exact)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          wv[2 * q] = __uint_as_float(wq[c][q] << 16);
-          wv[2 * q + 1] = __uint_as_float(wq[c][q] & 0xffff0000u);
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          wv[q] = __uint_as_float(wq[2 * c][q]);
-          wv[4 + q] = __uint_as_float(wq[2 * c + 1][q]);
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e)                                   // k ascending
-#pragma unroll
-        for (int mr = 0; mr < MR; ++mr)
-          acc[mr] = __builtin_amdgcn_mfma_f32_4x4x1f32(xq[mr][2 * c + (e >> 2)][e & 3], wv[e], acc[mr], S::CBSZ, 0, 0);
-    }
-  };
-#pragma unroll
-  for (int st = 0; st < S::STAGES - 1; ++st) f32m_issue<WT, RG, MR>(f32m_ring, rs_x, rs_w, voff_x, voff_w, st, steps);
-  __builtin_amdgcn_s_waitcnt(vmcnt_only(S::PENDING));                // stage 0 has landed
-  asm volatile("" ::: "memory");
-  read_phase(f32m_ring, 0, w_a, x_a);
-  for (int step = 0; step < steps; ++step) {
-    const unsigned char* stage = f32m_ring + (step % S::STAGES) * S::STAGE;
-    const unsigned char* next = f32m_ring + ((step + 1) % S::STAGES) * S::STAGE;
-    // stage step - 1 has been read (its last phase was read a phase ago): it may be asked for again
-    asm volatile("" ::: "memory");
-    f32m_issue<WT, RG, MR>(f32m_ring, rs_x, rs_w, voff_x, voff_w, step + S::STAGES - 1, steps);
-#pragma unroll
-    for (int ph = 0; ph < PH; ph += 2) {
-      read_phase(stage, ph + 1, w_b, x_b);
-      __builtin_amdgcn_sched_barrier(0);
-      run_phase(w_a, x_a);
-      __builtin_amdgcn_sched_barrier(0);
-      if (ph + 2 < PH) {
-        read_phase(stage, ph + 2, w_a, x_a);
-      } else {
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(S::PENDING));          // the next stage has landed (past K: zeros, unused)
-        asm volatile("" ::: "memory");
-        read_phase(next, 0, w_a, x_a);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      run_phase(w_b, x_b);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(vmcnt_only(0));                       // the padding loads too, before the wave ends
-  const int n = n0 + 4 * cg + i;
-  if (n >= N) return;
-#pragma unroll
-  for (int mr = 0; mr < MR; ++mr)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = 16 * mr + 4 * rg + r;
-      if (m >= M) continue;
-      float* o = y + (size_t)m * ldy + n;
-      *o = accumulate ? (*o + acc[mr][r]) : acc[mr][r];
-    }
-}
-
-template <typename WT, int RG, int MR>
-static void launch_f32_mfma(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate,
-                            hipStream_t s) {
-  using S = F32MShape<WT, RG, MR>;
-  hipLaunchKernelGGL((gemm_f32_mfma_kernel<WT, RG, MR>), dim3((N + S::NCW - 1) / S::NCW), dim3(64), S::STAGES * S::STAGE, s, x, w,
-                     y, M, N, K, ldx, ldy, accumulate);
-}
-
-template <typename WT>
-static void launch_f32_mfma_rows(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate,
-                                 hipStream_t s) {
-  if (M <= 32) launch_f32_mfma<WT, 4, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
-  else launch_f32_mfma<WT, 4, 4>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
-}
-
-// ------------------------------------------------------------------------------ prompt portions on the matrix cores
-
-// Tiles of 128 x 128 outputs, four waves of 64 x 64.  v_mfma_f32_32x32x1_2b_f32 is one step of k for two blocks of
-// 32 x 32 outputs: D[i][j] = fma(A[i], B[j], D[i][j]), the same single-rounding multiply-add as above; with the A
-// operand of the first block broadcast to the second, an instruction is 32 rows (A: lane i < 32 holds row i) against
-// 64 columns (B: lane l holds column l), and a wave issues two of them a step, for its upper and lower 32 rows: two
-// chains that are independent, so that neither waits for its own last result.  Every output is still one chain over k
-// ascending from zero.  A lane needs two elements of x and one of W a step for 4096 multiply-adds of the wave.
-// Operands come through a ring of four stages of 32 steps of k in LDS that the workgroup shares (buffer loads with
-// LDS as destination, chunks permuted against bank conflicts, one barrier a stage).  K a multiple of 32.
-#define F32P_BM 128
-#define F32P_BN 128
-#define F32P_KB 32
-#define F32P_STAGES 4
-
-template <typename WT>
-struct F32PShape {
-  static constexpr int XBYTES = F32P_BM * F32P_KB * 4;                        // 16 KB
-  static constexpr int WROW = F32P_KB * (int)sizeof(WT);                      // 64 or 128 bytes
-  static constexpr int WBYTES = F32P_BN * WROW;
-  static constexpr int STAGE = XBYTES + WBYTES;
-  static constexpr int X_LOADS = XBYTES / 1024 / 4, W_LOADS = WBYTES / 1024 / 4;   // per wave
-  static constexpr int LPW = X_LOADS + W_LOADS;
-  static constexpr int PENDING = LPW * (F32P_STAGES - 2);
-};
-
-template <typename WT>
-__device__ __forceinline__ void f32p_issue(unsigned char* ring, __amdgpu_buffer_rsrc_t rs_x, __amdgpu_buffer_rsrc_t rs_w,
-                                           const int* voff_x, const int* voff_w, int wave, int step, int steps) {
-  using S = F32PShape<WT>;
-  typedef __attribute__((address_space(3))) void* lds_ptr;
-  unsigned char* dst = ring + (step % F32P_STAGES) * S::STAGE;
-  const bool real = step < steps;                                  // scalar
-#pragma unroll
-  for (int t = 0; t < S::X_LOADS; ++t)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (lds_ptr)(dst + (wave * S::X_LOADS + t) * 1024), 16,
-                                             real ? voff_x[t] : 0x7ffffff0, step * F32P_KB * 4, 0, 0);
-#pragma unroll
-  for (int t = 0; t < S::W_LOADS; ++t)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, (lds_ptr)(dst + S::XBYTES + (wave * S::W_LOADS + t) * 1024), 16,
-                                             real ? voff_w[t] : 0x7ffffff0, step * S::WROW, 0, 0);
-}
-
-typedef __attribute__((ext_vector_type(32))) float f32x32;
-
-template <typename WT>
-__global__ __launch_bounds__(256) void gemm_f32_mfma_tile_kernel(const float* __restrict__ x, const WT* __restrict__ w,
-                                                                float* __restrict__ y, int M, int N, int K, int ldx, int ldy,
-                                                                int accumulate) {
-  using S = F32PShape<WT>;
-  constexpr bool BF = sizeof(WT) == 2;
-  extern __shared__ __attribute__((aligned(16))) unsigned char f32p_ring[];
-  const int wave = wave_index(), lane = threadIdx.x & 63;
-  const int wy = wave >> 1, wx = wave & 1;
-  const int m0 = blockIdx.y * F32P_BM, n0 = blockIdx.x * F32P_BN;
-  const int x_rows = min(F32P_BM, M - m0), w_rows = min(F32P_BN, N - n0);
-  const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(x + (size_t)m0 * ldx), 0, (int)((((size_t)x_rows - 1) * ldx + K) * sizeof(float)), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rs_w =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, (int)((size_t)w_rows * K * sizeof(WT)), 0x00020000);
-  // loads: 1 KB an instruction.  Rows of 128 bytes (x; 32-bit weights): 8 rows, lane l fills slot l % 8 of row l / 8 with
-  // chunk slot ^ (row % 8).  Rows of 64 bytes (bfloat16 weights): 16 rows, slot l % 4 of row l / 4, chunk
-  // slot ^ ((row / 2) % 4).  Rows past the operand are clamped to its last: their outputs are never stored.
-  int voff_x[S::X_LOADS], voff_w[S::W_LOADS];
-#pragma unroll
-  for (int t = 0; t < S::X_LOADS; ++t) {
-    const int row = 8 * (wave * S::X_LOADS + t) + (lane >> 3), chunk = (lane & 7) ^ (row & 7);
-    voff_x[t] = (min(row, x_rows - 1) * ldx + 4 * chunk) * 4;
-  }
-#pragma unroll
-  for (int t = 0; t < S::W_LOADS; ++t) {
-    if constexpr (BF) {
-      const int row = 16 * (wave * S::W_LOADS + t) + (lane >> 2), chunk = (lane & 3) ^ ((row >> 1) & 3);
-      voff_w[t] = (min(row, w_rows - 1) * K + 8 * chunk) * 2;
-    } else {
-      const int row = 8 * (wave * S::W_LOADS + t) + (lane >> 3), chunk = (lane & 7) ^ (row & 7);
-      voff_w[t] = (min(row, w_rows - 1) * K + 4 * chunk) * 4;
-    }
-  }
-  // operand reads: rows wy*64 + (lane % 32) and 32 further of x; column wx*64 + lane of W
-  const int xr0 = wy * 64 + (lane & 31), xr1 = xr0 + 32;
-  const int x_off0 = xr0 * 128, x_off1 = xr1 * 128, x_swz = xr0 & 7;     // (xr1 % 8 == xr0 % 8)
-  const int wc = wx * 64 + lane;
-  const int w_off = S::XBYTES + wc * S::WROW, w_swz = BF ? (wc >> 1) & 3 : wc & 7;
-  f32x32 acc0, acc1;
-#pragma unroll
-  for (int r = 0; r < 32; ++r) {
-    acc0[r] = 0.f;
-    acc1[r] = 0.f;
-  }
-  const int steps = K / F32P_KB;
-#pragma unroll
-  for (int st = 0; st < F32P_STAGES - 1; ++st) f32p_issue<WT>(f32p_ring, rs_x, rs_w, voff_x, voff_w, wave, st, steps);
-  for (int step = 0; step < steps; ++step) {
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(S::PENDING));
-    __builtin_amdgcn_s_barrier();                                    // everyone has the stage at hand and is done with the one before
-    asm volatile("" ::: "memory");
-    f32p_issue<WT>(f32p_ring, rs_x, rs_w, voff_x, voff_w, wave, step + F32P_STAGES - 1, steps);
-    const unsigned char* stage = f32p_ring + (step % F32P_STAGES) * S::STAGE;
-#pragma unroll
-    for (int c8 = 0; c8 < F32P_KB / 8; ++c8) {                        // 8 steps of k at a time
-      float wv[8];
-      if constexpr (BF) {
-        const u32x4 raw = *reinterpret_cast<const u32x4*>(stage + w_off + ((c8 ^ w_swz) * 16));
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {                                 // bfloat16 -> 32-bit: the bits, shifted (exact)
-          wv[2 * q] = __uint_as_float(raw[q] << 16);
-          wv[2 * q + 1] = __uint_as_float(raw[q] & 0xffff0000u);
-        }
-      } else {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const f32x4 raw = *reinterpret_cast<const f32x4*>(stage + w_off + (((2 * c8 + h) ^ w_swz) * 16));
-#pragma unroll
-          for (int q = 0; q < 4; ++q) wv[4 * h + q] = raw[q];
-        }
-      }
-      f32x4 xa[2], xb[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        xa[h] = *reinterpret_cast<const f32x4*>(stage + x_off0 + (((2 * c8 + h) ^ x_swz) * 16));
-        xb[h] = *reinterpret_cast<const f32x4*>(stage + x_off1 + (((2 * c8 + h) ^ x_swz) * 16));
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {                                   // k ascending; the two chains alternate
-        acc0 = __builtin_amdgcn_mfma_f32_32x32x1f32(xa[e >> 2][e & 3], wv[e], acc0, 1, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_32x32x1f32(xb[e >> 2][e & 3], wv[e], acc1, 1, 0, 0);
-      }
-    }
-    asm volatile("" ::: "memory");
-  }
-  __builtin_amdgcn_s_waitcnt(vmcnt_only(0));                         // the padding loads too, before the waves end
-  // lane l, register r of a block: row 8 * (r / 4) + 4 * (l / 32) + r % 4 of the 32, column l % 32 (+ 32 for the
-  // second block, registers 16 to 31)
-#pragma unroll
-  for (int half = 0; half < 2; ++half)
-#pragma unroll
-    for (int r = 0; r < 32; ++r) {
-      const int m = m0 + wy * 64 + 32 * half + 8 * ((r & 15) >> 2) + 4 * (lane >> 5) + (r & 3);
-      const int n = n0 + wx * 64 + 32 * (r >> 4) + (lane & 31);
-      if (m < M && n < N) {
-        float* o = y + (size_t)m * ldy + n;
-        const float v = half == 0 ? acc0[r] : acc1[r];
-        *o = accumulate ? (*o + v) : v;
-      }
-    }
-}
-
-// Tiles of 64 RB x 64 outputs, four waves of 16 RB x 64 (RB 1 or 2), for the same products: v_mfma_f32_16x16x1_4b_f32 is one step
-// of k for four blocks of 16 x 16 outputs; with the A operand of the first block broadcast, 16 rows (lane i < 16 holds row i)
-// against 64 columns.  A 128 x 128 tile keeps a SIMD busy with 64 x 64 outputs, 167 to 188 clocks a step of k whatever the
-// rest of the chip does: 450 rows against 2,048 columns are 64 workgroups above, a quarter of the chip, and 256 here.
-// What bounds it is the matrix instructions' own time (33 clocks and 4 a vector instruction, which does not run under
-// them, not even another wave's): a step of k measured 51 to 58 clocks a tile of 64 x 64, 90 to 104 of 128 x 64.
-// Measured with bfloat16 weights: 450 rows, 2048 x 8192: 571 -> 211 us, 2048 x 2048: 150 -> 55, 6144 x 2048: 163 -> 135.
-template <typename WT, int RB>
-struct F32QShape {
-  static constexpr int BM = 64 * RB, BN = 64, KB = 32, STAGES = 4;
-  static constexpr int XBYTES = BM * KB * 4, WROW = KB * (int)sizeof(WT), WBYTES = BN * WROW, STAGE = XBYTES + WBYTES;
-  static constexpr int X_LOADS = XBYTES / 1024 / 4, W_LOADS = WBYTES / 1024 / 4, LPW = X_LOADS + W_LOADS;   // 1 KB instructions a wave
-  static constexpr int XQ = 4, WQ = WROW / 32;                      // 16-byte reads of a half stage: of a row of x, of a column of W
-};
-
-template <typename WT, int RB>
-__device__ __forceinline__ void f32q_issue(unsigned char* ring, __amdgpu_buffer_rsrc_t rs_x, __amdgpu_buffer_rsrc_t rs_w,
-                                           const int* voff_x, const int* voff_w, int wave, int step, int steps) {
-  using S = F32QShape<WT, RB>;
-  typedef __attribute__((address_space(3))) void* lds_ptr;
-  unsigned char* dst = ring + (step % S::STAGES) * S::STAGE;
-  const bool real = step < steps;                                  // scalar
-#pragma unroll
-  for (int t = 0; t < S::X_LOADS; ++t)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (lds_ptr)(dst + (wave * S::X_LOADS + t) * 1024), 16,
-                                             real ? voff_x[t] : 0x7ffffff0, step * S::KB * 4, 0, 0);
-#pragma unroll
-  for (int t = 0; t < S::W_LOADS; ++t)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, (lds_ptr)(dst + S::XBYTES + (wave * S::W_LOADS + t) * 1024), 16,
-                                             real ? voff_w[t] : 0x7ffffff0, step * S::WROW, 0, 0);
-}
-
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-
-// The operands of half a stage (16 steps of k), and the 16 RB matrix instructions on them.
-template <typename WT, int RB>
-struct F32QHalf {
-  f32x4 x[RB][F32QShape<WT, RB>::XQ];
-  u32x4 w[F32QShape<WT, RB>::WQ];
-};
-
-template <typename WT, int RB>
-__device__ __forceinline__ void f32q_read(const unsigned char* stage, int half, int x_off, int x_swz, int w_off, int w_swz, F32QHalf<WT, RB>& h) {
-  using S = F32QShape<WT, RB>;
-#pragma unroll
-  for (int c = 0; c < S::WQ; ++c) h.w[c] = *reinterpret_cast<const u32x4*>(stage + w_off + (((S::WQ * half + c) ^ w_swz) * 16));
-#pragma unroll
-  for (int c = 0; c < S::XQ; ++c)
-#pragma unroll
-    for (int b = 0; b < RB; ++b) h.x[b][c] = *reinterpret_cast<const f32x4*>(stage + x_off + b * 16 * 128 + (((S::XQ * half + c) ^ x_swz) * 16));
-}
-
-template <typename WT, int RB>
-__device__ __forceinline__ void f32q_run(const F32QHalf<WT, RB>& h, f32x16 (&acc)[RB]) {
-  // every weight is widened before the first matrix instruction: between a vector instruction and a matrix instruction
-  // that reads its result there are two idle slots, and a wave's vector instructions do not run under its own matrix ones
-  float wv[16];
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    if constexpr (sizeof(WT) == 2) {                                 // bfloat16 -> 32-bit: the bits, shifted (exact)
-      const uint32_t two = h.w[k >> 3][(k >> 1) & 3];
-      wv[k] = __uint_as_float((k & 1) ? two & 0xffff0000u : two << 16);
-    } else {
-      wv[k] = __uint_as_float(h.w[k >> 2][k & 3]);
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int k = 0; k < 16; ++k)                                       // ascending
-#pragma unroll
-    for (int b = 0; b < RB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(h.x[b][k >> 2][k & 3], wv[k], acc[b], 2, 0, 0);
-}
-
-template <typename WT, int RB>
-__global__ __launch_bounds__(256) void gemm_f32_mfma_columns_kernel(const float* __restrict__ x, const WT* __restrict__ w,
-                                                                   float* __restrict__ y, int M, int N, int K, int ldx, int ldy,
-                                                                   int accumulate, int m_tiles) {
-  using S = F32QShape<WT, RB>;
-  constexpr bool BF = sizeof(WT) == 2;
-  extern __shared__ __attribute__((aligned(16))) unsigned char f32q_ring[];
-  const int wave = wave_index(), lane = threadIdx.x & 63;
-  // the row tiles of a column tile run one after the other on one die: its weights come from memory once
-  int bid = blockIdx.x;
-  if (gridDim.x % 8 == 0) bid = (bid % 8) * (gridDim.x / 8) + bid / 8;
-  const int m0 = (bid % m_tiles) * S::BM, n0 = (bid / m_tiles) * S::BN;
-  const int x_rows = min(S::BM, M - m0), w_rows = min(S::BN, N - n0);
-  const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(x + (size_t)m0 * ldx), 0, (int)((((size_t)x_rows - 1) * ldx + K) * sizeof(float)), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rs_w =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, (int)((size_t)w_rows * K * sizeof(WT)), 0x00020000);
-  // loads as in the kernel above.  The permutations are for the sixteen lanes that LDS serves together in a 16-byte read
-  // (0-3, 12-15, 20-27 of each half wave, and the others): rows of 128 bytes want the chunk exchanged by row / 2, rows of 64 by row / 4.
-  int voff_x[S::X_LOADS], voff_w[S::W_LOADS];
-#pragma unroll
-  for (int t = 0; t < S::X_LOADS; ++t) {
-    const int row = 8 * (wave * S::X_LOADS + t) + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
-    voff_x[t] = (min(row, x_rows - 1) * ldx + 4 * chunk) * 4;
-  }
-#pragma unroll
-  for (int t = 0; t < S::W_LOADS; ++t) {
-    if constexpr (BF) {
-      const int row = 16 * (wave * S::W_LOADS + t) + (lane >> 2), chunk = (lane & 3) ^ ((row >> 2) & 3);
-      voff_w[t] = (min(row, w_rows - 1) * K + 8 * chunk) * 2;
-    } else {
-      const int row = 8 * (wave * S::W_LOADS + t) + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
-      voff_w[t] = (min(row, w_rows - 1) * K + 4 * chunk) * 4;
-    }
-  }
-  // operand reads: rows 16 RB wave + 16 b + lane % 16 of x (the instruction uses the first sixteen lanes'), column ``lane`` of W
-  const int xr = 16 * RB * wave + (lane & 15), x_off = xr * 128, x_swz = (xr >> 1) & 7;
-  const int w_off = S::XBYTES + lane * S::WROW, w_swz = BF ? (lane >> 2) & 3 : (lane >> 1) & 7;
-  f32x16 acc[RB];
-#pragma unroll
-  for (int b = 0; b < RB; ++b)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
-  const int steps = K / S::KB;
-  // Half a stage is read from LDS while the matrix instructions of the half before run; the wait for the next stage
-  // and the barrier stand between a stage's two halves.
-  F32QHalf<WT, RB> h0, h1;
-#pragma unroll
-  for (int st = 0; st < S::STAGES - 1; ++st) f32q_issue<WT, RB>(f32q_ring, rs_x, rs_w, voff_x, voff_w, wave, st, steps);
-  __builtin_amdgcn_s_waitcnt(vmcnt_only(2 * S::LPW));                // this wave's share of stage 0 has landed
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  f32q_read<WT, RB>(f32q_ring, 0, x_off, x_swz, w_off, w_swz, h0);
-  for (int step = 0; step < steps; ++step) {
-    f32q_read<WT, RB>(f32q_ring + (step % S::STAGES) * S::STAGE, 1, x_off, x_swz, w_off, w_swz, h1);
-    __builtin_amdgcn_sched_barrier(0);
-    f32q_run<WT, RB>(h0, acc);
-    __builtin_amdgcn_sched_barrier(0);
-    // this wave's share of the next stage has landed (past K: zeros, unused); behind the barrier everyone's has, and
-    // everyone is done with the stage before this one, whose place the stage asked for next takes
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(S::LPW));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    f32q_issue<WT, RB>(f32q_ring, rs_x, rs_w, voff_x, voff_w, wave, step + S::STAGES - 1, steps);
-    f32q_read<WT, RB>(f32q_ring + ((step + 1) % S::STAGES) * S::STAGE, 0, x_off, x_swz, w_off, w_swz, h0);
-    __builtin_amdgcn_sched_barrier(0);
-    f32q_run<WT, RB>(h1, acc);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  __builtin_amdgcn_s_waitcnt(vmcnt_only(0));                         // the padding loads too, before the waves end
-  // block j, register i of it, lane l: row 4 * (l / 16) + i of the 16, column 16 j + l % 16
-#pragma unroll
-  for (int b = 0; b < RB; ++b)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = m0 + 16 * RB * wave + 16 * b + 4 * (lane >> 4) + i, n = n0 + 16 * j + (lane & 15);
-        if (m < M && n < N) {
-          float* o = y + (size_t)m * ldy + n;
-          *o = accumulate ? (*o + acc[b][4 * j + i]) : acc[b][4 * j + i];
-        }
-      }
-}
-
-template <typename WT, int RB>
-static void launch_f32_mfma_columns(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s) {
-  using S = F32QShape<WT, RB>;
-  constexpr int lds_bytes = S::STAGES * S::STAGE;
-  static bool allowed = false;                       // more than 64 KB of dynamic LDS has to be asked for once
-  if (lds_bytes > 48 * 1024 && !allowed) {
-    (void)hipFuncSetAttribute((const void*)gemm_f32_mfma_columns_kernel<WT, RB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    allowed = true;
-  }
-  const int m_tiles = (M + S::BM - 1) / S::BM, n_tiles = (N + S::BN - 1) / S::BN;
-  hipLaunchKernelGGL((gemm_f32_mfma_columns_kernel<WT, RB>), dim3(m_tiles * n_tiles), dim3(256), lds_bytes, s, x, w, y, M, N, K, ldx, ldy,
-                     accumulate, m_tiles);
-}
+// ------------------------------------------------------------------------------ which kernel a product gets
 
 // Which tiles a prompt's product gets, rows x columns: clocks a step of k a round of the compute units, as measured with bfloat16
-// weights (the comment at F32QShape), times the rounds.  With 32-bit weights, which need no widening, every tile takes about a tenth
-// less, so the same rule holds: over 65 to 2,048 rows, 512 to 16,384 columns and K of 512 to 8,192 its choice took 0.33 to 1.01
-// of the 128 x 128 tiles' time with either (450 rows, 2048 x 8192: 519 us -> 174 with 32-bit weights, 572 -> 194 with bfloat16).
+// weights (100 and 200 rows, K = 2048 and 8192: 15.8, 31 and 58 ns), times the rounds.  With 32-bit weights, which need no widening,
+// every tile takes 1.02 to 1.06 times as long (their loads are twice as wide), so the same rule holds.
 struct F32PromptTile {
   int rows, columns;
 };
@@ -1224,10 +579,10 @@ static F32PromptTile f32_prompt_tile(int M, int N) {
   auto cost = [&](int bm, int bn, int clocks) {
     return (long long)clocks * ((((long long)(M + bm - 1) / bm) * ((N + bn - 1) / bn) + 255) / 256);
   };
-  const long long big = cost(F32P_BM, F32P_BN, 185), one = cost(64, 64, 55), two = cost(128, 64, 103);
+  const long long big = cost(128, 128, 137), one = cost(64, 64, 37), two = cost(128, 64, 73);
   if (one < big && one <= two) return {64, 64};
   if (two < big) return {128, 64};
-  return {F32P_BM, F32P_BN};
+  return {128, 128};
 }
 
 extern "C" int bw_gemm_f32_prompt_tile(int M, int N, int* rows, int* columns) {
@@ -1239,20 +594,42 @@ extern "C" int bw_gemm_f32_prompt_tile(int M, int N, int* rows, int* columns) {
 }
 
 template <typename WT>
-static void launch_f32_mfma_tiles(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate,
-                                  hipStream_t s) {
-  using S = F32PShape<WT>;
+static void launch_f32_prompt(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s) {
   const F32PromptTile tile = f32_prompt_tile(M, N);
-  if (tile.rows == 64) return launch_f32_mfma_columns<WT, 1>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
-  if (tile.columns == 64) return launch_f32_mfma_columns<WT, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
-  constexpr int lds_bytes = F32P_STAGES * S::STAGE;
-  static bool allowed = false;                       // more than 64 KB of dynamic LDS has to be asked for once
-  if (!allowed) {
-    (void)hipFuncSetAttribute((const void*)gemm_f32_mfma_tile_kernel<WT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    allowed = true;
+  if (tile.rows == 64) {
+    // more than two workgroups a compute unit: without loading waves three of them fit (450 rows, 6144 x 2048: 96 us against 117);
+    // with no more than that their own loads cost the working waves more (2048 x 8192: 145 us against 133)
+    const long long wgs = ((M + 63) / 64) * (long long)((N + 63) / 64);
+    if (wgs > 512) return launch_f32_tiles<WT, 4, 1, 1, 4, 32, 4, 0>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+    return launch_f32_tiles<WT, 4, 1, 1, 4, 32, 4, 4>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
   }
-  hipLaunchKernelGGL(gemm_f32_mfma_tile_kernel<WT>, dim3((N + F32P_BN - 1) / F32P_BN, (M + F32P_BM - 1) / F32P_BM), dim3(256),
-                     lds_bytes, s, x, w, y, M, N, K, ldx, ldy, accumulate);
+  if (tile.columns == 64) return launch_f32_tiles<WT, 8, 1, 1, 4, 32, 4, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+  launch_f32_tiles<WT, 8, 2, 1, 4, 32, 4, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+}
+
+// Up to 64 rows, K a multiple of 64 (of 32 where the tiles of 64 x 64 take it); us with bfloat16 weights and K = 2048:
+//   as strips while those of 32 columns are one workgroup a compute unit at most (8 rows of 6144 columns 10.9, as tiles 14.8; 32 rows
+//   of 2048 columns 11.1 and 14.7; beyond that LDS bounds them: 32 rows of 6144 columns 20.6 and 14.9);
+//   up to 16 rows as tiles of 16 x 64 (16384 columns 15.8; strips 20);
+//   more rows as tiles of 32 x 32 (16384 columns 23, 6144 15 to 22), from 33 rows and 256 blocks of 64 columns on as tiles of 64 x 64
+//   (64 rows of 16384 columns 41 and 37; of 6144 columns 22 and 36).
+enum { F32_STRIPS, F32_TILES_16, F32_TILES_32, F32_TILES_64 };
+
+static int f32_few_rows_kernel(int M, int N, int K) {
+  if (K % 64 != 0) return F32_TILES_64;
+  if ((M + 15) / 16 * ((long long)(N + 31) / 32) <= 256) return F32_STRIPS;
+  if (M <= 16) return F32_TILES_16;
+  return M > 32 && (N + 63) / 64 >= 256 ? F32_TILES_64 : F32_TILES_32;
+}
+
+template <typename WT>
+static void launch_f32_few_rows(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s) {
+  switch (f32_few_rows_kernel(M, N, K)) {
+    case F32_STRIPS: return launch_f32_strips<WT, 2, 9>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+    case F32_TILES_16: return launch_f32_tiles<WT, 1, 1, 1, 4, 64, sizeof(WT) == 2 ? 6 : 5, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+    case F32_TILES_32: return launch_f32_tiles<WT, 1, 1, 2, 2, 64, 4, 0>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+    default: return launch_f32_tiles<WT, 4, 1, 1, 4, 32, 4, 4>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+  }
 }
 
 template <typename WT, int MR>
@@ -1284,43 +661,35 @@ extern "C" int bw_gemm_f32(const float* x, const void* w, int w_is_bf16, float* 
   hipStream_t s = (hipStream_t)stream;
   // which kernel runs depends on the shape alone, and both run the same chains
   const int wc = w_is_bf16 ? 8 : 4;
-  // 17 to 64 rows, K in whole stages: the chains run on the matrix cores (offsets within x and within a wave's rows
-  // of W must fit the buffer descriptors' 31 bits).  Up to 16 rows stay on the vector unit: a matrix instruction that
-  // depends on the one before it issues some 40 clocks later, a vector multiply-add 9, and so few rows have too few
-  // chains to fill the gap.
-  if (M > 16 && M <= 64 && K % 64 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 &&
-      (size_t)M * ldx * 4 < ((size_t)1 << 31) && (size_t)64 * K * 4 < ((size_t)1 << 31)) {
-    if (w_is_bf16) launch_f32_mfma_rows<bf16_t>(x, (const bf16_t*)w, y, M, N, K, ldx, ldy, accumulate, s);
-    else launch_f32_mfma_rows<float>(x, (const float*)w, y, M, N, K, ldx, ldy, accumulate, s);
-    return BW_LAUNCH_CHECK();
-  }
-  // up to 8 rows, many columns, K in whole stages: a wave a row, the row four elements a register, loader waves
-  if (M <= F32C_MAX_ROWS && (N + 63) / 64 >= F32L_MIN_BLOCKS && K % (w_is_bf16 ? 64 : 32) == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 &&
-      ((uintptr_t)w & 15) == 0 && (size_t)64 * K * 4 < ((size_t)1 << 31) && (size_t)M * ldx * 4 < ((size_t)1 << 31)) {
+  // offsets within a tile's rows of x and columns of W must fit the buffer descriptors' 31 bits
+  const bool vectors = ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
+  const int tile_rows = M > 64 ? 128 : (M < 64 ? M : 64), tile_columns = M > 64 ? 128 : 64;
+  const bool fits = vectors && (size_t)tile_rows * ldx * 4 < ((size_t)1 << 31) && (size_t)tile_columns * K * 4 < ((size_t)1 << 31);
+  // one row, many columns, K in whole stages: a chain a lane, the row four elements a register, loader waves
+  if (fits && M <= F32C_MAX_ROWS && (N + 63) / 64 >= F32C_MIN_BLOCKS && K % (w_is_bf16 ? 64 : 32) == 0) {
     if (w_is_bf16) launch_chain<bf16_t>(x, (const bf16_t*)w, y, M, N, K, ldx, ldy, accumulate, s);
     else launch_chain<float>(x, (const float*)w, y, M, N, K, ldx, ldy, accumulate, s);
     return BW_LAUNCH_CHECK();
   }
-  // up to 16 rows, many columns, K in whole stages: a wave a row, weights packed in LDS
-  if (M <= 16 && (N + 63) / 64 >= F32L_MIN_BLOCKS && K % (w_is_bf16 ? 64 : 32) == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 &&
-      ((uintptr_t)w & 15) == 0 && (size_t)64 * K * 4 < ((size_t)1 << 31) && (size_t)M * ldx * 4 < ((size_t)1 << 31)) {
-    if (w_is_bf16) launch_lanes<bf16_t>(x, (const bf16_t*)w, y, M, N, K, ldx, ldy, accumulate, s);
-    else launch_lanes<float>(x, (const float*)w, y, M, N, K, ldx, ldy, accumulate, s);
+  // up to 64 rows, K in whole stages: the chains run on the matrix cores (K % 64 == 32: for so many outputs only that the chains of
+  // the vector units, which take 16 rows by 16 columns a workgroup, are slower)
+  if (fits && M <= 64 && (K % 64 == 0 || (K % 32 == 0 && (M > 16 || (N + 63) / 64 >= 256)))) {
+    if (w_is_bf16) launch_f32_few_rows<bf16_t>(x, (const bf16_t*)w, y, M, N, K, ldx, ldy, accumulate, s);
+    else launch_f32_few_rows<float>(x, (const float*)w, y, M, N, K, ldx, ldy, accumulate, s);
     return BW_LAUNCH_CHECK();
   }
-  if (M <= 64 && K % wc == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0) {
+  if (M <= 64 && K % wc == 0 && vectors) {
     if (w_is_bf16) launch_rows<bf16_t>(x, (const bf16_t*)w, y, M, N, K, ldx, ldy, accumulate, s);
     else launch_rows<float>(x, (const float*)w, y, M, N, K, ldx, ldy, accumulate, s);
     return BW_LAUNCH_CHECK();
   }
   // prompt portions, K in whole stages: tiles on the matrix cores (the same chains)
-  if (M > 64 && K % F32P_KB == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 &&
-      (size_t)F32P_BM * ldx * 4 < ((size_t)1 << 31) && (size_t)F32P_BN * K * 4 < ((size_t)1 << 31)) {
-    if (w_is_bf16) launch_f32_mfma_tiles<bf16_t>(x, (const bf16_t*)w, y, M, N, K, ldx, ldy, accumulate, s);
-    else launch_f32_mfma_tiles<float>(x, (const float*)w, y, M, N, K, ldx, ldy, accumulate, s);
+  if (fits && M > 64 && K % 32 == 0) {
+    if (w_is_bf16) launch_f32_prompt<bf16_t>(x, (const bf16_t*)w, y, M, N, K, ldx, ldy, accumulate, s);
+    else launch_f32_prompt<float>(x, (const float*)w, y, M, N, K, ldx, ldy, accumulate, s);
     return BW_LAUNCH_CHECK();
   }
-  if (M > 64 && K % F32T_BK == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0) {
+  if (M > 64 && K % F32T_BK == 0 && vectors) {
     dim3 tgrid((N + F32T_BN - 1) / F32T_BN, (M + F32T_BM - 1) / F32T_BM);
     if (w_is_bf16)
       hipLaunchKernelGGL(gemm_f32_tile_kernel<bf16_t>, tgrid, block, 0, s, x, (const bf16_t*)w, y, M, N, K, ldx, ldy, accumulate);
