@@ -136,14 +136,15 @@ int bw_norm_shift(const float* x, int ldx, const float* w, const float* mix, flo
 // mode 6: mode 0 with the decays themselves in gate (bw_decay_rows; no bias).  Passes over chunks: this in place of mode 0.
 // q is multiplied by qscale, k by kscale; heads_per_key neighbouring heads share one q and one k.
 // (silu 1, fixed decay only: q, k and v pass SiLU on their way in; few 1: the requests bring a few rows each, which picks the
-// kernel that favours many waves over long walks, the same bits)
+// kernel that favours many waves over long walks, the same bits; in_stages 1, modes 1 (with gates, 3 heads floats a row of scratch) and
+// 6 with heads of 64 or 128 channels: portions that are long for the number of memories, columns in stages, the same bits)
 int bw_linear_recurrence(int mode, const float* proj, int ldp, int q_off, int k_off, int v_off, const float* gate, int ldg,
                          int gate_off, int gate2_off, const float* bias, const float* bias2, float param, float qscale,
                          float kscale, const float* skip, int heads_per_key, int silu, int few, float* state, long long state_ld, float* out,
                          int ldo, const int32_t* seq_rows,
                          const int32_t* slots, const int32_t* positions, int nseq, int heads, int dim, int vdim,
                          const int32_t* chunks, int nchunks, const int32_t* spans, int nspans, float* scan_local,
-                         float* scan_start, long long scan_floats, void* stream);
+                         float* scan_start, long long scan_floats, int in_stages, float* gates, void* stream);
 // z[r][c] <- exp(logsigmoid(z[r][c] + bias[c]) * param), in place: the decays of mode 0 for mode 6
 int bw_decay_rows(float* z, int ld, const float* bias, float param, int rows, int cols, void* stream);
 long long bw_recurrence_record(int dim, int vdim);      // floats that scan_local and scan_start hold per chunk and head

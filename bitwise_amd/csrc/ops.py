@@ -105,7 +105,8 @@ _SIGS = {
     "bw_decay_rows": [c_void_p, c_int, c_void_p, c_float, c_int, c_int, c_void_p],
     "bw_linear_recurrence": [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p,
                              c_float, c_float, c_float, c_void_p, c_int, c_int, c_int, c_void_p, c_longlong, c_void_p, c_int, c_void_p, c_void_p,
-                             c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_longlong, c_void_p],
+                             c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_longlong, c_int, c_void_p,
+                             c_void_p],
     "bw_head_norm_gate": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_int,
                           c_int, c_int, c_float, c_void_p],
     "bw_gated_part_norm": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_int, c_float,
@@ -931,7 +932,7 @@ def linear_recurrence(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_o
                       state: torch.Tensor, out: torch.Tensor, seq_rows: torch.Tensor, slots: torch.Tensor,
                       positions: torch.Tensor, nseq: int, heads: int, dim: int, vdim: int, scan=None, kscale: float = 1.0,
                       heads_per_key: int = 1, skip: Optional[torch.Tensor] = None, silu: bool = False,
-                      few_rows: bool = False) -> None:
+                      few_rows: bool = False, in_stages: bool = False, gates: Optional[torch.Tensor] = None) -> None:
     """The recurrence S <- decay * S + k v^T, o = S^T (q * qscale) per head over every request's rows in order, from and
     to ``state`` [slots, elements].  RECUR_DECAY_PER_CHANNEL: decay = exp(logsigmoid(gate + bias) * param) per key
     channel (``gate`` [rows, >= gate_off + heads*dim]).  RECUR_SCALAR_GATES: capped input and forget gates per head
@@ -947,7 +948,9 @@ def linear_recurrence(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_o
     behind the decays, from gate2_off + heads on, the products k.q of the key heads, as they enter; ``bias`` None):
     S <- a S, S <- S + k (b (v - S^T k))^T, then the read-out; always in one pass.
     ``silu`` (fixed decay): q, k and v are the SiLU of what ``proj`` holds.  ``few_rows``: every request brings a few rows (the same
-    bits; a kernel that favours many waves over long walks).
+    bits; a kernel that favours many waves over long walks).  ``in_stages`` (RECUR_DECAY_GIVEN, and RECUR_SCALAR_GATES with
+    ``gates``, float32 scratch of 3 * heads a row): the portions are long for the number of memories (the same bits; heads of 64 or
+    128 channels, others are walked as without it).
     k is multiplied by ``kscale``; ``heads_per_key`` neighbouring heads share one q and one k.  A head's state lies as
     [value column][key channel].  ``state`` may be a column slice of a wider tensor.
 
@@ -1027,6 +1030,10 @@ def linear_recurrence(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_o
         _need(start, torch.float32, "scan records")
         if chunks.numel() < 4 * nchunks or spans.numel() < 3 * nspans or start.numel() < local.numel():
             raise ValueError("linear_recurrence: the scan's tables or records do not fit")
+    if gates is not None:
+        _need(gates, torch.float32, "gates")
+        if gates.dim() != 2 or gates.shape[0] < out.shape[0] or gates.shape[1] != 3 * heads:
+            raise ValueError("linear_recurrence: the scratch for prepared gates does not fit the rows and heads")
     _check(_fn("bw_linear_recurrence")(int(mode), proj.data_ptr(), proj.stride(0), q_off, k_off, v_off,
                                        0 if gate is None else gate.data_ptr(), 0 if gate is None else gate.stride(0),
                                        gate_off, gate2_off, 0 if bias is None else bias.data_ptr(),
@@ -1037,7 +1044,8 @@ def linear_recurrence(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_o
                                        0 if chunks is None else chunks.data_ptr(), nchunks,
                                        0 if spans is None else spans.data_ptr(), nspans,
                                        0 if local is None else local.data_ptr(), 0 if start is None else start.data_ptr(),
-                                       0 if local is None else local.numel(), _stream()), "linear_recurrence")
+                                       0 if local is None else local.numel(), int(in_stages), 0 if gates is None else gates.data_ptr(),
+                                       _stream()), "linear_recurrence")
 
 
 def rotate_halves_rows(x: torch.Tensor, offsets: Sequence[int], heads: int, dim: int, rot: int, cos: torch.Tensor,

@@ -999,6 +999,8 @@ int launch_recurrence_passes(const RecurArgs& a, int nseq, bool few, int nchunks
   return rc;
 }
 
+#include "recurrence_stages.h"
+
 // ------------------------------------------------------------------------- per-head RMS norm and output gate
 
 enum { GATE_SIGMOID = 0, GATE_SILU = 1 };
@@ -1237,7 +1239,8 @@ extern "C" int bw_linear_recurrence(int mode, const float* proj, int ldp, int q_
                                     float qscale, float kscale, const float* skip, int heads_per_key, int silu, int few, float* state, long long state_ld, float* out, int ldo,
                                     const int32_t* seq_rows, const int32_t* slots, const int32_t* positions, int nseq,
                                     int heads, int dim, int vdim, const int32_t* chunks, int nchunks, const int32_t* spans,
-                                    int nspans, float* scan_local, float* scan_start, long long scan_floats, void* stream) {
+                                    int nspans, float* scan_local, float* scan_start, long long scan_floats, int in_stages, float* gates,
+                                    void* stream) {
   if (nseq <= 0 && nchunks <= 0) return 0;
   if (nchunks > 0) {
     if (chunks == nullptr || spans == nullptr || nspans <= 0 || scan_local == nullptr || scan_start == nullptr) return -2;
@@ -1252,6 +1255,8 @@ extern "C" int bw_linear_recurrence(int mode, const float* proj, int ldp, int q_
   RecurArgs a{proj, ldp, q_off, k_off, v_off, gate, ldg, gate_off, gate2_off, bias, bias2, skip, heads_per_key, param, qscale, kscale, silu, state, state_ld,
               out, ldo, seq_rows, slots, positions, heads, dim, vdim, chunks, scan_local, scan_start};
   hipStream_t s = (hipStream_t)stream;
+  if (in_stages && nchunks <= 0 && !few && (mode == RECUR_DECAY_GIVEN || (mode == RECUR_SCALAR_GATES && gates != nullptr)) && stages_fit(a, mode))
+    return launch_in_stages(mode, a, gates, nseq, s);
   if (mode == RECUR_SCALAR_GATES) return launch_recurrence_passes<RECUR_SCALAR_GATES>(a, nseq, few != 0, nchunks, spans, nspans, s);
   if (mode == RECUR_DECAY_PER_CHANNEL) return launch_recurrence_passes<RECUR_DECAY_PER_CHANNEL>(a, nseq, few != 0, nchunks, spans, nspans, s);
   if (mode == RECUR_BONUS_DECAY) return launch_recurrence_passes<RECUR_BONUS_DECAY>(a, nseq, few != 0, nchunks, spans, nspans, s);

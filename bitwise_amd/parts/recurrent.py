@@ -42,6 +42,11 @@ FEW_SEQ_ROWS = 4         # steps whose requests bring up to so many rows each ru
 # -> 8.7, 48 rows 12.3 -> 11.0; 16 of 16: 64 rows 11.6 -> 12.0, 96 rows 16.2 -> 15.5), heads of 64 channels and more sooner where
 # the step's requests together fill the chip (8 x 5 rows: 32 heads of 64 10.7 -> 9.3, 8 of 128 20.4 -> 15.8).
 DECAYS_AHEAD_CHAIN, DECAYS_AHEAD_COLUMNS = 1200, 40960
+# A long portion walks its memories in stages where they leave the chip idle: from so many rows on, and up to so many columns
+# (heads x value channels) times requests of the longest one's length: (decays given, scalar gates).  Microseconds, walk -> stages, 2,048 columns:
+# decays 48 rows 11.3 -> 10.9, 80 rows 14.9 -> 10.9, two requests of 64 rows 12.4 -> 12.1, three of 128 21.2 -> 26.3, of 683 93 -> 98; gates 64 rows 21.6
+# -> 22.1, 80 rows 26.8 -> 24.4, three requests of 128 rows 45.8 -> 43.6, four of 512 161 -> 142.
+STAGES_MIN_ROWS, STAGES_MAX_COLUMNS = (64, 80), (4096, 8192)
 SCAN_CHUNK = 32          # rows of a chunk of a long portion
 SCAN_MIN_ROWS = 96       # portions from this many rows on run in three passes over chunks (shorter ones are walked whole),
                          # where the engine allows logits to depend on the cut in their last bits (Workspace.exact_cuts False)
@@ -157,10 +162,14 @@ class _MatrixMemoryMixer(Mixer):
             local = ctx.ws.buffer("recur_scan_local", most * rec, torch.float32, rows=1)
             start = ctx.ws.buffer("recur_scan_start", most * rec, torch.float32, rows=1)
             scan = (chunks, nchunks, spans, nspans, local, start)
-        ops.linear_recurrence(self.mode if mode is None else mode, y, at["r"] if "q" not in at else at["q"], at["k"], at["v"], gate, gate_off, gate2_off,
+        mode = self.mode if mode is None else mode
+        stages = plan is None and mode in (ops.RECUR_DECAY_GIVEN, ops.RECUR_SCALAR_GATES) and in_stages(
+            max_seq_rows(ctx), ctx.rows, self.heads * self.vdim, mode == ops.RECUR_SCALAR_GATES)
+        gates = ctx.ws.buffer("recur_gates", 3 * self.heads, torch.float32) if stages and mode == ops.RECUR_SCALAR_GATES else None
+        ops.linear_recurrence(mode, y, at["r"] if "q" not in at else at["q"], at["k"], at["v"], gate, gate_off, gate2_off,
                               bias, bias2, param, self.qscale, call.state if state is None else state, raw, seq_rows, ctx.slots, ctx.positions, nseq,
                               self.heads, self.dim, self.vdim, scan=scan, kscale=kscale, heads_per_key=heads_per_key, skip=skip, silu=silu,
-                              few_rows=max_seq_rows(ctx) <= FEW_SEQ_ROWS)
+                              few_rows=max_seq_rows(ctx) <= FEW_SEQ_ROWS, in_stages=stages, gates=gates)
 
     def _finish(self, ctx, y, raw, target, add: bool = True, g_off: Optional[int] = None) -> None:
         act = ctx.ws.buffer("recur_gated", self.heads * self.vdim, self.rt.act_dtype)
@@ -170,6 +179,11 @@ class _MatrixMemoryMixer(Mixer):
             self.o.add_into(ctx.ws, act, target, ctx.rows)
         else:
             self.o.store(ctx.ws, act, target, ctx.rows)
+
+
+def in_stages(longest: int, rows: int, columns: int, gates: bool) -> bool:
+    """Whether a step of ``rows`` rows, up to ``longest`` a request, walks a layer's memories of ``columns`` value columns in stages."""
+    return longest >= STAGES_MIN_ROWS[gates] and rows * columns <= longest * STAGES_MAX_COLUMNS[gates]
 
 
 def decays_ahead(longest: int, rows: int, heads: int, dim: int, vdim: int) -> bool:
