@@ -1030,11 +1030,12 @@ struct FoldLds {
     lsum = mcol + 32;
     eights = lsum + 16;
     state = eights + fold_lds_eights(pcap, hpt);
-    parts = state + ((hpt * hd + 1) & ~1);
+    parts = state + ((hpt * hd + 3) & ~3);
   }
-  __host__ __device__ static int fold_lds_eights(int pcap, int hpt) { return (((pcap + 7) >> 3) * hpt + 1) & ~1; }
+  // (every part in whole vectors of four: the partials may come as loads with LDS as their destination)
+  __host__ __device__ static int fold_lds_eights(int pcap, int hpt) { return (((pcap + 7) >> 3) * hpt + 3) & ~3; }
   static size_t bytes(int pcap, int hpt, int hd) {
-    return ((size_t)3 * ((pcap + 7) & ~7) * hpt + 48 + fold_lds_eights(pcap, hpt) + (size_t)((hpt * hd + 1) & ~1) +
+    return ((size_t)3 * ((pcap + 7) & ~7) * hpt + 48 + fold_lds_eights(pcap, hpt) + (size_t)((hpt * hd + 3) & ~3) +
             (size_t)pcap * hpt * (hd + 2)) * sizeof(float);
   }
 };
@@ -1175,6 +1176,7 @@ __device__ __forceinline__ void store_partial(const AttnBf16Args& a, const Group
 }
 
 #define DECODE_W 8               // waves a workgroup of the decode kernel
+#define DEVICE_SCOPE_LOAD 16     // a load's cache policy: what another die has written is seen (sc1)
 // Partitions that a workgroup of a split launch takes by itself: the meeting in device memory costs some 2 us whatever the
 // head, a second round of loads behind the first as much as its bytes, so it grows with the head.  Up to a round it always pays
 // (300 keys, 1 to 16 rows: 32 heads of 64 8.5 us -> 6.4, 8 heads of 128 10.4 -> 8.6, 4 of 256 18.6 -> 16.5); 16 partitions
@@ -1421,24 +1423,15 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     for (int pass0 = first; pass0 <= last; pass0 += pcap) {
       const int count = (last - pass0) < pcap ? last - pass0 + 1 : pcap;
       const float* src = mine + (size_t)(pass0 - first) * a.hpt * CELL;
-      // eight loads of 8 bytes in flight a thread (a loop of one load and its store waits a memory round trip for
-      // each: 40 us for the 66 KB of a group of four heads of 128 over 32 partitions)
-      const int total = count * a.hpt * CELL / 2;
-      const unsigned long long* src64 = reinterpret_cast<const unsigned long long*>(src);
-      unsigned long long* parts64 = reinterpret_cast<unsigned long long*>(parts);
-      for (int base = 0; base < total; base += 8 * THREADS) {
-        unsigned long long v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int i = base + j * THREADS + (int)threadIdx.x;
-          v[j] = __hip_atomic_load(src64 + (i < total ? i : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int i = base + j * THREADS + (int)threadIdx.x;
-          if (i < total) parts64[i] = v[j];
-        }
-      }
+      // Straight into LDS, 1 KB a load and all of them in flight at once (device scope; the last one's lanes past the partials bring
+      // zeros into the KB behind them).  Through registers, eight loads of 8 bytes a thread at a time, the 148 KB of four heads of
+      // 128 over 71 partitions were five trips past the L2s, in four passes of 48 KB.
+      const int total = count * a.hpt * CELL * (int)sizeof(float);
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, total, 0x00020000);
+      typedef __attribute__((address_space(3))) void* lds_ptr;
+      for (int at = 1024 * wave; at < total; at += 1024 * W)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)(reinterpret_cast<unsigned char*>(parts) + at), 16, 16 * gc.lane, at, 0, DEVICE_SCOPE_LOAD);
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
       __syncthreads();
       decode_fold_pass<HD, W>(a, gc, lds, count, (pass0 - first) / pcap, pass0 + pcap > last, row);
       __syncthreads();
@@ -1487,6 +1480,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
 }
 
 #define BW_LDS_BYTES (160 * 1024 - 256)   // a compute unit's LDS less the kernels' few static words
+#define DECODE_LDS_HALF (79 * 1024)        // two workgroups a compute unit
 #define DECODE_MANY 257          // that many workgroups: more than there are compute units
 #define DECODE_MANY_LONG 1024    // heads of 128 or more in a cache laid out for long contexts (more than 80 partitions a
                                  // request): eight waves' loads in flight are worth more there up to this many (64
@@ -1545,6 +1539,16 @@ static int launch_attention(const AttnBf16Args& a, int decode, float* scratch, s
       nsplit = 1;
     }
     if (few_waves) lds_bytes = shape(WM, pcap);
+    // All of a context's partials at once, if they fit beside what else runs on the compute unit: nothing where workgroups have eight
+    // waves, one more of four waves.  A pass over 48 KB of them costs some 2 us (three barriers, the chains' starts), split also a trip
+    // to memory.  32 heads of 128 on 8, us: split 5 rows of 4,500 keys 34.5 -> 27.4, 1 row 23.0 -> 15.8, 8 of 8,192 75 -> 66; 32 rows of
+    // 3,000 75.0 -> 71.4; 40 of 6,000 234 -> 221; 64 of 2,000, 16 heads of 96 on 2, 31.4 -> 27.2.  Four waves and heads of up to 64 stay
+    // (300 rows of 2,000 keys, 16 heads on 1: 45.2 and 46.8).  Contexts that do not fit take passes as before.
+    const size_t behind = nsplit > 1 ? 1024 : 0;     // (the last KB that a split launch loads)
+    const size_t room = !few_waves ? BW_LDS_BYTES : HD > 64 ? DECODE_LDS_HALF : 0;
+    const int most = max_parts < 256 ? max_parts : 256;
+    while (pcap < most && FoldLds::bytes(pcap + 1, a.hpt, HD) + behind <= room) ++pcap;
+    lds_bytes = FoldLds::bytes(pcap, a.hpt, HD) + behind;
     if (lds_bytes > BW_LDS_BYTES) return -8;
     // more than 64 KB of dynamic LDS has to be asked for once per kernel
     static bool allowed[3] = {false, false, false};
