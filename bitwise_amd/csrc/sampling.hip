@@ -145,15 +145,25 @@ extern "C" int bw_sample(const float* logits, int vocab, int ld, int rows, const
 
 // Fingerprint chain of the reference (src/engine.cpp:18-29): h = (h ^ word) * 1099511628211
 // over the row's 8-byte words, single trailing bytes likewise, then the splitmix64 finaliser.
-// The chain is sequential by construction (an exclusive or, then a product modulo 2^64: no algebra in which both
-// are linear), so a row's time is its number of words times the latency of one link.  A wave takes a row: the row's
+//
+// One wave a row, link by link: the chain as it is written.  The row's
 // address is the same for every lane, so the words arrive through the scalar unit, sixteen of them a load and the
-// next sixteen asked for before these are used, and the chain runs in scalar registers, a link every dozen clocks;
-// rows run beside each other on as many compute units.  (One lane a row with loads of its own, as this kernel
-// was first written, spent a memory latency a word: 6.4 ms for 64 rows of 128,256 logits.)
+// next sixteen asked for before these are used, and the chain runs in scalar registers, a link every 13 ns (eight scalar
+// instructions): 318 us for 49,152 logits, whatever the number of rows.  For short rows, and for very many.
 #define FP_BLOCK 16        // words of 8 bytes a block
 __device__ __forceinline__ uint64_t fp_link(uint64_t h, uint32_t lo, uint32_t hi) {
   return (h ^ ((uint64_t)lo | ((uint64_t)hi << 32))) * 1099511628211ull;
+}
+
+// an odd row's last element byte by byte, and the finaliser
+__device__ __forceinline__ uint64_t fp_finish(uint64_t h, const uint32_t* __restrict__ p, int vocab) {
+  if (vocab & 1) {
+    const uint32_t t = p[vocab - 1];
+    for (int k = 0; k < 4; ++k) h = (h ^ ((t >> (8 * k)) & 0xffu)) * 1099511628211ull;
+  }
+  h = (h ^ (h >> 30)) * 0xBF58476D1CE4E5B9ull;
+  h = (h ^ (h >> 27)) * 0x94D049BB133111EBull;
+  return h ^ (h >> 31);
 }
 
 struct FpBlock {
@@ -200,19 +210,175 @@ __global__ __launch_bounds__(64) void fingerprint_kernel(const float* __restrict
   }
   if (b < blocks) h = fp_chain(h, even);                               // an odd number of blocks: the last one
   for (int i = blocks * FP_BLOCK; i < words; ++i) h = fp_link(h, p[2 * i], p[2 * i + 1]);
-  if (vocab & 1) {
-    const uint32_t t = p[vocab - 1];
-    for (int k = 0; k < 4; ++k) h = (h ^ ((t >> (8 * k)) & 0xffu)) * 1099511628211ull;
+  if (threadIdx.x == 0) h_out[row] = fp_finish(h, p, vocab);
+}
+
+// Bit by bit, all links at once.  The chain is serial in its links but not in its bits: bit j of a link's product
+// is bit j of x = h ^ word plus carries and shifted copies that depend on lower bits of x alone, so that
+//   h_j(n + 1) = h_j(n) ^ word_j(n) ^ K_j(n),      K_j made of bits below j of the same link,
+// and once the bits below j are known at every link, bit j of all of them is an exclusive or over the links before: a scan.  A
+// row is therefore 64 scans, one behind the other, instead of one step a word.
+//
+// A workgroup holds 32 links a thread as 64 slices of a bit each: link i * T + t is bit i of thread t's slices (T threads;
+// consecutive threads read consecutive words, and a 32 x 32 transposition in registers makes the slices).  The factor is
+// 2^40 + 3 (1 + 16 + 128): y = 3 x, z = y + 16 y, u = z + 128 y, v = u + 2^40 x, sums of two numbers each, a bit of all 32 links
+// in two instructions (exclusive or and majority of three).  A bit's scan runs over the lanes of a wave for all 32 values
+// of i at once, over the waves through LDS, and over i in scalar registers.  A row longer than a workgroup holds takes
+// several passes; slots past a pass's links hold zero words, and the first of them reads the pass's result.
+//
+// What bounds it: the 64 rounds, each some thirty instructions a wave and one meeting of the workgroup.  49,152 logits: 318 us as a
+// chain, 42 so (eight rows 43, 256 rows 46); 128,256: 831 and 85; 32,000: 208 and 31.
+__device__ __forceinline__ uint32_t fp_xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
+
+__device__ __forceinline__ uint32_t fp_major(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0xe8);
+#else
+  return (a & b) | (a & c) | (b & c);
+#endif
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t fp_scan_step(uint32_t v) {
+  return v ^ (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, true);
+}
+
+// bit i of a[j] and bit j of a[i] change places
+__device__ __forceinline__ void fp_transpose(uint32_t (&a)[32]) {
+#pragma unroll
+  for (int s = 16; s; s >>= 1) {
+    const uint32_t low = s == 16 ? 0x0000ffffu : s == 8 ? 0x00ff00ffu : s == 4 ? 0x0f0f0f0fu : s == 2 ? 0x33333333u : 0x55555555u;
+#pragma unroll
+    for (int k = 0; k < 32; ++k)
+      if (!(k & s)) {
+        const uint32_t x = a[k], y = a[k + s];
+        a[k] = (x & low) | ((y << s) & ~low);
+        a[k + s] = ((x >> s) & low) | (y & ~low);
+      }
   }
-  h = (h ^ (h >> 30)) * 0xBF58476D1CE4E5B9ull;
-  h = (h ^ (h >> 27)) * 0x94D049BB133111EBull;
-  if (threadIdx.x == 0) h_out[row] = h ^ (h >> 31);
+}
+
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 4) void fingerprint_slices_kernel(const float* __restrict__ logits, int vocab, int ld,
+                                                                        const uint64_t* __restrict__ h_in, uint64_t* __restrict__ h_out) {
+  constexpr int T = 64 * WAVES;
+  static_assert(WAVES == 4 || WAVES == 8 || WAVES == 16, "the waves' totals are scanned in a row of 16 lanes");
+  __shared__ uint32_t totals[2][16];
+  __shared__ uint32_t state[2];
+  const int row = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint32_t* __restrict__ p = reinterpret_cast<const uint32_t*>(logits + (size_t)row * ld);
+  const int words = vocab >> 1;
+  uint64_t h = h_in[row];
+  if (t < 16) totals[0][t] = totals[1][t] = 0;                       // (lanes past the waves read zeros)
+  __syncthreads();
+  for (int at = 0; at < words; at += 32 * T - 1) {
+    const int n = words - at < 32 * T - 1 ? words - at : 32 * T - 1;   // the pass's links
+    uint32_t x[64], y[64];
+    {
+      uint32_t lo[32], hi[32];
+#pragma unroll
+      for (int i = 0; i < 32; ++i) {
+        const int link = i * T + t;
+        lo[i] = link < n ? p[2 * (size_t)(at + link)] : 0u;
+        hi[i] = link < n ? p[2 * (size_t)(at + link) + 1] : 0u;
+      }
+      fp_transpose(lo);
+      fp_transpose(hi);
+#pragma unroll
+      for (int j = 0; j < 32; ++j) {
+        x[j] = lo[j];
+        x[32 + j] = hi[j];
+      }
+    }
+    uint32_t cy = 0, cz = 0, cu = 0, cv = 0;
+#pragma unroll
+    for (int j = 0; j < 64; ++j) {
+      const uint32_t x1 = j >= 1 ? x[j - 1] : 0u, y4 = j >= 4 ? y[j - 4] : 0u, y7 = j >= 7 ? y[j - 7] : 0u, x40 = j >= 40 ? x[j - 40] : 0u;
+      const uint32_t d = fp_xor3(fp_xor3(fp_xor3(x[j] ^ x40, y4, y7), x1, cy), cz, cu ^ cv);
+      uint32_t v = fp_scan_step<0x111, 0xf>(d);                       // row_shr 1, 2, 4, 8: sixteen lanes
+      v = fp_scan_step<0x112, 0xf>(v);
+      v = fp_scan_step<0x114, 0xf>(v);
+      v = fp_scan_step<0x118, 0xf>(v);
+      v = fp_scan_step<0x142, 0xa>(v);                                // row_bcast 15 and 31: the whole wave
+      v = fp_scan_step<0x143, 0xc>(v);
+      if (lane == 63) totals[j & 1][wave] = v;
+      __syncthreads();                                                // (a buffer is written again two meetings on)
+      uint32_t w = totals[j & 1][lane & 15];
+      w = fp_scan_step<0x111, 0xf>(w);
+      w = fp_scan_step<0x112, 0xf>(w);
+      if (WAVES > 4) w = fp_scan_step<0x114, 0xf>(w);
+      if (WAVES > 8) w = fp_scan_step<0x118, 0xf>(w);
+      const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)w, WAVES - 1);
+      const uint32_t before = wave ? (uint32_t)__builtin_amdgcn_readlane((int)w, wave - 1) : 0u;
+      uint32_t base = all << 1;                                       // exclusive or of the totals of smaller i
+      base ^= base << 1;
+      base ^= base << 2;
+      base ^= base << 4;
+      base ^= base << 8;
+      base ^= base << 16;
+      base ^= before ^ (0u - (uint32_t)((h >> j) & 1));
+      // v ^ d: the lanes before; ^ base: h_j at the own links; ^ the word's bit: x_j
+      const uint32_t xj = fp_xor3(v, x[j] ^ d, base);
+      x[j] = xj;
+      const uint32_t yj = fp_xor3(xj, x1, cy), zj = fp_xor3(yj, y4, cz), uj = fp_xor3(zj, y7, cu);
+      y[j] = yj;
+      cy = fp_major(xj, x1, cy);
+      cz = fp_major(yj, y4, cz);
+      cu = fp_major(zj, y7, cu);
+      cv = fp_major(uj, x40, cv);
+    }
+    // the slot behind the last link: its word is zero, so x is h there
+    const int slot = n / T;
+    if (t == n - slot * T) {
+      uint32_t lo = 0, hi = 0;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) {
+        lo |= ((x[j] >> slot) & 1u) << j;
+        hi |= ((x[32 + j] >> slot) & 1u) << j;
+      }
+      state[0] = lo;
+      state[1] = hi;
+    }
+    __syncthreads();
+    h = (uint64_t)__builtin_amdgcn_readfirstlane((int)state[0]) & 0xffffffffull;
+    h |= (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)state[1]) << 32;
+  }
+  if (t == 0) h_out[row] = fp_finish(h, p, vocab);
 }
 
 extern "C" int bw_fingerprint(const float* logits, int vocab, int ld, int rows, const void* h_in, void* h_out,
                               void* stream) {
   if (rows <= 0) return 0;
-  hipLaunchKernelGGL(fingerprint_kernel, dim3(rows), dim3(64), 0, (hipStream_t)stream, logits, vocab, ld,
-                     rows, (const uint64_t*)h_in, (uint64_t*)h_out);
+  const uint64_t* from = (const uint64_t*)h_in;
+  uint64_t* to = (uint64_t*)h_out;
+  const int words = vocab >> 1;
+  // Which kernel, by nanoseconds.  A link of the chain takes 13; beyond a few hundred rows its waves share compute units (1,024 rows
+  // take 1.2 to 1.9 times as long, 2,048 2.3 to 3.7 times).  A pass of 4, 8 or 16 waves over their 8,191, 16,383 or 32,767 words
+  // takes 26, 30 or 42 us on a compute unit of its own, and sixteen waves' worth of rows share one at about the last of these.
+  // 4,096 logits are 26 us so and 28 as a chain, 3,072 are 26 and 21; 1,024 rows of 8,192 45 and 63, 4,096 of them 237 as a chain.
+  const long long chain = (long long)words * 13 * (2048 + rows) / 2048;
+  const int pass_ns[3] = {26000, 30000, 42000};
+  int waves = 0;
+  long long best = chain;
+  for (int k = 0; k < 3; ++k) {
+    const int w = 4 << k, slots = 2048 * w - 1, a_round = 256 * 16 / w;
+    const long long passes = (words + slots - 1) / slots;
+    const long long ns = passes * (rows <= 256 ? pass_ns[k] : (rows + a_round - 1) / a_round * (long long)pass_ns[2]);
+    if (ns < best) {
+      best = ns;
+      waves = w;
+    }
+  }
+  const hipStream_t s = (hipStream_t)stream;
+  if (waves == 16) hipLaunchKernelGGL((fingerprint_slices_kernel<16>), dim3(rows), dim3(1024), 0, s, logits, vocab, ld, from, to);
+  else if (waves == 8) hipLaunchKernelGGL((fingerprint_slices_kernel<8>), dim3(rows), dim3(512), 0, s, logits, vocab, ld, from, to);
+  else if (waves == 4) hipLaunchKernelGGL((fingerprint_slices_kernel<4>), dim3(rows), dim3(256), 0, s, logits, vocab, ld, from, to);
+  else hipLaunchKernelGGL(fingerprint_kernel, dim3(rows), dim3(64), 0, s, logits, vocab, ld, rows, from, to);
   return BW_LAUNCH_CHECK();
 }
