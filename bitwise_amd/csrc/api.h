@@ -25,6 +25,8 @@ int bw_add(float* x, const float* y, long long n, void* stream);
 int bw_add_bias(float* x, const float* bias, int rows, int cols, int ldx, void* stream);
 int bw_convert(const void* src, int src_is_bf16, void* dst, int dst_is_bf16, int rows, int cols, int lds, int ldd,
                void* stream);
+int bw_gemm_f32_swiglu(const float* x, const void* w, int w_is_bf16, float* gate_up, float* h, int M, int outputs, int K, int ldx,
+                       void* stream);
 int bw_swiglu_f32(const float* gate_up, float* h, int rows, int inter, void* stream);
 int bw_gather_rows_f32(const float* x, const int32_t* idx, float* out, int count, int width, int ldx, void* stream);
 int bw_rope_kvwrite(float* qkv, void* q_out, const int32_t* positions, const int32_t* row_seq,

@@ -593,18 +593,19 @@ extern "C" int bw_gemm_f32_prompt_tile(int M, int N, int* rows, int* columns) {
   return 0;
 }
 
-template <typename WT>
+// (GATED: N counts the outputs; the tiles are chosen by the rows of the stacked weight)
+template <typename WT, bool GATED = false>
 static void launch_f32_prompt(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s) {
-  const F32PromptTile tile = f32_prompt_tile(M, N);
+  const F32PromptTile tile = f32_prompt_tile(M, GATED ? 2 * N : N);
   if (tile.rows == 64) {
     // more than two workgroups a compute unit: without loading waves three of them fit (450 rows, 6144 x 2048: 96 us against 117);
     // with no more than that their own loads cost the working waves more (2048 x 8192: 145 us against 133)
-    const long long wgs = ((M + 63) / 64) * (long long)((N + 63) / 64);
-    if (wgs > 512) return launch_f32_tiles<WT, 4, 1, 1, 4, 32, 4, 0>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
-    return launch_f32_tiles<WT, 4, 1, 1, 4, 32, 4, 4>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+    const long long wgs = ((M + 63) / 64) * (long long)(((GATED ? 2 * N : N) + 63) / 64);
+    if (wgs > 512) return launch_f32_tiles<WT, 4, 1, 1, 4, 32, 4, 0, GATED>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+    return launch_f32_tiles<WT, 4, 1, 1, 4, 32, 4, 4, GATED>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
   }
-  if (tile.columns == 64) return launch_f32_tiles<WT, 8, 1, 1, 4, 32, 4, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
-  launch_f32_tiles<WT, 8, 2, 1, 4, 32, 4, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+  if (tile.columns == 64) return launch_f32_tiles<WT, 8, 1, 1, 4, 32, 4, 2, GATED>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+  launch_f32_tiles<WT, 8, 2, 1, 4, 32, 4, 2, GATED>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
 }
 
 // Up to 64 rows, K a multiple of 64 (of 32 where the tiles of 64 x 64 take it); us with bfloat16 weights and K = 2048:
@@ -622,13 +623,13 @@ static int f32_few_rows_kernel(int M, int N, int K) {
   return M > 32 && (N + 63) / 64 >= 256 ? F32_TILES_64 : F32_TILES_32;
 }
 
-template <typename WT>
+template <typename WT, bool GATED = false>
 static void launch_f32_few_rows(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s) {
-  switch (f32_few_rows_kernel(M, N, K)) {
-    case F32_STRIPS: return launch_f32_strips<WT, 2, 9>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
-    case F32_TILES_16: return launch_f32_tiles<WT, 1, 1, 1, 4, 64, sizeof(WT) == 2 ? 6 : 5, 2>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
-    case F32_TILES_32: return launch_f32_tiles<WT, 1, 1, 2, 2, 64, 4, 0>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
-    default: return launch_f32_tiles<WT, 4, 1, 1, 4, 32, 4, 4>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+  switch (f32_few_rows_kernel(M, GATED ? 2 * N : N, K)) {
+    case F32_STRIPS: if constexpr (!GATED) return launch_f32_strips<WT, 2, 9>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+    case F32_TILES_16: return launch_f32_tiles<WT, 1, 1, 1, 4, 64, sizeof(WT) == 2 ? 6 : 5, 2, GATED>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+    case F32_TILES_32: return launch_f32_tiles<WT, 1, 1, 2, 2, 64, 4, 0, GATED>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
+    default: return launch_f32_tiles<WT, 4, 1, 1, 4, 32, 4, 4, GATED>(x, w, y, M, N, K, ldx, ldy, accumulate, s);
   }
 }
 
@@ -702,4 +703,29 @@ extern "C" int bw_gemm_f32(const float* x, const void* w, int w_is_bf16, float* 
   else
     hipLaunchKernelGGL(gemm_f32_kernel<float>, grid, block, 0, s, x, (const float*)w, y, M, N, K, ldx, ldy, accumulate);
   return BW_LAUNCH_CHECK();
+}
+
+// h = silu(x Wg^T) * (x Wu^T), w = [Wg; Wu] (outputs rows each).  Where the product goes in tiles its epilogue computes h; otherwise
+// the sums go to gate_up and swiglu_f32_kernel behind it.  The same operations on the same sums.  (One row too: a chain a lane and
+// the kernel behind it take 17.2 us for 8192 outputs of K = 2048, the tiles 16.3; with 32-bit weights 32.3 and 30.0.)
+extern "C" int bw_gemm_f32_swiglu(const float* x, const void* w, int w_is_bf16, float* gate_up, float* h, int M, int outputs, int K, int ldx,
+                                  void* stream) {
+  if (M <= 0 || outputs <= 0) return 0;
+  if (K <= 0 || ldx < K) return -2;
+  hipStream_t s = (hipStream_t)stream;
+  const bool vectors = ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
+  const size_t limit = (size_t)0x7ff00000;             // (a tile's descriptor spans the whole weight)
+  const bool fits = vectors && (size_t)(M < 128 ? M : 128) * ldx * 4 < limit && (size_t)2 * outputs * K * (w_is_bf16 ? 2 : 4) < limit;
+  if (fits && M > 64 && K % 32 == 0) {
+    if (w_is_bf16) launch_f32_prompt<bf16_t, true>(x, (const bf16_t*)w, h, M, outputs, K, ldx, outputs, 0, s);
+    else launch_f32_prompt<float, true>(x, (const float*)w, h, M, outputs, K, ldx, outputs, 0, s);
+    return BW_LAUNCH_CHECK();
+  }
+  if (fits && M <= 64 && K % 64 == 0 && f32_few_rows_kernel(M, 2 * outputs, K) != F32_STRIPS) {
+    if (w_is_bf16) launch_f32_few_rows<bf16_t, true>(x, (const bf16_t*)w, h, M, outputs, K, ldx, outputs, 0, s);
+    else launch_f32_few_rows<float, true>(x, (const float*)w, h, M, outputs, K, ldx, outputs, 0, s);
+    return BW_LAUNCH_CHECK();
+  }
+  const int rc = bw_gemm_f32(x, w, w_is_bf16, gate_up, M, 2 * outputs, K, ldx, 2 * outputs, 0, stream);
+  return rc != 0 ? rc : bw_swiglu_f32(gate_up, h, M, outputs, stream);
 }

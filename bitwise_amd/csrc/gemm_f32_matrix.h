@@ -135,7 +135,39 @@ __device__ __forceinline__ void f32_write(const f32x4 (&acc)[RBL][CB], float* y,
       }
 }
 
-template <typename S, typename WT, int RBL, int CB, int ST, int LW>
+// Gated: gate and up of an output meet in one wave (f32k_weight_row): as its two column blocks, or as the halves of one, whose lanes
+// then exchange half of their rows.  h = g * (1/(1+exp(-g))) * u, as swiglu_f32_kernel has it.
+__device__ __forceinline__ float f32_swiglu(float g, float u) { return g * (1.0f / (1.0f + bw_expf(-g))) * u; }
+
+template <int RBL, int CB>
+__device__ __forceinline__ void f32_write_gated(const f32x4 (&acc)[RBL][CB], float* h, int ldh, int m0, int n0, int M, int N) {
+  const int lane = threadIdx.x & 63;
+  if constexpr (CB == 2) {
+    const int n = n0 + (lane & 15);
+#pragma unroll
+    for (int r = 0; r < RBL; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = m0 + 16 * r + 4 * (lane >> 4) + i;
+        const float v = f32_swiglu(acc[r][0][i], acc[r][1][i]);
+        if (m < M && n < N) h[(size_t)m * ldh + n] = v;
+      }
+  } else {
+    const bool up = lane & 8;
+    const int n = n0 + (lane & 7);
+#pragma unroll
+    for (int r = 0; r < RBL; ++r)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float got = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(up ? acc[r][0][i] : acc[r][0][2 + i]), 0x128, 0xf, 0xf, true));
+        const int m = m0 + 16 * r + 4 * (lane >> 4) + i + (up ? 2 : 0);
+        const float v = f32_swiglu(up ? got : acc[r][0][i], up ? acc[r][0][2 + i] : got);
+        if (m < M && n < N) h[(size_t)m * ldh + n] = v;
+      }
+  }
+}
+
+template <typename S, typename WT, int RBL, int CB, int ST, int LW, bool GATED>
 __device__ __forceinline__ void f32k_tile(unsigned char* ring, __amdgpu_buffer_rsrc_t rs_x, __amdgpu_buffer_rsrc_t rs_w, const int* voff_x,
                                           const int* voff_w, int loader, const int* xa, const int* wa, int steps, float* y, int ldy, int m0, int n0,
                                           int M, int N, int accumulate) {
@@ -174,11 +206,26 @@ __device__ __forceinline__ void f32k_tile(unsigned char* ring, __amdgpu_buffer_r
     }
   }
   if constexpr (LW == 0) __builtin_amdgcn_s_waitcnt(vmcnt_only(0));             // the padding loads too, before the waves end
-  if constexpr (RBL > 0) f32_write<R, CB>(acc, y, ldy, m0, n0, M, N, accumulate);
+  if constexpr (RBL > 0) {
+    if constexpr (GATED) f32_write_gated<R, CB>(acc, y, ldy, m0, n0, M, N);
+    else f32_write<R, CB>(acc, y, ldy, m0, n0, M, N, accumulate);
+  }
+}
+
+// Which row of the stacked weight [gate; up] is a gated tile's column c: blocks of 16 in turn, or halves of a block of 16.
+// (Past the last output: the last one's again.)
+template <int CB>
+__device__ __forceinline__ int f32k_weight_row(int c, int first, int outputs) {
+  constexpr int H = 8 * CB;
+  const int row = min(first + c / (2 * H) * H + c % H, outputs - 1);
+  return c & H ? row + outputs : row;
 }
 #endif
 
-template <typename WT, int RB, int CB, int WR, int WC, int KB, int ST, int LW>
+// GATED: w is [gate; up], N counts the outputs, and y takes silu(gate) * up.  8 rows, 8192 outputs of K = 2048, bfloat16 weights: the sums to
+// memory and a kernel behind them 18.1 us, so 16.0; 64 rows 40.2 and 37.9, 2048 rows 1035 and 1025; 4104 outputs of K = 512, 8 rows,
+// 10.0 and 6.2.
+template <typename WT, int RB, int CB, int WR, int WC, int KB, int ST, int LW, bool GATED>
 __global__ __launch_bounds__(64 * (WR * WC + LW)) void gemm_f32_tiles_kernel(const float* __restrict__ x, const WT* __restrict__ w,
                                                                             float* __restrict__ y, int M, int N, int K, int ldx, int ldy,
                                                                             int accumulate, int row_tiles) {
@@ -191,12 +238,12 @@ __global__ __launch_bounds__(64 * (WR * WC + LW)) void gemm_f32_tiles_kernel(con
   if (gridDim.x % 8 == 0) bid = (bid % 8) * (gridDim.x / 8) + bid / 8;
   const int blocks = (M + 15) / 16, tile = bid % row_tiles;
   const int first = (int)((long long)blocks * tile / row_tiles), last = (int)((long long)blocks * (tile + 1) / row_tiles);
-  const int m0 = 16 * first, n0 = (bid / row_tiles) * S::COLS;
-  const int x_rows = min(16 * (last - first), M - m0), w_rows = min(S::COLS, N - n0);
+  const int m0 = 16 * first, n0 = (bid / row_tiles) * (GATED ? S::COLS / 2 : S::COLS);
+  const int x_rows = min(16 * (last - first), M - m0), w_rows = GATED ? 2 * N : min(S::COLS, N - n0);
   const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(x + (size_t)m0 * ldx), 0, (int)((((size_t)x_rows - 1) * ldx + K) * sizeof(float)), 0x00020000);
   const __amdgpu_buffer_rsrc_t rs_w =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, (int)((size_t)w_rows * K * sizeof(WT)), 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc((void*)(w + (GATED ? 0 : (size_t)n0 * K)), 0, (int)((size_t)w_rows * K * sizeof(WT)), 0x00020000);
   // loads: 1 KB an instruction, whole rows of a stage, lane l the 16 bytes at 16 l; which chunk of its row a lane asks for is permuted
   // (rows past the operand are clamped to its last: their outputs are never stored)
   const int loader = LW > 0 ? wave - S::WAVES : wave;                          // (negative: a wave that does not load)
@@ -211,7 +258,9 @@ __global__ __launch_bounds__(64 * (WR * WC + LW)) void gemm_f32_tiles_kernel(con
   for (int t = 0; t < S::WW; ++t) {
     constexpr int CH = S::WROW / 16;
     const int row = (loader + t * S::LOADERS) * (64 / CH) + lane / CH, chunk = (lane % CH) ^ f32k_swizzle<S::WROW>(row);
-    voff_w[t] = min(row, w_rows - 1) * K * (int)sizeof(WT) + 16 * chunk;
+    int w_row = min(row, w_rows - 1);
+    if constexpr (GATED) w_row = f32k_weight_row<CB>(row, n0, N);
+    voff_w[t] = w_row * K * (int)sizeof(WT) + 16 * chunk;
   }
   const int steps = K / KB;
   if (LW == 0 || wave >= S::WAVES) {
@@ -241,9 +290,9 @@ __global__ __launch_bounds__(64 * (WR * WC + LW)) void gemm_f32_tiles_kernel(con
   for (int c = 0; c < KB * (int)sizeof(WT) / 16; ++c)
     wa[c] = S::XBYTES + (wc * 16 * CB + row) * S::WROW + ((c ^ f32k_swizzle<S::WROW>(row)) * 16) + (int)sizeof(WT) * g;
   const int live = min(RB, last - first - wr * RB);                            // scalar: this wave's row blocks
-  const int mw = m0 + wr * 16 * RB, nw = n0 + wc * 16 * CB;
+  const int mw = m0 + wr * 16 * RB, nw = n0 + wc * (GATED ? 8 : 16) * CB;
 #define BW_F32K_TILE(L) \
-  return f32k_tile<S, WT, L, CB, ST, LW>(f32k_ring, rs_x, rs_w, voff_x, voff_w, loader, xa, wa, steps, y, ldy, mw, nw, M, N, accumulate)
+  return f32k_tile<S, WT, L, CB, ST, LW, GATED>(f32k_ring, rs_x, rs_w, voff_x, voff_w, loader, xa, wa, steps, y, ldy, mw, nw, M, N, accumulate)
   // (tiles of eight blocks are for more than 64 rows: evenly shared, four at least)
   if constexpr (RB == 8) {
     static_assert(WR == 1, "every wave has all rows");
@@ -267,16 +316,16 @@ __global__ __launch_bounds__(64 * (WR * WC + LW)) void gemm_f32_tiles_kernel(con
 #endif
 }
 
-template <typename WT, int RB, int CB, int WR, int WC, int KB, int ST, int LW>
+template <typename WT, int RB, int CB, int WR, int WC, int KB, int ST, int LW, bool GATED = false>
 static void launch_f32_tiles(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s) {
   using S = F32KShape<WT, RB, CB, WR, WC, KB, ST, LW>;
   static bool allowed = false;                       // more than 64 KB of dynamic LDS has to be asked for once
   if (S::LDS > 48 * 1024 && !allowed) {
-    (void)hipFuncSetAttribute((const void*)gemm_f32_tiles_kernel<WT, RB, CB, WR, WC, KB, ST, LW>, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
+    (void)hipFuncSetAttribute((const void*)gemm_f32_tiles_kernel<WT, RB, CB, WR, WC, KB, ST, LW, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
     allowed = true;
   }
   const int row_tiles = ((M + 15) / 16 + RB * WR - 1) / (RB * WR);
-  hipLaunchKernelGGL((gemm_f32_tiles_kernel<WT, RB, CB, WR, WC, KB, ST, LW>), dim3(row_tiles * ((N + S::COLS - 1) / S::COLS)),
+  hipLaunchKernelGGL((gemm_f32_tiles_kernel<WT, RB, CB, WR, WC, KB, ST, LW, GATED>), dim3(row_tiles * (((GATED ? 2 : 1) * N + S::COLS - 1) / S::COLS)),
                      dim3(64 * (S::WAVES + LW)), S::LDS, s, x, w, y, M, N, K, ldx, ldy, accumulate, row_tiles);
 }
 

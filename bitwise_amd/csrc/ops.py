@@ -47,6 +47,7 @@ _SIGS = {
     "bw_rope_kvwrite": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                         c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_f32": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    "bw_gemm_f32_swiglu": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_clamped_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],
     "bw_gemm_gelu_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
@@ -454,6 +455,24 @@ def gemm_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows: int, acc
         raise ValueError(f"gemm_f32: x {tuple(x.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not match")
     _check(_fn("bw_gemm_f32")(x.data_ptr(), w.data_ptr(), _is_bf16(w, "weight"), out.data_ptr(), rows, N, K,
                               x.stride(0), out.stride(0), int(accumulate), _stream()), "gemm_f32")
+
+
+def gemm_f32_swiglu(x: torch.Tensor, w: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, rows: int) -> None:
+    """out[:rows] = silu(g) * u with [g | u] = x[:rows] @ w.T, ``w`` = [gate; up] stacked: ``gemm_f32`` and ``swiglu_f32`` in one kernel
+    where the product goes in tiles of the matrix cores, the same bits.  ``gate_up``: room for the sums where it does not."""
+    if not x.is_cuda or x.dtype != torch.float32 or x.dim() != 2 or x.stride(1) != 1:
+        raise ValueError("gemm_f32_swiglu: x must be a float32 GPU matrix with contiguous rows")
+    _need(gate_up, torch.float32, "gate_up")
+    _need(out, torch.float32, "out")
+    if not w.is_cuda or not w.is_contiguous() or w.dim() != 2:
+        raise ValueError("gemm_f32_swiglu: weight must be a contiguous [2 * inter, K] GPU tensor")
+    N, K = w.shape
+    inter = out.shape[1]
+    if x.shape[1] != K or N != 2 * inter or gate_up.shape[1] != N or min(x.shape[0], out.shape[0], gate_up.shape[0]) < rows:
+        raise ValueError(f"gemm_f32_swiglu: x {tuple(x.shape)}, w {tuple(w.shape)}, gate_up {tuple(gate_up.shape)}, out {tuple(out.shape)} "
+                         "do not match")
+    _check(_fn("bw_gemm_f32_swiglu")(x.data_ptr(), w.data_ptr(), _is_bf16(w, "weight"), gate_up.data_ptr(), out.data_ptr(), rows, inter, K,
+                                     x.stride(0), _stream()), "gemm_f32_swiglu")
 
 
 def gemm_f32_prompt_tile(rows: int, N: int) -> Tuple[int, int]:

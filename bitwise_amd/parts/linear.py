@@ -64,6 +64,10 @@ class Linear:
         return (ws.buffer("gemm_add_split", floats, torch.float32, rows=1),
                 ws.buffer("gemm_add_split_count", counters, torch.int32, rows=1))
 
+    def store_swiglu(self, ws, x: torch.Tensor, sums: torch.Tensor, out: torch.Tensor, rows: int) -> None:
+        """out[:rows] = silu(g) * u with [g | u] = x[:rows] @ W.T, on the 32-bit kernels; ``sums``: room for [g | u]."""
+        ops.gemm_f32_swiglu(self._x32(ws, x, rows), self.weight, sums, out, rows)
+
     def store(self, ws, x: torch.Tensor, out: torch.Tensor, rows: int) -> None:
         """out[:rows] = x[:rows] @ W.T (out float32, or bfloat16 on the matrix-core path).  ``ws`` is the
         step's workspace (temporaries for a weight whose dtype is not the mode's)."""
