@@ -81,6 +81,7 @@ __device__ __forceinline__ float dot_canonical(const float* __restrict__ q_lds, 
 }
 
 #define ATT32_THREADS 256
+#define ATT32_KEEP_THREADS 512        // of the kernel that keeps its scores: eight waves
 
 // A workgroup barrier for data that meets in LDS: this wave's LDS writes are done, then the barrier.  (The
 // language's own barrier also waits for every load from memory that is still on its way, which would end the
@@ -144,10 +145,15 @@ __device__ __forceinline__ void walk_chunk(const float* __restrict__ ed, const f
 // window, can hold), turn into e_j there once the maximum is known, and pass 2 fetches values only: the keys are
 // read once and every dot product is computed once.  The e_j are the same function of the same numbers, so the bits
 // are those of the two-pass form, which remains for contexts whose scores do not fit.
+// Eight waves: a decoding workgroup often has a compute unit to itself, and pass 1 is a long run of dependent instructions a
+// key (a look-up, its loads, a chain, a tree); two waves a SIMD hide each other's waits and have twice the keys on
+// their way. Against four waves, 32-bit keys and values: eight rows of 1,024 keys, 32 heads of 64, 33.6 -> 27.2 us (4.9 TB/s, what a
+// copy reaches); one row 24.9 -> 18.1; 8 x 4,096 keys 113 -> 91; 40 x 700 121 -> 100; 32/8 heads of 128 39.9 -> 28.0, 8/4 of 256 60 -> 48.
+// Eight keys a group on their way in four waves: 31.3, in eight the same 27.9; sixteen waves: 47 (their registers do not fit).
 template <int HD, bool KEEP>
-__global__ __launch_bounds__(ATT32_THREADS) void attention_f32_kernel(AttnF32Args a) {
+__global__ __launch_bounds__(KEEP ? ATT32_KEEP_THREADS : ATT32_THREADS) void attention_f32_kernel(AttnF32Args a) {
   using S = Att32Shape<HD>;
-  constexpr int T = S::T, KC = S::KC, SEGS = S::SEGS, VJ = S::VJ;
+  constexpr int T = KEEP ? ATT32_KEEP_THREADS : S::T, KC = S::KC, SEGS = S::SEGS, VJ = S::VJ;
   extern __shared__ __attribute__((aligned(16))) float v_lds[];    // [2][KC][HD]: value rows of a chunk of keys; KEEP: then the scores
   float* scores = v_lds + 2 * KC * HD;
   __shared__ float q_lds[HD];
@@ -280,14 +286,14 @@ __global__ __launch_bounds__(ATT32_THREADS) void attention_f32_kernel(AttnF32Arg
     // Values only.  Three chunks of them are on their way at any time (three sets of registers in turn; a chunk in
     // flight is what keeps a compute unit's share of the memory system busy across a trip to memory), the first
     // three asked for before the scores turn into e_j.  Chunks past the last key fetch the last key again.
-    // Where the walk leaves two waves or more without an element (head sizes up to 128), those waves alone fetch
-    // and stash, and the walking waves only walk: a chunk then costs the longer of the two, not their sum.
-    constexpr int WW = (HD + 63) / 64, LW = T / 64 - WW;     // waves that walk, waves that do not
-    constexpr bool APART = LW >= 2;
-    constexpr int LT = APART ? 64 * LW : T;                  // threads that fetch and stash
+    // The waves without an element of the walk fetch and stash (four of them: whole turns of a chunk's pieces), and
+    // the walking waves only walk: a chunk then costs the longer of the two, not their sum.
+    constexpr int WW = (HD + 63) / 64, LW = 4;                // waves that walk, waves that load
+    constexpr int LT = 64 * LW;                              // threads that fetch and stash
+    static_assert(WW + LW <= T / 64, "walkers and loaders are different waves");
     constexpr int VL = (KC * SEGS + LT - 1) / LT;            // pieces of a chunk's value rows for each of them
-    const int lt = APART ? tid - 64 * WW : tid;              // (negative: this thread walks only)
-    const bool loads = lt >= 0;
+    const int lt = tid - 64 * WW;                            // (negative: this thread walks)
+    const bool loads = lt >= 0 && lt < LT;
     f32x4 r0[VL], r1[VL], r2[VL];
     auto fetch_into = [&](f32x4 (&reg)[VL], int j0) {
       size_t off[VL];                                        // (all the pages looked up before the first load goes out)
@@ -364,17 +370,11 @@ __global__ __launch_bounds__(ATT32_THREADS) void attention_f32_kernel(AttnF32Arg
     // one chunk's turn: the chunk three ahead is asked for into ``next``, the chunk in ``buf`` is walked, the
     // chunk one ahead goes from ``ready`` into the other buffer; the barrier publishes it
     auto turn = [&](f32x4 (&next)[VL], const f32x4 (&ready)[VL], int j0, int buf) {
-      if constexpr (APART) {
-        if (loads) {
-          fetch_into(next, j0 + 3 * KC);
-          stash_from(buf ^ 1, ready);
-        } else {
-          walk4(j0, buf);
-        }
-      } else {
+      if (loads) {
         fetch_into(next, j0 + 3 * KC);
-        walk4(j0, buf);
         stash_from(buf ^ 1, ready);
+      } else if (lt < 0) {
+        walk4(j0, buf);
       }
       lds_barrier();
     };
@@ -934,7 +934,7 @@ static void launch_attention_f32(const AttnF32Args& a, dim3 grid, hipStream_t s)
   if (a.chunk > 0 && a.chunk < capacity) capacity = a.chunk;
   const long long keep_bytes = Att32Shape<HD>::LDS_BYTES + ((capacity + 3) & ~3ll) * (long long)sizeof(float);
   if (keep_bytes <= ATT32_KEEP_LDS && a.table_stride <= ATT32_TABLE && a.page_shift >= 0)   // (and the table's row fits the kernel's copy of it)
-    hipLaunchKernelGGL((attention_f32_kernel<HD, true>), grid, dim3(ATT32_THREADS), (size_t)keep_bytes, s, a);
+    hipLaunchKernelGGL((attention_f32_kernel<HD, true>), grid, dim3(ATT32_KEEP_THREADS), (size_t)keep_bytes, s, a);
   else
     hipLaunchKernelGGL((attention_f32_kernel<HD, false>), grid, dim3(ATT32_THREADS), Att32Shape<HD>::LDS_BYTES, s, a);
 }
