@@ -41,6 +41,7 @@ int bw_gemm_bf16(const void* x, const void* w, void* out, int M, int N, int K, i
                  void* stream);
 // rows and rows of W of the tiles that a bfloat16 product of more than 64 rows gets where all of K is one workgroup's and the
 // kernels for few rows do not take it (K a multiple of 64; gated 1: the stacked weight of a gated epilogue, 2: the exact GELU)
+int bw_gemm_prompt_parts(int M, long long w_rows, int K, int gated, long long* first);
 int bw_gemm_prompt_tile(int M, long long w_rows, int K, int gated, int* rows, int* columns);
 int bw_gemm_clamped_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, float limit,
                              float alpha, void* stream);

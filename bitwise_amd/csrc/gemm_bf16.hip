@@ -486,7 +486,7 @@ static int launch_gemm_bf16(const bf16_t* x, const bf16_t* w, void* out, int M, 
     }
     // K in whole steps of 64: tiles through LDS rings, of the shape that takes the least time
     if (K % 64 == 0)
-      return launch_ring<EPI>(ring_choice(M, epi_is_glu(EPI) ? 2LL * N : N, K, epi_is_glu(EPI), nullptr, EPI == EPI_GELU_BF16), x, w, out, M, N, K, ldx, ldo, s, rp);
+      return launch_ring_tiles<EPI>(x, w, out, M, N, K, ldx, ldo, s, rp);
     constexpr int COLS = epi_is_glu(EPI) ? 64 : 128;
     const int m_tiles = (M + WIDE_BM - 1) / WIDE_BM, n_tiles = (N + COLS - 1) / COLS;
     dim3 grid(m_tiles * n_tiles), block(256);

@@ -52,6 +52,7 @@ _SIGS = {
     "bw_gemm_clamped_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],
     "bw_gemm_gelu_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_f32_prompt_tile": [c_int, c_int, c_void_p, c_void_p],
+    "bw_gemm_prompt_parts": [c_int, c_longlong, c_int, c_int, c_void_p],
     "bw_gemm_prompt_tile": [c_int, c_longlong, c_int, c_int, c_void_p, c_void_p],
     "bw_gemm_gelu_glu_wins": [c_int, c_int, c_int],
     "bw_gemm_split_tile": [c_int, c_int, c_int, c_int, c_void_p, c_void_p],
@@ -164,7 +165,7 @@ _fns = {}
 # what waits.
 _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
-    "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_gelu_glu_wins", "bw_gemm_split_tile", "bw_gemm_split_rows",
+    "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts", "bw_gemm_gelu_glu_wins", "bw_gemm_split_tile", "bw_gemm_split_rows",
     "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
     "bw_chain_flush", "bw_chain_end",
@@ -489,6 +490,14 @@ def gemm_prompt_tile(rows: int, w_rows: int, K: int, gated: bool = False, erf: b
     r, c = ctypes.c_int(0), ctypes.c_int(0)
     _check(_fn("bw_gemm_prompt_tile")(rows, w_rows, K, 2 if erf else int(gated), ctypes.addressof(r), ctypes.addressof(c)), "gemm_prompt_tile")
     return int(r.value), int(c.value)
+
+
+def gemm_prompt_parts(rows: int, w_rows: int, K: int, gated: bool = False) -> int:
+    """Of a product that ``gemm_prompt_tile`` describes: how many rows of W go in tiles of a first launch, the others in tiles of another
+    shape; 0: the product goes whole."""
+    first = ctypes.c_longlong(0)
+    _check(_fn("bw_gemm_prompt_parts")(rows, w_rows, K, int(gated), ctypes.addressof(first)), "gemm_prompt_parts")
+    return int(first.value)
 
 
 @functools.lru_cache(maxsize=None)
