@@ -42,11 +42,18 @@ FEW_SEQ_ROWS = 4         # steps whose requests bring up to so many rows each ru
 # -> 8.7, 48 rows 12.3 -> 11.0; 16 of 16: 64 rows 11.6 -> 12.0, 96 rows 16.2 -> 15.5), heads of 64 channels and more sooner where
 # the step's requests together fill the chip (8 x 5 rows: 32 heads of 64 10.7 -> 9.3, 8 of 128 20.4 -> 15.8).
 DECAYS_AHEAD_CHAIN, DECAYS_AHEAD_COLUMNS = 1200, 40960
-# A long portion walks its memories in stages where they leave the chip idle: from so many rows on, and up to so many columns
-# (heads x value channels) times requests of the longest one's length: (decays given, scalar gates).  Microseconds, walk -> stages, 2,048 columns:
-# decays 48 rows 11.3 -> 10.9, 80 rows 14.9 -> 10.9, two requests of 64 rows 12.4 -> 12.1, three of 128 21.2 -> 26.3, of 683 93 -> 98; gates 64 rows 21.6
-# -> 22.1, 80 rows 26.8 -> 24.4, three requests of 128 rows 45.8 -> 43.6, four of 512 161 -> 142.
-STAGES_MIN_ROWS, STAGES_MAX_COLUMNS = (64, 80), (4096, 8192)
+# A long portion walks its memories in stages where they leave the chip idle.  A stage launch has a workgroup for every request and
+# eight columns (heads x value channels), with rings to set up and to drain, so a request is counted as this many rows more than
+# it brings: 2,048 columns, decays given, 64 channels, microseconds walk / stages, a portion of 128 rows alone 20 / 14, beside 4
+# single tokens 22 / 21, beside 15 27 / 38, 64 60 / 119; of 2,048 rows beside 31 270 / 180, beside 128 330 / 339.
+STAGES_REQUEST_ROWS = 48
+# (gates?, heads of 128 channels?): the longest portion from this many rows on, and (columns a row of it is worth, rows of it that are
+# worth nothing).  Fitted to 920 steps (2 to 32 heads, one to eight portions of 5 to 2,048 rows, 0 to 255 single tokens beside them), of
+# which the rule takes 1 that is slower than the walk by more than 3 % (1.08 times), and leaves 1.01 times the time of the better one.
+STAGES_RULE = {(False, False): (64, 6144, 0), (False, True): (64, 3072, -16), (True, False): (80, 10240, 48), (True, True): (80, 10240, 48)}
+# Decays of 128 channels take a compute unit's LDS whole: requests that need a second round of workgroups (2,048 columns together)
+# want a portion of so many rows (8 heads of 128 x 64, 5 requests, the longest 96: 16.9 / 19.6; 256: 36.2 / 33.4).
+STAGES_ROUND, STAGES_SECOND_ROUND_ROWS = 2048, 150
 SCAN_CHUNK = 32          # rows of a chunk of a long portion
 SCAN_MIN_ROWS = 96       # portions from this many rows on run in three passes over chunks (shorter ones are walked whole),
                          # where the engine allows logits to depend on the cut in their last bits (Workspace.exact_cuts False)
@@ -164,7 +171,7 @@ class _MatrixMemoryMixer(Mixer):
             scan = (chunks, nchunks, spans, nspans, local, start)
         mode = self.mode if mode is None else mode
         stages = plan is None and mode in (ops.RECUR_DECAY_GIVEN, ops.RECUR_SCALAR_GATES) and in_stages(
-            max_seq_rows(ctx), ctx.rows, self.heads * self.vdim, mode == ops.RECUR_SCALAR_GATES)
+            max_seq_rows(ctx), ctx.rows, nseq, self.heads * self.vdim, self.dim, mode == ops.RECUR_SCALAR_GATES)
         gates = ctx.ws.buffer("recur_gates", 3 * self.heads, torch.float32) if stages and mode == ops.RECUR_SCALAR_GATES else None
         ops.linear_recurrence(mode, y, at["r"] if "q" not in at else at["q"], at["k"], at["v"], gate, gate_off, gate2_off,
                               bias, bias2, param, self.qscale, call.state if state is None else state, raw, seq_rows, ctx.slots, ctx.positions, nseq,
@@ -181,9 +188,15 @@ class _MatrixMemoryMixer(Mixer):
             self.o.store(ctx.ws, act, target, ctx.rows)
 
 
-def in_stages(longest: int, rows: int, columns: int, gates: bool) -> bool:
-    """Whether a step of ``rows`` rows, up to ``longest`` a request, walks a layer's memories of ``columns`` value columns in stages."""
-    return longest >= STAGES_MIN_ROWS[gates] and rows * columns <= longest * STAGES_MAX_COLUMNS[gates]
+def in_stages(longest: int, rows: int, requests: int, columns: int, dim: int, gates: bool) -> bool:
+    """Whether a step of ``rows`` rows of ``requests`` requests, up to ``longest`` a request, walks a layer's memories of ``columns`` value
+    columns and ``dim`` key channels in stages."""
+    if dim not in (64, 128):
+        return False
+    least, share, less = STAGES_RULE[gates, dim == 128]
+    if not gates and dim == 128 and requests * columns > STAGES_ROUND and longest < STAGES_SECOND_ROUND_ROWS:
+        return False
+    return longest >= least and columns * (rows + STAGES_REQUEST_ROWS * requests) <= share * (longest - less)
 
 
 def decays_ahead(longest: int, rows: int, heads: int, dim: int, vdim: int) -> bool:
