@@ -78,6 +78,8 @@ int bw_attention_f32(const float* q, int q_stride, const int32_t* positions, con
                      const int32_t* block_table, int table_stride, const float* k_cache, const float* v_cache,
                      float* out, int out_stride, int rows, int heads, int kv_heads, int head_dim, int page_size,
                      int window, float scale, const float* sink, int chunk, float softcap, void* stream);
+// waves (4 or 8) of a workgroup of bw_attention_f32 that keeps the scores of up to ``capacity`` keys in LDS
+int bw_attention_f32_waves(int head_dim, long long workgroups, long long capacity);
 int bw_attention_f32_tiles(const float* q, int q_stride, const int32_t* positions, const int32_t* block_table,
                            int table_stride, const int32_t* tiles, int num_tiles, int tiled, const float* k_cache,
                            const float* v_cache, float* out, int out_stride, int heads, int kv_heads, int head_dim,

@@ -81,7 +81,6 @@ __device__ __forceinline__ float dot_canonical(const float* __restrict__ q_lds, 
 }
 
 #define ATT32_THREADS 256
-#define ATT32_KEEP_THREADS 512        // of the kernel that keeps its scores: eight waves
 
 // A workgroup barrier for data that meets in LDS: this wave's LDS writes are done, then the barrier.  (The
 // language's own barrier also waits for every load from memory that is still on its way, which would end the
@@ -150,10 +149,12 @@ __device__ __forceinline__ void walk_chunk(const float* __restrict__ ed, const f
 // their way. Against four waves, 32-bit keys and values: eight rows of 1,024 keys, 32 heads of 64, 33.6 -> 27.2 us (4.9 TB/s, what a
 // copy reaches); one row 24.9 -> 18.1; 8 x 4,096 keys 113 -> 91; 40 x 700 121 -> 100; 32/8 heads of 128 39.9 -> 28.0, 8/4 of 256 60 -> 48.
 // Eight keys a group on their way in four waves: 31.3, in eight the same 27.9; sixteen waves: 47 (their registers do not fit).
-template <int HD, bool KEEP>
-__global__ __launch_bounds__(KEEP ? ATT32_KEEP_THREADS : ATT32_THREADS) void attention_f32_kernel(AttnF32Args a) {
+// Some head sizes keep four waves where there is more than a workgroup a compute unit (att32_waves).
+template <int HD, bool KEEP, int T>
+__global__ __launch_bounds__(T) void attention_f32_kernel(AttnF32Args a) {
   using S = Att32Shape<HD>;
-  constexpr int T = KEEP ? ATT32_KEEP_THREADS : S::T, KC = S::KC, SEGS = S::SEGS, VJ = S::VJ;
+  static_assert(KEEP || T == S::T, "the two-pass form has four waves");
+  constexpr int KC = S::KC, SEGS = S::SEGS, VJ = S::VJ;
   extern __shared__ __attribute__((aligned(16))) float v_lds[];    // [2][KC][HD]: value rows of a chunk of keys; KEEP: then the scores
   float* scores = v_lds + 2 * KC * HD;
   __shared__ float q_lds[HD];
@@ -286,13 +287,13 @@ __global__ __launch_bounds__(KEEP ? ATT32_KEEP_THREADS : ATT32_THREADS) void att
     // Values only.  Three chunks of them are on their way at any time (three sets of registers in turn; a chunk in
     // flight is what keeps a compute unit's share of the memory system busy across a trip to memory), the first
     // three asked for before the scores turn into e_j.  Chunks past the last key fetch the last key again.
-    // The waves without an element of the walk fetch and stash (four of them: whole turns of a chunk's pieces), and
-    // the walking waves only walk: a chunk then costs the longer of the two, not their sum.
-    constexpr int WW = (HD + 63) / 64, LW = 4;                // waves that walk, waves that load
-    constexpr int LT = 64 * LW;                              // threads that fetch and stash
-    static_assert(WW + LW <= T / 64, "walkers and loaders are different waves");
+    // Where the walk leaves two waves or more without an element, those (four of them at most: whole turns of a
+    // chunk's pieces) fetch and stash, and the walking waves only walk: a chunk then costs the longer of the two, not their sum.
+    constexpr int WW = (HD + 63) / 64, LEFT = T / 64 - WW;    // waves that walk, waves that do not
+    constexpr bool APART = LEFT >= 2;
+    constexpr int LT = APART ? 64 * (LEFT < 4 ? LEFT : 4) : T;   // threads that fetch and stash
     constexpr int VL = (KC * SEGS + LT - 1) / LT;            // pieces of a chunk's value rows for each of them
-    const int lt = tid - 64 * WW;                            // (negative: this thread walks)
+    const int lt = APART ? tid - 64 * WW : tid;              // (negative: this thread walks only)
     const bool loads = lt >= 0 && lt < LT;
     f32x4 r0[VL], r1[VL], r2[VL];
     auto fetch_into = [&](f32x4 (&reg)[VL], int j0) {
@@ -370,11 +371,17 @@ __global__ __launch_bounds__(KEEP ? ATT32_KEEP_THREADS : ATT32_THREADS) void att
     // one chunk's turn: the chunk three ahead is asked for into ``next``, the chunk in ``buf`` is walked, the
     // chunk one ahead goes from ``ready`` into the other buffer; the barrier publishes it
     auto turn = [&](f32x4 (&next)[VL], const f32x4 (&ready)[VL], int j0, int buf) {
-      if (loads) {
+      if constexpr (APART) {
+        if (loads) {
+          fetch_into(next, j0 + 3 * KC);
+          stash_from(buf ^ 1, ready);
+        } else if (lt < 0) {
+          walk4(j0, buf);
+        }
+      } else {
         fetch_into(next, j0 + 3 * KC);
-        stash_from(buf ^ 1, ready);
-      } else if (lt < 0) {
         walk4(j0, buf);
+        stash_from(buf ^ 1, ready);
       }
       lds_barrier();
     };
@@ -918,14 +925,33 @@ static void launch_attention_f32_tiles(const AttnF32Args& a, dim3 grid, hipStrea
 
 #define ATT32_KEEP_LDS (144 * 1024)     // dynamic LDS of the kernel that keeps its scores: the values' chunks and the scores
 
+// Waves of a workgroup that keeps its scores, by what both forms measure.  A compute unit holds (by registers) one workgroup of eight
+// waves or two of four, and up to 128 elements the one is done sooner.  Heads of 16 elements, and of 160 and more, get four waves once
+// there is more than one workgroup for every compute unit; of 160 and more also where at most 64 keys are seen.  Four -> eight, us, 8 heads on 4:
+//   heads of 16:   256 workgroups of 200 keys 10.3 -> 8.7, 400 11.5 -> 15.1, 2,400 48 -> 70; of 2,400 keys 44 -> 35, 49 -> 67, 230 -> 339
+//   heads of 160:  256 of 20 keys 7.1 -> 7.0, 400 8.5 -> 12.2, 2,400 37 -> 57; 400 of 200 and 800 keys 24 -> 26 and 69 -> 67
+//   heads of 256:  256 of 60 and 200 keys 8.5 -> 8.8 and 19 -> 18; 400 of 20, 200 and 2,400 keys 9.3 -> 13.5, 34 -> 37 and 338 -> 305;
+//                  2,400 of them 38 -> 63, 150 -> 181, 1993 -> 1965
+//   heads of 32:   400 of 20 keys 12.1 -> 10.2, 2,400 of 200 97 -> 79 (and so up to 128)
+// (How many keys a row sees is on the device; the host knows the most.)
+static int att32_waves(int head_dim, long long workgroups, long long capacity) {
+  if (head_dim != 16 && head_dim < 160) return 8;
+  return workgroups > 256 || (head_dim >= 160 && capacity <= 64) ? 4 : 8;
+}
+
+extern "C" int bw_attention_f32_waves(int head_dim, long long workgroups, long long capacity) {
+  return att32_waves(head_dim, workgroups, capacity);
+}
+
 template <int HD>
 static void launch_attention_f32(const AttnF32Args& a, dim3 grid, hipStream_t s) {
+  constexpr int FEW = HD == 16 || HD >= 160 ? 256 : 512;   // (the others have no kernel of four waves)
   static bool allowed = false;                         // 64 KB of dynamic LDS and more has to be asked for once
   if (!allowed) {
-    (void)hipFuncSetAttribute((const void*)attention_f32_kernel<HD, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    (void)hipFuncSetAttribute((const void*)attention_f32_kernel<HD, false, ATT32_THREADS>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               Att32Shape<HD>::LDS_BYTES);
-    (void)hipFuncSetAttribute((const void*)attention_f32_kernel<HD, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              ATT32_KEEP_LDS);
+    (void)hipFuncSetAttribute((const void*)attention_f32_kernel<HD, true, 512>, hipFuncAttributeMaxDynamicSharedMemorySize, ATT32_KEEP_LDS);
+    (void)hipFuncSetAttribute((const void*)attention_f32_kernel<HD, true, FEW>, hipFuncAttributeMaxDynamicSharedMemorySize, ATT32_KEEP_LDS);
     allowed = true;
   }
   // the most keys a query of this launch can see: what a row of the block table covers, or the window
@@ -933,10 +959,14 @@ static void launch_attention_f32(const AttnF32Args& a, dim3 grid, hipStream_t s)
   if (a.window > 0 && a.window < capacity) capacity = a.window;
   if (a.chunk > 0 && a.chunk < capacity) capacity = a.chunk;
   const long long keep_bytes = Att32Shape<HD>::LDS_BYTES + ((capacity + 3) & ~3ll) * (long long)sizeof(float);
-  if (keep_bytes <= ATT32_KEEP_LDS && a.table_stride <= ATT32_TABLE && a.page_shift >= 0)   // (and the table's row fits the kernel's copy of it)
-    hipLaunchKernelGGL((attention_f32_kernel<HD, true>), grid, dim3(ATT32_KEEP_THREADS), (size_t)keep_bytes, s, a);
-  else
-    hipLaunchKernelGGL((attention_f32_kernel<HD, false>), grid, dim3(ATT32_THREADS), Att32Shape<HD>::LDS_BYTES, s, a);
+  if (keep_bytes <= ATT32_KEEP_LDS && a.table_stride <= ATT32_TABLE && a.page_shift >= 0) {   // (and the table's row fits the kernel's copy of it)
+    if (FEW == 256 && att32_waves(HD, (long long)grid.x * grid.y, capacity) == 4)
+      hipLaunchKernelGGL((attention_f32_kernel<HD, true, FEW>), grid, dim3(FEW), (size_t)keep_bytes, s, a);
+    else
+      hipLaunchKernelGGL((attention_f32_kernel<HD, true, 512>), grid, dim3(512), (size_t)keep_bytes, s, a);
+  } else {
+    hipLaunchKernelGGL((attention_f32_kernel<HD, false, ATT32_THREADS>), grid, dim3(ATT32_THREADS), Att32Shape<HD>::LDS_BYTES, s, a);
+  }
 }
 
 static int attention_f32_dispatch(const AttnF32Args& a, int items, int tiled, hipStream_t s) {

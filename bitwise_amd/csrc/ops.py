@@ -70,6 +70,7 @@ _SIGS = {
                               c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_attention_f32_tiles": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p,
                                c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_int, c_float, c_void_p],
+    "bw_attention_f32_waves": [c_int, c_longlong, c_longlong],
     "bw_attention_f32": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
                          c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p, c_int, c_float, c_void_p],
     "bw_attention_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_int,
@@ -165,7 +166,7 @@ _fns = {}
 # what waits.
 _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
-    "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts", "bw_gemm_gelu_glu_wins", "bw_gemm_split_tile", "bw_gemm_split_rows",
+    "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts", "bw_gemm_gelu_glu_wins", "bw_attention_f32_waves", "bw_gemm_split_tile", "bw_gemm_split_rows",
     "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
     "bw_chain_flush", "bw_chain_end",
@@ -740,6 +741,11 @@ def attention_f32(q: torch.Tensor, positions: torch.Tensor, row_seq: torch.Tenso
                                    v_cache.data_ptr(), out.data_ptr(), out.stride(0), rows, heads, kv_heads, head_dim,
                                    page_size, int(window), float(scale), _sink_ptr(sink, heads), int(chunk), float(softcap),
                                    _stream()), "attention_f32")
+
+
+def attention_f32_waves(head_dim: int, workgroups: int, capacity: int) -> int:
+    """Waves of a workgroup (a row and head) of ``attention_f32`` that keeps the scores of up to ``capacity`` keys in LDS."""
+    return int(_fn("bw_attention_f32_waves")(head_dim, workgroups, capacity))
 
 
 def attention_f32_tiles(q: torch.Tensor, positions: torch.Tensor, block_table: torch.Tensor, tiles: torch.Tensor,
