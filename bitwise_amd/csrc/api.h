@@ -25,6 +25,8 @@ int bw_add(float* x, const float* y, long long n, void* stream);
 int bw_add_bias(float* x, const float* bias, int rows, int cols, int ldx, void* stream);
 int bw_convert(const void* src, int src_is_bf16, void* dst, int dst_is_bf16, int rows, int cols, int lds, int ldd,
                void* stream);
+// whether bw_gemm_f32 runs so few rows as chains on the vector units rather than on the matrix cores (16-byte alignments given)
+int bw_gemm_f32_by_chains(int M, int N, int K, int w_is_bf16);
 int bw_gemm_f32_swiglu(const float* x, const void* w, int w_is_bf16, float* gate_up, float* h, int M, int outputs, int K, int ldx,
                        void* stream);
 int bw_swiglu_f32(const float* gate_up, float* h, int rows, int inter, void* stream);

@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256) void gemm_f32_rows_kernel(const float* __restr
 
 // ------------------------------------------------------------------------------ a wave a row, the row four elements a register
 
-// A decoded token alone: a wave is a row and 64 columns, lane l the chain of (row, column n0 + l); weights and rows travel from
+// Few rows of many columns (f32_by_chains): a wave is a row and 64 columns, lane l the chain of (row, column n0 + l); weights and rows travel from
 // memory straight into an LDS ring (buffer loads with LDS as destination: 8 rows of W, 128 bytes each, or 4 rows of x, 256
 // bytes each, an instruction; whole cache lines, the 16-byte chunks of a row of W permuted against bank conflicts; a ring of
 // stages, waits by counting loads).  The weights stay packed there: a lane reads its column's 16-byte chunks and widens them in
@@ -541,12 +541,32 @@ __global__ __launch_bounds__(64 * (8 + F32C_LOADERS)) void gemm_f32_chain_kernel
   *o = accumulate ? (*o + acc) : acc;
 }
 
-// For one row and at least as many blocks of 64 columns as there are compute units: 16,384 columns, K = 2048: 14.4 us, 15.0 to 15.8
-// on the matrix cores (gemm_f32_matrix.h), a head of 49,152 columns 36.6 against 37.4.  From two rows on those are faster (15.4
-// against 15.0, 36.7 and 37.3; three rows 17.9 against 15.4, eight 25 against 16 and 62 against 38).
 #define F32C_STAGES 7
-#define F32C_MAX_ROWS 1
+#define F32C_MAX_ROWS 8
 #define F32C_MIN_BLOCKS 256                                           // blocks of 64 columns
+
+// Which products of up to eight rows and at least as many blocks of 64 columns as there are compute units go by chains and not on the
+// matrix cores (gemm_f32_matrix.h).  A workgroup of chains is two to a compute unit, its loaders ask for little at a time and its waves
+// start at once; a tile with 32-bit weights has a compute unit to itself, so columns cost a round of the chip for every 16,384 of them.
+// Tiles / chains, us (K: 64, 256, 1024, 2048):
+//   32-bit weights, 2 rows, 16,321 columns  3.9/3.3  6.2/5.6  12.6/13.0 29.4/30.5     28,000 columns  6.0/3.9  9.8/7.9  26.9/25.5 48.7/44.3
+//                   4 rows, 24,000          6.0/4.0  9.6/7.9  25.5/24.0 46.8/42.3     8 rows, 65,000  11.5/7.2 18.5/15.5 43.6/42.8 99/105
+//   bfloat16        2 rows, 24,000          4.4/3.8  6.8/6.5  14.9/15.1 24.2/23.6     4 rows, 100,000 10.7/9.7 17.3/16.7 42.6/42.2 91/91
+// Of 1,350 products of two to eight rows (16,321 to 128,256 columns, K of 64 to 8192) the rule leaves 1.004 times the time of the better
+// kernel, 1.11 times at most; tiles for all of them left 1.08 and 1.86.  One row: by chains whatever K (16,384 columns, K = 2048, bfloat16
+// weights, 14.4 and 15.0 to 15.8 us; a head of 49,152 columns 36.6 and 37.4).
+static bool f32_by_chains(int M, int N, int K, bool bf16) {
+  const int blocks = (N + 63) / 64;
+  if (M > F32C_MAX_ROWS || blocks < F32C_MIN_BLOCKS || K % (bf16 ? 64 : 32) != 0) return false;
+  if (M == 1) return true;
+  if (bf16) return M == 2 ? K <= 512 || (blocks >= 1024 && K <= 1536) : M <= 4 && K <= 128;
+  if (K <= 256) return true;
+  if (M > 4) return blocks >= 600 && K <= 1024;
+  // (more than 1,024 steps of k: where the tiles' last round is not a full one)
+  return blocks > 256 && (K <= 1024 || (blocks % 256 >= 1 && blocks % 256 <= 230));
+}
+
+extern "C" int bw_gemm_f32_by_chains(int M, int N, int K, int w_is_bf16) { return f32_by_chains(M, N, K, w_is_bf16 != 0); }
 
 template <typename WT>
 static void launch_chain(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s) {
@@ -666,8 +686,8 @@ extern "C" int bw_gemm_f32(const float* x, const void* w, int w_is_bf16, float* 
   const bool vectors = ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
   const int tile_rows = M > 64 ? 128 : (M < 64 ? M : 64), tile_columns = M > 64 ? 128 : 64;
   const bool fits = vectors && (size_t)tile_rows * ldx * 4 < ((size_t)1 << 31) && (size_t)tile_columns * K * 4 < ((size_t)1 << 31);
-  // one row, many columns, K in whole stages: a chain a lane, the row four elements a register, loader waves
-  if (fits && M <= F32C_MAX_ROWS && (N + 63) / 64 >= F32C_MIN_BLOCKS && K % (w_is_bf16 ? 64 : 32) == 0) {
+  // up to eight rows, many columns, K in whole stages: a chain a lane, the row four elements a register, loader waves
+  if (fits && f32_by_chains(M, N, K, w_is_bf16 != 0)) {
     if (w_is_bf16) launch_chain<bf16_t>(x, (const bf16_t*)w, y, M, N, K, ldx, ldy, accumulate, s);
     else launch_chain<float>(x, (const float*)w, y, M, N, K, ldx, ldy, accumulate, s);
     return BW_LAUNCH_CHECK();

@@ -47,6 +47,7 @@ _SIGS = {
     "bw_rope_kvwrite": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                         c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_f32": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    "bw_gemm_f32_by_chains": [c_int, c_int, c_int, c_int],
     "bw_gemm_f32_swiglu": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_clamped_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],
@@ -166,7 +167,7 @@ _fns = {}
 # what waits.
 _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
-    "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts", "bw_gemm_gelu_glu_wins", "bw_attention_f32_waves", "bw_gemm_split_tile", "bw_gemm_split_rows",
+    "bw_gemm_f32_by_chains", "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts", "bw_gemm_gelu_glu_wins", "bw_attention_f32_waves", "bw_gemm_split_tile", "bw_gemm_split_rows",
     "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
     "bw_chain_flush", "bw_chain_end",
@@ -457,6 +458,11 @@ def gemm_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows: int, acc
         raise ValueError(f"gemm_f32: x {tuple(x.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not match")
     _check(_fn("bw_gemm_f32")(x.data_ptr(), w.data_ptr(), _is_bf16(w, "weight"), out.data_ptr(), rows, N, K,
                               x.stride(0), out.stride(0), int(accumulate), _stream()), "gemm_f32")
+
+
+def gemm_f32_by_chains(rows: int, N: int, K: int, bf16_weights: bool) -> bool:
+    """Whether ``gemm_f32`` runs so few rows as chains on the vector units rather than on the matrix cores (the same bits)."""
+    return bool(_fn("bw_gemm_f32_by_chains")(rows, N, K, int(bf16_weights)))
 
 
 def gemm_f32_swiglu(x: torch.Tensor, w: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, rows: int) -> None:

@@ -19,8 +19,8 @@ SHAPES = [
     (17, 4097, 64), (31, 4128, 128), (33, 2754, 320), (49, 2080, 192), (64, 2049, 64),
     # 64 x 64 tiles: 33 rows and more of many columns, and K in stages of 32 only
     (33, 16384, 64), (64, 16400, 192), (17, 50, 96), (40, 200, 32), (5, 16390, 96),
-    # one row of many columns
-    (1, 16385, 128),
+    # chains: up to eight rows of many columns (two to eight with 32-bit weights, some with bfloat16 ones)
+    (1, 16385, 128), (1, 16321, 704), (2, 16385, 64), (3, 16330, 128), (4, 16449, 1024), (5, 16400, 256), (7, 16385, 96), (8, 16390, 192),
 ]
 
 
