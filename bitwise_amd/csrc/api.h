@@ -27,6 +27,8 @@ int bw_convert(const void* src, int src_is_bf16, void* dst, int dst_is_bf16, int
                void* stream);
 // whether bw_gemm_f32 runs so few rows as chains on the vector units rather than on the matrix cores (16-byte alignments given)
 int bw_gemm_f32_by_chains(int M, int N, int K, int w_is_bf16);
+// whether bw_gemm_f32_swiglu computes the activation in the product's epilogue (and leaves gate_up alone)
+int bw_gemm_f32_swiglu_in_tiles(const float* x, const void* w, int w_is_bf16, int M, int outputs, int K, int ldx);
 int bw_gemm_f32_swiglu(const float* x, const void* w, int w_is_bf16, float* gate_up, float* h, int M, int outputs, int K, int ldx,
                        void* stream);
 int bw_swiglu_f32(const float* gate_up, float* h, int rows, int inter, void* stream);

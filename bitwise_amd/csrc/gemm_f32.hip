@@ -725,27 +725,50 @@ extern "C" int bw_gemm_f32(const float* x, const void* w, int w_is_bf16, float* 
   return BW_LAUNCH_CHECK();
 }
 
+// Up to eight rows of more than 8,192 outputs: more than one gated tile for every compute unit, and the product as it goes without
+// the epilogue can be so much faster that two kernels are.  Tiles with the epilogue / two kernels, us, outputs x K:
+//   32-bit weights, one row   8200 x 64 6.1/5.5, x 1024 20.3/17.8, x 4096 68/51; 16384 x 512 15.1/15.8, x 1024 42/31; 50000 x 64 18.7/11.0
+//                   8 rows    8200 x 64 6.5/6.0, x 256 9.6/10.2; 16384 x 256 11.0/11.4; 32768 x 512 36.6/30.0
+//   bfloat16, one row         8200 x 512 9.0/8.9, x 1024 13.8/12.4, x 4096 43/29; 14336 x 1024 14.6/16.1, x 2048 23.8/23.7
+// Of 804 such products this leaves 1.007 times the time of the better way (tiles for all 1.043; 1.69 times at most, and now 1.27).
+// One row of 8,192 outputs, K = 2048: 16.3 us in tiles and 17.2; with 32-bit weights 30.0 and 32.3.
+static bool f32_gated_apart(int M, int outputs, int K, bool bf16) {
+  if (M > 8 || outputs <= 8192) return false;
+  if (bf16) return M == 1 && K >= 1024 && (outputs < 11000 || (K >= 2048 && K <= 4096 && outputs < 16000));
+  if (M <= 4) return K <= 2048 || (K <= 4096 && outputs < 10000);
+  return K <= 64 || (K <= 256 && outputs >= 18000) || (K <= 1024 && outputs >= 24000);
+}
+
+// Whether the product goes in tiles with the activation in their epilogue.
+static bool f32_gated_in_tiles(const float* x, const void* w, bool bf16, int M, int outputs, int K, int ldx) {
+  const size_t limit = (size_t)0x7ff00000;             // (a tile's descriptor spans the whole weight)
+  if (ldx % 4 != 0 || ((uintptr_t)x & 15) != 0 || ((uintptr_t)w & 15) != 0) return false;
+  if ((size_t)(M < 128 ? M : 128) * ldx * 4 >= limit || (size_t)2 * outputs * K * (bf16 ? 2 : 4) >= limit) return false;
+  if (M > 64) return K % 32 == 0;
+  return K % 64 == 0 && !f32_gated_apart(M, outputs, K, bf16) && f32_few_rows_kernel(M, 2 * outputs, K) != F32_STRIPS;
+}
+
+extern "C" int bw_gemm_f32_swiglu_in_tiles(const float* x, const void* w, int w_is_bf16, int M, int outputs, int K, int ldx) {
+  return M > 0 && outputs > 0 && K > 0 && ldx >= K && f32_gated_in_tiles(x, w, w_is_bf16 != 0, M, outputs, K, ldx);
+}
+
 // h = silu(x Wg^T) * (x Wu^T), w = [Wg; Wu] (outputs rows each).  Where the product goes in tiles its epilogue computes h; otherwise
-// the sums go to gate_up and swiglu_f32_kernel behind it.  The same operations on the same sums.  (One row too: a chain a lane and
-// the kernel behind it take 17.2 us for 8192 outputs of K = 2048, the tiles 16.3; with 32-bit weights 32.3 and 30.0.)
+// the sums go to gate_up and swiglu_f32_kernel behind it.  The same operations on the same sums.
 extern "C" int bw_gemm_f32_swiglu(const float* x, const void* w, int w_is_bf16, float* gate_up, float* h, int M, int outputs, int K, int ldx,
                                   void* stream) {
   if (M <= 0 || outputs <= 0) return 0;
   if (K <= 0 || ldx < K) return -2;
   hipStream_t s = (hipStream_t)stream;
-  const bool vectors = ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
-  const size_t limit = (size_t)0x7ff00000;             // (a tile's descriptor spans the whole weight)
-  const bool fits = vectors && (size_t)(M < 128 ? M : 128) * ldx * 4 < limit && (size_t)2 * outputs * K * (w_is_bf16 ? 2 : 4) < limit;
-  if (fits && M > 64 && K % 32 == 0) {
+  if (!f32_gated_in_tiles(x, w, w_is_bf16 != 0, M, outputs, K, ldx)) {
+    const int rc = bw_gemm_f32(x, w, w_is_bf16, gate_up, M, 2 * outputs, K, ldx, 2 * outputs, 0, stream);
+    return rc != 0 ? rc : bw_swiglu_f32(gate_up, h, M, outputs, stream);
+  }
+  if (M > 64) {
     if (w_is_bf16) launch_f32_prompt<bf16_t, true>(x, (const bf16_t*)w, h, M, outputs, K, ldx, outputs, 0, s);
     else launch_f32_prompt<float, true>(x, (const float*)w, h, M, outputs, K, ldx, outputs, 0, s);
-    return BW_LAUNCH_CHECK();
-  }
-  if (fits && M <= 64 && K % 64 == 0 && f32_few_rows_kernel(M, 2 * outputs, K) != F32_STRIPS) {
+  } else {
     if (w_is_bf16) launch_f32_few_rows<bf16_t, true>(x, (const bf16_t*)w, h, M, outputs, K, ldx, outputs, 0, s);
     else launch_f32_few_rows<float, true>(x, (const float*)w, h, M, outputs, K, ldx, outputs, 0, s);
-    return BW_LAUNCH_CHECK();
   }
-  const int rc = bw_gemm_f32(x, w, w_is_bf16, gate_up, M, 2 * outputs, K, ldx, 2 * outputs, 0, stream);
-  return rc != 0 ? rc : bw_swiglu_f32(gate_up, h, M, outputs, stream);
+  return BW_LAUNCH_CHECK();
 }

@@ -48,6 +48,7 @@ _SIGS = {
                         c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_f32": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_f32_by_chains": [c_int, c_int, c_int, c_int],
+    "bw_gemm_f32_swiglu_in_tiles": [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int],
     "bw_gemm_f32_swiglu": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_clamped_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],
@@ -167,7 +168,8 @@ _fns = {}
 # what waits.
 _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
-    "bw_gemm_f32_by_chains", "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts", "bw_gemm_gelu_glu_wins", "bw_attention_f32_waves", "bw_gemm_split_tile", "bw_gemm_split_rows",
+    "bw_gemm_f32_by_chains", "bw_gemm_f32_swiglu_in_tiles", "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts",
+    "bw_gemm_gelu_glu_wins", "bw_gemm_split_tile", "bw_gemm_split_rows", "bw_attention_f32_waves",
     "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
     "bw_chain_flush", "bw_chain_end",
@@ -465,9 +467,14 @@ def gemm_f32_by_chains(rows: int, N: int, K: int, bf16_weights: bool) -> bool:
     return bool(_fn("bw_gemm_f32_by_chains")(rows, N, K, int(bf16_weights)))
 
 
+def gemm_f32_swiglu_in_tiles(x: torch.Tensor, w: torch.Tensor, rows: int) -> bool:
+    """Whether ``gemm_f32_swiglu`` computes the activation in the product's epilogue (and leaves ``gate_up`` alone)."""
+    return bool(_fn("bw_gemm_f32_swiglu_in_tiles")(x.data_ptr(), w.data_ptr(), int(w.dtype == torch.bfloat16), rows, w.shape[0] // 2, w.shape[1], x.stride(0)))
+
+
 def gemm_f32_swiglu(x: torch.Tensor, w: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, rows: int) -> None:
     """out[:rows] = silu(g) * u with [g | u] = x[:rows] @ w.T, ``w`` = [gate; up] stacked: ``gemm_f32`` and ``swiglu_f32`` in one kernel
-    where the product goes in tiles of the matrix cores, the same bits.  ``gate_up``: room for the sums where it does not."""
+    where that is faster (``gemm_f32_swiglu_in_tiles``), the same bits.  ``gate_up``: room for the sums where it does not."""
     if not x.is_cuda or x.dtype != torch.float32 or x.dim() != 2 or x.stride(1) != 1:
         raise ValueError("gemm_f32_swiglu: x must be a float32 GPU matrix with contiguous rows")
     _need(gate_up, torch.float32, "gate_up")

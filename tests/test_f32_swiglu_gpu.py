@@ -16,6 +16,7 @@ pytestmark = pytest.mark.gpu
     (33, 8200, 64, 0), (64, 8193, 128, 0),                             # 64 x 64 of few rows
     (65, 97, 32, 0), (100, 1000, 96, 0), (450, 1021, 64, 0),           # 64 x 64 and 128 x 64 of a prompt
     (300, 4099, 32, 0), (1000, 2050, 96, 0), (2050, 700, 64, 0),       # 128 x 128, and three 64 x 64 a compute unit
+    (1, 8200, 1024, 0), (4, 8193, 128, 0), (8, 18000, 64, 0),             # more than 8,192 outputs: the epilogue or two kernels
     (8, 200, 256, 0), (3, 4104, 100, 0), (70, 130, 50, 0), (70, 130, 64, 1), (9, 5000, 96, 0),   # strips; no tile
 ])
 def test_bits_of_two_kernels(gpu, dtype, rows, inter, K, offset):
