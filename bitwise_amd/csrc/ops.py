@@ -472,22 +472,29 @@ def gemm_f32_swiglu_in_tiles(x: torch.Tensor, w: torch.Tensor, rows: int) -> boo
     return bool(_fn("bw_gemm_f32_swiglu_in_tiles")(x.data_ptr(), w.data_ptr(), int(w.dtype == torch.bfloat16), rows, w.shape[0] // 2, w.shape[1], x.stride(0)))
 
 
-def gemm_f32_swiglu(x: torch.Tensor, w: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, rows: int) -> None:
+def gemm_f32_swiglu(x: torch.Tensor, w: torch.Tensor, gate_up: Optional[torch.Tensor], out: torch.Tensor, rows: int) -> None:
     """out[:rows] = silu(g) * u with [g | u] = x[:rows] @ w.T, ``w`` = [gate; up] stacked: ``gemm_f32`` and ``swiglu_f32`` in one kernel
-    where that is faster (``gemm_f32_swiglu_in_tiles``), the same bits.  ``gate_up``: room for the sums where it does not."""
+    where that is faster (``gemm_f32_swiglu_in_tiles``), the same bits.  ``gate_up``: room for the sums where it is not
+    (None where it is)."""
     if not x.is_cuda or x.dtype != torch.float32 or x.dim() != 2 or x.stride(1) != 1:
         raise ValueError("gemm_f32_swiglu: x must be a float32 GPU matrix with contiguous rows")
-    _need(gate_up, torch.float32, "gate_up")
+    if gate_up is not None:
+        _need(gate_up, torch.float32, "gate_up")
     _need(out, torch.float32, "out")
     if not w.is_cuda or not w.is_contiguous() or w.dim() != 2:
         raise ValueError("gemm_f32_swiglu: weight must be a contiguous [2 * inter, K] GPU tensor")
     N, K = w.shape
     inter = out.shape[1]
-    if x.shape[1] != K or N != 2 * inter or gate_up.shape[1] != N or min(x.shape[0], out.shape[0], gate_up.shape[0]) < rows:
-        raise ValueError(f"gemm_f32_swiglu: x {tuple(x.shape)}, w {tuple(w.shape)}, gate_up {tuple(gate_up.shape)}, out {tuple(out.shape)} "
-                         "do not match")
-    _check(_fn("bw_gemm_f32_swiglu")(x.data_ptr(), w.data_ptr(), _is_bf16(w, "weight"), gate_up.data_ptr(), out.data_ptr(), rows, inter, K,
-                                     x.stride(0), _stream()), "gemm_f32_swiglu")
+    if x.shape[1] != K or N != 2 * inter or min(x.shape[0], out.shape[0]) < rows:
+        raise ValueError(f"gemm_f32_swiglu: x {tuple(x.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not match")
+    bf16 = _is_bf16(w, "weight")
+    if gate_up is None:
+        if not gemm_f32_swiglu_in_tiles(x, w, rows):
+            raise ValueError("gemm_f32_swiglu: this product needs gate_up for its sums")
+    elif gate_up.dim() != 2 or gate_up.shape[1] != N or gate_up.shape[0] < rows:
+        raise ValueError(f"gemm_f32_swiglu: gate_up {tuple(gate_up.shape)} does not match w {tuple(w.shape)} and {rows} rows")
+    _check(_fn("bw_gemm_f32_swiglu")(x.data_ptr(), w.data_ptr(), bf16, 0 if gate_up is None else gate_up.data_ptr(), out.data_ptr(), rows, inter,
+                                     K, x.stride(0), _stream()), "gemm_f32_swiglu")
 
 
 def gemm_f32_prompt_tile(rows: int, N: int) -> Tuple[int, int]:

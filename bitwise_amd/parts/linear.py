@@ -64,9 +64,20 @@ class Linear:
         return (ws.buffer("gemm_add_split", floats, torch.float32, rows=1),
                 ws.buffer("gemm_add_split_count", counters, torch.int32, rows=1))
 
-    def store_swiglu(self, ws, x: torch.Tensor, sums: torch.Tensor, out: torch.Tensor, rows: int) -> None:
-        """out[:rows] = silu(g) * u with [g | u] = x[:rows] @ W.T, on the 32-bit kernels; ``sums``: room for [g | u]."""
-        ops.gemm_f32_swiglu(self._x32(ws, x, rows), self.weight, sums, out, rows)
+    SUMS_ROWS = 64         # products of up to so many rows share one small buffer for sums that a kernel behind them reads
+
+    def store_swiglu(self, ws, x: torch.Tensor, out: torch.Tensor, rows: int) -> None:
+        """out[:rows] = silu(g) * u (32-bit) with [g | u] what ``store`` gives.  Where the product's epilogue computes it, which it does for
+        nearly every prompt, [g | u] is never in memory, and no room is held for it."""
+        if not self.mfma:
+            x = self._x32(ws, x, rows)
+            if ops.gemm_f32_swiglu_in_tiles(x, self.weight, rows):
+                ops.gemm_f32_swiglu(x, self.weight, None, out, rows)
+                return
+        few = rows <= self.SUMS_ROWS < ws.max_rows
+        sums = ws.buffer("gate_up", self.out_features, torch.float32, rows=self.SUMS_ROWS if few else None)
+        self.store(ws, x, sums, rows)
+        ops.swiglu_f32(sums, out, rows)
 
     def store(self, ws, x: torch.Tensor, out: torch.Tensor, rows: int) -> None:
         """out[:rows] = x[:rows] @ W.T (out float32, or bfloat16 on the matrix-core path).  ``ws`` is the

@@ -67,9 +67,8 @@ class SwiGLU(FeedForward):
             act = ws.buffer("mlp_h", self.inter, torch.bfloat16)
             ops.gemm_bf16(h, self.gate_up.weight, act, rows, ops.EPI_SWIGLU_BF16)   # SwiGLU in the epilogue
         else:
-            gu = ws.buffer("gate_up", 2 * self.inter, torch.float32)
             act32 = ws.buffer("mlp_h32", self.inter, torch.float32)
-            self.gate_up.store_swiglu(ws, h, gu, act32, rows)
+            self.gate_up.store_swiglu(ws, h, act32, rows)
             if rt.bf16:
                 # bfloat16 mode rounds the activation here whatever dtype the weights are stored in, so that
                 # the mode has one set of rounding points (a 32-bit down projection widens it again)

@@ -5,6 +5,9 @@ import pytest
 import torch
 
 from bitwise_amd.csrc import ops
+from bitwise_amd.parts.linear import Linear
+from bitwise_amd.parts.mlp import SwiGLU
+from bitwise_amd.runtime import Runtime, Workspace
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +34,27 @@ def test_bits_of_two_kernels(gpu, dtype, rows, inter, K, offset):
     got = torch.full((rows + 1, inter), 7.0, device=gpu)
     ops.gemm_f32_swiglu(x, w, torch.empty_like(sums), got, rows)
     assert torch.equal(got[:rows].view(torch.int32), want.view(torch.int32)) and bool((got[rows] == 7.0).all())
+
+
+def _feed_forward(gpu, width, inter, bias=None):
+    rt = Runtime("float32", gpu)
+    g = torch.Generator(device=gpu).manual_seed(width)
+    part = SwiGLU({"width": width, "inter": inter}, rt)
+    part.bind({n: torch.randn(*s.shape, generator=g, device=gpu) * 0.1 for n, s in part.tensors().items()})
+    if bias is not None:
+        part.gate_up = Linear(part.gate_up.weight, rt, bias=bias)
+    return part, torch.randn(300, width, generator=g, device=gpu)
+
+
+def test_no_room_is_held_for_sums_that_never_reach_memory(gpu):
+    width, inter = 256, 4200
+    part, x = _feed_forward(gpu, width, inter)
+    ws = Workspace(gpu, max_rows=300, page_size=16)
+    act = torch.empty(300, inter, device=gpu)
+    for rows in (1, 8, 40, 64, 65, 300):
+        part.gate_up.store_swiglu(ws, x, act, rows)
+    assert ws.nbytes() == 0
+    small, y = _feed_forward(gpu, 128, 200)                             # strips up to 64 rows, tiles for more
+    for rows in (1, 64, 65, 300):
+        small.gate_up.store_swiglu(ws, y, act.view(-1)[:300 * 200].view(300, 200), rows)
+    assert ws.nbytes() == 64 * 2 * 200 * 4
