@@ -69,7 +69,7 @@ class Linear:
     def store_swiglu(self, ws, x: torch.Tensor, out: torch.Tensor, rows: int) -> None:
         """out[:rows] = silu(g) * u (32-bit) with [g | u] what ``store`` gives.  Where the product's epilogue computes it, which it does for
         nearly every prompt, [g | u] is never in memory, and no room is held for it."""
-        if not self.mfma:
+        if self.bias is None and not self.mfma:
             x = self._x32(ws, x, rows)
             if ops.gemm_f32_swiglu_in_tiles(x, self.weight, rows):
                 ops.gemm_f32_swiglu(x, self.weight, None, out, rows)

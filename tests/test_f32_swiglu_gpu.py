@@ -58,3 +58,17 @@ def test_no_room_is_held_for_sums_that_never_reach_memory(gpu):
     for rows in (1, 64, 65, 300):
         small.gate_up.store_swiglu(ws, y, act.view(-1)[:300 * 200].view(300, 200), rows)
     assert ws.nbytes() == 64 * 2 * 200 * 4
+
+
+def test_a_bias_of_the_stacked_projection_counts(gpu):
+    width, inter = 256, 4200
+    bias = torch.linspace(-1, 1, 2 * inter, device=gpu)
+    part, x = _feed_forward(gpu, width, inter, bias)
+    ws, act, want = Workspace(gpu, max_rows=300, page_size=16), torch.empty(300, inter, device=gpu), torch.empty(300, inter, device=gpu)
+    sums = torch.empty(300, 2 * inter, device=gpu)
+    part.gate_up.store(ws, x, sums, 300)
+    ops.swiglu_f32(sums, want, 300)
+    for rows in (300, 40):
+        act.zero_()
+        part.gate_up.store_swiglu(ws, x, act, rows)
+        assert torch.equal(act[:rows].view(torch.int32), want[:rows].view(torch.int32))
