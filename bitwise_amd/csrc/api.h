@@ -124,6 +124,8 @@ int bw_chain_flush(void* stream);
 int bw_chain_end(void* stream);
 int bw_sample(const float* logits, int vocab, int ld, int rows, const float* temperature, const double* uniform,
               int32_t* out, void* stream);
+// waves of a workgroup that chains a row bit by bit; 0: the row goes word by word
+int bw_fingerprint_waves(int rows, int vocab);
 int bw_fingerprint(const float* logits, int vocab, int ld, int rows, const void* h_in, void* h_out, void* stream);
 // Mixers with a fixed-size state per request (sequence_mix.hip).  seq_rows: [requests, 2] = (first row, rows) of every
 // request of the step; slots: its state slot.  A request without rows, with a negative slot or a negative first

@@ -92,6 +92,7 @@ _SIGS = {
     "bw_chain_flush": [c_void_p],
     "bw_chain_end": [c_void_p],
     "bw_sample": [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
+    "bw_fingerprint_waves": [c_int, c_int],
     "bw_fingerprint": [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
     "bw_norm_shift": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p, c_void_p,
                       c_void_p, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p],
@@ -169,7 +170,7 @@ _fns = {}
 _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
     "bw_gemm_f32_by_chains", "bw_gemm_f32_swiglu_in_tiles", "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts",
-    "bw_gemm_gelu_glu_wins", "bw_gemm_split_tile", "bw_gemm_split_rows", "bw_attention_f32_waves",
+    "bw_gemm_gelu_glu_wins", "bw_gemm_split_tile", "bw_gemm_split_rows", "bw_attention_f32_waves", "bw_fingerprint_waves",
     "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
     "bw_chain_flush", "bw_chain_end",
@@ -1978,6 +1979,11 @@ def sample(logits: torch.Tensor, rows: int, temperature: torch.Tensor, uniform: 
         raise ValueError("sample: buffers shorter than the number of rows")
     _check(_fn("bw_sample")(logits.data_ptr(), logits.shape[1], logits.stride(0), rows, temperature.data_ptr(),
                             uniform.data_ptr(), out.data_ptr(), _stream()), "sample")
+
+
+def fingerprint_waves(rows: int, vocab: int) -> int:
+    """Waves of a workgroup that chains a row of logits bit by bit, or 0 where ``fingerprint`` goes word by word (the same values)."""
+    return int(_fn("bw_fingerprint_waves")(rows, vocab))
 
 
 def fingerprint(logits: torch.Tensor, rows: int, h_in: torch.Tensor, h_out: torch.Tensor) -> None:

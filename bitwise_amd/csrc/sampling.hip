@@ -352,29 +352,38 @@ __global__ __launch_bounds__(64 * WAVES, 4) void fingerprint_slices_kernel(const
   if (t == 0) h_out[row] = fp_finish(h, p, vocab);
 }
 
+// Which kernel, by nanoseconds: the waves of a workgroup of slices, or 0 for the chain.  A link of the chain takes 13, 15 with 787 rows and
+// 16 with 1,024, whose waves share compute units; 1,100 rows take 1.8 times as long, 2,048 2 to 3.7 times.  A pass of 4, 8 or 16 waves
+// over their 8,191, 16,383 or 32,767 words takes 26, 30 or 42 us on a compute unit of its own, 34 with two of four waves on one, 47 with
+// four; beyond that sixteen waves' worth of rows share one at about 42.
+// 4,096 logits are 26 us so and 28 as a chain, 3,072 are 26 and 21; 787 rows of 5,645 47 and 42, 1,024 rows of 7,000 47 and 59, of 8,192 47 and
+// 67, 4,096 of them 237 as a chain.
+static int fingerprint_waves(int rows, int words) {
+  const long long link = rows <= 512 ? 13000 : rows <= 1024 ? 13000 + 6ll * (rows - 512) : 13000ll * (2048 + rows) / 2048;   // ps
+  const int pass_ns[3] = {26000, 30000, 42000};
+  int waves = 0;
+  long long best = words * link / 1000;
+  for (int k = 0; k < 3; ++k) {
+    const int w = 4 << k, slots = 2048 * w - 1, a_round = 256 * 16 / w;
+    const long long passes = (words + slots - 1) / slots;
+    long long ns = rows <= 256 ? pass_ns[k] : (rows + a_round - 1) / a_round * (long long)pass_ns[2];
+    if (k == 0 && rows > 256 && rows <= 1024) ns = rows <= 512 ? 34000 : 47000;
+    if (passes * ns < best) {
+      best = passes * ns;
+      waves = w;
+    }
+  }
+  return waves;
+}
+
+extern "C" int bw_fingerprint_waves(int rows, int vocab) { return rows > 0 && vocab > 0 ? fingerprint_waves(rows, vocab >> 1) : 0; }
+
 extern "C" int bw_fingerprint(const float* logits, int vocab, int ld, int rows, const void* h_in, void* h_out,
                               void* stream) {
   if (rows <= 0) return 0;
   const uint64_t* from = (const uint64_t*)h_in;
   uint64_t* to = (uint64_t*)h_out;
-  const int words = vocab >> 1;
-  // Which kernel, by nanoseconds.  A link of the chain takes 13; beyond a few hundred rows its waves share compute units (1,024 rows
-  // take 1.2 to 1.9 times as long, 2,048 2.3 to 3.7 times).  A pass of 4, 8 or 16 waves over their 8,191, 16,383 or 32,767 words
-  // takes 26, 30 or 42 us on a compute unit of its own, and sixteen waves' worth of rows share one at about the last of these.
-  // 4,096 logits are 26 us so and 28 as a chain, 3,072 are 26 and 21; 1,024 rows of 8,192 45 and 63, 4,096 of them 237 as a chain.
-  const long long chain = (long long)words * 13 * (2048 + rows) / 2048;
-  const int pass_ns[3] = {26000, 30000, 42000};
-  int waves = 0;
-  long long best = chain;
-  for (int k = 0; k < 3; ++k) {
-    const int w = 4 << k, slots = 2048 * w - 1, a_round = 256 * 16 / w;
-    const long long passes = (words + slots - 1) / slots;
-    const long long ns = passes * (rows <= 256 ? pass_ns[k] : (rows + a_round - 1) / a_round * (long long)pass_ns[2]);
-    if (ns < best) {
-      best = ns;
-      waves = w;
-    }
-  }
+  const int waves = fingerprint_waves(rows, vocab >> 1);
   const hipStream_t s = (hipStream_t)stream;
   if (waves == 16) hipLaunchKernelGGL((fingerprint_slices_kernel<16>), dim3(rows), dim3(1024), 0, s, logits, vocab, ld, from, to);
   else if (waves == 8) hipLaunchKernelGGL((fingerprint_slices_kernel<8>), dim3(rows), dim3(512), 0, s, logits, vocab, ld, from, to);
