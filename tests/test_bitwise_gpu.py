@@ -50,7 +50,7 @@ def test_matrix_product_at_layer_widths(gpu):
 
 
 def test_matrix_product_on_the_matrix_cores_is_the_same_chain(gpu):
-    """17 to 64 rows and prompt portions run their chains as 32-bit matrix instructions of one step of k each:
+    """17 to 64 rows and prompt portions run their chains as 32-bit matrix instructions of four steps of k each:
     shapes around the kernels' tile edges, 32-bit and bfloat16 weights, store and residual add, against std::fma."""
     g = torch.Generator().manual_seed(15)
     shapes = [(17, 33, 64), (24, 16, 128), (32, 100, 192), (33, 17, 64), (64, 130, 256), (48, 64, 2048),

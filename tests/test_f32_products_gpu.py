@@ -24,19 +24,62 @@ SHAPES = [
 ]
 
 
+def _check(gpu, x, w, wdt):
+    """``x`` (rows farther apart than they are long) times ``w`` against std::fma, written and added."""
+    (M, K), N = x.shape, w.shape[0]
+    want = ps.linear(x.contiguous().numpy(), w.float().numpy())
+    out = torch.full((M, N + 4), 5.0, device=gpu)
+    wide = torch.zeros(M, K + 8)
+    wide[:, :K] = x
+    there, weight = wide.to(gpu)[:, :K], w.to(wdt).to(gpu)
+    ops.gemm_f32(there, weight, out[:, :N], M)
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:, :N].view(np.uint32), want.view(np.uint32))
+    assert (got[:, N:] == 5.0).all()
+    ops.gemm_f32(there, weight, out[:, :N], M, accumulate=True)
+    assert np.array_equal(out.cpu().numpy()[:, :N], want + want)
+    return want
+
+
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("wdt", [torch.bfloat16, torch.float32])
 def test_few_rows_are_the_scalar_chains(gpu, M, N, K, wdt):
     g = torch.Generator().manual_seed(M * 31 + N + K)
-    wide = torch.randn(M, K + 8, generator=g)
-    wide[0, :4] = torch.tensor([-0.0, 1e-38, -3e38, 1e-42])
-    w = (torch.randn(N, K, generator=g) * 0.2).to(wdt)
-    want = ps.linear(wide[:, :K].contiguous().numpy(), w.float().numpy())
-    out = torch.full((M, N + 4), 5.0, device=gpu)
-    x = wide.to(gpu)[:, :K]                                     # rows farther apart than they are long
-    ops.gemm_f32(x, w.to(gpu), out[:, :N], M)
-    got = out.cpu().numpy()
-    assert np.array_equal(got[:, :N].view(np.uint32), want.view(np.uint32))
-    assert (got[:, N:] == 5.0).all()
-    ops.gemm_f32(x, w.to(gpu), out[:, :N], M, accumulate=True)
-    assert np.array_equal(out.cpu().numpy()[:, :N], want + want)
+    x, w = torch.randn(M, K, generator=g), (torch.randn(N, K, generator=g) * 0.2).to(wdt)
+    want = _check(gpu, x, w, wdt)
+    # (what a missing, repeated or exchanged step of k would give is another number in nearly every output)
+    swapped = x.clone()
+    swapped[:, [0, K - 1]] = x[:, [K - 1, 0]]
+    assert (ps.linear(swapped.numpy(), w[:8].float().numpy()) != want[:, :8]).mean() > 0.5
+
+
+# a shape for every kernel that takes a 32-bit product
+KERNELS = [(1, 33, 64), (8, 40, 192), (1, 16385, 128), (4, 16330, 128), (8, 16390, 64), (9, 8256, 128), (20, 4128, 128), (40, 16400, 64), (5, 40, 72),
+           (30, 50, 72), (70, 200, 96), (100, 130, 48), (1000, 2040, 64), (257, 300, 64)]
+
+
+@pytest.mark.parametrize("M,N,K", KERNELS)
+@pytest.mark.parametrize("wdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["denormal sums", "denormal operands", "cancelling", "infinite", "zeros"])
+def test_special_values_are_the_scalar_chains(gpu, M, N, K, wdt, kind):
+    g = torch.Generator().manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g), (torch.randn(N, K, generator=g) * 0.2).to(wdt).float()
+    if kind == "denormal sums":                                 # products of about 1e-41: sums that are denormal throughout
+        x, w = x * 1e-20, (w * 5e-21).to(wdt).float()
+    elif kind == "denormal operands":
+        x = x * 1e-40
+    elif kind == "cancelling":                                  # huge steps next to each other take each other back: their order shows
+        at = torch.randint(0, K // 2, (M,), generator=g) * 2
+        w[:, 1::2] = w[:, 0::2]
+        rows = torch.arange(M)
+        x[rows, at], x[rows, at + 1] = 1e7, -1e7
+    elif kind == "infinite":                                    # one a row: no sum is the difference of two
+        x[torch.arange(M), torch.randint(0, K, (M,), generator=g)] = float("inf")
+        w[w == 0] = 1.0
+    else:
+        x[:] = torch.where(torch.rand(M, K, generator=g) < 0.5, 0.0, -0.0)
+    want = _check(gpu, x, w, wdt)
+    if kind.startswith("denormal"):
+        assert (want != 0).mean() > 0.9 and (np.abs(want) < np.finfo(np.float32).tiny).all()
+    elif kind == "infinite":
+        assert np.isinf(want).all()

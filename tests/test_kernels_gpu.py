@@ -9,6 +9,7 @@ import pytest
 import torch
 
 import plain_llama as pl
+import plain_scalar as ps
 from bitwise_amd.csrc import ops
 
 pytestmark = pytest.mark.gpu
@@ -85,7 +86,7 @@ def test_gemm_f32_grid_rows_and_accumulate(gpu):
     ops.gemm_f32(x, wb, batch, 9, accumulate=True)
     assert torch.equal(batch, before + before)                     # y + acc, one addition per output
     # prompt portions (64 x 64 tiles on the matrix cores, or on the vector units where K is no multiple of 32): a row's bits are those of the row alone
-    # (and 17 to 64 rows: the chain-per-thread kernel with two or four blocks of rows)
+    # (and 17 to 64 rows: the chain-per-thread kernel with two or four blocks of rows, and strips on the matrix cores)
     for M, N, K in [(150, 200, 1024), (129, 130, 64), (300, 77, 48), (70, 140, 1000), (40, 130, 1024), (20, 77, 264),
                     (64, 50, 136), (33, 16, 8)]:
         x, w = torch.randn(M, K, generator=g).to(gpu), torch.randn(N, K, generator=g).to(gpu)
@@ -99,9 +100,9 @@ def test_gemm_f32_grid_rows_and_accumulate(gpu):
             before = batch.clone()
             ops.gemm_f32(x, weight, batch, M, accumulate=True)
             assert torch.equal(batch, before + before)
-    # many columns and up to 16 rows (a wave a row, weights packed in LDS; up to 8 rows with loader waves and the row
-    # four elements a register): the bits of the same rows inside a product of 20 rows (matrix cores) and of the
-    # chain-per-thread kernel (K + 8 is no whole stage of the first)
+    # many columns and up to 16 rows (chains with the row four elements a register, or tiles of 16 x 64 on the matrix cores; K = 96
+    # with bfloat16 weights, tiles of 64 x 64): the bits of the same rows inside a product of 20 rows (tiles of 32 x 32) and of the
+    # chain-per-thread kernel of the vector units (K + 8 is no whole stage of the others)
     for M, N, K in [(1, 16400, 64), (8, 16384, 2048), (16, 20000, 128), (5, 16385, 192), (13, 16500, 96), (3, 16390, 128),
                     (7, 16384, 320), (2, 17000, 64), (9, 16384, 64)]:
         x, w = torch.randn(20, K + 8, generator=g).to(gpu), (torch.randn(N, K + 8, generator=g) * 0.1).to(gpu)
@@ -139,7 +140,8 @@ def test_gemm_f32_prompt_products_reach_every_tile():
 @pytest.mark.parametrize("wdt", [torch.bfloat16, torch.float32])
 def test_gemm_f32_prompt_tiles_are_the_chains_of_few_rows(gpu, M, N, K, wdt):
     """Every tile shape of the 32-bit prompt products at the edges of its rows, columns and stages: the bits of the same rows
-    given sixteen at a time (the vector units' chains), written or added, from rows farther apart than they are long."""
+    given sixteen at a time (K a multiple of 64: on the matrix cores too; of 32 only: the vector units' chains, or tiles of 64 x 64),
+    written or added, from rows farther apart than they are long; and some rows and columns against the scalar std::fma program."""
     g = torch.Generator(device=gpu).manual_seed(M + N + K)
     wide = torch.randn(M, K + 12, generator=g, device=gpu)
     x, w = wide[:, :K], torch.randn(N, K, generator=g, device=gpu).to(wdt)
@@ -150,6 +152,9 @@ def test_gemm_f32_prompt_tiles_are_the_chains_of_few_rows(gpu, M, N, K, wdt):
         ops.gemm_f32(x[r:r + n], w, want[r:r + n], n)
     got = torch.empty(M, N, device=gpu)
     ops.gemm_f32(x, w, got, M)
+    some, columns = sorted({0, 15, 16, M // 2, M - 17, M - 1}), sorted({*range(0, N, 61), N - 1})
+    scalar = ps.linear(x[some].contiguous().cpu().numpy(), w[columns].float().cpu().numpy())
+    assert np.array_equal(got[some][:, columns].cpu().numpy().view(np.uint32), scalar.view(np.uint32))
     base = torch.randn(M, N, generator=g, device=gpu)
     added = base.clone()
     ops.gemm_f32(x, w, added, M, accumulate=True)
