@@ -43,10 +43,13 @@ int bw_gemm_f32(const float* x, const void* w, int w_is_bf16, float* y, int M, i
 int bw_gemm_f32_prompt_tile(int M, int N, int* rows, int* columns);
 int bw_gemm_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, int epilogue,
                  void* stream);
-// rows and rows of W of the tiles that a bfloat16 product of more than 64 rows gets where all of K is one workgroup's and the
-// kernels for few rows do not take it (K a multiple of 64; gated 1: the stacked weight of a gated epilogue, 2: the exact GELU)
-int bw_gemm_prompt_parts(int M, long long w_rows, int K, int gated, long long* first);
+// rows and rows of W of the tiles that are best for a bfloat16 product of more than 64 rows in one launch, where all of K is one
+// workgroup's and the kernels for few rows do not take it (K a multiple of 64; gated 1: the stacked weight of a gated epilogue, 2: the
+// exact GELU).  It goes so where bw_gemm_prompt_parts leaves 0
 int bw_gemm_prompt_tile(int M, long long w_rows, int K, int gated, int* rows, int* columns);
+// in two launches of tiles of two shapes: the rows of W (of both halves together, gated) of the first; 0: the product goes whole, as
+// one with the rotary epilogue always does
+int bw_gemm_prompt_parts(int M, long long w_rows, int K, int gated, long long* first);
 int bw_gemm_clamped_glu_bf16(const void* x, const void* w, void* out, int M, int N, int K, int ldx, int ldo, float limit,
                              float alpha, void* stream);
 // the same with the GELU (tanh form) of the gate instead of the clamped unit

@@ -506,19 +506,19 @@ def gemm_f32_prompt_tile(rows: int, N: int) -> Tuple[int, int]:
 
 
 def gemm_prompt_tile(rows: int, w_rows: int, K: int, gated: bool = False, erf: bool = False) -> Tuple[int, int]:
-    """(rows, rows of W) of the tiles that ``gemm_bf16`` gives a product of more than 64 rows, K in whole steps of 64, where
+    """(rows, rows of W) of the tiles that are best for a product of more than 64 rows in one launch, K in whole steps of 64, where
     all of K is one workgroup's and the kernels for few rows do not take it; ``gated``: of a gated epilogue, ``erf``: of the exact
-    GELU."""
+    GELU.  What ``gemm_bf16`` gives it unless ``gemm_prompt_parts`` sends it in two launches."""
     r, c = ctypes.c_int(0), ctypes.c_int(0)
     _check(_fn("bw_gemm_prompt_tile")(rows, w_rows, K, 2 if erf else int(gated), ctypes.addressof(r), ctypes.addressof(c)), "gemm_prompt_tile")
     return int(r.value), int(c.value)
 
 
-def gemm_prompt_parts(rows: int, w_rows: int, K: int, gated: bool = False) -> int:
+def gemm_prompt_parts(rows: int, w_rows: int, K: int, gated: bool = False, erf: bool = False) -> int:
     """Of a product that ``gemm_prompt_tile`` describes: how many rows of W go in tiles of a first launch, the others in tiles of another
-    shape; 0: the product goes whole."""
+    shape; 0: the product goes whole, as one with the rotary epilogue always does."""
     first = ctypes.c_longlong(0)
-    _check(_fn("bw_gemm_prompt_parts")(rows, w_rows, K, int(gated), ctypes.addressof(first)), "gemm_prompt_parts")
+    _check(_fn("bw_gemm_prompt_parts")(rows, w_rows, K, 2 if erf else int(gated), ctypes.addressof(first)), "gemm_prompt_parts")
     return int(first.value)
 
 

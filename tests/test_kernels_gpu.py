@@ -179,7 +179,8 @@ BF16_PROMPT_TILES = {       # tile -> products (M, rows of W, K) that the rule g
 def test_gemm_bf16_prompt_products_reach_every_tile():
     for tile, shapes in BF16_PROMPT_TILES.items():
         assert [ops.gemm_prompt_tile(M, N, K) for M, N, K in shapes] == [tile] * len(shapes)
-    assert ops.gemm_prompt_tile(1345, 8200, 64, gated=True) == (256, 256)
+        assert not any(ops.gemm_prompt_parts(M, N, K) for M, N, K in shapes)
+    assert ops.gemm_prompt_tile(1345, 8200, 64, gated=True) == (256, 256) and ops.gemm_prompt_parts(1345, 8200, 64, gated=True) == 0
     for M, K in ((64, 64), (65, 72)):
         with pytest.raises(RuntimeError, match="out of the kernel's range"):
             ops.gemm_prompt_tile(M, 200, K)

@@ -34,3 +34,36 @@ def test_both_launches_keep_the_bits(gpu, M, N, K, gated):
             want = base[r:r + n].clone()
             ops.gemm_bf16(x[r:r + n], w, want, n, epi)
             assert torch.equal(got[r:r + n], want), (epi, r)
+
+
+@pytest.mark.parametrize("M,N,K", [(514, 22414, 512), (641, 22343, 512), (961, 19014, 1024), (911, 16396, 2048)])
+def test_exact_gelu_of_both_launches(gpu, M, N, K):
+    assert 0 < ops.gemm_prompt_parts(M, N, K, erf=True) < N
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    x = torch.randn(M, K + 16, generator=g, device=gpu).bfloat16()[:, :K]
+    w = (torch.randn(N, K, generator=g, device=gpu) * K ** -0.5).bfloat16()
+    got, sums = torch.zeros(M, N, device=gpu, dtype=torch.bfloat16), torch.zeros(M, N, device=gpu)
+    ops.gemm_bf16(x, w, got, M, ops.EPI_GELU_BF16)
+    for r in range(0, M, 16):
+        n = min(16, M - r)
+        ops.gemm_bf16(x[r:r + n], w, sums[r:r + n], n, ops.EPI_F32)
+    want = torch.zeros_like(got)
+    ops.activate(sums, want, M, ops.PLAIN_GELU_ERF)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M,N,K", [(518, 10962, 512), (642, 11141, 512), (395, 11323, 2112), (1287, 5927, 2048), (777, 14336, 4096)])
+def test_other_gated_epilogues_of_both_launches(gpu, M, N, K):
+    assert 0 < ops.gemm_prompt_parts(M, 2 * N, K, gated=True) < 2 * N
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    x = torch.randn(M, K + 16, generator=g, device=gpu).bfloat16()[:, :K]
+    w = (torch.randn(2 * N, K, generator=g, device=gpu) * 3 * K ** -0.5).bfloat16()
+    sums = torch.zeros(M, 2 * N, device=gpu)
+    for r in range(0, M, 16):
+        n = min(16, M - r)
+        ops.gemm_bf16(x[r:r + n], w, sums[r:r + n], n, ops.EPI_F32)
+    for act, entry, more in ((ops.ACT_CLAMPED_SWISH, "bw_gemm_clamped_glu_bf16", (1.5, 1.702)), (ops.ACT_GELU_TANH, "bw_gemm_gelu_glu_bf16", ())):
+        want, got = torch.zeros(M, N, device=gpu, dtype=torch.bfloat16), torch.full((M + 1, N), 7.0, device=gpu, dtype=torch.bfloat16)
+        ops.glu(sums, want, M, act, **({"limit": 1.5, "alpha": 1.702} if more else {}))
+        assert ops._fn(entry)(x.data_ptr(), w.data_ptr(), got.data_ptr(), M, N, K, x.stride(0), N, *more, ops._stream()) == 0
+        assert torch.equal(got[:M], want) and bool((got[M] == 7.0).all()), act

@@ -68,7 +68,7 @@ def store(entry, x, w, M, N, dtype, pad, *more):
 @pytest.mark.parametrize("tile", list(STORED))
 def test_stores_and_adds_row_by_row(gpu, tile):
     M, N, K = STORED[tile]
-    assert ops.gemm_prompt_tile(M, N, K) == tile
+    assert ops.gemm_prompt_tile(M, N, K) == tile and ops.gemm_prompt_parts(M, N, K) == 0
     x, w, g = operands(gpu, M, N, K)
     want = by_sixteen(x, w, torch.zeros(M, N, device=gpu), ops.EPI_F32)
     got = store("bw_gemm_bf16", x, w, M, N, torch.float32, 4, ops.EPI_F32)
@@ -89,7 +89,7 @@ def test_stores_and_adds_row_by_row(gpu, tile):
 @pytest.mark.parametrize("tile", list(STORED))
 def test_exact_gelu_of_every_tile(gpu, tile):
     M, N, K = STORED[tile]
-    assert ops.gemm_prompt_tile(M, N, K, erf=True) == tile
+    assert ops.gemm_prompt_tile(M, N, K, erf=True) == tile and ops.gemm_prompt_parts(M, N, K, erf=True) == 0
     x, w, _ = operands(gpu, M, N, K)
     sums = by_sixteen(x, w, torch.zeros(M, N, device=gpu), ops.EPI_F32)
     want = torch.zeros(M, N, device=gpu, dtype=torch.bfloat16)
@@ -100,7 +100,7 @@ def test_exact_gelu_of_every_tile(gpu, tile):
 @pytest.mark.parametrize("tile,M,N,K", [(t, *s) for t, shapes in GATED.items() for s in shapes])
 def test_gated_epilogues_of_every_tile(gpu, tile, M, N, K):
     """SwiGLU, the clamped unit and the gated GELU: stores of 16 bytes (rows of whole pieces) and element by element."""
-    assert ops.gemm_prompt_tile(M, 2 * N, K, gated=True) == tile
+    assert ops.gemm_prompt_tile(M, 2 * N, K, gated=True) == tile and ops.gemm_prompt_parts(M, 2 * N, K, gated=True) == 0
     x, w, _ = operands(gpu, M, 2 * N, K)
     w = w * 3.0                                                     # (sums large enough for the clamps to bite)
     sums = by_sixteen(x, w, torch.zeros(M, 2 * N, device=gpu), ops.EPI_F32)
@@ -121,7 +121,7 @@ def test_gated_epilogues_of_every_tile(gpu, tile, M, N, K):
 def test_gated_epilogues_pass_on_infinities_and_nan(gpu):
     """Sums that are infinite or no number, and gates of every size, through the epilogues themselves."""
     M, N, K = 581, 8264, 64
-    assert ops.gemm_prompt_tile(M, 2 * N, K, gated=True) == (256, 256)
+    assert ops.gemm_prompt_tile(M, 2 * N, K, gated=True) == (256, 256) and ops.gemm_prompt_parts(M, 2 * N, K, gated=True) == 0
     x, w, _ = operands(gpu, M, 2 * N, K, apart=0)
     x, w = x.contiguous(), w.contiguous()
     x[3], x[40], x[300, 5], x[301, 6], x[580] = float("inf"), float("nan"), 3e38, -3e38, 1e20
