@@ -542,3 +542,50 @@ def test_gelu_unit_takes_rows_of_a_wider_matrix(gpu):
         ops.gemm_gelu_glu_bf16(wide.T[:200], w[:, :200].contiguous(), got, 200)
     with pytest.raises(RuntimeError):
         ops.gemm_gelu_glu_bf16(wide[:, 3:195], w, got, 200)          # (16-byte loads: not from any column)
+
+
+# ----------------------------------------------------------------------------- memories walked in stages
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_portions_on_both_sides_of_the_stages(tmp_path, gpu, dtype, monkeypatch):
+    """Heads of 64 and of 128 channels with given decays and with scalar gates, whose long portions are walked in stages: a request's
+    logits have the same bits however its portions fall on either side of the rule, alone and beside other requests, and its memory
+    goes from stages to the walk and back."""
+    from bitwise_amd.csrc import ops
+    from bitwise_amd.parts import recurrent
+
+    cfg = config(96, 61, 1e-5, [gla(2, 64, 16, 8.0, 6, 64), mlstm(1, 128, 24, 12.0, None), gla(1, 128, 8, 4.0, 3, None), mlstm(3, 64, 8, 8.0, 48)])
+    folder = bw.write_random_model(tmp_path / "staged", cfg, 23, SIGMA)
+    g = torch.Generator().manual_seed(5)
+    toks, other = (torch.randint(0, 61, (n,), generator=g).tolist() for n in (201, 90))
+    seen = []
+    real = ops.linear_recurrence
+
+    def note(mode, *args, **kw):
+        seen.append((mode, kw["in_stages"]))
+        if mode == ops.RECUR_SCALAR_GATES:
+            assert (kw["gates"] is not None) == kw["in_stages"]
+        return real(mode, *args, **kw)
+
+    monkeypatch.setattr(ops, "linear_recurrence", note)
+    rp = replayer(str(folder), dtype, 640, use_graphs=False)
+    whole = run_cut(rp, "whole", toks, [201])
+    assert close(whole, pk.forward(cfg, weights(folder), toks, rnd=RND[dtype]).numpy(), dtype)
+    assert set(seen) == {(ops.RECUR_DECAY_GIVEN, True), (ops.RECUR_SCALAR_GATES, True)}
+    for k, cuts in enumerate(([63, 138], [64, 137], [79, 122], [80, 121], [40, 65, 96], [100, 1, 2, 80], [3, 150], [20] * 10)):
+        seen.clear()
+        assert np.array_equal(run_cut(rp, f"r{k}", toks, cuts).view(np.uint32), whole.view(np.uint32)), cuts
+        staged = {s for _, s in seen}
+        assert staged == ({False} if max(cuts) < 64 else {True} if min(cuts) >= 80 else {True, False}), cuts
+    # two portions in one step, one long and one short, then single tokens beside a portion that is long and one that is not
+    alone = run_cut(rp, "other", other, [90])
+    lg = [rp.step([{"id": "a", "tokens": toks[:100], "want": list(range(100))}, {"id": "b", "tokens": other[:7], "want": list(range(7))}]),
+          rp.step([{"id": "b", "tokens": other[7:89], "want": list(range(82))}, {"id": "a", "tokens": toks[100:101], "want": [0]}]),
+          rp.step([{"id": "b", "tokens": other[89:], "want": [0]}, {"id": "a", "tokens": toks[101:], "want": list(range(100))}], ["a", "b"])]
+    a = np.concatenate([lg[0][:100], lg[1][82:], lg[2][1:]])
+    b = np.concatenate([lg[0][100:], lg[1][:82], lg[2][:1]])
+    assert np.array_equal(a.view(np.uint32), whole.view(np.uint32)) and np.array_equal(b.view(np.uint32), alone.view(np.uint32))
+    # with portions that the rule leaves to the walk: the same bits again
+    monkeypatch.setattr(recurrent, "in_stages", lambda *a: False)
+    assert np.array_equal(run_cut(rp, "walked", toks, [201]).view(np.uint32), whole.view(np.uint32))
+    assert rp.manager.all_free()
