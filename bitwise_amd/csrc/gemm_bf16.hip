@@ -293,7 +293,8 @@ static long long add_join_time(int M, int N, int S) { return (8LL * S + 8) * M *
 // for: the weights' way from memory takes the time there, not the matrix cores, and the times below do not see it (33 products of 129
 // to 192 rows, 4096 to 8192 columns and K of 4096 to 14336, every shape timed, split and whole: by the count four take more than 5 %
 // longer than the best, up to 27 %; by the times ten, up to 18 %).  More rows: the shape that takes less time than all of K a
-// workgroup; -1: none does (204 products of up to 2,048 rows: 0.8 % from the best in the mean).
+// workgroup in one launch (not in the two that ring_parts might make of it); -1: none does (204 products of up to 2,048 rows: 0.8 %
+// from the best in the mean).
 static int add_split_shape(int M, int N, int K) {
   const int S = (K + GEMM_SEG - 1) / GEMM_SEG;
   if (M <= 192) {

@@ -335,8 +335,8 @@ __global__ __launch_bounds__(256) void gemm_f32_rows_kernel(const float* __restr
 
 // ------------------------------------------------------------------------------ a wave a row, the row four elements a register
 
-// Few rows of many columns (f32_by_chains): a wave is a row and 64 columns, lane l the chain of (row, column n0 + l); weights and rows travel from
-// memory straight into an LDS ring (buffer loads with LDS as destination: 8 rows of W, 128 bytes each, or 4 rows of x, 256
+// Few rows of many columns (f32_by_chains): a wave is a row and 64 columns, lane l the chain of (row, column n0 + l); weights and
+// rows travel from memory straight into an LDS ring (buffer loads with LDS as destination: 8 rows of W, 128 bytes each, or 4 rows of x, 256
 // bytes each, an instruction; whole cache lines, the 16-byte chunks of a row of W permuted against bank conflicts; a ring of
 // stages, waits by counting loads).  The weights stay packed there: a lane reads its column's 16-byte chunks and widens them in
 // registers.  x[row][k] is the same number for every lane of the wave; read as such from LDS it costs what any read costs.  Here lane

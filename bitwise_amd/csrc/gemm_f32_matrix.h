@@ -15,8 +15,10 @@
 
 // Workgroups of WR x WC working waves, each with RB x CB blocks of 16 x 16 outputs, and LW waves that only load (none: every wave
 // loads its share).  x and W (as it is in memory) travel straight into a ring of ST stages of KB steps of k; a lane reads its
-// elements one at a time, sixteen rows' in distinct banks, and bfloat16 ones are widened in registers: RB matrix instructions
-// for every shift.  The row blocks are shared out evenly over the row tiles (450 rows are 29 blocks: four tiles of seven or eight, not
+// elements one at a time, and bfloat16 ones are widened in registers: RB matrix instructions for every shift.  (Sixteen rows' elements
+// are in distinct ones of 64 banks, but two rows each share one of 32, and every such read is replayed once: SQ_LDS_BANK_CONFLICT is half
+// of SQ_LDS_IDX_ACTIVE in all tiles.  In those of 128 x 128 that is under matrix instructions that are at work all the time; in those
+// of 16 x 64, 8 rows of 16384 x 2048, LDS is at work for 8 of 17 us, half of that replays.)  The row blocks are shared out evenly over the row tiles (450 rows are 29 blocks: four tiles of seven or eight, not
 // three of eight and one of five), and a block without rows costs nothing.
 // Against the kernels before it (one step of k an instruction: 16x16x1, 32x32x1 and 4x4x1), bfloat16 weights, us:
 //   rows   16384 x 2048   6144 x 2048   2048 x 8192   2048 x 2048      (columns x K)
@@ -43,7 +45,7 @@ struct F32KShape {
 };
 
 // Which 16-byte chunk of a row of BYTES lies in slot 0: sixteen rows' equal chunks (of bfloat16: halves of chunks) then lie in
-// different banks.
+// different ones of 64 banks.
 template <int BYTES>
 __device__ __forceinline__ int f32k_swizzle(int row) {
   if constexpr (BYTES == 64) return (row >> 2) & 3;
