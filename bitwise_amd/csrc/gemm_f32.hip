@@ -561,6 +561,8 @@ static bool f32_by_chains(int M, int N, int K, bool bf16) {
   if (M == 1) return true;
   if (bf16) return M == 2 ? K <= 512 || (blocks >= 1024 && K <= 1536) : M <= 4 && K <= 128;
   if (K <= 256) return true;
+  // (no whole stages of 64: the other way is tiles of 64 x 64, whatever the rows; 8 rows of 39,549 columns, K = 1824, 59 and 53 us, 65,000 82 and 88)
+  if (K % 64 != 0 && K > 1024 && (blocks == 256 || (blocks >= 600 && blocks % 256 <= 230))) return true;
   if (M > 4) return blocks >= 600 && K <= 1024;
   // (more than 1,024 steps of k: where the tiles' last round is not a full one)
   return blocks > 256 && (K <= 1024 || (blocks % 256 >= 1 && blocks % 256 <= 230));

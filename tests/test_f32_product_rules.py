@@ -10,7 +10,8 @@ CHAINS = [(False, 2, 16321, 64, 3.9, 3.3), (False, 4, 16321, 1024, 12.7, 13.9), 
           (False, 4, 24000, 1024, 25.5, 24.0), (False, 2, 32768, 4096, 99.8, 119.4), (False, 8, 24000, 512, 13.1, 14.3),
           (False, 8, 65000, 256, 18.5, 15.5), (False, 6, 65000, 512, 31.4, 27.2), (False, 2, 100000, 64, 16.9, 9.2), (True, 2, 24000, 64, 4.4, 3.8),
           (True, 2, 100000, 1024, 42.6, 38.7), (True, 4, 100000, 64, 10.7, 9.7), (True, 4, 24000, 2048, 24.0, 25.2),
-          (True, 8, 24000, 1024, 15.0, 22.4), (True, 8, 65000, 2048, 45.6, 90.3)]
+          (True, 8, 24000, 1024, 15.0, 22.4), (True, 8, 65000, 2048, 45.6, 90.3), (False, 2, 16384, 1824, 29.3, 24.4),
+          (False, 8, 39549, 1824, 59.3, 53.2), (False, 6, 49152, 1056, 43.3, 39.2), (False, 8, 65000, 1824, 82.4, 88.0)]
 
 
 @pytest.mark.parametrize("bf16,rows,columns,K,tiles,chains", CHAINS)

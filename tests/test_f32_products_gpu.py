@@ -21,6 +21,7 @@ SHAPES = [
     (33, 16384, 64), (64, 16400, 192), (17, 50, 96), (40, 200, 32), (5, 16390, 96),
     # chains: up to eight rows of many columns (two to eight with 32-bit weights, some with bfloat16 ones)
     (1, 16385, 128), (1, 16321, 704), (2, 16385, 64), (3, 16330, 128), (4, 16449, 1024), (5, 16400, 256), (7, 16385, 96), (8, 16390, 192),
+    (3, 16384, 1056),
 ]
 
 
