@@ -114,7 +114,7 @@ def build(force: bool = False, verbose: bool = True) -> Path:
         objs = list(pool.map(compile_one, SOURCES))
     tmp_lib = out_dir / (LIB_NAME + f".tmp{os.getpid()}")
     # -z defs: a kernel template that the host pass failed to instantiate (it can do so without a
-    # word) leaves an undefined symbol; better the link fails here than the load on the GPU box
+    # word) leaves an undefined symbol; better the link fails here than the load on a machine with a GPU
     p = subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,-z,defs", "-o", str(tmp_lib), *objs],
                        capture_output=True, text=True, env=env)
     if p.returncode != 0:

@@ -18,8 +18,9 @@
 // elements one at a time, and bfloat16 ones are widened in registers: RB matrix instructions for every shift.  (Sixteen rows' elements
 // are in distinct ones of 64 banks, but two rows each share one of 32, and every such read is replayed once: SQ_LDS_BANK_CONFLICT is half
 // of SQ_LDS_IDX_ACTIVE in all tiles.  In those of 128 x 128 that is under matrix instructions that are at work all the time; in those
-// of 16 x 64, 8 rows of 16384 x 2048, LDS is at work for 8 of 17 us, half of that replays.)  The row blocks are shared out evenly over the row tiles (450 rows are 29 blocks: four tiles of seven or eight, not
-// three of eight and one of five), and a block without rows costs nothing.
+// of 16 x 64, 8 rows of 16384 x 2048, LDS is at work for 8 of 17 us, half of that replays.)
+// The row blocks are shared out evenly over the row tiles (450 rows are 29 blocks: four tiles of seven or eight, not three of eight
+// and one of five), and a block without rows costs nothing.
 // Against the kernels before it (one step of k an instruction: 16x16x1, 32x32x1 and 4x4x1), bfloat16 weights, us:
 //   rows   16384 x 2048   6144 x 2048   2048 x 8192   2048 x 2048      (columns x K)
 //    452    334 -> 247      119 -> 97     190 -> 134     54 -> 39
@@ -235,7 +236,8 @@ __global__ __launch_bounds__(64 * (WR * WC + LW)) void gemm_f32_tiles_kernel(con
   using S = F32KShape<WT, RB, CB, WR, WC, KB, ST, LW>;
   extern __shared__ __attribute__((aligned(16))) unsigned char f32k_ring[];
   const int wave = wave_index(), lane = threadIdx.x & 63;
-  // the row tiles of a column tile run one after the other on one die: its weights come from memory once
+  // the row tiles of a column tile run one after the other on one die: its weights come from memory once (where the workgroups divide
+  // by the dies; other grids are dealt as they come, and a column tile's weights go to several dies)
   int bid = blockIdx.x;
   if (gridDim.x % 8 == 0) bid = (bid % 8) * (gridDim.x / 8) + bid / 8;
   const int blocks = (M + 15) / 16, tile = bid % row_tiles;
