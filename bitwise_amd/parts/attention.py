@@ -23,6 +23,14 @@ from .linear import Linear
 # own once its context is at least this long (same bits either way; this only buys parallelism).
 DECODE_MIN_CONTEXT = 128
 
+# Beside a prompt portion all single tokens of a step go into the portion's launch, as tiles of one row, if none of them walks
+# more 64-key partitions than the longest of the portion's rows does, and this many: a launch of its own costs what a dozen partitions
+# take there, and the portion's longest workgroups leave room beside them.  Heads of 64 and 128, microseconds, two launches -> one: 1,341 tokens at
+# 640 and 7 singles of up to 592 keys (32 heads of 64) 50.6 -> 39.9; 854 tokens and 60 of up to 1,186 (32 heads of 128 on 8) 74.5 -> 53.3; 65 tokens and 22 of
+# up to 416 19.1 -> 13.6.  80 drawn mixes: ten partitions more 0.63 to 1.02 of the time, 15 more 1.05 to 1.08, 35 more 1.8.
+JOIN_PARTITIONS = 8
+PARTITION = 64
+
 
 @dataclass
 class AttentionPlan:
@@ -33,21 +41,36 @@ class AttentionPlan:
     decode_count: int
 
 
-def plan_tiles(ctx, tokens_per_tile: int, group_tiles: int = 1) -> AttentionPlan:
+def _partitions(pos: int, window: int, chunk: int) -> int:
+    """64-key partitions that the query at ``pos`` walks."""
+    first = pos - pos % chunk if chunk else max(0, pos - window + 1) if window else 0
+    return pos // PARTITION - first // PARTITION + 1
+
+
+def plan_tiles(ctx, tokens_per_tile: int, group_tiles: int = 1, join: bool = False, window: int = 0, chunk: int = 0) -> AttentionPlan:
     """Cut a step's segments into tiles of up to ``tokens_per_tile`` consecutive rows of one request; every
     request's run of tiles is padded with empty tiles to a multiple of ``group_tiles`` (the tiles one wave owns
     must belong to one request).  Single decoded tokens with a long context go to the decode kernel (a wave per
     64-key partition).  A step of nothing but one row per request (``ctx.one_row_per_request``, the shape of a
-    captured decode step) needs no tile list: tile t is row t of request t.  The plan is made once per step
+    captured decode step) needs no tile list: tile t is row t of request t.  ``join``: single tokens may go into the
+    portions' launch (JOIN_PARTITIONS), with the layer's ``window`` or ``chunk``.  The plan is made once per step
     and kept in the context for the other layers."""
     if getattr(ctx, "one_row_per_request", False):
         return AttentionPlan(None, 0, None, ctx.rows)
 
     def make() -> AttentionPlan:
         fold, split = [], []
-        for i, s in enumerate(ctx.segments):
+        singles = [i for i, s in enumerate(ctx.segments) if len(s.tokens) == 1]
+        longest = max((_partitions(s.pos0 + len(s.tokens) - 1, window, chunk) for s in ctx.segments if len(s.tokens) > 1), default=0)
+        joined = join and longest > 0 and all(_partitions(ctx.segments[i].pos0, window, chunk) <= longest + JOIN_PARTITIONS for i in singles)
+        # (the kernel starts a list's last tiles first: the singles, the shortest in front, start behind the portions)
+        order = range(len(ctx.segments))
+        if joined:
+            order = sorted(singles, key=lambda i: ctx.segments[i].pos0) + [i for i in order if len(ctx.segments[i].tokens) > 1]
+        for i in order:
+            s = ctx.segments[i]
             n, r0 = len(s.tokens), ctx.seq_start[i]
-            if n == 1 and s.pos0 + 1 >= DECODE_MIN_CONTEXT:
+            if n == 1 and not joined and s.pos0 + 1 >= DECODE_MIN_CONTEXT:
                 split.append((r0, 1, i, 0))
                 continue
             for off in range(0, n, tokens_per_tile):
@@ -60,7 +83,7 @@ def plan_tiles(ctx, tokens_per_tile: int, group_tiles: int = 1) -> AttentionPlan
         return AttentionPlan(dev[:len(fold)].contiguous() if fold else None, len(fold),
                              dev[len(fold):].contiguous() if split else None, len(split))
 
-    return ctx.memo(("attention_tiles", tokens_per_tile, group_tiles), make)
+    return ctx.memo(("attention_tiles", tokens_per_tile, group_tiles, join, window, chunk), make)
 
 
 def _split_scratch(ws, tiles: int, table_width: int, heads: int, kv_heads: int, head_dim: int):
@@ -99,7 +122,9 @@ def attend_bf16(ctx, call, q, out, heads: int, kv_heads: int, head_dim: int, win
     table = ctx.block_tables[call.group]
     extra = _mask_and_cap(sink, chunk, softcap)
     tokens_per_tile = 16 // min(heads // kv_heads, 16)
-    plan = plan_tiles(ctx, tokens_per_tile, ops.fold_group_tiles(head_dim))
+    # (the sizes whose fold kernel is the fast one)
+    join = head_dim in (64, 128) and ws.page_size >= 16
+    plan = plan_tiles(ctx, tokens_per_tile, ops.fold_group_tiles(head_dim), join, window, chunk)
     common = (call.k_cache, call.v_cache, out, heads, kv_heads, head_dim, ws.page_size, window, scale)
     if plan.fold_count:
         ops.attention_bf16(q, ctx.positions, table, plan.fold_tiles, plan.fold_count, *common, **extra)

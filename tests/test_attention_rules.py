@@ -1,8 +1,14 @@
-"""How many waves a workgroup of 32-bit decode attention gets: host code, held against both forms' measured times."""
+"""How many waves a workgroup of 32-bit decode attention gets, held against both forms' measured times; and which rows of a step
+the bfloat16 kernels treat together: host code."""
+
+from types import SimpleNamespace
 
 import pytest
+import torch
 
 from bitwise_amd.csrc import ops
+from bitwise_amd.engine.batch import Segment, StepContext
+from bitwise_amd.parts.attention import JOIN_PARTITIONS, plan_tiles
 
 # head size, workgroups, keys (and the most of them), microseconds in four waves, in eight
 MEASURED = [(16, 64, 2400, 44.1, 33.1), (16, 256, 200, 10.3, 8.7), (16, 400, 200, 11.5, 15.1), (16, 2400, 2400, 229.8, 338.6),
@@ -20,3 +26,34 @@ def test_the_form_that_is_taken_is_the_faster_one(head_dim, workgroups, keys, fo
 def test_heads_without_a_kernel_of_four_waves_get_eight():
     for head_dim in (32, 48, 64, 80, 96, 112, 128):
         assert {ops.attention_f32_waves(head_dim, n, c) for n in (1, 256, 257, 60000) for c in (1, 64, 65, 30000)} == {8}
+
+
+def tiles_of(rows, window=0, chunk=0, tokens=4, group=8, join=True):
+    """Plan of requests given as (position of the first row, rows): (fold tiles, decode tiles) as lists, and the context."""
+    segments = [Segment([0] * n, pos, [list(range((pos + n + 15) // 16))], i) for i, (pos, n) in enumerate(rows)]
+    ctx = StepContext(segments, 1, SimpleNamespace(device=torch.device("cpu"), page_size=16))
+    plan = plan_tiles(ctx, tokens, group, join, window, chunk)
+    return [[] if t is None else t.tolist() for t in (plan.fold_tiles, plan.decode_tiles)], ctx
+
+
+PORTION = 64 * 4          # walks 4 partitions at its last row
+EDGE = 64 * (4 + JOIN_PARTITIONS)
+
+
+@pytest.mark.parametrize("rows,window,chunk,joined", [
+    ([(0, PORTION), (EDGE - 1, 1)], 0, 0, True), ([(0, PORTION), (EDGE, 1)], 0, 0, False),
+    ([(EDGE - 1, 1), (0, PORTION), (5, 1), (200, 1)], 0, 0, True), ([(200, 1), (0, PORTION), (EDGE + 7, 1)], 0, 0, False),
+    ([(0, 17), (0, PORTION), (300, 1)], 0, 0, True), ([(9000, 1), (0, PORTION)], 100, 0, True), ([(9000, 1), (0, PORTION)], 64 * 13, 0, False),
+    ([(9000, 1), (0, PORTION)], 0, 256, True), ([(300, 1), (10, 1)], 0, 0, False), ([(300, 1)], 0, 0, False), ([(0, PORTION)], 0, 0, True)])
+def test_single_tokens_join_a_portion_whose_walk_is_about_as_long(rows, window, chunk, joined):
+    (fold, decode), ctx = tiles_of(rows, window, chunk)
+    single = {ctx.seq_start[i] for i, s in enumerate(ctx.segments) if len(s.tokens) == 1 and s.pos0 + 1 >= 128}
+    assert {t[0] for t in decode} == (set() if joined else single)
+    # every row of the step is in one tile, a group of tiles is one request's, and the singles stand in front, the shortest first
+    rows_seen = sorted(r for t in fold + decode for r in range(t[0], t[0] + t[1]))
+    assert rows_seen == list(range(ctx.rows)) and len(fold) % 8 == 0
+    for g in range(0, len(fold), 8):
+        assert len({t[2] for t in fold[g:g + 8]}) == 1
+    if joined:
+        lone = [ctx.segments[t[2]].pos0 for t in fold if t[1] and len(ctx.segments[t[2]].tokens) == 1]
+        assert lone == sorted(lone) and all(len(ctx.segments[t[2]].tokens) == 1 for t in fold[:8 * len(lone)])

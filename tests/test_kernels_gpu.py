@@ -1021,6 +1021,35 @@ def test_prompt_attention_of_common_heads_equals_the_decode_kernel(gpu, heads, k
                 assert (outs[0].cpu().double() - ref).abs().max() <= 2.0 ** -7 * v.double().abs().max()
 
 
+@pytest.mark.parametrize("heads,kvh,hd,page", [(2, 2, 64, 16), (6, 2, 64, 32), (4, 1, 128, 16), (17, 1, 128, 64)])
+def test_single_tokens_in_a_portions_launch_equal_the_decode_kernel(gpu, heads, kvh, hd, page):
+    """Tiles of one row beside a portion's, as a step of both gives them to the fold kernel: the bits of the decode kernel, for the
+    first and last slots of pages and partitions, with dead slots full of NaN, windows, chunks and a sink."""
+    n_keys = 700
+    k, v, kc, vc, tab = paged_setup(gpu, True, heads, kvh, hd, page, 74 if page == 16 else 41, n_keys, seed=heads + hd, poison=True)
+    g = torch.Generator().manual_seed(page + hd)
+    sink = torch.randn(heads, generator=g).to(gpu)
+    group, tpt = ops.fold_group_tiles(hd), 16 // min(heads // kvh, 16)
+    singles = [0, 15, 16, 63, 64, 127, 128, 500, 639, 640, 699]
+    first, rows = 100, 5 * tpt + 3
+    positions = singles + list(range(first, first + rows))
+    q = torch.randn(len(positions), heads * hd, generator=g).to(torch.bfloat16).to(gpu)
+    pos = torch.tensor(positions, dtype=torch.int32, device=gpu)
+    tiles = []
+    for i in range(len(singles)):
+        tiles += [(i, 1, 0, 0)] + [(i, 0, 0, 0)] * (group - 1)
+    tiles += [(len(singles) + off, min(tpt, rows - off), 0, 0) for off in range(0, rows, tpt)]
+    tiles += [(0, 0, 0, 0)] * (-len(tiles) % group)
+    for window, extra in ((0, {}), (70, {}), (0, {"chunk": 48}), (0, {"sink": sink})):
+        outs = []
+        for decode, ts in ((False, tiles), (True, [(r, 1, 0, 0) for r in range(len(positions))])):
+            out = torch.zeros(len(positions), heads * hd, device=gpu, dtype=torch.bfloat16)
+            ops.attention_bf16(q, pos, tab, torch.tensor(ts, dtype=torch.int32, device=gpu), len(ts), kc, vc, out, heads, kvh, hd, page,
+                               window, float(hd) ** -0.5, decode=decode, **extra)
+            outs.append(out)
+        assert torch.equal(outs[0], outs[1]), (window, extra)
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 def test_attention_finds_a_far_key_and_respects_the_window(gpu, bf16):
     """One key among hundreds is made to stand out by scaling it and the query: the output must
