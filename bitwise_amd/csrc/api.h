@@ -106,6 +106,8 @@ int bw_attention_fold_group_tiles(int head_dim);
 int bw_norm_gemm_supported(int M, int K);
 // rows wider than one 2048-segment of K: whether the fused norm + product kernel with ``cols`` columns a workgroup takes them
 int bw_norm_gemm_wide_supported(int M, int N, int K, int cols);
+// strips of 16 rows of W (SwiGLU: 8 outputs) a workgroup of it takes, a wave each; 0: not that kernel
+int bw_norm_gemm_strips(int M, int N, int K, int epilogue);
 int bw_norm_gemm_bf16(const float* x, int ldx, const void* norm_w, int norm_w_is_bf16, float eps, const void* w,
                       void* out, int ldo, int M, int N, int K, int epilogue, void* stream);
 int bw_norm_qkv_rope_bf16(const float* x, int ldx, const void* norm_w, int norm_w_is_bf16, float eps,

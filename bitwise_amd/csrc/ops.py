@@ -82,6 +82,7 @@ _SIGS = {
     "bw_attention_fold_group_tiles": [c_int],
     "bw_norm_gemm_supported": [c_int, c_int],
     "bw_norm_gemm_wide_supported": [c_int, c_int, c_int, c_int],
+    "bw_norm_gemm_strips": [c_int, c_int, c_int, c_int],
     "bw_norm_gemm_bf16": [c_void_p, c_int, c_void_p, c_int, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                           c_int, c_void_p],
     "bw_norm_qkv_rope_bf16": [c_void_p, c_int, c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -171,7 +172,7 @@ _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
     "bw_gemm_f32_by_chains", "bw_gemm_f32_swiglu_in_tiles", "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts",
     "bw_gemm_gelu_glu_wins", "bw_gemm_split_tile", "bw_gemm_split_rows", "bw_attention_f32_waves", "bw_fingerprint_waves",
-    "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_attention_decode_scratch",
+    "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_norm_gemm_strips", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
     "bw_chain_flush", "bw_chain_end",
 })
@@ -668,6 +669,11 @@ def can_fuse_norm(rows: int, weight: torch.Tensor, x: torch.Tensor, columns: int
     if not (weight.dtype == torch.bfloat16 and x.dtype == torch.float32 and x.shape[1] == K and x.stride(0) % 4 == 0):
         return False
     return norm_gemm_supported(rows, K) or norm_gemm_wide_supported(rows, weight.shape[0] // stacked, columns, K)
+
+
+def norm_gemm_strips(rows: int, columns: int, inner: int, epilogue: int) -> int:
+    """Strips of 16 rows of W (SwiGLU: of 8 outputs) that a workgroup of ``norm_gemm_bf16`` takes, a wave each; 0: another kernel runs it."""
+    return int(_fn("bw_norm_gemm_strips")(rows, columns, inner, epilogue))
 
 
 def norm_gemm_bf16(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w: torch.Tensor, out: torch.Tensor,

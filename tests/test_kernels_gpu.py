@@ -1216,6 +1216,29 @@ def test_fused_norm_products_equal_the_separate_kernels(gpu):
         assert torch.equal(outs[0][1], outs[1][1]) and torch.equal(outs[0][2], outs[1][2])
 
 
+@pytest.mark.parametrize("M,N,K,strips", [(1, 8208, 64, 6), (8, 8256, 512, 6), (16, 11000, 128, 7), (5, 11008, 2048, 7), (9, 14329, 192, 7), (8, 8200, 2560, 5),
+                                          (3, 14336, 4096, 7), (2, 16384, 2048, 8), (13, 16377, 1024, 8), (8, 18440, 4096, 5), (1, 24576, 2176, 6)])
+@pytest.mark.parametrize("glu", [True, False])
+def test_normalised_rows_by_strips_of_their_own_equal_the_separate_kernels(gpu, M, N, K, strips, glu):
+    """Products of more workgroups than compute units, a wave a strip: last strips and workgroups that are part empty, one to eight
+    rows and up to sixteen, K shorter than the ring, one segment and two; the bits of RMSNorm and product one after the other."""
+    g = torch.Generator().manual_seed(M + N + K)
+    columns = N if glu else 2 * N
+    epilogue = ops.EPI_SWIGLU_BF16 if glu else ops.EPI_F32
+    if glu:
+        assert ops.norm_gemm_strips(M, N, K, epilogue) == strips
+    x = (torch.randn(M, K, generator=g) * 2).to(gpu)
+    nw = (1 + 0.1 * torch.randn(K, generator=g)).bfloat16().to(gpu)
+    w = (torch.randn(2 * N, K, generator=g) * 0.05).bfloat16().to(gpu)
+    h = torch.zeros(M, K, device=gpu, dtype=torch.bfloat16)
+    ops.rmsnorm(x, nw, h, M, 1e-5)
+    kind = torch.bfloat16 if glu else torch.float32
+    sep, fused = torch.zeros(M, columns, device=gpu, dtype=kind), torch.full((M + 1, columns), 5.0, device=gpu, dtype=kind)
+    ops.gemm_bf16(h, w, sep, M, epilogue)
+    ops.norm_gemm_bf16(x, nw, 1e-5, w, fused, M, epilogue)
+    assert torch.equal(fused[:M], sep) and (fused[M] == 5.0).all()
+
+
 @pytest.mark.parametrize("heads,kvh,M,tile", [(71, 13, 300, (64, 128)), (101, 12, 250, (128, 64)), (71, 13, 384, (128, 128)),
                                               (72, 12, 700, (128, 256)), (71, 13, 1345, (160, 256)), (125, 17, 1000, (192, 256)),
                                               (71, 12, 2041, (256, 192)), (75, 11, 2041, (256, 256))])
