@@ -27,6 +27,12 @@ int bw_convert(const void* src, int src_is_bf16, void* dst, int dst_is_bf16, int
                void* stream);
 // whether bw_gemm_f32 runs so few rows as chains on the vector units rather than on the matrix cores (16-byte alignments given)
 int bw_gemm_f32_by_chains(int M, int N, int K, int w_is_bf16);
+// whether bw_gemm_f32_qkv_rope takes the stacked q|k|v product, which it leaves with q and k rotated, and k and v in their 32-bit page slots
+int bw_gemm_f32_rope_in_strips(const float* x, const void* w, int w_is_bf16, int M, int all_heads, int head_dim, int K, int ldx);
+int bw_gemm_f32_qkv_rope(const float* x, const void* w, int w_is_bf16, float* y, int M, int K, int ldx, int ldy, const int32_t* positions,
+                         const int32_t* row_seq, const int32_t* block_table, int table_stride, const float* cos_table,
+                         const float* sin_table, float* k_cache, float* v_cache, int heads, int kv_heads, int head_dim, int page_size,
+                         int write_cache, void* stream);
 // whether bw_gemm_f32_swiglu computes the activation in the product's epilogue (and leaves gate_up alone)
 int bw_gemm_f32_swiglu_in_tiles(const float* x, const void* w, int w_is_bf16, int M, int outputs, int K, int ldx);
 int bw_gemm_f32_swiglu(const float* x, const void* w, int w_is_bf16, float* gate_up, float* h, int M, int outputs, int K, int ldx,

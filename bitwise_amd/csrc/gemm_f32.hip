@@ -774,3 +774,30 @@ extern "C" int bw_gemm_f32_swiglu(const float* x, const void* w, int w_is_bf16, 
   }
   return BW_LAUNCH_CHECK();
 }
+
+// Whether bw_gemm_f32_qkv_rope takes the stacked product: up to 64 rows that go as strips, whole tiles of 16 pairs.
+extern "C" int bw_gemm_f32_rope_in_strips(const float* x, const void* w, int w_is_bf16, int M, int all_heads, int head_dim, int K, int ldx) {
+  const long long N = (long long)all_heads * head_dim;
+  if (M <= 0 || M > 64 || all_heads <= 0 || head_dim <= 0 || head_dim % 32 || K <= 0 || K % 64 || ldx < K || N > (1 << 28)) return 0;
+  const size_t limit = (size_t)1 << 31;                // (a tile's descriptors: 16 rows of x, a head's columns of W)
+  if (ldx % 4 || (((uintptr_t)x | (uintptr_t)w) & 15) || (size_t)64 * ldx * 4 >= limit || (size_t)head_dim * K * 4 >= limit) return 0;
+  return !f32_by_chains(M, (int)N, K, w_is_bf16 != 0) && f32_few_rows_kernel(M, (int)N, K) == F32_STRIPS;
+}
+
+// y = x W^T with q and k rotated and k and v in their page slots: the bits of bw_gemm_f32 followed by bw_rope_kvwrite on 32-bit
+// caches, in one kernel; -7: not this shape (bw_gemm_f32_rope_in_strips).
+extern "C" int bw_gemm_f32_qkv_rope(const float* x, const void* w, int w_is_bf16, float* y, int M, int K, int ldx, int ldy, const int32_t* positions,
+                                    const int32_t* row_seq, const int32_t* block_table, int table_stride, const float* cos_table,
+                                    const float* sin_table, float* k_cache, float* v_cache, int heads, int kv_heads, int head_dim, int page_size,
+                                    int write_cache, void* stream) {
+  if (M <= 0) return 0;
+  const int all_heads = heads + 2 * kv_heads, N = all_heads * head_dim;
+  if (page_size <= 0 || ldy < N || kv_heads <= 0 || heads <= 0) return -2;
+  if (!bw_gemm_f32_rope_in_strips(x, w, w_is_bf16, M, all_heads, head_dim, K, ldx)) return -7;
+  const F32RopeArgs ra{positions, row_seq, block_table, cos_table, sin_table, k_cache, v_cache,
+                       heads, kv_heads, head_dim, page_size, page_size & (page_size - 1) ? -1 : __builtin_ctz((unsigned)page_size), table_stride, write_cache};
+  hipStream_t s = (hipStream_t)stream;
+  if (w_is_bf16) launch_f32_strips<bf16_t, 2, 9, true>(x, (const bf16_t*)w, y, M, N, K, ldx, ldy, 0, s, ra);
+  else launch_f32_strips<float, 2, 9, true>(x, (const float*)w, y, M, N, K, ldx, ldy, 0, s, ra);
+  return BW_LAUNCH_CHECK();
+}

@@ -406,19 +406,41 @@ __device__ __forceinline__ void f32s_store(unsigned char* stage, const int (*at_
 }
 #endif
 
-template <typename WT, int WC, int D>
+// What rotation and cache write in the epilogue need (rope_kvwrite_kernel's arguments).
+struct F32RopeArgs {
+  const int32_t* positions;
+  const int32_t* row_seq;
+  const int32_t* block_table;
+  const float* cos_table;    // [positions, head_dim / 2]
+  const float* sin_table;
+  float* k_cache;
+  float* v_cache;
+  int heads, kv_heads, head_dim, page_size, page_shift, table_stride, write_cache;      // (page_shift: log2 of page_size, or -1)
+};
+
+// ROPE (two working waves): y is the stacked q|k|v product with q and k rotated, k and v also in their page slots: the statements of
+// rope_kvwrite_kernel, which as a launch of its own reads and writes the 32-bit sums once more.  A workgroup's columns are 16 pairs of
+// one head, first halves with one wave and second halves with the other, so that a lane's partner lies in the same lane of
+// the other wave.  Replayed as graphs, us, product and kernel -> one: 8 rows of 96 heads of 64, K = 2048, 15.1 -> 13.2 (the product alone
+// 12.0), 32-bit weights 19.4 -> 16.1; 8 rows of 48 heads of 128, K = 4096, 23.8 -> 22.4; 64 rows of 12 heads, K = 1024, 9.6 -> 8.2; 0.72 to 0.94 of
+// the time at 14 such products.
+template <typename WT, int WC, int D, bool ROPE>
 __global__ __launch_bounds__(64 * (WC + 2)) void gemm_f32_strips_kernel(const float* __restrict__ x, const WT* __restrict__ w, float* __restrict__ y, int M,
-                                                                       int N, int K, int ldx, int ldy, int accumulate, int row_tiles) {
+                                                                       int N, int K, int ldx, int ldy, int accumulate, int row_tiles, F32RopeArgs ra) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using S = F32SShape<WT, WC, D>;
   extern __shared__ __attribute__((aligned(16))) unsigned char f32s_lds[];
   const int wave = wave_index(), lane = threadIdx.x & 63;
-  const int m0 = 16 * ((int)blockIdx.x % row_tiles), n0 = ((int)blockIdx.x / row_tiles) * S::COLS;
+  static_assert(!ROPE || WC == 2, "a wave for the first halves of the pairs, one for the second");
+  const int m0 = 16 * ((int)blockIdx.x % row_tiles), tile = (int)blockIdx.x / row_tiles;
+  const int half = ROPE ? ra.head_dim >> 1 : S::COLS;                          // (a tile's second 16 columns are half a head behind its first)
+  const int head = ROPE ? tile / (half >> 4) : 0, pair0 = ROPE ? 16 * (tile % (half >> 4)) : 0;
+  const int n0 = ROPE ? head * ra.head_dim + pair0 : tile * S::COLS;
   const int steps = K / S::KB;
   if (wave >= WC) {
     // ---- a loading wave: runs of 8 k, lane l run l % 8 of row (column) l / 8 of its 8
     const int loader = wave - WC;
-    const int x_rows = min(16, M - m0), w_rows = min(S::COLS, N - n0);
+    const int x_rows = min(16, M - m0), w_rows = ROPE ? half + 16 : min(S::COLS, N - n0);   // (ROPE: whole tiles)
     const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(x + (size_t)m0 * ldx), 0, (int)((((size_t)x_rows - 1) * ldx + K) * sizeof(float)), 0x00020000);
     const __amdgpu_buffer_rsrc_t rs_w =
@@ -435,7 +457,7 @@ __global__ __launch_bounds__(64 * (WC + 2)) void gemm_f32_strips_kernel(const fl
 #pragma unroll
     for (int t = 0; t < S::WW; ++t) {
       const int row = (loader + t * S::LW) * (64 / S::RUNS) + lane / S::RUNS;
-      voff_w[t] = min(row, w_rows - 1) * K * (int)sizeof(WT) + run * 8 * (int)sizeof(WT);
+      voff_w[t] = (ROPE ? (row < 16 ? row : row - 16 + half) : min(row, w_rows - 1)) * K * (int)sizeof(WT) + run * 8 * (int)sizeof(WT);
 #pragma unroll
       for (int g = 0; g < 4; ++g) at_w[t][g] = S::XBYTES + (run >> 1) * S::WBLOCK + row * 64 + f32s_chunk(g, row, run >> 1) + 8 * (run & 1);
     }
@@ -469,6 +491,17 @@ __global__ __launch_bounds__(64 * (WC + 2)) void gemm_f32_strips_kernel(const fl
   }
   f32x4 acc[1][1] = {{{0.f, 0.f, 0.f, 0.f}}};
   f32x4 hx[2][2], hw[2][2];
+  int pos[4] = {-1, -1, -1, -1}, page[4] = {0, 0, 0, 0};
+  float cosine[4] = {}, sine[4] = {};
+  int seq[4] = {0, 0, 0, 0};
+  if constexpr (ROPE) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = min(m0 + 4 * g + i, M - 1);
+      pos[i] = ra.positions[m];
+      seq[i] = ra.row_seq[m];
+    }
+  }
   __builtin_amdgcn_s_barrier();                                                // stages 0 and 1 are there
   asm volatile("" ::: "memory");
 #pragma unroll
@@ -477,6 +510,19 @@ __global__ __launch_bounds__(64 * (WC + 2)) void gemm_f32_strips_kernel(const fl
     hx[0][i] = *reinterpret_cast<const f32x4*>(f32s_lds + i * S::XBLOCK + xa[i]);
   }
   for (int base = 0; base < steps; base += 3) {
+    if constexpr (ROPE) {
+      // what hangs on the positions is asked for once those are there for certain, a turn later (in front of the first stage the wait
+      // for them took 0.3 us a layer more)
+      if (base == (steps > 3 ? 3 : 0)) {                                       // scalar
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int at = max(pos[i], 0);                                       // (a padding row: the product as it is, whatever is loaded)
+          cosine[i] = ra.cos_table[(size_t)at * half + pair0 + row];
+          sine[i] = ra.sin_table[(size_t)at * half + pair0 + row];
+          page[i] = ra.block_table[(size_t)(pos[i] < 0 ? 0 : seq[i]) * ra.table_stride + (ra.page_shift >= 0 ? at >> ra.page_shift : at / ra.page_size)];
+        }
+      }
+    }
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
       if (base + u >= steps) break;                                            // scalar
@@ -506,14 +552,42 @@ __global__ __launch_bounds__(64 * (WC + 2)) void gemm_f32_strips_kernel(const fl
       }
     }
   }
-  f32_write<1, 1>(acc, y, ldy, m0, n0 + 16 * wave, M, N, accumulate);
+  if constexpr (ROPE) {
+    // (the loading waves are done: their last stores lie before the barrier behind the last stage)
+    const f32x4 own = acc[0][0];
+    f32x4* sums = reinterpret_cast<f32x4*>(f32s_lds);
+    sums[64 * wave + lane] = own;
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const f32x4 other = sums[64 * (wave ^ 1) + lane];
+    const int n = n0 + half * wave + row, in_head = pair0 + half * wave + row;
+    const bool turns = head < ra.heads + ra.kv_heads;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = m0 + 4 * g + i;
+      if (m >= M) continue;
+      float v = own[i];
+      if (turns && pos[i] >= 0) v = wave == 0 ? own[i] * cosine[i] - other[i] * sine[i] : own[i] * cosine[i] + other[i] * sine[i];
+      y[(size_t)m * ldy + n] = v;
+      if (head >= ra.heads && pos[i] >= 0 && ra.write_cache) {
+        float* cache = turns ? ra.k_cache : ra.v_cache;
+        const int kv = head - ra.heads - (turns ? 0 : ra.kv_heads);
+        const int slot = ra.page_shift >= 0 ? pos[i] & (ra.page_size - 1) : pos[i] % ra.page_size;
+        cache[(((size_t)page[i] * ra.kv_heads + kv) * ra.page_size + slot) * ra.head_dim + in_head] = v;
+      }
+    }
+  } else {
+    f32_write<1, 1>(acc, y, ldy, m0, n0 + 16 * wave, M, N, accumulate);
+  }
 #endif
 }
 
-template <typename WT, int WC, int D>
-static void launch_f32_strips(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s) {
+template <typename WT, int WC, int D, bool ROPE = false>
+static void launch_f32_strips(const float* x, const WT* w, float* y, int M, int N, int K, int ldx, int ldy, int accumulate, hipStream_t s,
+                              const F32RopeArgs& ra = F32RopeArgs{}) {
   using S = F32SShape<WT, WC, D>;
   const int row_tiles = (M + 15) / 16;
-  hipLaunchKernelGGL((gemm_f32_strips_kernel<WT, WC, D>), dim3(row_tiles * ((N + S::COLS - 1) / S::COLS)), dim3(64 * (WC + S::LW)), S::LDS, s, x, w, y, M, N,
-                     K, ldx, ldy, accumulate, row_tiles);
+  hipLaunchKernelGGL((gemm_f32_strips_kernel<WT, WC, D, ROPE>), dim3(row_tiles * ((N + S::COLS - 1) / S::COLS)), dim3(64 * (WC + S::LW)), S::LDS, s, x, w, y, M, N,
+                     K, ldx, ldy, accumulate, row_tiles, ra);
 }

@@ -49,6 +49,9 @@ _SIGS = {
     "bw_gemm_f32": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_f32_by_chains": [c_int, c_int, c_int, c_int],
     "bw_gemm_f32_swiglu_in_tiles": [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int],
+    "bw_gemm_f32_rope_in_strips": [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int],
+    "bw_gemm_f32_qkv_rope": [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
+                             c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_f32_swiglu": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "bw_gemm_clamped_glu_bf16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_void_p],
@@ -170,7 +173,7 @@ _fns = {}
 # what waits.
 _CHAIN_KEEPS = frozenset({
     "bw_gemm_bf16", "bw_gemm_add_bf16", "bw_gemm_store_bf16", "bw_norm_gemm_bf16", "bw_norm_qkv_rope_bf16",
-    "bw_gemm_f32_by_chains", "bw_gemm_f32_swiglu_in_tiles", "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts",
+    "bw_gemm_f32_by_chains", "bw_gemm_f32_rope_in_strips", "bw_gemm_f32_swiglu_in_tiles", "bw_gemm_f32_prompt_tile", "bw_gemm_prompt_tile", "bw_gemm_prompt_parts",
     "bw_gemm_gelu_glu_wins", "bw_gemm_split_tile", "bw_gemm_split_rows", "bw_attention_f32_waves", "bw_fingerprint_waves",
     "bw_gemm_add_scratch", "bw_norm_gemm_supported", "bw_norm_gemm_wide_supported", "bw_norm_gemm_strips", "bw_attention_decode_scratch",
     "bw_attention_fold_group_tiles", "bw_gemm_add_bf16_static_max", "bw_moe_max_tiles", "bw_shared_key_piece", "bw_chain_sync_words", "bw_chain_begin",
@@ -467,6 +470,43 @@ def gemm_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rows: int, acc
 def gemm_f32_by_chains(rows: int, N: int, K: int, bf16_weights: bool) -> bool:
     """Whether ``gemm_f32`` runs so few rows as chains on the vector units rather than on the matrix cores (the same bits)."""
     return bool(_fn("bw_gemm_f32_by_chains")(rows, N, K, int(bf16_weights)))
+
+
+def gemm_f32_rope_in_strips(x: torch.Tensor, w: torch.Tensor, rows: int, head_dim: int) -> bool:
+    """Whether ``gemm_f32_qkv_rope`` takes the stacked q|k|v product of so many rows."""
+    return (x.is_cuda and w.is_cuda and x.dtype == torch.float32 and x.dim() == 2 and x.stride(1) == 1 and w.is_contiguous()
+            and w.dtype in (torch.float32, torch.bfloat16) and x.shape[1] == w.shape[1] and w.shape[0] % head_dim == 0
+            and bool(_fn("bw_gemm_f32_rope_in_strips")(x.data_ptr(), w.data_ptr(), int(w.dtype == torch.bfloat16), rows, w.shape[0] // head_dim,
+                                                       head_dim, w.shape[1], x.stride(0))))
+
+
+def gemm_f32_qkv_rope(x: torch.Tensor, w: torch.Tensor, qkv: torch.Tensor, positions: torch.Tensor, row_seq: torch.Tensor,
+                      block_table: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                      rows: int, heads: int, kv_heads: int, head_dim: int, page_size: int, write_cache: bool = True) -> None:
+    """``gemm_f32`` of the stacked q|k|v product followed by ``rope_kvwrite`` on 32-bit caches in one kernel, the same bits
+    (``gemm_f32_rope_in_strips``: where it takes them)."""
+    _need(x, torch.float32, "x")
+    _need(qkv, torch.float32, "qkv")
+    _need(positions, torch.int32, "positions")
+    _need(row_seq, torch.int32, "row_seq")
+    _need(block_table, torch.int32, "block_table")
+    _need(cos, torch.float32, "cos table")
+    _need(sin, torch.float32, "sin table")
+    _need(k_cache, torch.float32, "k_cache")
+    _need(v_cache, torch.float32, "v_cache")
+    width = (heads + 2 * kv_heads) * head_dim
+    if tuple(w.shape) != (width, x.shape[1]) or x.shape[0] < rows or not gemm_f32_rope_in_strips(x, w, rows, head_dim):
+        raise ValueError(f"gemm_f32_qkv_rope: {rows} rows of x {tuple(x.shape)} against weight {tuple(w.shape)} do not go as strips")
+    if qkv.shape[1] != width or qkv.shape[0] < rows or positions.numel() < rows or row_seq.numel() < rows:
+        raise ValueError(f"gemm_f32_qkv_rope: qkv must be [>= {rows}, {width}]")
+    if cos.shape[1] != head_dim // 2 or sin.shape != cos.shape:
+        raise ValueError("gemm_f32_qkv_rope: tables must be [positions, head_dim/2]")
+    if k_cache.numel() % (kv_heads * page_size * head_dim) or v_cache.numel() != k_cache.numel():
+        raise ValueError("gemm_f32_qkv_rope: cache size is no multiple of a page")
+    _check(_fn("bw_gemm_f32_qkv_rope")(x.data_ptr(), w.data_ptr(), _is_bf16(w, "weight"), qkv.data_ptr(), rows, w.shape[1], x.stride(0), qkv.stride(0),
+                                       positions.data_ptr(), row_seq.data_ptr(), block_table.data_ptr(), block_table.stride(0), cos.data_ptr(),
+                                       sin.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), heads, kv_heads, head_dim, page_size,
+                                       int(write_cache), _stream()), "gemm_f32_qkv_rope")
 
 
 def gemm_f32_swiglu_in_tiles(x: torch.Tensor, w: torch.Tensor, rows: int) -> bool:

@@ -272,7 +272,9 @@ class Attention(Mixer):
             self._attend(ctx, call, q, residual)
             return
         qkv = ws.buffer("qkv", self.q_dim + 2 * self.kv_dim, torch.float32)
-        self.qkv.store(ws, h, qkv, rows)
+        turned = not rt.bf16 and self.qkv.store_rotated(ctx, call, h, qkv, self.cos, self.sin, self.heads, self.kv_heads, self.head_dim)
+        if not turned:
+            self.qkv.store(ws, h, qkv, rows)
         if rt.bf16:
             q = ws.buffer("q_rot", self.q_dim, torch.bfloat16)
             ops.rope_kvwrite(qkv, q, ctx.positions, ctx.row_seq, table, self.cos, self.sin,
@@ -280,9 +282,10 @@ class Attention(Mixer):
                              ws.page_size, call.writes_cache)
             self._attend(ctx, call, q, residual)
         else:
-            ops.rope_kvwrite(qkv, None, ctx.positions, ctx.row_seq, table, self.cos, self.sin,
-                             call.k_cache, call.v_cache, rows, self.heads, self.kv_heads, self.head_dim,
-                             ws.page_size, call.writes_cache)
+            if not turned:
+                ops.rope_kvwrite(qkv, None, ctx.positions, ctx.row_seq, table, self.cos, self.sin,
+                                 call.k_cache, call.v_cache, rows, self.heads, self.kv_heads, self.head_dim,
+                                 ws.page_size, call.writes_cache)
             out = ws.buffer("attn_out", self.q_dim, torch.float32)
             attend_f32(ctx, call, qkv, out, self.heads, self.kv_heads, self.head_dim, window, self.scale)
             self.o.add_into(ws, out, residual, rows)

@@ -104,6 +104,16 @@ class Linear:
             ops.gemm_f32(self._x32(ws, x, rows), self.weight, tmp, rows)
             ops.convert(tmp, out, rows)
 
+    def store_rotated(self, ctx, call, x: torch.Tensor, out: torch.Tensor, cos, sin, heads: int, kv_heads: int, head_dim: int) -> bool:
+        """``store`` of a stacked q|k|v product in the 32-bit mode with rotation and cache write (``ops.rope_kvwrite``) in one kernel.
+        False (and nothing is done) where that kernel does not take this step."""
+        rows = ctx.rows
+        if self.bias is not None or self.mfma or x.dtype != torch.float32 or not ops.gemm_f32_rope_in_strips(x, self.weight, rows, head_dim):
+            return False
+        ops.gemm_f32_qkv_rope(x, self.weight, out, ctx.positions, ctx.row_seq, ctx.block_tables[call.group], cos, sin, call.k_cache,
+                              call.v_cache, rows, heads, kv_heads, head_dim, ctx.ws.page_size, call.writes_cache)
+        return True
+
     def store_normed(self, x: torch.Tensor, norm, out: torch.Tensor, rows: int) -> bool:
         """out[:rows] = norm(x[:rows]) @ W.T as one kernel (32-bit store), with the bits of the norm followed by ``store``.
         False (and nothing is done) where the fused kernel does not take this step: many rows, the 32-bit mode, a norm of

@@ -1216,6 +1216,57 @@ def test_fused_norm_products_equal_the_separate_kernels(gpu):
         assert torch.equal(outs[0][1], outs[1][1]) and torch.equal(outs[0][2], outs[1][2])
 
 
+@pytest.mark.parametrize("M,heads,kvh,hd,page,K", [(1, 4, 2, 32, 16, 64), (8, 32, 32, 64, 16, 2048), (5, 3, 1, 96, 8, 128), (16, 8, 2, 128, 32, 192),
+                                                   (17, 6, 3, 64, 24, 320), (33, 5, 1, 160, 16, 448), (64, 12, 2, 64, 64, 128)])
+@pytest.mark.parametrize("bf16_weights", [False, True])
+def test_rotation_in_the_32_bit_product_equals_the_separate_kernels(gpu, M, heads, kvh, hd, page, K, bf16_weights):
+    """q|k|v of one to four tiles of rows with rotation and cache write in the epilogue: every element of the product, of the caches
+    (slots that no row writes among them) and of padding rows as the two kernels leave them."""
+    g = torch.Generator().manual_seed(M + heads + hd + K)
+    width, limit = (heads + 2 * kvh) * hd, 4 * page
+    x = torch.randn(M, K, generator=g).to(gpu)
+    w = (torch.randn(width, K, generator=g) * 0.05).to(torch.bfloat16 if bf16_weights else torch.float32).to(gpu)
+    angles = torch.randn(limit, hd // 2, generator=g)
+    cos, sin = torch.cos(angles).to(gpu), torch.sin(angles).to(gpu)
+    # a request a row; padding rows among them
+    pos = torch.randint(0, limit, (M,), generator=g)
+    if M > 2:
+        pos[::4] = -1
+    seq = torch.randperm(M, generator=g).to(torch.int32).to(gpu)
+    table = torch.randperm(4 * M, generator=g).view(M, 4).to(torch.int32).to(gpu)
+    positions = pos.to(torch.int32).to(gpu)
+    assert ops.gemm_f32_rope_in_strips(x, w, M, hd)
+    for writes in (True, False):
+        got = []
+        for fused in (False, True):
+            qkv = torch.full((M + 1, width), 3.0, device=gpu)
+            kc, vc = (torch.full((4 * M, kvh * page * hd), f, device=gpu) for f in (5.0, 7.0))
+            args = (positions, seq, table, cos, sin, kc, vc, M, heads, kvh, hd, page, writes)
+            if fused:
+                ops.gemm_f32_qkv_rope(x, w, qkv, *args)
+            else:
+                ops.gemm_f32(x, w, qkv, M)
+                ops.rope_kvwrite(qkv, None, *args)
+            got.append((qkv, kc, vc))
+        for a, b in zip(*got):
+            assert torch.equal(a, b), writes
+
+
+def test_32_bit_products_that_keep_their_rotation_as_a_kernel(gpu):
+    """Halves of heads that are no whole tiles, K in no whole stages, more rows or columns than strips suit, rows that start at no vector."""
+    x, w = torch.zeros(65, 2052, device=gpu), torch.zeros(320, 2048, device=gpu)
+    assert ops.gemm_f32_rope_in_strips(x[:, :2048], w, 8, 64) and not ops.gemm_f32_rope_in_strips(x[:, :2048], w, 65, 64)
+    assert not ops.gemm_f32_rope_in_strips(x[:, :2048], w, 8, 80) and not ops.gemm_f32_rope_in_strips(x[:, :2048], w, 8, 16)
+    assert not ops.gemm_f32_rope_in_strips(x[:, 1:2049], w, 8, 64)
+    assert not ops.gemm_f32_rope_in_strips(x[:, :2016].contiguous(), w[:, :2016].contiguous(), 8, 64)
+    assert not ops.gemm_f32_rope_in_strips(x[:, :64], torch.zeros(16384, 64, device=gpu), 8, 64)
+    with pytest.raises(ValueError):
+        cache = torch.zeros(1, 16 * 64, device=gpu)
+        ids = torch.zeros(65, dtype=torch.int32, device=gpu)
+        ops.gemm_f32_qkv_rope(x[:, :2048].contiguous(), w, torch.zeros(65, 320, device=gpu), ids, ids, ids.view(65, 1), torch.zeros(16, 32, device=gpu),
+                              torch.zeros(16, 32, device=gpu), cache, cache.clone(), 65, 3, 1, 64, 16)
+
+
 @pytest.mark.parametrize("M,N,K,strips", [(1, 8208, 64, 6), (8, 8256, 512, 6), (16, 11000, 128, 7), (5, 11008, 2048, 7), (9, 14329, 192, 7), (8, 8200, 2560, 5),
                                           (3, 14336, 4096, 7), (2, 16384, 2048, 8), (13, 16377, 1024, 8), (8, 18440, 4096, 5), (1, 24576, 2176, 6)])
 @pytest.mark.parametrize("glu", [True, False])
