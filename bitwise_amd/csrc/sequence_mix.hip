@@ -55,6 +55,7 @@ __device__ __forceinline__ float row_sumsq(const float* __restrict__ xr, int dim
 // row above, or for the first row of a request in this step what the state slot holds (zeros for a new request).
 // The wave of a request's first row also leaves the h of the request's last row in the slot, after it has read it:
 // nothing else reads or writes that slot in this launch.  A wave a row.
+#define SHIFT_REGS 8      // 16-byte vectors of a row a lane keeps (rows of up to 2,048 elements)
 template <typename OT>
 __global__ __launch_bounds__(256) void norm_shift_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w,
                                                          const float* __restrict__ mix, float* __restrict__ state,
@@ -85,6 +86,53 @@ __global__ __launch_bounds__(256) void norm_shift_kernel(const float* __restrict
     const f32x4* lv = reinterpret_cast<const f32x4*>(x + (size_t)last * ldx);
     const f32x4* wv = reinterpret_cast<const f32x4*>(w);
     const f32x4* mv = reinterpret_cast<const f32x4*>(mix);
+    if (!is_first && nvec <= 64 * SHIFT_REGS) {
+      // both rows, the weight and the first mixing vector in registers, asked for once and at once: the rows came twice, the second time
+      // behind two sums.  2,048 rows to bfloat16, us: 2,048 wide 8.6 -> 7.4, 1,028 7.1 -> 5.8.
+      f32x4 xq[SHIFT_REGS], pq[SHIFT_REGS], wq[SHIFT_REGS], mq[SHIFT_REGS];
+#pragma unroll
+      for (int j = 0; j < SHIFT_REGS; ++j) {
+        if (64 * j >= nvec) continue;                                          // (scalar)
+        const int c = min(64 * j + lane, nvec - 1);
+        xq[j] = xv[c];
+        pq[j] = pv[c];
+        wq[j] = wv[c];
+        mq[j] = mv[c];
+      }
+      // (row_sumsq_vec's chains)
+      float sx = 0.0f, sp = 0.0f;
+#pragma unroll
+      for (int j = 0; j < SHIFT_REGS; ++j) {
+        if (64 * j + lane >= nvec) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sx = fmaf(xq[j][e], xq[j][e], sx);
+          sp = fmaf(pq[j][e], pq[j][e], sp);
+        }
+      }
+      const float inv = 1.0f / sqrtf(wave_sum(sx) / (float)dim + eps), invp = 1.0f / sqrtf(wave_sum(sp) / (float)dim + eps);
+#pragma unroll
+      for (int j = 0; j < SHIFT_REGS; ++j) {
+        const int c = 64 * j + lane;
+        if (c >= nvec) continue;
+        f32x4 hq, dq;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          hq[e] = (xq[j][e] * inv) * wq[j][e];
+          dq[e] = (pq[j][e] * invp) * wq[j][e] - hq[e];
+        }
+        for (int m = 0; m < nmix; ++m) {
+          const f32x4 mm = m == 0 ? mq[j] : mv[(size_t)m * nvec + c];
+          f32x4 r;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) r[e] = fmaf(dq[e], mm[e], hq[e]);
+          OT* om = o + (size_t)m * dim;
+          if constexpr (sizeof(OT) == 2) *reinterpret_cast<u32x2*>(om + 4 * c) = (u32x2){pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
+          else *reinterpret_cast<f32x4*>(om + 4 * c) = r;
+        }
+      }
+      return;
+    }
     const float inv = 1.0f / sqrtf(row_sumsq_vec(xv, nvec, lane) / (float)dim + eps);
     const float invp = is_first ? 1.0f : 1.0f / sqrtf(row_sumsq_vec(pv, nvec, lane) / (float)dim + eps);
     const float invl = !is_first || last == row ? inv : 1.0f / sqrtf(row_sumsq_vec(lv, nvec, lane) / (float)dim + eps);
@@ -1029,6 +1077,64 @@ __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __rest
   }
 }
 
+// The same for heads of whole rows of lanes and many (row, head) items: a wave takes HG_ITEMS neighbouring items and asks for all
+// they need before the first sum.  One item a wave was a chain of four trips to memory beside 64 to 256 elements.
+// bfloat16, us: 2048 x 16 heads of 128 15.6 -> 11.9, 2048 x 8 of 256 13.9 -> 11.4; 10,000 items of 64 to 128 as they were or 3 to 6 % slower.
+#define HG_ITEMS 4
+#define HG_MIN_ITEMS 16384
+template <typename OT, int EV>
+__global__ __launch_bounds__(256) void head_norm_gate_items_kernel(const float* __restrict__ o, int ldi, const float* __restrict__ weight,
+                                                                   int wstride, const float* __restrict__ g, int ldg, int gate,
+                                                                   OT* __restrict__ out, int ldo, const int32_t* __restrict__ positions,
+                                                                   int items, int heads, float eps) {
+  constexpr int VD = 64 * EV;
+  const int lane = threadIdx.x & 63;
+  const int item0 = (blockIdx.x * 4 + wave_index()) * HG_ITEMS;
+  if (item0 >= items) return;
+  float ov[HG_ITEMS][EV], gv[HG_ITEMS][EV], wv[HG_ITEMS][EV], sum[HG_ITEMS];
+  int row[HG_ITEMS], head[HG_ITEMS], pos[HG_ITEMS];
+#pragma unroll
+  for (int k = 0; k < HG_ITEMS; ++k) {
+    const int item = min(item0 + k, items - 1);
+    row[k] = item / heads;
+    head[k] = item - row[k] * heads;
+    pos[k] = positions[row[k]];
+#pragma unroll
+    for (int e = 0; e < EV; ++e) {
+      const int at = head[k] * VD + lane + 64 * e;
+      ov[k][e] = o[(size_t)row[k] * ldi + at];
+      gv[k][e] = g[(size_t)row[k] * ldg + at];
+      wv[k][e] = weight[(size_t)head[k] * wstride + lane + 64 * e];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < HG_ITEMS; ++k) {
+    sum[k] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < EV; ++e) sum[k] = fmaf(ov[k][e], ov[k][e], sum[k]);      // (row_sumsq's chain)
+    sum[k] = wave_sum(sum[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < HG_ITEMS; ++k) {
+    if (item0 + k >= items || pos[k] < 0) continue;
+    const float inv = 1.0f / sqrtf(sum[k] / (float)VD + eps);
+#pragma unroll
+    for (int e = 0; e < EV; ++e) {
+      const float z = gv[k][e], sg = 1.0f / (1.0f + bw_expf(-z));
+      store_act(out + (size_t)row[k] * ldo + head[k] * VD + lane + 64 * e, ((ov[k][e] * inv) * wv[k][e]) * (gate == GATE_SILU ? z * sg : sg));
+    }
+  }
+}
+
+template <typename OT>
+static void launch_head_norm_items(const float* o, int ldi, const float* weight, int wstride, const float* g, int ldg, int gate, OT* out, int ldo,
+                                   const int32_t* positions, int items, int heads, int vdim, float eps, hipStream_t s) {
+  const dim3 grid((items + 4 * HG_ITEMS - 1) / (4 * HG_ITEMS)), block(256);
+  if (vdim == 64) hipLaunchKernelGGL((head_norm_gate_items_kernel<OT, 1>), grid, block, 0, s, o, ldi, weight, wstride, g, ldg, gate, out, ldo, positions, items, heads, eps);
+  else if (vdim == 128) hipLaunchKernelGGL((head_norm_gate_items_kernel<OT, 2>), grid, block, 0, s, o, ldi, weight, wstride, g, ldg, gate, out, ldo, positions, items, heads, eps);
+  else hipLaunchKernelGGL((head_norm_gate_items_kernel<OT, 4>), grid, block, 0, s, o, ldi, weight, wstride, g, ldg, gate, out, ldo, positions, items, heads, eps);
+}
+
 // ------------------------------------------------------------------------- output gate and an RMS norm in equal parts
 
 // A row's parts are equal stretches of ``size`` elements.  BEHIND false: v = o[r][e] * act(z[r][e]), out = v / sqrt(mean of v^2
@@ -1283,6 +1389,12 @@ extern "C" int bw_head_norm_gate(const float* o, int ldi, const float* weight, i
   if (rows <= 0) return 0;
   if (heads <= 0 || vdim <= 0 || ldi < heads * vdim || ldo < heads * vdim) return -2;
   hipStream_t s = (hipStream_t)stream;
+  const long long items = (long long)rows * heads;
+  if (items >= HG_MIN_ITEMS && items < (1LL << 30) && (vdim == 64 || vdim == 128 || vdim == 256)) {
+    if (out_is_bf16) launch_head_norm_items(o, ldi, weight, wstride, g, ldg, gate, (bf16_t*)out, ldo, positions, (int)items, heads, vdim, eps, s);
+    else launch_head_norm_items(o, ldi, weight, wstride, g, ldg, gate, (float*)out, ldo, positions, (int)items, heads, vdim, eps, s);
+    return BW_LAUNCH_CHECK();
+  }
   const dim3 grid((rows * heads + 3) / 4), block(256);
   if (out_is_bf16)
     hipLaunchKernelGGL(head_norm_gate_kernel<bf16_t>, grid, block, 0, s, o, ldi, weight, wstride, g, ldg, gate, (bf16_t*)out,
