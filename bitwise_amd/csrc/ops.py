@@ -485,7 +485,6 @@ def gemm_f32_qkv_rope(x: torch.Tensor, w: torch.Tensor, qkv: torch.Tensor, posit
                       rows: int, heads: int, kv_heads: int, head_dim: int, page_size: int, write_cache: bool = True) -> None:
     """``gemm_f32`` of the stacked q|k|v product followed by ``rope_kvwrite`` on 32-bit caches in one kernel, the same bits
     (``gemm_f32_rope_in_strips``: where it takes them)."""
-    _need(x, torch.float32, "x")
     _need(qkv, torch.float32, "qkv")
     _need(positions, torch.int32, "positions")
     _need(row_seq, torch.int32, "row_seq")

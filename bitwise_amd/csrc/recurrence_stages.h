@@ -439,10 +439,12 @@ __global__ __launch_bounds__(64 * RW) void recurrence_stages_kernel(RecurArgs a)
 // of 32 tokens behind one another, a barrier a chunk: the running maximum, which is the one chain; the factors (a token a lane); the
 // normaliser (a channel a lane); its product with q, summed over the lanes.
 // What bounds it: the instructions of a compute unit's four SIMDs, of which the keeping waves and the summing ones share two.  Sums of
-// eight tokens go through the lanes together (wave_sums_of_eight): 2,048 tokens of 8 heads of 128 77 -> 72 us.
+// eight tokens go through the lanes together (wave_sums_of_eight): 2,048 tokens of 8 heads of 128 77 -> 72 us.  Then the keys' way: loads a token were more than a
+// wave may count, so no more than two chunks were on their way; four tokens a load, straight into LDS, five chunks ahead: 72 -> 61.
 #define SG_CHUNK 32
 #define SG_TOKENS 2048   // whose gates lie in LDS together
 #define SG_SUMS 4        // waves that sum
+#define SG_SLOTS 6       // chunks of keys in LDS
 
 // wave_sum of eight values: the same additions, but where a step of a butterfly leaves both halves with the same sums, here each half
 // goes on with another value's (20 instructions for what eight butterflies take some 90).  A lane has the sum of value number
@@ -474,7 +476,7 @@ __global__ __launch_bounds__(64 * (2 + NN + SG_SUMS)) void scalar_gates_kernel(R
 #if defined(__HIP_DEVICE_COMPILE__)                                            // (buffer descriptors are a type of the device pass)
   constexpr int T = SG_CHUNK, DIM = 64 * NN, THREADS = 64 * (2 + NN + SG_SUMS), MINE = T / SG_SUMS;
   __shared__ __attribute__((aligned(16))) float gi[SG_TOKENS], gf[SG_TOKENS], mx[2][T], before[2], ems[4][T], fib[2][T][2];
-  extern __shared__ __attribute__((aligned(16))) float sg_n[];                // [2][T][DIM]
+  extern __shared__ __attribute__((aligned(16))) float sg_n[];                // [2][T][DIM], then the keeping waves' keys
   const int lane = threadIdx.x & 63, wave = wave_index(), h = blockIdx.x;
   const int first = a.seq_rows[2 * blockIdx.y], count = a.seq_rows[2 * blockIdx.y + 1], slot = a.slots[blockIdx.y];
   if (count <= 0 || slot < 0) return;
@@ -553,21 +555,30 @@ __global__ __launch_bounds__(64 * (2 + NN + SG_SUMS)) void scalar_gates_kernel(R
         }
       });
     } else {
-      // keys and queries: four chunks in registers, three of them on their way
+      // queries: four chunks in registers, three of them on their way
       const bool sums = wave >= 2 + NN;
       const float* from = a.proj + (size_t)(first + base) * a.ldp + (sums ? a.q_off : a.k_off) + hk * DIM;   // (scalar)
       const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc((void*)from, 0, (int)((((size_t)tokens - 1) * a.ldp + DIM) * 4), 0x00020000);
       const int row_bytes = a.ldp * 4;
       if (!sums) {
-        float k0[T], k1[T], k2[T], k3[T];
-        auto fetch = [&](float (&k)[T], int c) {
+        // A wave's keys: [SG_SLOTS chunks][T][64 channels] of LDS that nobody else touches, filled straight from memory (four tokens
+        // a load), SG_SLOTS - 1 chunks ahead.  Rows past the portion's end lie outside the descriptor (zeros, never used).
+        float* keys = sg_n + 2 * T * DIM + (wave - 2) * SG_SLOTS * T * 64;
+        const unsigned at = (unsigned)(lane >> 4) * row_bytes + 256 * (wave - 2) + 16 * (lane & 15);
+        auto fetch = [&](int c, int slot) {
+          typedef __attribute__((address_space(3))) void* lds_ptr;
 #pragma unroll
-          for (int t = 0; t < T; ++t) k[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows, ch * 4, min(c * T + t, tokens - 1) * row_bytes, 0));
+          for (int t = 0; t < T / 4; ++t)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (lds_ptr)(keys + (slot * T + 4 * t) * 64), 16, (int)(at + (unsigned)(c * T + 4 * t) * row_bytes), 0, 0, 0);
         };
-        auto run = [&](const float (&k)[T], int c) {
+        auto run = [&](int c, int slot) {
           const int tc = rows_of(c);
+          const float* kc = keys + slot * T * 64 + lane;
           float* out = sg_n + (c & 1) * T * DIM + ch;
           if (tc == T) {
+            float k[T];
+#pragma unroll
+            for (int t = 0; t < T; ++t) k[t] = kc[t * 64];
 #pragma unroll
             for (int t = 0; t < T; t += 2) {
               const f32x4 two = *reinterpret_cast<const f32x4*>(&fib[c & 1][t][0]);
@@ -577,24 +588,24 @@ __global__ __launch_bounds__(64 * (2 + NN + SG_SUMS)) void scalar_gates_kernel(R
               out[(t + 1) * DIM] = n;
             }
           } else {
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-              if (t >= tc) break;                                              // (scalar; a branch a token costs as much as the token)
-              n = fmaf(fib[c & 1][t][0], n, fib[c & 1][t][1] * (k[t] * a.kscale));
+            for (int t = 0; t < tc; ++t) {
+              n = fmaf(fib[c & 1][t][0], n, fib[c & 1][t][1] * (kc[t * 64] * a.kscale));
               out[t * DIM] = n;
             }
           }
         };
-        fetch(k0, 0);
-        fetch(k1, 1);
-        fetch(k2, 2);
+        for (int c = 0; c < SG_SLOTS - 1; ++c) fetch(c, c);
         for (int i = 0; i < 2; ++i) __syncthreads();
-        for (int c = 0;;) {                                                     // (left in the middle, as the walk in stages is)
-          fetch(k3, c + 3); run(k0, c); __syncthreads(); if (++c == chunks) break;
-          fetch(k0, c + 3); run(k1, c); __syncthreads(); if (++c == chunks) break;
-          fetch(k1, c + 3); run(k2, c); __syncthreads(); if (++c == chunks) break;
-          fetch(k2, c + 3); run(k3, c); __syncthreads(); if (++c == chunks) break;
+        int slot = 0;
+        for (int c = 0; c < chunks; ++c) {
+          fetch(c + SG_SLOTS - 1, slot == 0 ? SG_SLOTS - 1 : slot - 1);        // (where the chunk before lay)
+          __builtin_amdgcn_s_waitcnt(vmcnt_only((SG_SLOTS - 1) * (T / 4)));    // this chunk's have landed: loads land in order
+          asm volatile("" ::: "memory");
+          run(c, slot);
+          slot = slot == SG_SLOTS - 1 ? 0 : slot + 1;
+          __syncthreads();
         }
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));                             // (those past the end, too, before the places are used again)
         for (int i = 2; i < 3; ++i) __syncthreads();
       } else {
         float q0[MINE][NN], q1[MINE][NN], q2[MINE][NN], q3[MINE][NN];
@@ -661,7 +672,7 @@ static int launch_stages(const RecurArgs& a, int nseq, hipStream_t s) {
 
 template <int NN>
 static int launch_scalar_gates(const RecurArgs& a, float* gates, int nseq, hipStream_t s) {
-  constexpr int lds = 2 * SG_CHUNK * 64 * NN * 4;
+  constexpr int lds = (2 + SG_SLOTS) * SG_CHUNK * 64 * NN * 4;
   static bool allowed = false;
   if (lds > 48 * 1024 && !allowed) {
     (void)hipFuncSetAttribute((const void*)scalar_gates_kernel<NN>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);

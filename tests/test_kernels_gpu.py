@@ -1224,7 +1224,7 @@ def test_rotation_in_the_32_bit_product_equals_the_separate_kernels(gpu, M, head
     (slots that no row writes among them) and of padding rows as the two kernels leave them."""
     g = torch.Generator().manual_seed(M + heads + hd + K)
     width, limit = (heads + 2 * kvh) * hd, 4 * page
-    x = torch.randn(M, K, generator=g).to(gpu)
+    x = torch.randn(M, K + 8, generator=g).to(gpu)[:, 4:K + 4]                  # (rows apart by a stride of their own)
     w = (torch.randn(width, K, generator=g) * 0.05).to(torch.bfloat16 if bf16_weights else torch.float32).to(gpu)
     angles = torch.randn(limit, hd // 2, generator=g)
     cos, sin = torch.cos(angles).to(gpu), torch.sin(angles).to(gpu)
