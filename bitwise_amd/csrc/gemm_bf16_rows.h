@@ -708,7 +708,7 @@ static int launch_norm_strips(const bf16_t* w, void* out, int M, int N, int K, i
 //   stores          128256 x 4096 206 -> 194 (7)   20000 x 1024 14.6 -> 10.9 (7)
 // Where both make whole rounds the variant is as fast or faster (8192 x 2048 17.6 and 17.9 with 4 strips; stores of K = 2048: 49152
 // columns 46.0 and 47.0 with 6, 32000 30.5 and 31.7 with 8; of K = 2176 47936 39.7 and 42.2 with 7), so it stays unless the count says
-// 4 % less, 10 % for stores of one segment, 6 % for those of two.  66 products drawn over all of that: 0.71 to 1.02 of the variant's time.
+// 4 % less, 10 % for stores of one segment, 6 % for those of two.  57 products drawn over all of that: 0.71 to 1.02 of the variant's time.
 extern "C" int bw_norm_gemm_strips(int M, int N, int K, int epilogue) {
   const bool glu = epilogue == EPI_SWIGLU_BF16;
   if ((!glu && epilogue != EPI_F32) || !mid_norm_admits(M, K, (N + (glu ? 31 : 63)) / (glu ? 32 : 64))) return 0;
