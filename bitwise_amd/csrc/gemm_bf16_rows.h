@@ -558,15 +558,14 @@ static int launch_mid(const bf16_t* x, const bf16_t* w, void* out, int M, int N,
 // The NORM variant above gives a workgroup 32 outputs of SwiGLU or 64 columns, whatever the product: one of more workgroups than
 // compute units pays the workgroup's beginning (rows asked for, normalised, the ring's first loads: 6 us) once a round.  Here a
 // workgroup takes up to eight strips of 16 rows of W, a wave each (SwiGLU: eight gate rows and the eight up rows of the same outputs, whose
-// sums meet by a lane exchange), so that the rounds are the product's choice (norm_strips_shape).  A wave streams its strip
+// sums meet by a lane exchange), so that the rounds are the product's choice (norm_strips_admits).  A wave streams its strip
 // through a ring of its own, which nobody else touches: no barrier behind the one that ends the normalising.
-// LDS: [strips][STAGES][16 rows of W, 128 bytes each, chunks permuted as above], then the rows as in the NORM variant.
 __device__ __forceinline__ void norm_strips_issue(unsigned char* slot, __amdgpu_buffer_rsrc_t rs0, __amdgpu_buffer_rsrc_t rs1, int voff0, int voff1,
                                                   int step, int steps) {
   typedef __attribute__((address_space(3))) void* lds_ptr;
   const bool real = step < steps;                                     // scalar; past K: zeros from outside the descriptors
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs0, (lds_ptr)slot, 16, real ? voff0 : 0x7ffffff0, step * 128, 0, 0);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs1, (lds_ptr)(slot + 1024), 16, real ? voff1 : 0x7ffffff0, step * 128, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs1, (lds_ptr)(slot + norm_strips_half(1)), 16, real ? voff1 : 0x7ffffff0, step * 128, 0, 0);
 }
 
 // A wave's rows: asked for before its ring's first stages, normalised behind them.
@@ -585,7 +584,7 @@ __device__ __forceinline__ void norm_strips_rows(const MidNormArgs& na, int M, i
   __builtin_amdgcn_sched_barrier(0);
   if (working) {
 #pragma unroll
-    for (int st = 0; st < STAGES - 1; ++st) norm_strips_issue(ring + st * 2048, rs0, rs1, voff0, voff1, st, steps);
+    for (int st = 0; st < STAGES - 1; ++st) norm_strips_issue(ring + st * NORM_STRIP_STAGE, rs0, rs1, voff0, voff1, st, steps);
   }
   __builtin_amdgcn_sched_barrier(0);
   unsigned char* rl = rows_lds;
@@ -599,32 +598,26 @@ template <int EPI, int STAGES>
 __device__ __forceinline__ void norm_strips_body(const bf16_t* __restrict__ w, void* __restrict__ out, int M, int N, int K, int ldo, const MidNormArgs& na,
                                                  int strips) {
   constexpr bool GLU = EPI == EPI_SWIGLU_BF16;
-  constexpr int COLS = GLU ? 8 : 16;                                  // outputs a strip
   static_assert(2 * (STAGES - 2) < 64 && STAGES >= 3, "the wait count has six bits");
   extern __shared__ __attribute__((aligned(16))) unsigned char strips_lds[];
   const int wave = wave_index(), lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
-  const int first = ((int)blockIdx.x * strips + wave) * COLS;
-  const bool working = wave < strips && first < N;                    // (scalar; the others only normalise)
-  const int n0 = working ? first : 0;
-  const int have = min(COLS, N - n0);
-  // the strip's rows 0 to 7 and 8 to 15: a descriptor each
-  const __amdgpu_buffer_rsrc_t rs0 = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, min(8, have) * K * 2, 0x00020000);
-  const int second = GLU ? have : max(have - 8, 0);
-  const __amdgpu_buffer_rsrc_t rs1 = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(w + (size_t)(GLU ? N + n0 : (second ? n0 + 8 : n0)) * K), 0, second * K * 2, 0x00020000);
-  const int lrow = lane >> 3, lslot = lane & 7;
-  const int voff0 = (lrow * K + 8 * (lslot ^ (lrow >> 1))) * 2, voff1 = (lrow * K + 8 * (lslot ^ ((8 + lrow) >> 1))) * 2;
+  const NormStrip own = norm_strips_of_wave(GLU, (int)blockIdx.x, strips, wave, N);   // (scalar)
+  const bool working = own.working;
+  const int n0 = own.n0;
+  const __amdgpu_buffer_rsrc_t rs0 = __builtin_amdgcn_make_buffer_rsrc((void*)(w + own.row[0] * K), 0, own.rows[0] * K * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs1 = __builtin_amdgcn_make_buffer_rsrc((void*)(w + own.row[1] * K), 0, own.rows[1] * K * 2, 0x00020000);
+  const int voff0 = norm_strips_load_offset(0, lane, K), voff1 = norm_strips_load_offset(1, lane, K);
   const int steps = K / 64;
-  unsigned char* ring = strips_lds + wave * STAGES * 2048;
-  unsigned char* rows_lds = strips_lds + strips * STAGES * 2048;
+  unsigned char* ring = strips_lds + norm_strips_ring_of(wave, STAGES);
+  unsigned char* rows_lds = strips_lds + norm_strips_ring(strips, STAGES);
   if (wave < M) {
     if (mid_norm_vectors_a_lane(K) == 16) norm_strips_rows<1, 16, STAGES>(na, M, K, wave, lane, rows_lds, ring, rs0, rs1, voff0, voff1, steps, working);
     else if (M <= 8) norm_strips_rows<1, 8, STAGES>(na, M, K, wave, lane, rows_lds, ring, rs0, rs1, voff0, voff1, steps, working);
     else norm_strips_rows<2, 8, STAGES>(na, M, K, wave, lane, rows_lds, ring, rs0, rs1, voff0, voff1, steps, working);
   } else if (working) {
 #pragma unroll
-    for (int st = 0; st < STAGES - 1; ++st) norm_strips_issue(ring + st * 2048, rs0, rs1, voff0, voff1, st, steps);
+    for (int st = 0; st < STAGES - 1; ++st) norm_strips_issue(ring + st * NORM_STRIP_STAGE, rs0, rs1, voff0, voff1, st, steps);
   }
   __builtin_amdgcn_s_waitcnt(0xc07f);                                  // this wave's normalised rows are in LDS
   __builtin_amdgcn_s_barrier();
@@ -649,8 +642,8 @@ __device__ __forceinline__ void norm_strips_body(const bf16_t* __restrict__ w, v
     for (int kk = 0; kk < 2; ++kk) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(fa[kk]), as_bf16x8(fb[kk]), acc, 0, 0, 0);
     asm volatile("" ::: "memory");
     // the stage of the step before: its operands have been used
-    norm_strips_issue(ring + (at == 0 ? (STAGES - 1) * 2048 : at - 2048), rs0, rs1, voff0, voff1, step + STAGES - 1, steps);
-    at = at == (STAGES - 1) * 2048 ? 0 : at + 2048;
+    norm_strips_issue(ring + norm_strips_before(at, STAGES), rs0, rs1, voff0, voff1, step + STAGES - 1, steps);
+    at = norm_strips_next(at, STAGES);
     const int kn = (step + 1) * 64;
     if (kn % GEMM_SEG == 0 && kn < K) {                               // a segment ends before the last: left to right
       tot = kn == GEMM_SEG ? acc : tot + acc;
@@ -677,8 +670,8 @@ __global__ __launch_bounds__(512) void gemm_bf16_norm_strips_kernel(const bf16_t
 
 template <int EPI, int STAGES>
 static int launch_norm_strips_deep(const bf16_t* w, void* out, int M, int N, int K, int ldo, const MidNormArgs& na, int strips, hipStream_t s) {
-  const int cols = strips * (EPI == EPI_SWIGLU_BF16 ? 8 : 16);
-  const int lds_bytes = mid_norm_lds_bytes(strips * STAGES * 2048, K, na.row_step);
+  const int cols = strips * norm_strips_cols(EPI == EPI_SWIGLU_BF16);
+  const int lds_bytes = mid_norm_lds_bytes(norm_strips_ring(strips, STAGES), K, na.row_step);
   if (lds_bytes > BW_LDS_LIMIT) return -2;
   static bool allowed = false;                       // more than 64 KB of dynamic LDS has to be asked for once
   if (!allowed) {
@@ -689,47 +682,17 @@ static int launch_norm_strips_deep(const bf16_t* w, void* out, int M, int N, int
   return BW_LAUNCH_CHECK();
 }
 
-// (as many stages as LDS holds beside the rows' 65 KB)
 template <int EPI>
 static int launch_norm_strips(const bf16_t* w, void* out, int M, int N, int K, int ldo, const MidNormArgs& na, int strips, hipStream_t s) {
   switch (strips) {
-    case 5: return launch_norm_strips_deep<EPI, 9>(w, out, M, N, K, ldo, na, strips, s);
-    case 6: return launch_norm_strips_deep<EPI, 7>(w, out, M, N, K, ldo, na, strips, s);
-    case 7: return launch_norm_strips_deep<EPI, 6>(w, out, M, N, K, ldo, na, strips, s);
-    default: return launch_norm_strips_deep<EPI, 5>(w, out, M, N, K, ldo, na, strips, s);
+    case 5: return launch_norm_strips_deep<EPI, norm_strips_stages(5)>(w, out, M, N, K, ldo, na, strips, s);
+    case 6: return launch_norm_strips_deep<EPI, norm_strips_stages(6)>(w, out, M, N, K, ldo, na, strips, s);
+    case 7: return launch_norm_strips_deep<EPI, norm_strips_stages(7)>(w, out, M, N, K, ldo, na, strips, s);
+    default: return launch_norm_strips_deep<EPI, norm_strips_stages(8)>(w, out, M, N, K, ldo, na, strips, s);
   }
 }
 
-// How many strips a workgroup takes, or 0: the NORM variant of the kernel for up to 64 rows.  Counted in what a strip of a full round
-// of the compute units takes (2.9 us for K = 2048, at 5.4 TB/s): a round its strips and 0.8 for its beginning, a part-empty last
-// round no less than 0.44 of its strips (what one compute unit pulls).  us, that variant -> strips:
-//   SwiGLU, 5 rows  11008 x 4096 46.2 -> 37.2 (7 strips)   14336 x 4096 50.7 -> 45.8 (7)   18432 x 4096 70.5 -> 65.1 (5)
-//                   9728 x 2560 29.0 -> 22.3 (6)   12000 x 2048 26.3 -> 23.6 (7)   16384 x 2048 31.9 -> 29.8 (8)
-//   stores          128256 x 4096 206 -> 194 (7)   20000 x 1024 14.6 -> 10.9 (7)
-// Where both make whole rounds the variant is as fast or faster (8192 x 2048 17.6 and 17.9 with 4 strips; stores of K = 2048: 49152
-// columns 46.0 and 47.0 with 6, 32000 30.5 and 31.7 with 8; of K = 2176 47936 39.7 and 42.2 with 7), so it stays unless the count says
-// 4 % less, 10 % for stores of one segment, 6 % for those of two.  57 products drawn over all of that: 0.71 to 1.02 of the variant's time.
-extern "C" int bw_norm_gemm_strips(int M, int N, int K, int epilogue) {
-  const bool glu = epilogue == EPI_SWIGLU_BF16;
-  if ((!glu && epilogue != EPI_F32) || !mid_norm_admits(M, K, (N + (glu ? 31 : 63)) / (glu ? 32 : 64))) return 0;
-  const auto cost = [&](int strips) {                                  // in 1/10000
-    const int cols = strips * (glu ? 8 : 16);
-    const long long wgs = (N + cols - 1) / cols, left = wgs % 256;
-    const long long rounds = wgs / 256 * 10000 + (left ? (left * 10000 / 256 > 4400 ? left * 10000 / 256 : 4400) : 0);
-    return strips * rounds + (wgs + 255) / 256 * 8000;
-  };
-  const long long variant = cost(4);
-  long long least = variant * (glu ? 96 : K <= GEMM_SEG ? 90 : 94) / 100;
-  int best = 0;
-  for (int strips = 5; strips <= 8; ++strips) {
-    const long long c = strips == 8 ? cost(strips) * 103 / 100 : cost(strips);     // (a ring of five stages)
-    if (c < least) {
-      least = c;
-      best = strips;
-    }
-  }
-  return best;
-}
+extern "C" int bw_norm_gemm_strips(int M, int N, int K, int epilogue) { return norm_strips_admits(M, N, K, epilogue); }
 
 // RMSNorm of up to 16 rows of the residual stream + product with many columns in one kernel; -7: not this shape.
 int bw_norm_gemm_mid(const float* x32, int ldx32, const void* norm_w, int norm_w_is_bf16, float eps, const void* w, void* out,

@@ -143,6 +143,77 @@ BW_HD int mid_norm_lds_bytes(int ring, int K, int row_step) {
   return ring + (K / 64) * row_step + (row_step == 1024 ? 1024 : 0);
 }
 
+// ------------------------------------------------------------------------------ gemm_bf16_norm_strips_kernel
+
+// A workgroup of eight waves takes ``strips`` (five to eight) strips of 16 rows of W, a wave each (SwiGLU: eight gate rows and the
+// eight up rows of the same outputs).  LDS: [strips][stages][16 rows of W of a step, 128 bytes each, chunks permuted as above], then the
+// rows as in the NORM variant.
+#define NORM_STRIP_STAGE 2048
+BW_HD constexpr int norm_strips_cols(bool glu) { return glu ? 8 : 16; }                                  // outputs a strip
+BW_HD constexpr int norm_strips_stages(int strips) { return strips == 5 ? 9 : strips == 6 ? 7 : strips == 7 ? 6 : 5; }   // (as many as LDS holds beside the rows' 65 KB)
+BW_HD constexpr int norm_strips_ring(int strips, int stages) { return strips * stages * NORM_STRIP_STAGE; }
+BW_HD constexpr int norm_strips_ring_of(int wave, int stages) { return wave * stages * NORM_STRIP_STAGE; }
+BW_HD constexpr int norm_strips_next(int at, int stages) { return at == (stages - 1) * NORM_STRIP_STAGE ? 0 : at + NORM_STRIP_STAGE; }
+BW_HD constexpr int norm_strips_before(int at, int stages) { return at == 0 ? (stages - 1) * NORM_STRIP_STAGE : at - NORM_STRIP_STAGE; }
+
+// A wave's strip: its first output, and the rows of W behind its two descriptors (strip rows 0 to 7 and 8 to 15; ``working`` false: the wave
+// has no strip and only normalises).  A descriptor of no rows gives zeros wherever a lane points in it.
+struct NormStrip {
+  bool working;
+  int n0, have;                        // first output, and how many of the strip's outputs there are
+  size_t row[2];                       // first row of W of each half
+  int rows[2];
+};
+BW_HD NormStrip norm_strips_of_wave(bool glu, int block, int strips, int wave, int N) {
+  NormStrip s;
+  const int cols = norm_strips_cols(glu), first = (block * strips + wave) * cols;
+  s.working = wave < strips && first < N;
+  s.n0 = s.working ? first : 0;
+  s.have = cols < N - s.n0 ? cols : N - s.n0;
+  s.rows[0] = s.have < 8 ? s.have : 8;
+  s.rows[1] = glu ? s.have : (s.have > 8 ? s.have - 8 : 0);
+  s.row[0] = (size_t)s.n0;
+  s.row[1] = (size_t)(glu ? N + s.n0 : (s.rows[1] ? s.n0 + 8 : s.n0));
+  return s;
+}
+// Where a lane points in the descriptor of half ``half``, in bytes (a step further: 128 more), and where its 16 bytes land in the stage.
+BW_HD int norm_strips_load_offset(int half, int lane, int K) {
+  const int row = lane >> 3, slot = lane & 7;
+  return (row * K + 8 * (slot ^ ((8 * half + row) >> 1))) * 2;
+}
+BW_HD constexpr int norm_strips_half(int half) { return half * 1024; }
+
+// How many strips a workgroup takes, or 0: the NORM variant of the kernel for up to 64 rows.  Counted in what a strip of a full round
+// of the compute units takes (2.9 us for K = 2048, at 5.4 TB/s): a round its strips and 0.8 for its beginning, a part-empty last
+// round no less than 0.44 of its strips (what one compute unit pulls).  us, that variant -> strips:
+//   SwiGLU, 5 rows  11008 x 4096 46.2 -> 37.2 (7 strips)   14336 x 4096 50.7 -> 45.8 (7)   18432 x 4096 70.5 -> 65.1 (5)
+//                   9728 x 2560 29.0 -> 22.3 (6)   12000 x 2048 26.3 -> 23.6 (7)   16384 x 2048 31.9 -> 29.8 (8)
+//   stores          128256 x 4096 206 -> 194 (7)   20000 x 1024 14.6 -> 10.9 (7)
+// Where both make whole rounds the variant is as fast or faster (8192 x 2048 17.6 and 17.9 with 4 strips; stores of K = 2048: 49152
+// columns 46.0 and 47.0 with 6, 32000 30.5 and 31.7 with 8; of K = 2176 47936 39.7 and 42.2 with 7), so it stays unless the count says
+// 4 % less, 10 % for stores of one segment, 6 % for those of two.  66 products drawn over all of that: 0.71 to 1.02 of the variant's time.
+inline int norm_strips_admits(int M, int N, int K, int epilogue) {
+  const bool glu = epilogue == EPI_SWIGLU_BF16;
+  if ((!glu && epilogue != EPI_F32) || !mid_norm_admits(M, K, (N + (glu ? 31 : 63)) / (glu ? 32 : 64))) return 0;
+  const auto cost = [&](int strips) {                                  // in 1/10000
+    const int cols = strips * norm_strips_cols(glu);
+    const long long wgs = (N + cols - 1) / cols, left = wgs % 256;
+    const long long rounds = wgs / 256 * 10000 + (left ? (left * 10000 / 256 > 4400 ? left * 10000 / 256 : 4400) : 0);
+    return strips * rounds + (wgs + 255) / 256 * 8000;
+  };
+  const long long variant = cost(4);
+  long long least = variant * (glu ? 96 : K <= GEMM_SEG ? 90 : 94) / 100;
+  int best = 0;
+  for (int strips = 5; strips <= 8; ++strips) {
+    const long long c = strips == 8 ? cost(strips) * 103 / 100 : cost(strips);     // (a ring of five stages)
+    if (c < least) {
+      least = c;
+      best = strips;
+    }
+  }
+  return best;
+}
+
 // ------------------------------------------------------------------------------ decode_gemm_kernel (fused_decode.hip)
 
 #define DEC_SEG 2048

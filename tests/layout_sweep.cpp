@@ -6,7 +6,10 @@
 //     and what lane (g, r) of a matrix instruction reads for step s is exactly what was stored for row r, elements
 //     64 s + 32 kk + 8 g .. + 7 (a model of LDS holds, for every byte, which row and element was stored there);
 //   * every load of the weights' ring lands inside the ring, the loads of a stage tile the stage exactly, and the
-//     operand reads of a step stay inside the step.
+//     operand reads of a step stay inside the step;
+//   * of the kernel that gives a wave a strip of W: every descriptor lies inside W, every load of a lane inside its
+//     descriptor's row or outside the descriptor, a lane of a matrix instruction reads the row and elements of W that it
+//     wants, every output is one wave's, and a stage is asked for again only behind the step that read it.
 // It is compiled with -fsanitize=address,undefined, so an index that leaves the model's arrays aborts the run.
 // A second part applies the same checks to a variant that is not in the library any more (rows of up to 4096
 // elements in every fused kernel, up to 16 rows, two rows a wave, sixteen vectors a lane) in the two forms it may
@@ -253,6 +256,131 @@ static long sweep_decode(int waves, int stages, int stage_bytes, int rope_lw) {
   return n;
 }
 
+// ------------------------------------------------------------------------------ gemm_bf16_norm_strips_kernel
+template <int STRIPS_A_WG>
+struct StripsShape {                   // as sweep_mid_norm_launch wants it: eight waves, all of which work on the one block of rows
+  static constexpr int NW = 8, NI = 1, STRIPS = 8, RING = norm_strips_ring(STRIPS_A_WG, norm_strips_stages(STRIPS_A_WG));
+};
+
+// the normalised rows beside the rings, for every (M, K) that the launcher can take
+template <int STRIPS_A_WG>
+static long sweep_strips_rows() {
+  using S = StripsShape<STRIPS_A_WG>;
+  long n = 0;
+  for (int K = 64; K <= 2 * GEMM_SEG; K += 64)
+    for (int M = 1; M <= 16; ++M) {
+      if (!mid_norm_admits(M, K, 64)) continue;
+      const int nv = mid_norm_vectors_a_lane(K), row_step = mid_norm_row_step(K);
+      CHECK(nv == 8 || M <= 8, "strips: %d rows of %d, sixteen vectors a lane", M, K);
+      n += sweep_mid_norm_launch<S>("norm+product, a wave a strip", M, K, nv == 16 || M <= 8 ? 1 : 2, nv, row_step, mid_norm_lds_bytes(S::RING, K, row_step), true);
+    }
+  return n;
+}
+
+// a wave's ring: stages in turn, the one of the step before asked for again
+static long sweep_strips_ring(int strips) {
+  long n = 0;
+  const int stages = norm_strips_stages(strips);
+  std::vector<int> owner((size_t)norm_strips_ring(strips, stages) / NORM_STRIP_STAGE, -1);
+  for (int wave = 0; wave < strips; ++wave) {
+    const int base = norm_strips_ring_of(wave, stages);
+    for (int st = 0; st < stages; ++st) {
+      const int off = base + st * NORM_STRIP_STAGE;
+      CHECK(off >= 0 && off + NORM_STRIP_STAGE <= norm_strips_ring(strips, stages), "strips: stage %d of wave %d at %d", st, wave, off);
+      CHECK(owner[off / NORM_STRIP_STAGE] == -1, "strips: stage %d of wave %d is wave %d's", st, wave, owner[off / NORM_STRIP_STAGE]);
+      owner[off / NORM_STRIP_STAGE] = wave;
+    }
+    std::vector<int> holds(stages, -1);                             // the step whose weights a stage holds
+    for (int st = 0; st < stages - 1; ++st) holds[st] = st;
+    int at = 0;
+    for (int step = 0; step < 70; ++step) {
+      CHECK(at >= 0 && at % NORM_STRIP_STAGE == 0 && at < stages * NORM_STRIP_STAGE && holds[at / NORM_STRIP_STAGE] == step, "strips: step %d reads the stage at %d", step, at);
+      const int again = norm_strips_before(at, stages);
+      CHECK(again >= 0 && again < stages * NORM_STRIP_STAGE && holds[again / NORM_STRIP_STAGE] < step, "strips: step %d asks for the stage at %d, which has not been read", step, again);
+      holds[again / NORM_STRIP_STAGE] = step + stages - 1;
+      at = norm_strips_next(at, stages);
+      n += 2;
+    }
+  }
+  return n;
+}
+
+// W [N (SwiGLU: 2 N), K] through the strips' descriptors into a stage, and the outputs
+static long sweep_strips_weights(bool glu, int N, int K, int strips) {
+  long n = 0;
+  const int cols = norm_strips_cols(glu), wgs = (N + strips * cols - 1) / (strips * cols), all = glu ? 2 * N : N;
+  std::vector<int> outputs(N, 0);
+  for (int block = 0; block < wgs; ++block)
+    for (int wave = 0; wave < 8; ++wave) {
+      const NormStrip s = norm_strips_of_wave(glu, block, strips, wave, N);
+      if (!s.working) continue;
+      CHECK(s.have >= 1 && s.have <= cols && s.n0 + s.have <= N, "strips: %d outputs from %d of %d", s.have, s.n0, N);
+      int in_stage[16];                                             // row of W behind each of the stage's rows, or -1
+      for (int half = 0; half < 2; ++half) {
+        CHECK(s.rows[half] >= 0 && s.rows[half] <= 8 && s.row[half] < (size_t)all && s.row[half] + s.rows[half] <= (size_t)all,
+              "strips: descriptor of %d rows from %zu of %d", s.rows[half], s.row[half], all);
+        for (int row = 0; row < 8; ++row) in_stage[8 * half + row] = row < s.rows[half] ? (int)s.row[half] + row : -1;
+      }
+      for (int c = 0; c < cols; ++c) {
+        const int out = s.n0 + c;
+        if (out < N) ++outputs[out];
+        if (out >= N) continue;
+        CHECK(in_stage[c] == out, "strips: output %d has row %d of W", out, in_stage[c]);
+        if (glu) CHECK(in_stage[8 + c] == N + out, "strips: output %d has up row %d of W", out, in_stage[8 + c]);
+      }
+      // (the lanes' ways do not hang on the strip)
+      if (block > 0 || wave > 0) continue;
+      const int steps = K / 64;
+      for (int step = 0; step < steps; ++step) {
+        std::vector<int> who(NORM_STRIP_STAGE / 2, -1);             // per 2 bytes of the stage: stage row * 65536 + element of the row
+        for (int half = 0; half < 2; ++half)
+          for (int lane = 0; lane < 64; ++lane) {
+            const int off = norm_strips_load_offset(half, lane, K) + step * 128, dst = norm_strips_half(half) + lane * 16;
+            const int row = off / (2 * K), element = off % (2 * K) / 2;
+            CHECK(off >= 0 && row == lane >> 3 && element % 8 == 0 && element / 64 == step && element + 8 <= K, "strips: lane %d of half %d loads from %d of a row of %d", lane, half, off, K);
+            CHECK(dst >= 0 && dst + 16 <= NORM_STRIP_STAGE, "strips: a load lands at %d", dst);
+            for (int e = 0; e < 8; ++e) {
+              CHECK(who[dst / 2 + e] == -1, "strips: two loads land at %d", dst);
+              who[dst / 2 + e] = (8 * half + row) * 65536 + element + e;
+            }
+            ++n;
+          }
+        for (int lane = 0; lane < 64; ++lane)
+          for (int kk = 0; kk < 2; ++kk) {
+            const int r = lane & 15, g = lane >> 4, off = mid_operand_offset(r, g, kk);
+            CHECK(off >= 0 && off + 16 <= NORM_STRIP_STAGE, "strips: operand read at %d", off);
+            for (int e = 0; e < 8; ++e)
+              CHECK(who[off / 2 + e] == r * 65536 + 64 * step + 32 * kk + 8 * g + e, "strips: lane %d reads row %d element %d", lane, who[off / 2 + e] >> 16, who[off / 2 + e] & 0xffff);
+            ++n;
+          }
+      }
+    }
+  for (int c = 0; c < N; ++c) CHECK(outputs[c] == 1, "strips: output %d of %d is stored %d times", c, N, outputs[c]);
+  return n;
+}
+
+static long sweep_strips() {
+  long n = sweep_strips_rows<5>() + sweep_strips_rows<6>() + sweep_strips_rows<7>() + sweep_strips_rows<8>();
+  for (int strips = 5; strips <= 8; ++strips) {
+    n += sweep_strips_ring(strips);
+    for (int glu = 0; glu < 2; ++glu) {
+      for (int N = 1; N <= 300; ++N) n += sweep_strips_weights(glu, N, 64, strips);
+      for (int N : {8200, 11008, 14329, 16377, 32749, 128256}) n += sweep_strips_weights(glu, N, 192, strips);
+      for (int K = 64; K <= 2 * GEMM_SEG; K += 64) n += sweep_strips_weights(glu, 17, K, strips);
+    }
+  }
+  // what the launcher's choice can be: none, or one of the forms above
+  for (int epilogue : {EPI_F32, EPI_SWIGLU_BF16, EPI_BF16, EPI_ADD_F32, EPI_QKV_ROPE})
+    for (int N = 64; N < 140000; N += 61)
+      for (int K : {32, 64, 2048, 2112, 2176, 4096, 4160})
+        for (int M : {0, 1, 8, 9, 16, 17}) {
+          const int s = norm_strips_admits(M, N, K, epilogue);
+          CHECK(s == 0 || (s >= 5 && s <= 8 && mid_norm_admits(M, K, 64) && (epilogue == EPI_F32 || epilogue == EPI_SWIGLU_BF16)), "strips: %d for %d x %d x %d", s, M, N, K);
+          ++n;
+        }
+  return n;
+}
+
 int main() {
   std::printf("ok row-vectors-8 %ld\n", sweep_row_vectors(8, GEMM_SEG));
   std::printf("ok row-vectors-16 %ld\n", sweep_row_vectors(16, 2 * GEMM_SEG));
@@ -285,6 +413,7 @@ int main() {
   rows += sweep_mid_norm<MidShape<EPI_QKV_ROPE, 1, true, true, false>>("norm+q|k|v, half a head a workgroup, four waves", false);
   rows += sweep_mid_norm<MidShape<EPI_F32, 1, true, false, false>>("norm+product, 64 columns, four waves", false);
   std::printf("ok mid-norm-rows %ld\n", rows);
+  std::printf("ok norm-strips %ld\n", sweep_strips());
 
   long dec = 0;
   dec += sweep_decode(4, 8, 2048, 0);       // plain epilogues: four strips a workgroup, eight stages

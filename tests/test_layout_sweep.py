@@ -37,6 +37,7 @@ def test_every_admitted_shape_stays_inside_its_row_and_its_lds(sweep_output):
     # each part of the sweep ran, over a number of addresses that says it was not empty
     assert counts["row-vectors-8"] > 1e4 and counts["row-vectors-16"] > 5e4 and counts["mid-ring"] > 3e4
     assert counts["mid-norm-rows"] > 1e7 and counts["decode-rows"] > 1e7
+    assert counts["norm-strips"] > 1e7
     assert "ok in-library failures 0" in out
 
 
