@@ -55,7 +55,6 @@ __device__ __forceinline__ float row_sumsq(const float* __restrict__ xr, int dim
 // row above, or for the first row of a request in this step what the state slot holds (zeros for a new request).
 // The wave of a request's first row also leaves the h of the request's last row in the slot, after it has read it:
 // nothing else reads or writes that slot in this launch.  A wave a row.
-#define SHIFT_REGS 8      // 16-byte vectors of a row a lane keeps (rows of up to 2,048 elements)
 template <typename OT>
 __global__ __launch_bounds__(256) void norm_shift_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w,
                                                          const float* __restrict__ mix, float* __restrict__ state,
@@ -86,53 +85,6 @@ __global__ __launch_bounds__(256) void norm_shift_kernel(const float* __restrict
     const f32x4* lv = reinterpret_cast<const f32x4*>(x + (size_t)last * ldx);
     const f32x4* wv = reinterpret_cast<const f32x4*>(w);
     const f32x4* mv = reinterpret_cast<const f32x4*>(mix);
-    if (!is_first && nvec <= 64 * SHIFT_REGS) {
-      // both rows, the weight and the first mixing vector in registers, asked for once and at once: the rows came twice, the second time
-      // behind two sums.  2,048 rows to bfloat16, us: 2,048 wide 8.6 -> 7.4, 1,028 7.1 -> 5.8.
-      f32x4 xq[SHIFT_REGS], pq[SHIFT_REGS], wq[SHIFT_REGS], mq[SHIFT_REGS];
-#pragma unroll
-      for (int j = 0; j < SHIFT_REGS; ++j) {
-        if (64 * j >= nvec) continue;                                          // (scalar)
-        const int c = min(64 * j + lane, nvec - 1);
-        xq[j] = xv[c];
-        pq[j] = pv[c];
-        wq[j] = wv[c];
-        mq[j] = mv[c];
-      }
-      // (row_sumsq_vec's chains)
-      float sx = 0.0f, sp = 0.0f;
-#pragma unroll
-      for (int j = 0; j < SHIFT_REGS; ++j) {
-        if (64 * j + lane >= nvec) continue;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          sx = fmaf(xq[j][e], xq[j][e], sx);
-          sp = fmaf(pq[j][e], pq[j][e], sp);
-        }
-      }
-      const float inv = 1.0f / sqrtf(wave_sum(sx) / (float)dim + eps), invp = 1.0f / sqrtf(wave_sum(sp) / (float)dim + eps);
-#pragma unroll
-      for (int j = 0; j < SHIFT_REGS; ++j) {
-        const int c = 64 * j + lane;
-        if (c >= nvec) continue;
-        f32x4 hq, dq;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          hq[e] = (xq[j][e] * inv) * wq[j][e];
-          dq[e] = (pq[j][e] * invp) * wq[j][e] - hq[e];
-        }
-        for (int m = 0; m < nmix; ++m) {
-          const f32x4 mm = m == 0 ? mq[j] : mv[(size_t)m * nvec + c];
-          f32x4 r;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) r[e] = fmaf(dq[e], mm[e], hq[e]);
-          OT* om = o + (size_t)m * dim;
-          if constexpr (sizeof(OT) == 2) *reinterpret_cast<u32x2*>(om + 4 * c) = (u32x2){pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
-          else *reinterpret_cast<f32x4*>(om + 4 * c) = r;
-        }
-      }
-      return;
-    }
     const float inv = 1.0f / sqrtf(row_sumsq_vec(xv, nvec, lane) / (float)dim + eps);
     const float invp = is_first ? 1.0f : 1.0f / sqrtf(row_sumsq_vec(pv, nvec, lane) / (float)dim + eps);
     const float invl = !is_first || last == row ? inv : 1.0f / sqrtf(row_sumsq_vec(lv, nvec, lane) / (float)dim + eps);

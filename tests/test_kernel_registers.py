@@ -45,3 +45,10 @@ def test_memory_walk_leaves_room_for_a_second_wave(mode, dim):
     found = [k for name, k in kernels().items() if f"linear_recurrence_kernelILi{mode}ELi{dim}ELi0E" in name]
     assert len(found) == 1
     assert found[0][".vgpr_count"] <= 256          # (accumulation registers included)
+
+
+def test_norm_with_shift_leaves_room_for_four_waves():
+    """Four waves of up to 128 registers share a SIMD; with both rows kept in registers the kernel took 142, three waves."""
+    found = [k for name, k in kernels().items() if "norm_shift_kernelI" in name]
+    assert len(found) == 2
+    assert all(k[".vgpr_count"] <= 128 for k in found)
