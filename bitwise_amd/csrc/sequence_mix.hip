@@ -1030,10 +1030,15 @@ __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __rest
 }
 
 // The same for heads of whole rows of lanes and many (row, head) items: a wave takes HG_ITEMS neighbouring items and asks for all
-// they need before the first sum.  One item a wave was a chain of four trips to memory beside 64 to 256 elements.
-// bfloat16, us: 2048 x 16 heads of 128 15.6 -> 11.9, 2048 x 8 of 256 13.9 -> 11.4; 10,000 items of 64 to 128 as they were or 3 to 6 % slower.
+// they need before the first sum.  One item a wave was a chain of four trips to memory beside 64 to 256 elements; four leave a quarter of
+// the waves, which few items feel.  One item a wave -> four, us to bfloat16, behind a kernel that has just written o (to 32 bit alike):
+//   items                  6,144         8,192         10,240        12,288        16,384        32,768
+//   heads of 64            3.8 -> 4.4    4.4 -> 4.5    5.2 -> 5.1    5.5 -> 5.0    6.3 -> 5.6    10.8 -> 8.3
+//   heads of 128           4.9 -> 5.2    5.4 -> 5.3    7.0 -> 6.2    7.5 -> 6.4    9.1 -> 8.1    19.7 -> 13.1
+//   heads of 256           6.5 -> 7.0    8.1 -> 7.9    13.2 -> 10.0  14.7 -> 10.7  18.0 -> 13.2  33.4 -> 18.5
+// so from 10,240 on.  Inside a Kuponex prompt of 2,048 tokens, 32,768 items of 128: 16.6 -> 13.3.
 #define HG_ITEMS 4
-#define HG_MIN_ITEMS 16384
+#define HG_MIN_ITEMS 10240
 template <typename OT, int EV>
 __global__ __launch_bounds__(256) void head_norm_gate_items_kernel(const float* __restrict__ o, int ldi, const float* __restrict__ weight,
                                                                    int wstride, const float* __restrict__ g, int ldg, int gate,

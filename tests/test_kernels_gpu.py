@@ -1290,6 +1290,42 @@ def test_normalised_rows_by_strips_of_their_own_equal_the_separate_kernels(gpu, 
     assert torch.equal(fused[:M], sep) and (fused[M] == 5.0).all()
 
 
+@pytest.mark.parametrize("vdim", [64, 128, 256])
+@pytest.mark.parametrize("rows,heads", [(1463, 7), (10241, 1), (641, 16), (2341, 7), (81, 127)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_gated_head_norms_of_many_items_equal_those_of_few(gpu, vdim, rows, heads, bf16):
+    """From 10,240 (row, head) items on a wave takes four of them, fewer go one a wave: one call and the same rows in slices, last
+    waves of one to four items, both gates, weights a head and shared, gates of wider rows, padding rows among a wave's four; the same bits, and within
+    what 32-bit sums of squares, an exponential and six roundings give of the 64-bit result."""
+    assert rows * heads >= 10240 > rows * heads // 2
+    g = torch.Generator().manual_seed(rows + vdim)
+    o = (torch.randn(rows, heads * vdim, generator=g) * 3).to(gpu)
+    gates = torch.randn(rows, heads * vdim + 12, generator=g).to(gpu)
+    pos = torch.arange(rows, dtype=torch.int32)
+    pos[3::5] = -1
+    pos[-1] = rows
+    positions = pos.to(gpu)
+    kind, live = torch.bfloat16 if bf16 else torch.float32, (pos >= 0).to(gpu)
+    for gate, per_head in ((ops.GATE_SILU, True), (ops.GATE_SIGMOID, False)):
+        w = torch.randn(heads * vdim if per_head else vdim, generator=g).to(gpu)
+        one, cut = (torch.full((rows, heads * vdim), 5.0, device=gpu, dtype=kind) for _ in range(2))
+        ops.head_norm_gate(o, w, per_head, gates, 8, gate, one, positions, rows, heads, vdim, 1e-6)
+        at, step = 0, (rows + 1) // 2
+        while at < rows:
+            n = min(step, rows - at)
+            assert n * heads < 10240
+            ops.head_norm_gate(o[at:at + n], w, per_head, gates[at:at + n], 8, gate, cut[at:at + n], positions[at:at + n], n, heads, vdim, 1e-6)
+            at += n
+        assert torch.equal(one, cut)
+        assert (one[~live] == 5.0).all()
+        o64, z = o.double().view(rows, heads, vdim), gates[:, 8:8 + heads * vdim].double().view(rows, heads, vdim)
+        act = torch.sigmoid(z) * (z if gate == ops.GATE_SILU else 1.0)
+        ref = (o64 / torch.sqrt((o64 * o64).mean(-1, keepdim=True) + 1e-6) * w.double().view(-1, vdim) * act).view(rows, -1)
+        # sum of squares: vdim / 64 + 6 roundings, halved by the root; the rest: root, division, exponential, sum, reciprocal, four products
+        bound = ((vdim / 64 + 6) / 2 + 12) * 2.0 ** -24 + (2.0 ** -8 if bf16 else 0.0)
+        assert ((one[live].double() - ref[live]).abs() <= bound * ref[live].abs()).all()
+
+
 @pytest.mark.parametrize("heads,kvh,M,tile", [(71, 13, 300, (64, 128)), (101, 12, 250, (128, 64)), (71, 13, 384, (128, 128)),
                                               (72, 12, 700, (128, 256)), (71, 13, 1345, (160, 256)), (125, 17, 1000, (192, 256)),
                                               (71, 12, 2041, (256, 192)), (75, 11, 2041, (256, 256))])
