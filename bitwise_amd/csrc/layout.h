@@ -185,13 +185,13 @@ BW_HD constexpr int norm_strips_half(int half) { return half * 1024; }
 
 // How many strips a workgroup takes, or 0: the NORM variant of the kernel for up to 64 rows.  Counted in what a strip of a full round
 // of the compute units takes (2.9 us for K = 2048, at 5.4 TB/s): a round its strips and 0.8 for its beginning, a part-empty last
-// round no less than 0.44 of its strips (what one compute unit pulls).  us, that variant -> strips:
-//   SwiGLU, 5 rows  11008 x 4096 46.2 -> 37.2 (7 strips)   14336 x 4096 50.7 -> 45.8 (7)   18432 x 4096 70.5 -> 65.1 (5)
-//                   9728 x 2560 29.0 -> 22.3 (6)   12000 x 2048 26.3 -> 23.6 (7)   16384 x 2048 31.9 -> 29.8 (8)
-//   stores          128256 x 4096 206 -> 194 (7)   20000 x 1024 14.6 -> 10.9 (7)
-// Where both make whole rounds the variant is as fast or faster (8192 x 2048 17.6 and 17.9 with 4 strips; stores of K = 2048: 49152
-// columns 46.0 and 47.0 with 6, 32000 30.5 and 31.7 with 8; of K = 2176 47936 39.7 and 42.2 with 7), so it stays unless the count says
-// 4 % less, 10 % for stores of one segment, 6 % for those of two.  66 products drawn over all of that: 0.71 to 1.02 of the variant's time.
+// round no less than 0.44 of its strips (what one compute unit pulls).  5 rows, us, that variant -> strips as many as the count takes (the best of 5 to 8):
+//   SwiGLU   11008 x 4096 46.4 -> 38.4 (7)   14336 x 4096 50.1 -> 47.7 (7)   18432 x 4096 68.6 -> 63.4 with 6 (62.6 with 5)
+//            9728 x 2560 28.7 -> 22.6 with 7 (22.1 with 6)   12000 x 2048 25.5 -> 24.6 with 6 (23.8 with 8)   16384 x 2048 32.0 -> 31.4 (8)
+//   stores   128256 x 4096 202 -> 194 (7)   20000 x 1024 14.6 -> 11.2 with 5 (10.9 with 7)
+// Where both make whole rounds the variant is as fast or faster (8192 x 2048 17.7, 17.9 with 8; stores of K = 2048: 49152 columns 44.4
+// and 46.1 with 7, 32000 29.7 and 30.7 with 8), so it stays unless the count says 4 % less, 10 % for stores of one segment, 6 % for those of
+// two (47936 x 2176 stays at 42.8, 42.2 with 6).  66 products drawn over all of that: 0.71 to 1.02 of the variant's time.
 inline int norm_strips_admits(int M, int N, int K, int epilogue) {
   const bool glu = epilogue == EPI_SWIGLU_BF16;
   if ((!glu && epilogue != EPI_F32) || !mid_norm_admits(M, K, (N + (glu ? 31 : 63)) / (glu ? 32 : 64))) return 0;

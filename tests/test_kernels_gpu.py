@@ -1267,24 +1267,33 @@ def test_32_bit_products_that_keep_their_rotation_as_a_kernel(gpu):
                               torch.zeros(16, 32, device=gpu), cache, cache.clone(), 65, 3, 1, 64, 16)
 
 
-@pytest.mark.parametrize("M,N,K,strips", [(1, 8208, 64, 6), (8, 8256, 512, 6), (16, 11000, 128, 7), (5, 11008, 2048, 7), (9, 14329, 192, 7), (8, 8200, 2560, 5),
-                                          (3, 14336, 4096, 7), (2, 16384, 2048, 8), (13, 16377, 1024, 8), (8, 18440, 4096, 5), (1, 24576, 2176, 6)])
-@pytest.mark.parametrize("glu", [True, False])
-def test_normalised_rows_by_strips_of_their_own_equal_the_separate_kernels(gpu, M, N, K, strips, glu):
+@pytest.mark.parametrize("M,N,K,strips,epilogue", [
+    (1, 8208, 64, 6, ops.EPI_SWIGLU_BF16), (8, 8256, 512, 6, ops.EPI_SWIGLU_BF16), (16, 11000, 128, 7, ops.EPI_SWIGLU_BF16), (5, 11008, 2048, 7, ops.EPI_SWIGLU_BF16),
+    (9, 14329, 192, 7, ops.EPI_SWIGLU_BF16), (8, 8200, 2560, 5, ops.EPI_SWIGLU_BF16), (3, 14336, 4096, 7, ops.EPI_SWIGLU_BF16), (2, 16384, 2048, 8, ops.EPI_SWIGLU_BF16),
+    (13, 16377, 1024, 8, ops.EPI_SWIGLU_BF16), (8, 18440, 4096, 5, ops.EPI_SWIGLU_BF16), (1, 24576, 2176, 6, ops.EPI_SWIGLU_BF16),
+    # columns of the last strip: 1, 7 and 8 (none for its second descriptor), 9 and 15; the last workgroup's strips: all, one, some
+    (1, 16385, 64, 5, ops.EPI_F32), (16, 16391, 192, 5, ops.EPI_F32), (9, 16400, 512, 5, ops.EPI_F32), (8, 16392, 2176, 5, ops.EPI_F32), (3, 16409, 2048, 6, ops.EPI_F32),
+    (16, 16424, 1024, 7, ops.EPI_F32), (5, 16431, 4096, 7, ops.EPI_F32), (13, 24577, 1024, 7, ops.EPI_F32), (4, 28673, 2560, 8, ops.EPI_F32),
+    (8, 28688, 4096, 8, ops.EPI_F32), (1, 28687, 2176, 8, ops.EPI_F32)])
+@pytest.mark.parametrize("norm_bf16", [True, False])
+def test_normalised_rows_by_strips_of_their_own_equal_the_separate_kernels(gpu, M, N, K, strips, epilogue, norm_bf16):
     """Products of more workgroups than compute units, a wave a strip: last strips and workgroups that are part empty, one to eight
-    rows and up to sixteen, K shorter than the ring, one segment and two; the bits of RMSNorm and product one after the other."""
+    rows and up to sixteen, K shorter than the ring, one segment and two, the norm's weight in both types; the bits of RMSNorm and product one
+    after the other."""
+    glu = epilogue == ops.EPI_SWIGLU_BF16
+    assert ops.norm_gemm_strips(M, N, K, epilogue) == strips
     g = torch.Generator().manual_seed(M + N + K)
-    columns = N if glu else 2 * N
-    epilogue = ops.EPI_SWIGLU_BF16 if glu else ops.EPI_F32
-    if glu:
-        assert ops.norm_gemm_strips(M, N, K, epilogue) == strips
     x = (torch.randn(M, K, generator=g) * 2).to(gpu)
-    nw = (1 + 0.1 * torch.randn(K, generator=g)).bfloat16().to(gpu)
-    w = (torch.randn(2 * N, K, generator=g) * 0.05).bfloat16().to(gpu)
+    nw = 1 + 0.1 * torch.randn(K, generator=g)
+    nw = (nw.bfloat16() if norm_bf16 else nw).to(gpu)
+    # (rows of NaN behind the weight's own: what a strip reads past its columns must not matter)
+    held = torch.full(((2 * N if glu else N) + 16, K), float("nan"), dtype=torch.bfloat16)
+    held[:-16] = torch.randn(held.shape[0] - 16, K, generator=g) * 0.05
+    w = held.to(gpu)[:-16]
     h = torch.zeros(M, K, device=gpu, dtype=torch.bfloat16)
     ops.rmsnorm(x, nw, h, M, 1e-5)
     kind = torch.bfloat16 if glu else torch.float32
-    sep, fused = torch.zeros(M, columns, device=gpu, dtype=kind), torch.full((M + 1, columns), 5.0, device=gpu, dtype=kind)
+    sep, fused = torch.zeros(M, N, device=gpu, dtype=kind), torch.full((M + 1, N), 5.0, device=gpu, dtype=kind)
     ops.gemm_bf16(h, w, sep, M, epilogue)
     ops.norm_gemm_bf16(x, nw, 1e-5, w, fused, M, epilogue)
     assert torch.equal(fused[:M], sep) and (fused[M] == 5.0).all()
