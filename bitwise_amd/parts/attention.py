@@ -54,19 +54,23 @@ def plan_tiles(ctx, tokens_per_tile: int, group_tiles: int = 1, join: bool = Fal
     64-key partition).  A step of nothing but one row per request (``ctx.one_row_per_request``, the shape of a
     captured decode step) needs no tile list: tile t is row t of request t.  ``join``: single tokens may go into the
     portions' launch (JOIN_PARTITIONS), with the layer's ``window`` or ``chunk``.  The plan is made once per step
-    and kept in the context for the other layers."""
+    and kept in the context for the other layers, those with other windows too where it is the same."""
     if getattr(ctx, "one_row_per_request", False):
         return AttentionPlan(None, 0, None, ctx.rows)
 
+    def joins() -> bool:
+        singles = [s.pos0 for s in ctx.segments if len(s.tokens) == 1]
+        longest = max((_partitions(s.pos0 + len(s.tokens) - 1, window, chunk) for s in ctx.segments if len(s.tokens) > 1), default=0)
+        return bool(singles) and longest > 0 and all(_partitions(p, window, chunk) <= longest + JOIN_PARTITIONS for p in singles)
+
+    joined = join and ctx.memo(("attention_join", window, chunk), joins)
+
     def make() -> AttentionPlan:
         fold, split = [], []
-        singles = [i for i, s in enumerate(ctx.segments) if len(s.tokens) == 1]
-        longest = max((_partitions(s.pos0 + len(s.tokens) - 1, window, chunk) for s in ctx.segments if len(s.tokens) > 1), default=0)
-        joined = join and longest > 0 and all(_partitions(ctx.segments[i].pos0, window, chunk) <= longest + JOIN_PARTITIONS for i in singles)
         # (the kernel starts a list's last tiles first: the singles, the shortest in front, start behind the portions)
-        order = range(len(ctx.segments))
+        order = list(range(len(ctx.segments)))
         if joined:
-            order = sorted(singles, key=lambda i: ctx.segments[i].pos0) + [i for i in order if len(ctx.segments[i].tokens) > 1]
+            order.sort(key=lambda i: (0, ctx.segments[i].pos0) if len(ctx.segments[i].tokens) == 1 else (1, 0))
         for i in order:
             s = ctx.segments[i]
             n, r0 = len(s.tokens), ctx.seq_start[i]
@@ -83,7 +87,7 @@ def plan_tiles(ctx, tokens_per_tile: int, group_tiles: int = 1, join: bool = Fal
         return AttentionPlan(dev[:len(fold)].contiguous() if fold else None, len(fold),
                              dev[len(fold):].contiguous() if split else None, len(split))
 
-    return ctx.memo(("attention_tiles", tokens_per_tile, group_tiles, join, window, chunk), make)
+    return ctx.memo(("attention_tiles", tokens_per_tile, group_tiles, joined), make)
 
 
 def _split_scratch(ws, tiles: int, table_width: int, heads: int, kv_heads: int, head_dim: int):

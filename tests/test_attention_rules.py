@@ -57,3 +57,14 @@ def test_single_tokens_join_a_portion_whose_walk_is_about_as_long(rows, window, 
     if joined:
         lone = [ctx.segments[t[2]].pos0 for t in fold if t[1] and len(ctx.segments[t[2]].tokens) == 1]
         assert lone == sorted(lone) and all(len(ctx.segments[t[2]].tokens) == 1 for t in fold[:8 * len(lone)])
+
+
+@pytest.mark.parametrize("rows,join,same", [([(0, 300), (500, 1)], False, True), ([(0, 300), (5, 40)], True, True), ([(300, 1), (9, 1)], True, True),
+                                            ([(0, 300), (9, 1), (200, 1)], True, True), ([(9000, 1), (0, 64)], True, False)])
+def test_layers_whose_windows_change_nothing_share_a_plan(rows, join, same):
+    """A plan is a list made on the host and a copy to the device: layers of different windows and chunks make another one only
+    where it differs (here the last: with a window the far token joins the portion, without it does not)."""
+    segments = [Segment([0] * n, pos, [list(range((pos + n + 15) // 16))], i) for i, (pos, n) in enumerate(rows)]
+    ctx = StepContext(segments, 1, SimpleNamespace(device=torch.device("cpu"), page_size=16))
+    plans = [plan_tiles(ctx, 4, 8, join, window, chunk) for window, chunk in ((0, 0), (70, 0), (128, 0), (0, 64))]
+    assert all(p is plans[1] for p in plans[2:]) and (plans[0] is plans[1]) == same
