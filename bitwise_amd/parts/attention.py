@@ -23,12 +23,19 @@ from .linear import Linear
 # own once its context is at least this long (same bits either way; this only buys parallelism).
 DECODE_MIN_CONTEXT = 128
 
-# Beside a prompt portion all single tokens of a step go into the portion's launch, as tiles of one row, if none of them walks
-# more 64-key partitions than the longest of the portion's rows does, and this many: a launch of its own costs what a dozen partitions
-# take there, and the portion's longest workgroups leave room beside them.  Heads of 64 and 128, microseconds, two launches -> one: 1,341 tokens at
-# 640 and 7 singles of up to 592 keys (32 heads of 64) 50.6 -> 39.9; 854 tokens and 60 of up to 1,186 (32 heads of 128 on 8) 74.5 -> 53.3; 65 tokens and 22 of
-# up to 416 19.1 -> 13.6.  80 drawn mixes: ten partitions more 0.63 to 1.02 of the time, 15 more 1.05 to 1.08, 35 more 1.8.
+# Beside a prompt portion all single tokens of a step go into the portion's launch, as tiles of one row, where that launch takes no longer with
+# them than a second one behind it.  Two things decide.  None of them may walk more 64-key partitions than the longest of the
+# portion's rows does, and JOIN_PARTITIONS: a launch of its own costs what a dozen partitions take there (80 drawn mixes: ten more 0.63 to
+# 1.02 of the time, 15 more 1.05 to 1.08, 35 more 1.8).  And all of them together may walk no more, over the kernel's items (a request's
+# key heads), than JOIN_WORK: so much, and so much more for each partition of the longest row.  A launch of many workgroups is bound by
+# what the chip does at once, where the decode kernel does a walk of ten partitions in up to 0.8 of the fold kernel's time; what joining saves is the
+# portion's own time, some 6 us and one a partition.  Two launches -> one, us: 1,341 tokens at 640 and 7 singles of up to 592 keys (32 heads of
+# 64) 50.6 -> 39.9; 854 tokens and 60 of up to 1,186 (32 heads of 128 on 8) 74.5 -> 53.3; a portion of 2 to 16 rows behind 8,000 keys and 14 of up to
+# 2,048 185 -> 168, 5,000 keys and 177 of up to 5,500 713 -> 610; a short portion and 230 of 400 to 500 keys (32 heads of 128) 242 -> 290, so two.
+# 961 drawn mixes of 1 to 4 portions of 2 to 1,900 rows at 0 to 8,000 with 1 to 256 singles: 0.49 to 1.03 of two launches' time by this
+# rule (1.20 by the walks' lengths alone), 1.001 (heads of 64) and 1.002 (128) of the better choice's in the mean.
 JOIN_PARTITIONS = 8
+JOIN_WORK = {64: (20000, 3200), 128: (5600, 1600)}       # head size -> partitions times items; the sizes whose fold kernel is the fast one
 PARTITION = 64
 
 
@@ -47,23 +54,25 @@ def _partitions(pos: int, window: int, chunk: int) -> int:
     return pos // PARTITION - first // PARTITION + 1
 
 
-def plan_tiles(ctx, tokens_per_tile: int, group_tiles: int = 1, join: bool = False, window: int = 0, chunk: int = 0) -> AttentionPlan:
+def plan_tiles(ctx, tokens_per_tile: int, group_tiles: int = 1, join: bool = False, window: int = 0, chunk: int = 0, items: int = 1,
+               head_dim: int = 64) -> AttentionPlan:
     """Cut a step's segments into tiles of up to ``tokens_per_tile`` consecutive rows of one request; every
     request's run of tiles is padded with empty tiles to a multiple of ``group_tiles`` (the tiles one wave owns
     must belong to one request).  Single decoded tokens with a long context go to the decode kernel (a wave per
     64-key partition).  A step of nothing but one row per request (``ctx.one_row_per_request``, the shape of a
     captured decode step) needs no tile list: tile t is row t of request t.  ``join``: single tokens may go into the
-    portions' launch (JOIN_PARTITIONS), with the layer's ``window`` or ``chunk``.  The plan is made once per step
+    portions' launch (JOIN_PARTITIONS, JOIN_WORK), with the layer's ``window`` or ``chunk``, ``items`` and ``head_dim``.  The plan is made once per step
     and kept in the context for the other layers, those with other windows too where it is the same."""
     if getattr(ctx, "one_row_per_request", False):
         return AttentionPlan(None, 0, None, ctx.rows)
 
     def joins() -> bool:
-        singles = [s.pos0 for s in ctx.segments if len(s.tokens) == 1]
+        singles = [_partitions(s.pos0, window, chunk) for s in ctx.segments if len(s.tokens) == 1]
         longest = max((_partitions(s.pos0 + len(s.tokens) - 1, window, chunk) for s in ctx.segments if len(s.tokens) > 1), default=0)
-        return bool(singles) and longest > 0 and all(_partitions(p, window, chunk) <= longest + JOIN_PARTITIONS for p in singles)
+        fixed, more = JOIN_WORK[head_dim]
+        return bool(singles) and longest > 0 and max(singles) <= longest + JOIN_PARTITIONS and sum(singles) * items <= fixed + more * longest
 
-    joined = join and ctx.memo(("attention_join", window, chunk), joins)
+    joined = join and ctx.memo(("attention_join", window, chunk, items, head_dim), joins)
 
     def make() -> AttentionPlan:
         fold, split = [], []
@@ -125,10 +134,9 @@ def attend_bf16(ctx, call, q, out, heads: int, kv_heads: int, head_dim: int, win
     ws = ctx.ws
     table = ctx.block_tables[call.group]
     extra = _mask_and_cap(sink, chunk, softcap)
-    tokens_per_tile = 16 // min(heads // kv_heads, 16)
-    # (the sizes whose fold kernel is the fast one)
-    join = head_dim in (64, 128) and ws.page_size >= 16
-    plan = plan_tiles(ctx, tokens_per_tile, ops.fold_group_tiles(head_dim), join, window, chunk)
+    heads_per_tile = min(heads // kv_heads, 16)
+    tokens_per_tile, items = 16 // heads_per_tile, kv_heads * -(-(heads // kv_heads) // heads_per_tile)
+    plan = plan_tiles(ctx, tokens_per_tile, ops.fold_group_tiles(head_dim), head_dim in JOIN_WORK and ws.page_size >= 16, window, chunk, items, head_dim)
     common = (call.k_cache, call.v_cache, out, heads, kv_heads, head_dim, ws.page_size, window, scale)
     if plan.fold_count:
         ops.attention_bf16(q, ctx.positions, table, plan.fold_tiles, plan.fold_count, *common, **extra)

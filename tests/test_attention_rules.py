@@ -68,3 +68,18 @@ def test_layers_whose_windows_change_nothing_share_a_plan(rows, join, same):
     ctx = StepContext(segments, 1, SimpleNamespace(device=torch.device("cpu"), page_size=16))
     plans = [plan_tiles(ctx, 4, 8, join, window, chunk) for window, chunk in ((0, 0), (70, 0), (128, 0), (0, 64))]
     assert all(p is plans[1] for p in plans[2:]) and (plans[0] is plans[1]) == same
+
+
+# head size, key heads, (position, rows) of the longest portion, single tokens' positions (the mean of those measured), microseconds in two launches, in one
+MIXES = [(128, 32, (188, 2), [480] * 230, 241.8, 289.9), (128, 32, (0, 5), [310] * 141, 128.6, 151.2), (128, 8, (0, 40), [540] * 202, 89.8, 94.8),
+         (64, 32, (190, 2), [650] * 254, 231.4, 253.0), (64, 32, (500, 10), [550] * 216, 180.2, 192.4), (128, 32, (890, 6), [730] * 176, 357.9, 383.4),
+         (128, 8, (0, 20), [280] * 112, 46.1, 44.1), (128, 8, (6, 70), [340] * 118, 47.2, 39.3), (64, 32, (2350, 9), [1530] * 160, 371.6, 360.4),
+         (128, 8, (1880, 900), [2100] * 100, 226.1, 194.6), (64, 32, (570, 6), [580] * 76, 84.5, 78.0), (128, 8, (7860, 9), [460] * 14, 185.2, 168.4)]
+
+
+@pytest.mark.parametrize("head_dim,items,portion,singles,two,one", MIXES)
+def test_single_tokens_join_a_portion_where_that_is_faster(head_dim, items, portion, singles, two, one):
+    segments = [Segment([0] * n, pos, [list(range((pos + n + 15) // 16))], i) for i, (pos, n) in enumerate([portion] + [(p, 1) for p in singles])]
+    ctx = StepContext(segments, 1, SimpleNamespace(device=torch.device("cpu"), page_size=16))
+    plan = plan_tiles(ctx, 4, 8, True, items=items, head_dim=head_dim)
+    assert (plan.decode_count == 0) == (one < two) and plan.decode_count in (0, len(singles))
