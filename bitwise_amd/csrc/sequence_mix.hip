@@ -1036,7 +1036,7 @@ __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __rest
 //   heads of 64            3.8 -> 4.4    4.4 -> 4.5    5.2 -> 5.1    5.5 -> 5.0    6.3 -> 5.6    10.8 -> 8.3
 //   heads of 128           4.9 -> 5.2    5.4 -> 5.3    7.0 -> 6.2    7.5 -> 6.4    9.1 -> 8.1    19.7 -> 13.1
 //   heads of 256           6.5 -> 7.0    8.1 -> 7.9    13.2 -> 10.0  14.7 -> 10.7  18.0 -> 13.2  33.4 -> 18.5
-// so from 10,240 on.  Inside a Kuponex prompt of 2,048 tokens, 32,768 items of 128: 16.6 -> 13.3.
+// so from 10,240 on.  Inside a Kuponex prompt of 2,048 tokens, 32,768 items of 128: 15.7 to 16.6 -> 12.3 to 13.4.
 #define HG_ITEMS 4
 #define HG_MIN_ITEMS 10240
 template <typename OT, int EV>

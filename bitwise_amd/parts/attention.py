@@ -31,7 +31,7 @@ DECODE_MIN_CONTEXT = 128
 # what the chip does at once, where the decode kernel does a walk of ten partitions in up to 0.8 of the fold kernel's time; what joining saves is the
 # portion's own time, some 6 us and one a partition.  Two launches -> one, us: 1,341 tokens at 640 and 7 singles of up to 592 keys (32 heads of
 # 64) 50.6 -> 39.9; 854 tokens and 60 of up to 1,186 (32 heads of 128 on 8) 74.5 -> 53.3; a portion of 2 to 16 rows behind 8,000 keys and 14 of up to
-# 2,048 185 -> 168, 5,000 keys and 177 of up to 5,500 713 -> 610; a short portion and 230 of 400 to 500 keys (32 heads of 128) 242 -> 290, so two.
+# 2,048 185 -> 168, 5,000 keys and 177 of up to 5,500 713 -> 610; a short portion and 230 of 230 to 470 keys (32 heads of 128) 242 -> 290, so two.
 # 961 drawn mixes of 1 to 4 portions of 2 to 1,900 rows at 0 to 8,000 with 1 to 256 singles: 0.49 to 1.03 of two launches' time by this
 # rule (1.20 by the walks' lengths alone), 1.001 (heads of 64) and 1.002 (128) of the better choice's in the mean.
 JOIN_PARTITIONS = 8

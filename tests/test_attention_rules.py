@@ -71,10 +71,10 @@ def test_layers_whose_windows_change_nothing_share_a_plan(rows, join, same):
 
 
 # head size, key heads, (position, rows) of the longest portion, single tokens' positions (the mean of those measured), microseconds in two launches, in one
-MIXES = [(128, 32, (188, 2), [480] * 230, 241.8, 289.9), (128, 32, (0, 5), [310] * 141, 128.6, 151.2), (128, 8, (0, 40), [540] * 202, 89.8, 94.8),
-         (64, 32, (190, 2), [650] * 254, 231.4, 253.0), (64, 32, (500, 10), [550] * 216, 180.2, 192.4), (128, 32, (890, 6), [730] * 176, 357.9, 383.4),
-         (128, 8, (0, 20), [280] * 112, 46.1, 44.1), (128, 8, (6, 70), [340] * 118, 47.2, 39.3), (64, 32, (2350, 9), [1530] * 160, 371.6, 360.4),
-         (128, 8, (1880, 900), [2100] * 100, 226.1, 194.6), (64, 32, (570, 6), [580] * 76, 84.5, 78.0), (128, 8, (7860, 9), [460] * 14, 185.2, 168.4)]
+MIXES = [(128, 32, (180, 5), [360] * 230, 241.8, 289.9), (128, 32, (0, 5), [286] * 141, 128.6, 151.2), (128, 8, (0, 40), [499] * 202, 89.8, 94.8),
+         (64, 32, (180, 20), [617] * 254, 231.4, 253.0), (64, 32, (490, 10), [526] * 216, 180.2, 192.4), (128, 32, (880, 6), [698] * 176, 357.9, 383.4),
+         (128, 8, (0, 10), [303] * 136, 46.1, 44.1), (128, 8, (0, 190), [342] * 108, 47.2, 39.3), (64, 32, (2340, 9), [1501] * 160, 371.6, 360.4),
+         (128, 8, (300, 1540), [2080] * 100, 226.1, 194.6), (64, 32, (0, 560), [544] * 76, 84.5, 78.0), (128, 8, (7850, 9), [430] * 14, 185.2, 168.4)]
 
 
 @pytest.mark.parametrize("head_dim,items,portion,singles,two,one", MIXES)
