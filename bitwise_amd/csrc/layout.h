@@ -191,7 +191,7 @@ BW_HD constexpr int norm_strips_half(int half) { return half * 1024; }
 //   stores   128256 x 4096 202 -> 194 (7)   20000 x 1024 14.6 -> 11.2 with 5 (10.9 with 7)
 // Where both make whole rounds the variant is as fast or faster (8192 x 2048 17.7, 17.9 with 8; stores of K = 2048: 49152 columns 44.4
 // and 46.1 with 7, 32000 29.7 and 30.7 with 8), so it stays unless the count says 4 % less, 10 % for stores of one segment, 6 % for those of
-// two (47936 x 2176 stays at 42.8, 42.2 with 6).  66 products drawn over all of that: 0.71 to 1.02 of the variant's time.
+// two (47936 x 2176 stays at 42.8, 42.2 with 6).  385 products drawn over all of that: 0.62 to 1.03 of the variant's time (two above 1.01), 0.88 in the mean.
 inline int norm_strips_admits(int M, int N, int K, int epilogue) {
   const bool glu = epilogue == EPI_SWIGLU_BF16;
   if ((!glu && epilogue != EPI_F32) || !mid_norm_admits(M, K, (N + (glu ? 31 : 63)) / (glu ? 32 : 64))) return 0;
@@ -205,7 +205,10 @@ inline int norm_strips_admits(int M, int N, int K, int epilogue) {
   long long least = variant * (glu ? 96 : K <= GEMM_SEG ? 90 : 94) / 100;
   int best = 0;
   for (int strips = 5; strips <= 8; ++strips) {
-    const long long c = strips == 8 ? cost(strips) * 103 / 100 : cost(strips);     // (a ring of five stages)
+    // eight: a ring of five stages; seven in more than one round: where the count is even with six those are faster (21000 x 2944 46.8 and
+    // 50.1, variant 47.3; stores of 42000 x 2944 49.0 and 52.3, 51.3)
+    const bool rounds = (N + strips * norm_strips_cols(glu) - 1) / (strips * norm_strips_cols(glu)) > 256;
+    const long long c = strips == 8 ? cost(strips) * 103 / 100 : strips == 7 && rounds ? cost(strips) * 1005 / 1000 : cost(strips);
     if (c < least) {
       least = c;
       best = strips;
